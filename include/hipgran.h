@@ -372,7 +372,7 @@ hg_status hg_pool_set_wide_threshold(hg_pool *pool, size_t wide_min);
  * the interval's wide steps, then the chunk kernel, each on the whole GPU.
  * 0 <= wide_cus < CU count. */
 hg_status hg_pool_set_wide_cus(hg_pool *pool, int wide_cus);
-/* The wide launches of one interval (2 per step + 1) are recorded once into a
+/* The wide launches of one interval (one per step + 1) are recorded once into a
  * HIP graph per (interval length, dt, wide set) and replayed; enable = 0
  * launches them one by one instead. Default on. */
 hg_status hg_pool_set_wide_graph(hg_pool *pool, int enable);
@@ -476,8 +476,9 @@ hg_status hg_server_get_stats(hg_server *srv, hg_server_stats *out);
  * which only times whole runs with std::chrono, main.cpp:146-164).
  * hg_profile_enable(sys, 1) resets and starts; 0 stops. hg_profile_read
  * synchronises the stream and returns, per phase, the launch count and the
- * summed device milliseconds: [0] acceleration pass, [1] kick/drift and
- * final kick, [2] neighbour rebuild (all of its kernels), [3] reserved. */
+ * summed device milliseconds: [0] acceleration pass (with the kick and drift
+ * that the same launch does), [1] kick/drift and final kick in launches of
+ * their own, [2] neighbour rebuild (all of its kernels), [3] reserved. */
 hg_status hg_profile_enable(hg_system *sys, int enable);
 hg_status hg_profile_read(hg_system *sys, uint64_t *launches, double *device_ms);
 /* Small FP64 systems (up to 256 particles) step through one launch per

@@ -3,11 +3,12 @@
 // Kept in FP64: positions and the centre distance |x_i - x_j| with everything
 // derived from it by subtraction (contact overlap, Hamaker gap h, cutoff
 // test), the facet closest point, and the spring vectors: their rotation into
-// the contact plane, rescaling and the accumulation xi += v dt. In FP32 with
-// a*b+c contraction allowed: the normal, relative velocities, normal force,
-// Coulomb test and cap, torques and the Hamaker scalar. Dot and cross
-// products and a*x+y vector updates, FP64 and FP32, are explicit fused
-// multiply-adds (one rounding where the FP64 path has two). The gap h must stay
+// the contact plane, rescaling and the accumulation xi += v dt. In FP32: the
+// normal, relative velocities, normal force, Coulomb test and cap, torques and
+// the Hamaker scalar. Every fused multiply-add is written out, FP64 and FP32
+// (one rounding where the FP64 path has two), and nothing is left to the
+// compiler's contraction, which fuses by basic block and so rounds the same
+// expression differently in different kernels. The gap h must stay
 // FP64: h = |d| - 2r near h0 = 0.1 nm loses eps_32 * 2r/h0 ~ 1.7e-5 of
 // relative precision in FP32. Accelerations are summed in FP32 per particle.
 //
@@ -68,9 +69,8 @@ HGD f3 fmamf(float s, f3 a, f3 b) {
 // 1e-8 of itself). FP32: v_rsq_f32 / v_rcp_f32 (1 ulp). Arguments must be
 // > 0.
 __device__ __forceinline__ double rsqrt64(double a) {
-#pragma clang fp contract(fast)
     const double y = __builtin_amdgcn_rsq(a);
-    return y * (1.5 - 0.5 * a * y * y);
+    return y * __builtin_fma(-(0.5 * a * y), y, 1.5);
 }
 __device__ __forceinline__ float rsqrt32(float a) { return __builtin_amdgcn_rsqf(a); }
 __device__ __forceinline__ float rcp32(float a) { return __builtin_amdgcn_rcpf(a); }
@@ -160,7 +160,6 @@ inline mixed_consts make_mixed_consts(const hg_params &p) {
 // The rescale |xi| / |xr| is x2 / sqrt(x2 l2): one reciprocal square root
 // (x2 l2 stays a normal number for springs longer than 1e-77 m).
 __device__ __forceinline__ d3 rotate_spring(d3 xi, d3 n) {
-#pragma clang fp contract(fast)
     d3 xr = fmam(-dotm(xi, n), n, xi);
     const double l2 = dotm(xr, xr);
     if (l2 > 0.0) {
@@ -176,7 +175,6 @@ __device__ __forceinline__ d3 rotate_spring(d3 xi, d3 n) {
 // test force) set the direction that the next step's projection keeps.
 __device__ __forceinline__ f3 shear_contact_mx(d3 &xi, d3 n64, float k, float g, float fn, float mus, float mud,
                                                f3 rv, d3 rv64, double dt) {
-#pragma clang fp contract(fast)
     xi = rotate_spring(xi, n64);
     const f3 f0 = fmamf(-k, tof(xi), (-g) * rv);
     const float sf = mus * fn, df = mud * fn;
@@ -201,7 +199,6 @@ __device__ __forceinline__ f3 shear_contact_mx(d3 &xi, d3 n64, float k, float g,
 
 // alt_sinter_bridge.h:137-156 with FP32 forces and an FP64 spring.
 __device__ __forceinline__ f3 shear_sinter_mx(d3 &xi, d3 n64, float k, float g, f3 rv, d3 rv64, double dt) {
-#pragma clang fp contract(fast)
     xi = rotate_spring(xi, n64);
     const f3 f0 = fmamf(-k, tof(xi), (-g) * rv);
     xi = fmam(dt, rv64, xi);
@@ -210,7 +207,6 @@ __device__ __forceinline__ f3 shear_sinter_mx(d3 &xi, d3 n64, float k, float g, 
 
 // Shared kinematics of contact and bonded pairs: n from the FP64 distance.
 __device__ __forceinline__ void pair_kinematics_mx(d3 xi, d3 xj, double &dist, d3 &n64, f3 &n) {
-#pragma clang fp contract(fast)
     const d3 d = xi - xj;
     const double d2 = dotm(d, d);
     // coincident particles (d2 == 0) get a zero normal, as normalized() of a
@@ -233,7 +229,6 @@ __device__ __forceinline__ void pair_kinematics_mx(d3 xi, d3 xj, double &dist, d
 template <bool BONDED, class VW>
 __device__ __forceinline__ accf bonded_or_contact_mx(const mixed_consts &m, double dist, d3 n64, f3 n, d3 vi, d3 wi,
                                                      VW &&vw, spring9 &sp, bool &active) {
-#pragma clang fp contract(fast)
     const double ovd = (BONDED ? m.s_r2 : m.c_r2) - dist;
     if (!BONDED && ovd <= 0.0) {
         active = false;
@@ -249,7 +244,7 @@ __device__ __forceinline__ accf bonded_or_contact_mx(const mixed_consts &m, doub
     const float r = float(rd), rpp = float(rppd);
     const d3 dv = vi - vj, dw = wi - wj, sw = wi + wj;
     const float v_n = float(-dotm(dv, n64));
-    const float f_n = (BONDED ? m.s_k : m.c_k) * ov + (BONDED ? m.s_gn : m.c_gn) * v_n;
+    const float f_n = __builtin_fmaf(BONDED ? m.s_k : m.c_k, ov, (BONDED ? m.s_gn : m.c_gn) * v_n);
     const d3 v_ij = fmam(rppd, crossm(n64, sw), dv);
     const d3 vt64 = fmam(-dotm(v_ij, n64), n64, v_ij);
     const d3 vr64 = (-rppd) * crossm(n64, dw);
@@ -273,7 +268,6 @@ __device__ __forceinline__ accf bonded_or_contact_mx(const mixed_consts &m, doub
 // direction is normalized(x_j - x_i) = -n.
 template <int HAM>
 __device__ __forceinline__ f3 hamaker_at_mx(const mixed_consts &m, float h, f3 n) {
-#pragma clang fp contract(fast)
     const float rp = m.h_r;
     if constexpr (HAM == HG_HAMAKER_SIMPLIFIED) {
         // simplified_hamaker_force.h:26: 2 A r / h^2 along x_j - x_i = -n
@@ -281,16 +275,17 @@ __device__ __forceinline__ f3 hamaker_at_mx(const mixed_consts &m, float h, f3 n
         return (-(m.h_2ar * ih * ih) * m.h_im) * n;
     }
     const float a = 4.0f * rp + h, b = 2.0f * rp + h;
-    const float ia = rcp32(a), ib = rcp32(b), ih = rcp32(h);
-    const float s = m.h_a6 * ((a + h) * ia * ih - 2.0f * ib - 4.0f * rp * rp * ib * ib * ib -
-                              2.0f * rp * rp * (a + h) * ia * ia * ih * ih);
+    const float ia = rcp32(a), ib = rcp32(b), ih = rcp32(h), q = a + h;
+    float t = __builtin_fmaf(ih, q * ia, -2.0f * ib);
+    t = __builtin_fmaf(-ib, 4.0f * rp * rp * ib * ib, t);
+    t = __builtin_fmaf(-ih, 2.0f * rp * rp * q * ia * ia * ih, t);
+    const float s = m.h_a6 * t;
     return (-s * m.h_im) * n;
 }
 
 // Hamaker (full, limited range or simplified) with an FP64 gap.
 template <int HAM>
 __device__ __forceinline__ f3 hamaker_mx(const mixed_consts &m, double dist, f3 n) {
-#pragma clang fp contract(fast)
     if (HAM == HG_HAMAKER_LIMITED && dist > m.h_cut) return zerof();
     double hd = dist - m.h_r2;
     if (hd < m.h_h0) hd = m.h_h0;
@@ -303,24 +298,21 @@ __device__ __forceinline__ f3 hamaker_mx(const mixed_consts &m, double dist, f3 
 // itself, below what the FP32 force arithmetic resolves anyway.
 template <int HAM>
 __device__ __forceinline__ f3 hamaker_far_mx(const mixed_consts &m, d3 d, double d2) {
-#pragma clang fp contract(fast)
     if (HAM == HG_HAMAKER_LIMITED && d2 > m.h_cut2) return zerof();
     const float q = float(d2);
     const float inv = rsqrt32(q);
     const f3 n = tof(d) * inv;
-    return hamaker_at_mx<HAM>(m, q * inv - m.h_r2f, n);
+    return hamaker_at_mx<HAM>(m, __builtin_fmaf(q, inv, -m.h_r2f), n);
 }
 
 __device__ __forceinline__ accf surface_contact_mx(const mixed_consts &m, d3 xf, d3 vf_, d3 xi, d3 vi_, d3 w64,
                                                    spring9 &sp) {
-#pragma clang fp contract(fast)
     const d3 d = xi - xf;
     const double d2 = dot(d, d);
     // a centre on its facet point (d2 == 0) gets a zero normal, as normalized()
     // of a zero vector gives in the reference (Eigen) and in the FP64 path
     const double inv = d2 > 0.0 ? rsqrt64(d2) : 0.0;
-    const double dist = d2 * inv;
-    const double ovd = m.sc_rd - dist;
+    const double ovd = __builtin_fma(-d2, inv, m.sc_rd);
     if (ovd <= 0.0) {
         sp = zero_spring();
         return {zerof(), zerof()};
@@ -332,7 +324,7 @@ __device__ __forceinline__ accf surface_contact_mx(const mixed_consts &m, d3 xf,
     const float rpp = float(rppd);
     const d3 dv = vi_ - vf_;
     const float v_n = float(-dot(dv, n64));
-    const float f_n = m.sc_k * ov + m.sc_gn * v_n;
+    const float f_n = __builtin_fmaf(m.sc_k, ov, m.sc_gn * v_n);
     const d3 v_ij = dv + rppd * cross(n64, w64);
     const d3 vt64 = v_ij - dot(v_ij, n64) * n64;
     const d3 vr64 = (-rppd) * cross(n64, w64);
@@ -346,14 +338,12 @@ __device__ __forceinline__ accf surface_contact_mx(const mixed_consts &m, d3 xf,
 }
 
 __device__ __forceinline__ f3 surface_hamaker_mx(const mixed_consts &m, d3 xf, d3 xi) {
-#pragma clang fp contract(fast)
     const d3 r = xf - xi;
     const double d2 = dot(r, r);
     // a centre on its facet point (d2 == 0) gets a zero normal, as normalized()
     // of a zero vector gives in the reference (Eigen) and in the FP64 path
     const double inv = d2 > 0.0 ? rsqrt64(d2) : 0.0;
-    const double dist = d2 * inv;
-    double hd = dist - m.sh_r;
+    double hd = __builtin_fma(d2, inv, -m.sh_r);
     if (hd < m.sh_h0) hd = m.sh_h0;
     const float h = float(hd), rp = float(m.sh_r);
     const float q = h + 2.0f * rp;

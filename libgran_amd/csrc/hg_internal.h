@@ -142,6 +142,14 @@ struct hg_system_impl {
     double *red = nullptr;
     double *energy = nullptr;  // per-particle ledger terms, 8 per particle (allocated on first use)
     double *tiny = nullptr;    // per-pair springs of the pair-parallel pass (n*n*kSpringRec, on first use)
+    // per-step launches (tile_step.h), on first use: the second x, v, omega
+    // and facets, the system's meta and its tiles
+    double *tile_state = nullptr;
+    facet_dev *tile_facets = nullptr;
+    void *tile_meta = nullptr, *tile_map = nullptr;
+    unsigned tile_blocks = 0;
+    int tile_cur = -1;  // the table half `tile_map` names
+    int tile_nf = -1;   // the facet count `tile_meta` holds
     // host copies of the topology
     std::vector<std::pair<uint32_t, uint32_t>> bonds;
     size_t bonds_skipped = 0;
@@ -176,6 +184,8 @@ hg_status fail(hg_status st, const std::string &msg);
     } while (0)
 
 // kernel launchers (kernels.hip)
+// The per-particle walk: the legacy functor, and the contact and alt_sinter
+// functors with dissipation tracking (sv.diss).
 hipError_t launch_force(const hg_params &p, const sys_view &sv, hipStream_t s);
 hipError_t launch_kick_drift(double *x, double *v, double *th, double *w, const double *a, const double *al,
                              uint32_t n, bool pending, double half_prev, double half, double dt, facet_dev *facets,

@@ -59,28 +59,6 @@ __global__ void __launch_bounds__(256) k_force_nl(hg_params P, sys_view S) {
     force_nl_one<BIN, HAM, TRACK>(P, S, i);
 }
 
-// Mixed-precision neighbour-list pass (HG_PRECISION_MIXED, dem_mixed.h).
-template <int BIN, int HAM>
-__global__ void __launch_bounds__(256) k_force_nl_mx(hg_params P, mixed_consts MC, sys_view S) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= S.n) return;
-    const d3 xi = ld3(S.x, i), vi = ld3(S.v, i), wi = ld3(S.w, i);
-    accf acc{zerof(), zerof()};
-    walker_t<true> W;
-    if constexpr (BIN != HG_BINARY_NONE) W.init(S.pt, i);
-    id_list ids;
-    ids.init(S.nb, S.ncnt, S.n, i, S.cap_n);
-    nl_partners(ids, [&](uint32_t j) { return pstate{ld3(S.x, j), ld3(S.v, j), ld3(S.w, j)}; },
-                [&](uint32_t j, const pstate &sj) {
-                    pair_fold_mx<BIN, HAM>(MC, j, xi, vi, wi, sj.x, [&](d3 &v, d3 &w) { v = sj.v, w = sj.w; }, W,
-                                           acc);
-                });
-    close_table<BIN>(W, S.pt.pcnt_new, i, S.flags);
-    if (S.nf > 0) acc = acc + facet_fold_mx(P, MC, S.facets, S.nf, S.ss, S.n, i, xi, vi, wi);
-    st3(S.a, i, tod(acc.lin));
-    st3(S.al, i, tod(acc.ang));
-}
-
 // All-pairs acceleration pass (granular_system): every j != i in ascending
 // order. Partner state is staged through LDS one tile per block-wide step;
 // all lanes read the same LDS word, a broadcast with no bank conflict.
@@ -572,52 +550,36 @@ __global__ void __launch_bounds__(256) k_energy(hg_params P, energy_view E, doub
 
 inline unsigned blocks_for(size_t n, unsigned bs) { return unsigned((n + bs - 1) / bs); }
 
-template <int BIN, int HAM>
+template <int BIN, int HAM, bool TRACK>
 hipError_t launch_force_t(const hg_params &p, const sys_view &sv, hipStream_t s) {
     if (sv.n == 0) return hipSuccess;
-    if (p.pair_mode == HG_PAIRS_NEIGHBOR_LIST && p.precision == HG_PRECISION_MIXED) {
-        if constexpr (BIN == HG_BINARY_SINTER_LEGACY) return hipErrorInvalidValue;  // FP64 only
-        else k_force_nl_mx<BIN, HAM><<<blocks_for(sv.n, 64), 64, 0, s>>>(p, make_mixed_consts(p), sv);
-    } else if (sv.diss) {
-        // dissipation tracking (FP64 contact and alt_sinter bonds only)
-        if constexpr (BIN == HG_BINARY_CONTACT || BIN == HG_BINARY_SINTER) {
-            if (p.pair_mode == HG_PAIRS_NEIGHBOR_LIST)
-                k_force_nl<BIN, HAM, true><<<blocks_for(sv.n, 64), 64, 0, s>>>(p, sv);
-            else
-                k_force_all<BIN, HAM, true><<<blocks_for(sv.n, kTile), kTile, 0, s>>>(p, sv);
-        } else {
-            return hipErrorInvalidValue;
-        }
-    } else if (p.pair_mode == HG_PAIRS_NEIGHBOR_LIST) {
-        // 64-lane blocks spread a modest particle count over more CUs.
-        k_force_nl<BIN, HAM, false><<<blocks_for(sv.n, 64), 64, 0, s>>>(p, sv);
-    } else {
-        k_force_all<BIN, HAM, false><<<blocks_for(sv.n, kTile), kTile, 0, s>>>(p, sv);
-    }
+    // 64-lane blocks spread a modest particle count over more CUs.
+    if (p.pair_mode == HG_PAIRS_NEIGHBOR_LIST)
+        k_force_nl<BIN, HAM, TRACK><<<blocks_for(sv.n, 64), 64, 0, s>>>(p, sv);
+    else
+        k_force_all<BIN, HAM, TRACK><<<blocks_for(sv.n, kTile), kTile, 0, s>>>(p, sv);
     return hipGetLastError();
 }
 
 }  // namespace
 
 hipError_t launch_force(const hg_params &p, const sys_view &sv, hipStream_t s) {
-#define HG_CASE(B, H)                                                       \
-    if (p.binary_model == B && p.hamaker_model == H) return launch_force_t<B, H>(p, sv, s);
-    HG_CASE(HG_BINARY_NONE, HG_HAMAKER_NONE)
-    HG_CASE(HG_BINARY_NONE, HG_HAMAKER_FULL)
-    HG_CASE(HG_BINARY_NONE, HG_HAMAKER_LIMITED)
-    HG_CASE(HG_BINARY_NONE, HG_HAMAKER_SIMPLIFIED)
-    HG_CASE(HG_BINARY_CONTACT, HG_HAMAKER_NONE)
-    HG_CASE(HG_BINARY_CONTACT, HG_HAMAKER_FULL)
-    HG_CASE(HG_BINARY_CONTACT, HG_HAMAKER_LIMITED)
-    HG_CASE(HG_BINARY_CONTACT, HG_HAMAKER_SIMPLIFIED)
-    HG_CASE(HG_BINARY_SINTER, HG_HAMAKER_NONE)
-    HG_CASE(HG_BINARY_SINTER, HG_HAMAKER_FULL)
-    HG_CASE(HG_BINARY_SINTER, HG_HAMAKER_LIMITED)
-    HG_CASE(HG_BINARY_SINTER, HG_HAMAKER_SIMPLIFIED)
-    HG_CASE(HG_BINARY_SINTER_LEGACY, HG_HAMAKER_NONE)
-    HG_CASE(HG_BINARY_SINTER_LEGACY, HG_HAMAKER_FULL)
-    HG_CASE(HG_BINARY_SINTER_LEGACY, HG_HAMAKER_LIMITED)
-    HG_CASE(HG_BINARY_SINTER_LEGACY, HG_HAMAKER_SIMPLIFIED)
+#define HG_CASE(B, H, TRACK)                                                                        \
+    if (p.binary_model == B && p.hamaker_model == H && p.precision == HG_PRECISION_FP64 &&          \
+        (sv.diss != nullptr) == TRACK)                                                              \
+        return launch_force_t<B, H, TRACK>(p, sv, s);
+    HG_CASE(HG_BINARY_CONTACT, HG_HAMAKER_NONE, true)
+    HG_CASE(HG_BINARY_CONTACT, HG_HAMAKER_FULL, true)
+    HG_CASE(HG_BINARY_CONTACT, HG_HAMAKER_LIMITED, true)
+    HG_CASE(HG_BINARY_CONTACT, HG_HAMAKER_SIMPLIFIED, true)
+    HG_CASE(HG_BINARY_SINTER, HG_HAMAKER_NONE, true)
+    HG_CASE(HG_BINARY_SINTER, HG_HAMAKER_FULL, true)
+    HG_CASE(HG_BINARY_SINTER, HG_HAMAKER_LIMITED, true)
+    HG_CASE(HG_BINARY_SINTER, HG_HAMAKER_SIMPLIFIED, true)
+    HG_CASE(HG_BINARY_SINTER_LEGACY, HG_HAMAKER_NONE, false)
+    HG_CASE(HG_BINARY_SINTER_LEGACY, HG_HAMAKER_FULL, false)
+    HG_CASE(HG_BINARY_SINTER_LEGACY, HG_HAMAKER_LIMITED, false)
+    HG_CASE(HG_BINARY_SINTER_LEGACY, HG_HAMAKER_SIMPLIFIED, false)
 #undef HG_CASE
     return hipErrorInvalidValue;
 }

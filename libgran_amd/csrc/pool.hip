@@ -27,10 +27,9 @@
 #include <string>
 #include <vector>
 
-#include "force_device.h"
-#include "hg_internal.h"
 #include "pool_internal.h"
 #include "snapshot.h"
+#include "tile_step.h"
 
 // Device scratch of hg_pool_energy_noalloc, the entry point that allocates
 // nothing: the per-particle ledger terms of one system (8 doubles per
@@ -44,666 +43,7 @@ static __device__ __align__(256) double scratch[8 * kNoAllocParticles + 8];
 
 namespace hg {
 
-// slot: the system's own index, naming its fault word in pool_view::sflags.
-struct pool_meta {
-    uint32_t offset, n, cur, acc_valid, nf, rebuild, slot, pad1;
-};
-
-struct pool_view {
-    double *x, *v, *th, *w, *a, *al;
-    const uint32_t *nb;
-    const uint32_t *ncnt;
-    uint32_t *pj0, *pj1, *pcnt0, *pcnt1;
-    double *ps0, *ps1;
-    uint32_t cap_s, cap_n;
-    const uint32_t *bj;  // neck-strength lists (see pair_table), null unless bonds break
-    const double *bstr;
-    const uint32_t *bcnt;
-    facet_dev *facets;
-    uint32_t max_facets;
-    double *ss;
-    const pool_meta *meta;
-    size_t stride;
-    int *flags;
-    int *sflags;  // per-system fault words (HG_FAULT_* bits), indexed by slot
-};
-
 namespace {
-
-// Where a running system's particle state lives during a chunk (chosen per
-// system from its size and the workgroup's LDS; local index g - offset):
-//   STATE_FULL   all of x, v, omega, theta, a, alpha in LDS (18 doubles per
-//                particle), read from global memory at the start of the
-//                chunk and written back once at its end;
-//   STATE_MIRROR x, v, omega copied into LDS (9 doubles per particle) and
-//                refreshed by each owner lane in the kick/drift phase, so
-//                partner gathers read LDS; the state itself stays global;
-//   STATE_POS    x alone copied into LDS (3 doubles per particle) and
-//                refreshed likewise: every partner needs its position, only
-//                the bonded and overlapping ones (a few of a 3.2r list) its
-//                velocities, which then come from global memory;
-//   STATE_GLOBAL everything in global memory.
-enum { STATE_GLOBAL = 0, STATE_MIRROR = 1, STATE_FULL = 2, STATE_POS = 3 };
-#ifndef HG_CHUNK_EAGER
-#define HG_CHUNK_EAGER 1
-#endif
-#ifndef HG_CHUNK_PREFETCH
-#define HG_CHUNK_PREFETCH 1
-#endif
-#ifndef HG_CHUNK_MIN_BLOCKS
-#define HG_CHUNK_MIN_BLOCKS 1
-#endif
-constexpr bool kChunkEager = HG_CHUNK_EAGER, kChunkPrefetch = HG_CHUNK_PREFETCH;
-extern __shared__ double pool_lds[];
-constexpr uint32_t kPosStride = 3, kMirrorStride = 9, kFullStride = 18;
-template <int MODE>
-constexpr uint32_t lds_stride() {
-    return MODE == STATE_FULL ? kFullStride : (MODE == STATE_MIRROR ? kMirrorStride : kPosStride);
-}
-
-template <int MODE>
-__device__ __forceinline__ double *lds_rec(uint32_t offset, uint32_t g) {
-    return pool_lds + size_t(g - offset) * lds_stride<MODE>();
-}
-__device__ __forceinline__ d3 lds3(const double *q) { return d3{q[0], q[1], q[2]}; }
-__device__ __forceinline__ void sds3(double *q, d3 a) {
-    q[0] = a.x;
-    q[1] = a.y;
-    q[2] = a.z;
-}
-
-template <int MODE>
-__device__ __forceinline__ d3 load_x(const pool_view &V, uint32_t offset, uint32_t g) {
-    if constexpr (MODE == STATE_GLOBAL) return ld3(V.x, g);
-    else return lds3(lds_rec<MODE>(offset, g));
-}
-template <int MODE>
-__device__ __forceinline__ void load_vw(const pool_view &V, uint32_t offset, uint32_t g, d3 &v, d3 &w) {
-    if constexpr (MODE == STATE_GLOBAL || MODE == STATE_POS) {
-        v = ld3(V.v, g);
-        w = ld3(V.w, g);
-    } else {
-        const double *q = lds_rec<MODE>(offset, g);
-        v = lds3(q + 3);
-        w = lds3(q + 6);
-    }
-}
-
-template <int MODE>
-__device__ __forceinline__ void load_state(const pool_view &V, uint32_t offset, uint32_t g, d3 &x, d3 &v, d3 &w) {
-    if constexpr (MODE == STATE_GLOBAL) {
-        x = ld3(V.x, g);
-        v = ld3(V.v, g);
-        w = ld3(V.w, g);
-    } else if constexpr (MODE == STATE_POS) {
-        x = lds3(lds_rec<MODE>(offset, g));
-        v = ld3(V.v, g);
-        w = ld3(V.w, g);
-    } else {
-        const double *q = lds_rec<MODE>(offset, g);
-        x = lds3(q);
-        v = lds3(q + 3);
-        w = lds3(q + 6);
-    }
-}
-
-template <int MODE>
-__device__ __forceinline__ void store_acc(const pool_view &V, uint32_t offset, uint32_t g, d3 a, d3 al) {
-    if constexpr (MODE == STATE_FULL) {
-        double *q = lds_rec<MODE>(offset, g);
-        sds3(q + 12, a);
-        sds3(q + 15, al);
-    } else {
-        st3(V.a, g, a);
-        st3(V.al, g, al);
-    }
-}
-
-// Fills the LDS records of a system at the start of its chunk.
-template <int MODE>
-__device__ __forceinline__ void lds_fill(const pool_view &V, const pool_meta &M) {
-    for (uint32_t g = M.offset + threadIdx.x; g < M.offset + M.n; g += blockDim.x) {
-        double *q = lds_rec<MODE>(M.offset, g);
-        sds3(q, ld3(V.x, g));
-        if constexpr (MODE == STATE_POS) continue;
-        sds3(q + 3, ld3(V.v, g));
-        sds3(q + 6, ld3(V.w, g));
-        if constexpr (MODE == STATE_FULL) {
-            sds3(q + 9, ld3(V.th, g));
-            sds3(q + 12, ld3(V.a, g));
-            sds3(q + 15, ld3(V.al, g));
-        }
-    }
-}
-
-// LDS copy of a neighbour-list system's partner ids for one rebuild interval:
-// kmax slots per particle (kmax = the system's longest list), slot k of local
-// particle t at lids[k*n + t] as a halfword offset from the system's first
-// particle, then the list counts at lids[kmax*n + t]. A system of at most
-// 65,535 particles fits the halfwords.
-__host__ __device__ inline size_t lds_ids_bytes(uint32_t n, uint32_t kmax) { return size_t(n) * 2 * (kmax + 1); }
-
-__device__ __forceinline__ void lds_ids_fill(const pool_view &V, const pool_meta &M, uint32_t kmax, uint16_t *lids) {
-    for (uint32_t t = threadIdx.x; t < M.n; t += blockDim.x) {
-        const uint32_t g = M.offset + t, c = V.ncnt[g];
-        lids[kmax * M.n + t] = uint16_t(c);
-        for (uint32_t k = 0; k < c; k++) lids[k * M.n + t] = uint16_t(V.nb[size_t(k) * V.stride + g] - M.offset);
-    }
-}
-
-// Largest value of v over the workgroup (s_red: one word per wavefront).
-__device__ __forceinline__ uint32_t block_max_u32(uint32_t v, uint32_t *s_red) {
-    for (int o = 32; o > 0; o >>= 1) v = max(v, uint32_t(__shfl_xor(int(v), o)));
-    if ((threadIdx.x & 63u) == 0) s_red[threadIdx.x >> 6] = v;
-    __syncthreads();
-    uint32_t r = 0;
-    for (uint32_t w = 0; w < (blockDim.x + 63u) / 64u; w++) r = max(r, s_red[w]);
-    __syncthreads();
-    return r;
-}
-
-// Acceleration pass for particles g = g_first, g_first + g_step, ... < g_end
-// of system M (a workgroup strides over the whole system; a wide launch gives
-// each thread one particle). With LIDS the partner ids come from the system's
-// LDS copy `lids` (lds_ids_fill). after(g, x, v, w, a, alpha) runs once a
-// particle's accelerations are stored, with its state and accelerations
-// still in registers.
-struct no_after {
-    __device__ void operator()(uint32_t, d3, d3, d3, d3, d3) const {}
-};
-// The FP64 pair path's bond constants held in vector registers for a pass
-// (as pinned() does for the mixed path): kept as scalars they are spilled and
-// re-read lane by lane inside the pair loop.
-__device__ __forceinline__ hg_params pinned64(const hg_params &P) {
-    hg_params p = P;
-    hg_sinter_params &s = p.sinter;
-    double *f[] = {&s.k, &s.gamma_n, &s.k_t, &s.gamma_t, &s.k_r, &s.gamma_r,
-                   &s.k_o, &s.gamma_o, &s.r_part, &s.mass, &s.inertia, &s.dt};
-#pragma unroll
-    for (double *q : f) pin_vgpr(*q);
-    return p;
-}
-template <int BIN, int HAM, int PAIRS, int PREC, int LDS, bool LIDS = false, bool FAC = true, class AFTER = no_after>
-__device__ __forceinline__ void pool_force_phase(const hg_params &P, const mixed_consts &MC, const pool_view &V,
-                                                 const pool_meta &M, uint32_t cur, const facet_dev *F,
-                                                 uint32_t g_first, uint32_t g_end, uint32_t g_step,
-                                                 const uint16_t *lids = nullptr, uint32_t kmax = 0,
-                                                 AFTER after = AFTER{}) {
-    pair_table T;
-    T.pj_old = cur ? V.pj1 : V.pj0;
-    T.ps_old = cur ? V.ps1 : V.ps0;
-    T.pcnt_old = cur ? V.pcnt1 : V.pcnt0;
-    T.pj_new = cur ? V.pj0 : V.pj1;
-    T.ps_new = cur ? V.ps0 : V.ps1;
-    T.pcnt_new = cur ? V.pcnt0 : V.pcnt1;
-    T.cap = V.cap_s;
-    T.stride = V.stride;
-    T.bj = V.bj;
-    T.bstr = V.bstr;
-    T.bcnt = V.bcnt;
-    const uint32_t end = M.offset + M.n;
-    for (uint32_t g = g_first; g < g_end; g += g_step) {
-        d3 xi, vi, wi;
-        load_state<LDS>(V, M.offset, g, xi, vi, wi);
-        walker_t<PREC == HG_PRECISION_MIXED && kChunkEager> W;
-        if constexpr (BIN != HG_BINARY_NONE) W.init(T, g);
-        id_list ids;
-        if constexpr (PAIRS == HG_PAIRS_NEIGHBOR_LIST && !LIDS) ids.init(V.nb, V.ncnt, V.stride, g, V.cap_n);
-        // listed partners of g through fold(j, xj, vw), in list order: vw
-        // gives a partner's velocities when its pair needs them, from LDS or
-        // from a global gather made a pair ahead with its position
-        auto partners = [&](auto &&fold) {
-            auto run = [&](const auto &ids_) {
-                if constexpr (LDS == STATE_GLOBAL) {
-                    nl_partners<kChunkPrefetch>(
-                        ids_, [&](uint32_t j) { return pstate{ld3(V.x, j), ld3(V.v, j), ld3(V.w, j)}; },
-                        [&](uint32_t j, const pstate &sj) {
-                            fold(j, sj.x, [&](d3 &v, d3 &w) { v = sj.v, w = sj.w; });
-                        });
-                } else {
-                    nl_partners<kChunkPrefetch>(
-                        ids_, [&](uint32_t j) { return load_x<LDS>(V, M.offset, j); },
-                        [&](uint32_t j, d3 xj) {
-                            fold(j, xj, [&](d3 &v, d3 &w) { load_vw<LDS>(V, M.offset, j, v, w); });
-                        });
-                }
-            };
-            if constexpr (LIDS) {
-                const uint32_t t = g - M.offset;
-                run(lds_id_list{lids, M.n, t, M.offset, lids[kmax * M.n + t]});
-            } else {
-                run(ids);
-            }
-        };
-        auto vw_of = [&](uint32_t j) { return [&V, &M, j](d3 &v, d3 &w) { load_vw<LDS>(V, M.offset, j, v, w); }; };
-        if constexpr (PREC == HG_PRECISION_FP64) {
-            acc6 acc{zero3(), zero3()};
-            const hg_params pp = pinned64(P);
-            if constexpr (PAIRS == HG_PAIRS_NEIGHBOR_LIST) {
-                partners([&](uint32_t j, d3 xj, auto &&vw) { pair_fold_vw<BIN, HAM>(pp, j, xi, vi, wi, xj, vw, W, acc); });
-            } else {
-                for (uint32_t j = M.offset; j < end; j++) {
-                    if (j == g) continue;
-                    pair_fold_vw<BIN, HAM>(P, j, xi, vi, wi, load_x<LDS>(V, M.offset, j), vw_of(j), W, acc);
-                }
-            }
-            close_table<BIN>(W, T.pcnt_new, g, V.flags, V.sflags + M.slot);
-            if (FAC && M.nf > 0) acc = acc + facet_fold(P, F, int(M.nf), V.ss, V.stride, g, xi, vi, wi);
-            store_acc<LDS>(V, M.offset, g, acc.lin, acc.ang);
-            after(g, xi, vi, wi, acc.lin, acc.ang);
-        } else {
-            accf acc{zerof(), zerof()};
-            const mixed_consts m = pinned(MC);
-            if constexpr (PAIRS == HG_PAIRS_NEIGHBOR_LIST) {
-                partners([&](uint32_t j, d3 xj, auto &&vw) { pair_fold_mx<BIN, HAM>(m, j, xi, vi, wi, xj, vw, W, acc); });
-            } else {
-                for (uint32_t j = M.offset; j < end; j++) {
-                    if (j == g) continue;
-                    pair_fold_mx<BIN, HAM>(MC, j, xi, vi, wi, load_x<LDS>(V, M.offset, j), vw_of(j), W, acc);
-                }
-            }
-            close_table<BIN>(W, T.pcnt_new, g, V.flags, V.sflags + M.slot);
-            if (FAC && M.nf > 0) acc = acc + facet_fold_mx(P, MC, F, int(M.nf), V.ss, V.stride, g, xi, vi, wi);
-            const d3 a64 = tod(acc.lin), al64 = tod(acc.ang);
-            store_acc<LDS>(V, M.offset, g, a64, al64);
-            after(g, xi, vi, wi, a64, al64);
-        }
-    }
-}
-
-// Kick (completing the previous step when `pending`), kick, drift; the same
-// operations in the same order as k_kick_drift.
-template <int LDS>
-__device__ __forceinline__ void pool_kick_drift(const pool_view &V, const pool_meta &M, bool pending, double half,
-                                                double dt, uint32_t g_first, uint32_t g_end, uint32_t g_step) {
-    for (uint32_t g = g_first; g < g_end; g += g_step) {
-        double *q = lds_rec<LDS>(M.offset, g);
-        d3 vi, wi, ai, ali, x0, th0;
-        if constexpr (LDS == STATE_FULL) {
-            vi = lds3(q + 3); wi = lds3(q + 6); ai = lds3(q + 12); ali = lds3(q + 15); x0 = lds3(q); th0 = lds3(q + 9);
-        } else {
-            vi = ld3(V.v, g); wi = ld3(V.w, g); ai = ld3(V.a, g); ali = ld3(V.al, g); x0 = ld3(V.x, g);
-            th0 = ld3(V.th, g);
-        }
-        if (pending) {
-            vi = vi + ai * half;
-            wi = wi + ali * half;
-        }
-        vi = vi + ai * half;
-        wi = wi + ali * half;
-        const d3 xi = x0 + vi * dt;
-        const d3 thi = th0 + wi * dt;
-        if constexpr (LDS != STATE_FULL) {
-            st3(V.x, g, xi);
-            st3(V.th, g, thi);
-            st3(V.v, g, vi);
-            st3(V.w, g, wi);
-        }
-        if constexpr (LDS != STATE_GLOBAL) sds3(q, xi);
-        if constexpr (LDS == STATE_MIRROR || LDS == STATE_FULL) {
-            sds3(q + 3, vi);
-            sds3(q + 6, wi);
-        }
-        if constexpr (LDS == STATE_FULL) sds3(q + 9, thi);
-    }
-}
-
-// Final kick; a system kept wholly in LDS is written back here. A non-finite
-// velocity or angular velocity faults the system (HG_FAULT_NUMERIC).
-template <int LDS>
-__device__ __forceinline__ void pool_final_kick(const pool_view &V, const pool_meta &M, double half,
-                                                uint32_t g_first, uint32_t g_end, uint32_t g_step) {
-    bool bad = false;
-    for (uint32_t g = g_first; g < g_end; g += g_step) {
-        d3 vi, wi;
-        if constexpr (LDS == STATE_FULL) {
-            const double *q = lds_rec<LDS>(M.offset, g);
-            const d3 a = lds3(q + 12), al = lds3(q + 15);
-            vi = lds3(q + 3) + a * half;
-            wi = lds3(q + 6) + al * half;
-            st3(V.x, g, lds3(q));
-            st3(V.th, g, lds3(q + 9));
-            st3(V.a, g, a);
-            st3(V.al, g, al);
-        } else {
-            vi = ld3(V.v, g) + ld3(V.a, g) * half;
-            wi = ld3(V.w, g) + ld3(V.al, g) * half;
-        }
-        st3(V.v, g, vi);
-        st3(V.w, g, wi);
-        bad |= nonfinite(vi, wi);
-    }
-    if (bad) {
-        atomicOr(&V.flags[FLAG_NUMERIC], 1);
-        atomicOr(&V.sflags[M.slot], HG_FAULT_NUMERIC);
-    }
-}
-
-// All steps of one rebuild interval for one system, by one workgroup. With
-// LIDS the system's partner ids (kmax slots per particle) are copied to LDS
-// after its state records.
-template <int BIN, int HAM, int PAIRS, int PREC, int LDS, bool LIDS, bool FAC>
-__device__ __forceinline__ void run_system(const hg_params &P, const mixed_consts &MC, const pool_view &V,
-                                           const pool_meta &M, facet_dev *F, uint32_t nsteps, double dt,
-                                           uint32_t kmax) {
-    const double half = dt / 2.0;
-    uint32_t cur = M.cur;
-    const uint32_t g0 = M.offset + threadIdx.x, g_end = M.offset + M.n, gs = blockDim.x;
-    if constexpr (LDS != STATE_GLOBAL) lds_fill<LDS>(V, M);
-    uint16_t *lids = nullptr;
-    if constexpr (LIDS) {
-        lids = reinterpret_cast<uint16_t *>(
-            pool_lds + (LDS == STATE_GLOBAL ? 0 : size_t(M.n) * lds_stride<LDS>()));
-        lds_ids_fill(V, M, kmax, lids);
-    }
-    if constexpr (LDS != STATE_GLOBAL || LIDS) __syncthreads();
-    // step -1 is the initial acceleration pass of a system without valid
-    // accelerations; one call site keeps a single copy of the pass in the code
-    for (int s = M.acc_valid ? 0 : -1; s < int(nsteps); s++) {
-        if (s >= 0) {
-            pool_kick_drift<LDS>(V, M, s > 0, half, dt, g0, g_end, gs);
-            if (s > 0 && threadIdx.x == 0) advance_facets(F, int(M.nf), dt);
-            __syncthreads();
-        }
-        pool_force_phase<BIN, HAM, PAIRS, PREC, LDS, LIDS, FAC>(P, MC, V, M, cur, F, g0, g_end, gs, lids, kmax);
-        cur ^= 1u;
-        __syncthreads();
-    }
-    if (nsteps > 0) {
-        pool_final_kick<LDS>(V, M, half, g0, g_end, gs);
-        if (threadIdx.x == 0) advance_facets(F, int(M.nf), dt);
-    } else if constexpr (LDS == STATE_FULL) {
-        // only the initial pass ran: its accelerations go back to global
-        for (uint32_t g = M.offset + threadIdx.x; g < M.offset + M.n; g += blockDim.x) {
-            const double *q = lds_rec<LDS>(M.offset, g);
-            st3(V.a, g, lds3(q + 12));
-            st3(V.al, g, lds3(q + 15));
-        }
-    }
-    __syncthreads();
-}
-
-// One system's interval by the whole workgroup, in the state tier its size
-// allows (s_red: block_max_u32's scratch words).
-template <int BIN, int HAM, int PAIRS, int PREC, bool FAC>
-__device__ __forceinline__ void run_one(const hg_params &P, const mixed_consts &MC, const pool_view &V,
-                                        uint32_t slot, uint32_t nsteps, double dt, uint32_t lds_bytes,
-                                        uint32_t *s_red) {
-    const pool_meta M = V.meta[slot];
-    facet_dev *F = V.facets + size_t(slot) * V.max_facets;
-    const size_t need = size_t(M.n) * sizeof(double);
-    if constexpr (PAIRS == HG_PAIRS_NEIGHBOR_LIST) {
-        // the partner ids go to LDS too wherever they fit beside the state
-        uint32_t kmax = 0;
-        for (uint32_t t = threadIdx.x; t < M.n; t += blockDim.x) kmax = max(kmax, V.ncnt[M.offset + t]);
-        kmax = block_max_u32(kmax, s_red);
-        const size_t ids = M.n <= 65535u ? lds_ids_bytes(M.n, kmax) : ~size_t(0) / 2;
-        if (need * kFullStride + ids <= lds_bytes)
-            run_system<BIN, HAM, PAIRS, PREC, STATE_FULL, true, FAC>(P, MC, V, M, F, nsteps, dt, kmax);
-        else if (need * kMirrorStride + ids <= lds_bytes)
-            run_system<BIN, HAM, PAIRS, PREC, STATE_MIRROR, true, FAC>(P, MC, V, M, F, nsteps, dt, kmax);
-        else if (need * kPosStride + ids <= lds_bytes)
-            run_system<BIN, HAM, PAIRS, PREC, STATE_POS, true, FAC>(P, MC, V, M, F, nsteps, dt, kmax);
-        else if (ids <= lds_bytes)
-            run_system<BIN, HAM, PAIRS, PREC, STATE_GLOBAL, true, FAC>(P, MC, V, M, F, nsteps, dt, kmax);
-        else
-            run_system<BIN, HAM, PAIRS, PREC, STATE_GLOBAL, false, FAC>(P, MC, V, M, F, nsteps, dt, 0);
-    } else {
-        if (need * kFullStride <= lds_bytes)
-            run_system<BIN, HAM, PAIRS, PREC, STATE_FULL, false, FAC>(P, MC, V, M, F, nsteps, dt, 0);
-        else if (need * kMirrorStride <= lds_bytes)
-            run_system<BIN, HAM, PAIRS, PREC, STATE_MIRROR, false, FAC>(P, MC, V, M, F, nsteps, dt, 0);
-        else
-            run_system<BIN, HAM, PAIRS, PREC, STATE_GLOBAL, false, FAC>(P, MC, V, M, F, nsteps, dt, 0);
-    }
-}
-
-// Several small systems (a pack: count members, all of them at most one
-// particle per thread together) stepped side by side by one workgroup, so
-// that a system of 100 particles does not leave 400 lanes idle through every
-// step. Neighbour-list mode, all state in LDS: member m's particles take pack
-// positions base_m .. base_m + n_m - 1 (thread = position). Each thread steps
-// its own particle with the single-system device code, given its member's
-// meta with offset_m - base_m in place of the offset: LDS records and partner
-// ids are addressed by (arena index - that offset) = pack position (unsigned
-// arithmetic), and the ids are stored as pack positions. Every operation of a
-// particle is that of run_system, so a system's result does not depend on
-// packing. Returns false, having done nothing, when the pack needs more
-// threads or LDS than the workgroup has; the caller then steps the members
-// one at a time.
-constexpr uint32_t kMaxPack = 8;
-template <int BIN, int HAM, int PREC, bool FAC>
-__device__ __forceinline__ bool run_pack(const hg_params &P, const mixed_consts &MC, const pool_view &V,
-                                         const uint32_t *slots, uint32_t cnt, uint32_t nsteps, double dt,
-                                         uint32_t lds_bytes, uint32_t *s_red, pool_meta *s_pm, uint32_t *s_base) {
-    if (threadIdx.x == 0) {
-        uint32_t base = 0;
-        for (uint32_t m = 0; m < cnt; m++) {
-            s_pm[m] = V.meta[slots[m]];
-            s_base[m] = base;
-            base += s_pm[m].n;
-        }
-        s_base[cnt] = base;
-    }
-    __syncthreads();
-    const uint32_t N = s_base[cnt], t = threadIdx.x;
-    uint32_t m = 0;
-    bool all_valid = true;
-    for (uint32_t k = 0; k < cnt; k++) {
-        if (k > 0 && t >= s_base[k]) m = k;
-        all_valid = all_valid && s_pm[k].acc_valid;
-    }
-    const bool own = t < N;
-    const pool_meta Pm = s_pm[m];
-    const uint32_t g = Pm.offset + (t - s_base[m]);
-    pool_meta Mv = Pm;
-    Mv.offset = Pm.offset - s_base[m];
-    Mv.n = N;
-    uint32_t kmax = own ? V.ncnt[g] : 0u;
-    kmax = block_max_u32(kmax, s_red);
-    if (N > blockDim.x || size_t(N) * sizeof(double) * kFullStride + lds_ids_bytes(N, kmax) > lds_bytes) return false;
-    facet_dev *F = V.facets + size_t(Pm.slot) * V.max_facets;
-    uint16_t *lids = reinterpret_cast<uint16_t *>(pool_lds + size_t(N) * kFullStride);
-    if (own) {
-        double *q = pool_lds + size_t(t) * kFullStride;
-        sds3(q, ld3(V.x, g));
-        sds3(q + 3, ld3(V.v, g));
-        sds3(q + 6, ld3(V.w, g));
-        sds3(q + 9, ld3(V.th, g));
-        sds3(q + 12, ld3(V.a, g));
-        sds3(q + 15, ld3(V.al, g));
-        const uint32_t c = V.ncnt[g];
-        lids[kmax * N + t] = uint16_t(c);
-        for (uint32_t k = 0; k < c; k++) lids[k * N + t] = uint16_t(V.nb[size_t(k) * V.stride + g] - Mv.offset);
-    }
-    __syncthreads();
-    const double half = dt / 2.0;
-    uint32_t cur = Pm.cur;
-    auto advance_all = [&]() {
-        for (uint32_t k = 0; k < cnt; k++)
-            advance_facets(V.facets + size_t(s_pm[k].slot) * V.max_facets, int(s_pm[k].nf), dt);
-    };
-    for (int s = all_valid ? 0 : -1; s < int(nsteps); s++) {
-        if (s >= 0) {
-            if (own) pool_kick_drift<STATE_FULL>(V, Mv, s > 0, half, dt, g, g + 1, 1);
-            if (s > 0 && t == 0) advance_all();
-            __syncthreads();
-        }
-        if (own && (s >= 0 || !Pm.acc_valid)) {
-            pool_force_phase<BIN, HAM, HG_PAIRS_NEIGHBOR_LIST, PREC, STATE_FULL, true, FAC>(P, MC, V, Mv, cur, F, g,
-                                                                                           g + 1, 1, lids, kmax);
-            cur ^= 1u;
-        }
-        __syncthreads();
-    }
-    if (nsteps > 0) {
-        if (own) pool_final_kick<STATE_FULL>(V, Mv, half, g, g + 1, 1);
-        if (t == 0) advance_all();
-    } else if (own) {
-        const double *q = pool_lds + size_t(t) * kFullStride;
-        st3(V.a, g, lds3(q + 12));
-        st3(V.al, g, lds3(q + 15));
-    }
-    __syncthreads();
-    return true;
-}
-
-// One rebuild interval of every queued system. The queue holds packs
-// (packs[i] = first | count << 24 over the slots in `order`): a pack of one
-// is a system stepped by the whole workgroup, a larger one small systems
-// stepped side by side (run_pack). Exit: every workgroup leaves once the
-// shared counter passes `count`. lds_bytes of dynamic LDS per workgroup
-// decide each system's state placement. FAC = false leaves the facet fold
-// out (every queued system has nf = 0): it holds the kernel's largest
-// register set. TPB threads per workgroup (256 or 512): a 512-thread
-// workgroup alone on a CU has the same waves per SIMD as two of 256 and twice
-// the LDS for one system.
-template <int BIN, int HAM, int PAIRS, int PREC, bool FAC, int TPB>
-// The model constants come by value: the scalar registers they spill to are
-// re-read with v_readlane, which measured faster than reloading them through
-// a pointer inside the pair loop (scalar loads add memory latency there).
-__global__ void __launch_bounds__(TPB, HG_CHUNK_MIN_BLOCKS)
-    k_pool_chunk(hg_params P, mixed_consts MC, pool_view V, const uint32_t *order, const uint32_t *packs,
-                 uint32_t count, uint32_t *counter, uint32_t nsteps, double dt, uint32_t lds_bytes) {
-    __shared__ uint32_t s_item;
-    __shared__ uint32_t s_red[TPB / 64];
-    __shared__ pool_meta s_pm[kMaxPack];
-    __shared__ uint32_t s_base[kMaxPack + 1];
-    for (;;) {
-        if (threadIdx.x == 0) s_item = atomicAdd(counter, 1u);
-        __syncthreads();
-        const uint32_t item = s_item;
-        __syncthreads();
-        if (item >= count) break;
-        const uint32_t pk = packs[item];
-        const uint32_t first = pk & 0xFFFFFFu, cnt = pk >> 24;
-        if constexpr (PAIRS == HG_PAIRS_NEIGHBOR_LIST) {
-            if (cnt > 1 &&
-                run_pack<BIN, HAM, PREC, FAC>(P, MC, V, order + first, cnt, nsteps, dt, lds_bytes, s_red, s_pm, s_base))
-                continue;
-        }
-        for (uint32_t k = 0; k < cnt; k++)
-            run_one<BIN, HAM, PAIRS, PREC, FAC>(P, MC, V, order[first + k], nsteps, dt, lds_bytes, s_red);
-    }
-}
-
-// ------------------------------------------------- wide (large) systems -----
-// Systems of at least wide_min particles skip the chunk kernel, where one
-// workgroup would carry the whole system and set the interval's critical
-// path. They are stepped by per-step launches over all their particles at
-// once, one thread per particle: wide_block b covers particles
-// [start, start + kWideBlock) of system `slot`. The operations and their order
-// per particle are those of run_system, so results are the same either way.
-constexpr uint32_t kWideBlock = 128;
-constexpr uint32_t kDefaultWideMin = 2048;
-constexpr double kDefaultWideCuFraction = 0.25;
-enum { TUNE_OFF = 0, TUNE_START = 1, TUNE_RUNNING = 2, TUNE_DONE = 3 };
-struct wide_block {
-    uint32_t slot, start;
-};
-
-// pass < 0: the initial acceleration pass of the systems without valid
-// accelerations (others return); pass s >= 0: the pass of step s.
-template <int BIN, int HAM, int PAIRS, int PREC>
-__global__ void __launch_bounds__(kWideBlock) k_pool_wide_force(hg_params P, mixed_consts MC, pool_view V,
-                                                                const wide_block *map, int pass) {
-    const wide_block b = map[blockIdx.x];
-    const pool_meta M = V.meta[b.slot];
-    uint32_t cur = M.cur;
-    if (pass < 0) {
-        if (M.acc_valid) return;
-    } else {
-        cur ^= (uint32_t(pass) + (M.acc_valid ? 0u : 1u)) & 1u;
-    }
-    const uint32_t g = M.offset + b.start + threadIdx.x;
-    const uint32_t end = M.offset + M.n;
-    if (g >= end) return;
-    const facet_dev *F = V.facets + size_t(b.slot) * V.max_facets;
-    pool_force_phase<BIN, HAM, PAIRS, PREC, STATE_GLOBAL>(P, MC, V, M, cur, F, g, g + 1, 1);
-}
-
-// Kick/drift of step s (pending = s > 0 completes step s-1 and moves the
-// facets by one step first, as run_system does).
-__global__ void __launch_bounds__(kWideBlock) k_pool_wide_kick_drift(pool_view V, const wide_block *map, int pending,
-                                                                     double half, double dt) {
-    const wide_block b = map[blockIdx.x];
-    const pool_meta M = V.meta[b.slot];
-    if (pending && b.start == 0 && threadIdx.x == 0)
-        advance_facets(V.facets + size_t(b.slot) * V.max_facets, int(M.nf), dt);
-    const uint32_t g = M.offset + b.start + threadIdx.x;
-    if (g >= M.offset + M.n) return;
-    pool_kick_drift<STATE_GLOBAL>(V, M, pending != 0, half, dt, g, g + 1, 1);
-}
-
-__global__ void __launch_bounds__(kWideBlock) k_pool_wide_final_kick(pool_view V, const wide_block *map, double half,
-                                                                     double dt) {
-    const wide_block b = map[blockIdx.x];
-    const pool_meta M = V.meta[b.slot];
-    if (b.start == 0 && threadIdx.x == 0) advance_facets(V.facets + size_t(b.slot) * V.max_facets, int(M.nf), dt);
-    const uint32_t g = M.offset + b.start + threadIdx.x;
-    if (g >= M.offset + M.n) return;
-    pool_final_kick<STATE_GLOBAL>(V, M, half, g, g + 1, 1);
-}
-
-// Fused wide steps (no wide system has facets, whose one-per-step advance
-// other blocks of the same launch would race): positions, velocities and
-// angular velocities alternate between two buffers, so that one launch can
-// read every particle's step-s state (Vi) while it writes step s+1's (Vo).
-// theta, the accelerations and the pair tables stay in place (Vi and Vo share
-// them; only a particle's own thread touches its theta and accelerations).
-// Kick/drift of the next step for particle g: pool_kick_drift's operations
-// with pending = true, on the state and accelerations the pass leaves in
-// registers, written into Vo (theta in place).
-__device__ __forceinline__ void kick_drift_io(const pool_view &Vi, const pool_view &Vo, double half, double dt,
-                                              uint32_t g, d3 x0, d3 vi, d3 wi, d3 ai, d3 ali, d3 th0) {
-    vi = vi + ai * half;
-    wi = wi + ali * half;
-    vi = vi + ai * half;
-    wi = wi + ali * half;
-    const d3 xi = x0 + vi * dt;
-    const d3 thi = th0 + wi * dt;
-    st3(Vo.x, g, xi);
-    st3(Vi.th, g, thi);
-    st3(Vo.v, g, vi);
-    st3(Vo.w, g, wi);
-}
-
-// The pass of step `pass` from Vi, then the kick/drift of step pass+1 into Vo.
-template <int BIN, int HAM, int PAIRS, int PREC>
-__global__ void __launch_bounds__(kWideBlock) k_pool_wide_step(hg_params P, mixed_consts MC, pool_view Vi,
-                                                               pool_view Vo, const wide_block *map, int pass,
-                                                               double half, double dt) {
-    const wide_block b = map[blockIdx.x];
-    const pool_meta M = Vi.meta[b.slot];
-    const uint32_t cur = M.cur ^ ((uint32_t(pass) + (M.acc_valid ? 0u : 1u)) & 1u);
-    const uint32_t g = M.offset + b.start + threadIdx.x;
-    if (g >= M.offset + M.n) return;
-    const facet_dev *F = Vi.facets + size_t(b.slot) * Vi.max_facets;
-    const d3 th0 = ld3(Vi.th, g);
-    pool_force_phase<BIN, HAM, PAIRS, PREC, STATE_GLOBAL, false, true>(
-        P, MC, Vi, M, cur, F, g, g + 1, 1, nullptr, 0, [&](uint32_t gg, d3 x0, d3 v0, d3 w0, d3 a, d3 al) {
-            kick_drift_io(Vi, Vo, half, dt, gg, x0, v0, w0, a, al, th0);
-        });
-}
-
-// Final kick of the fused steps: pool_final_kick's operations from Vi into
-// Vo (the pool's own buffers), positions copied across when they differ.
-__global__ void __launch_bounds__(kWideBlock) k_pool_wide_final_kick_io(pool_view Vi, pool_view Vo,
-                                                                        const wide_block *map, double half) {
-    const wide_block b = map[blockIdx.x];
-    const pool_meta M = Vi.meta[b.slot];
-    const uint32_t g = M.offset + b.start + threadIdx.x;
-    if (g >= M.offset + M.n) return;
-    const d3 vi = ld3(Vi.v, g) + ld3(Vi.a, g) * half;
-    const d3 wi = ld3(Vi.w, g) + ld3(Vi.al, g) * half;
-    if (Vi.x != Vo.x) st3(Vo.x, g, ld3(Vi.x, g));
-    st3(Vo.v, g, vi);
-    st3(Vo.w, g, wi);
-    if (nonfinite(vi, wi)) {
-        atomicOr(&Vi.flags[FLAG_NUMERIC], 1);
-        atomicOr(&Vi.sflags[M.slot], HG_FAULT_NUMERIC);
-    }
-}
 
 // Sums the per-particle ledger terms in particle order, the order sum_energy
 // uses on the host: lane c < 7 adds term c of every particle, then lane 0 adds
@@ -890,115 +230,42 @@ __global__ void k_zero_rows_f64(double *p, size_t stride, size_t offset, size_t 
 
 inline unsigned nblk(size_t n, unsigned bs) { return unsigned((n + bs - 1) / bs); }
 
-template <int BIN, int HAM, int PAIRS, int PREC, bool FAC, int TPB>
-hipError_t launch_chunk_k(const hg_params &p, const pool_view &V, const uint32_t *order, const uint32_t *packs,
-                          uint32_t count,
-                          uint32_t *counter, uint32_t nsteps, double dt, unsigned grid, uint32_t lds_cap,
-                          hipStream_t s) {
-    const size_t lds_bytes = lds_cap;
-    if (lds_bytes > 0) {
-        hipError_t e =
-            hipFuncSetAttribute(reinterpret_cast<const void *>(&k_pool_chunk<BIN, HAM, PAIRS, PREC, FAC, TPB>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, int(lds_bytes));
-        if (e != hipSuccess) return e;
-    }
-    k_pool_chunk<BIN, HAM, PAIRS, PREC, FAC, TPB><<<grid, TPB, lds_bytes, s>>>(p, make_mixed_consts(p), V, order,
-                                                                                packs, count, counter, nsteps, dt,
-                                                                                lds_cap);
+}  // namespace
+hipError_t launch_tile_kick(const pool_view &V, const pool_view &Vo, const wide_block *map, unsigned blocks, int pairs,
+                            double half, double dt, hipStream_t s) {
+    if (blocks == 0) return hipSuccess;
+    k_tile_kick<<<blocks, 64, 0, s>>>(V, Vo, map, uint32_t(tile_width(pairs)), half, dt);
     return hipGetLastError();
 }
-
-template <int BIN, int HAM, int PAIRS>
-hipError_t launch_chunk_t(const hg_params &p, const pool_view &V, const uint32_t *order, const uint32_t *packs,
-                          uint32_t count,
-                          uint32_t *counter, uint32_t nsteps, double dt, unsigned grid, uint32_t lds_cap,
-                          bool facets, int tpb, hipStream_t s) {
-#define HG_KCASE(PREC, FAC, TPB)                                                                                \
-    if (p.precision == PREC && facets == FAC && tpb == TPB)                                                    \
-        return launch_chunk_k<BIN, HAM, PAIRS, PREC, FAC, TPB>(p, V, order, packs, count, counter, nsteps, dt, \
-                                                                grid, lds_cap, s);
-    HG_KCASE(HG_PRECISION_MIXED, true, 256)
-    HG_KCASE(HG_PRECISION_MIXED, false, 256)
-    HG_KCASE(HG_PRECISION_FP64, true, 256)
-    HG_KCASE(HG_PRECISION_FP64, false, 256)
-    HG_KCASE(HG_PRECISION_MIXED, true, 512)
-    HG_KCASE(HG_PRECISION_MIXED, false, 512)
-    HG_KCASE(HG_PRECISION_FP64, true, 512)
-    HG_KCASE(HG_PRECISION_FP64, false, 512)
-#undef HG_KCASE
+hipError_t launch_tile(const hg_params &p, const pool_view &Vi, const pool_view &Vo, const wide_block *map,
+                              unsigned blocks, int mode, bool facets, double half, double dt, hipStream_t s) {
+#define HG_TCASE(B, A)                                       \
+    if (p.binary_model == B && p.pair_mode == A)             \
+        return launch_tile_b<B, A>(p, Vi, Vo, map, blocks, mode, facets, half, dt, s);
+    HG_TCASE(HG_BINARY_NONE, HG_PAIRS_ALL)
+    HG_TCASE(HG_BINARY_NONE, HG_PAIRS_NEIGHBOR_LIST)
+    HG_TCASE(HG_BINARY_CONTACT, HG_PAIRS_ALL)
+    HG_TCASE(HG_BINARY_CONTACT, HG_PAIRS_NEIGHBOR_LIST)
+    HG_TCASE(HG_BINARY_SINTER, HG_PAIRS_ALL)
+    HG_TCASE(HG_BINARY_SINTER, HG_PAIRS_NEIGHBOR_LIST)
+#undef HG_TCASE
     return hipErrorInvalidValue;
 }
-
-// facets: whether any queued system has facets (else the kernel without the
-// facet fold runs); tpb: threads per workgroup (256 or 512).
-template <int PAIRS>
-hipError_t launch_chunk_p(const hg_params &p, const pool_view &V, const uint32_t *order, const uint32_t *packs,
-                          uint32_t count,
-                          uint32_t *counter, uint32_t nsteps, double dt, unsigned grid, uint32_t lds_cap,
-                          bool facets, int tpb, hipStream_t s) {
-#define HG_PCASE(B, H) \
-    if (p.binary_model == B && p.hamaker_model == H) \
-        return launch_chunk_t<B, H, PAIRS>(p, V, order, packs, count, counter, nsteps, dt, grid, lds_cap, facets, \
-                                           tpb, s);
-    HG_PCASE(HG_BINARY_NONE, HG_HAMAKER_NONE)
-    HG_PCASE(HG_BINARY_NONE, HG_HAMAKER_FULL)
-    HG_PCASE(HG_BINARY_NONE, HG_HAMAKER_LIMITED)
-    HG_PCASE(HG_BINARY_NONE, HG_HAMAKER_SIMPLIFIED)
-    HG_PCASE(HG_BINARY_CONTACT, HG_HAMAKER_NONE)
-    HG_PCASE(HG_BINARY_CONTACT, HG_HAMAKER_FULL)
-    HG_PCASE(HG_BINARY_CONTACT, HG_HAMAKER_LIMITED)
-    HG_PCASE(HG_BINARY_CONTACT, HG_HAMAKER_SIMPLIFIED)
-    HG_PCASE(HG_BINARY_SINTER, HG_HAMAKER_NONE)
-    HG_PCASE(HG_BINARY_SINTER, HG_HAMAKER_FULL)
-    HG_PCASE(HG_BINARY_SINTER, HG_HAMAKER_LIMITED)
-    HG_PCASE(HG_BINARY_SINTER, HG_HAMAKER_SIMPLIFIED)
-#undef HG_PCASE
-    return hipErrorInvalidValue;
-}
-
-// Vo null: the pass alone (k_pool_wide_force); else the fused step into Vo.
-template <int BIN, int HAM, int PAIRS>
-hipError_t launch_wide_force_t(const hg_params &p, const pool_view &V, const wide_block *map, unsigned blocks,
-                               int pass, hipStream_t s, const pool_view *Vo, double half, double dt) {
-    const mixed_consts mc = make_mixed_consts(p);
-    if (p.precision == HG_PRECISION_MIXED) {
-        if (Vo)
-            k_pool_wide_step<BIN, HAM, PAIRS, HG_PRECISION_MIXED>
-                <<<blocks, kWideBlock, 0, s>>>(p, mc, V, *Vo, map, pass, half, dt);
-        else
-            k_pool_wide_force<BIN, HAM, PAIRS, HG_PRECISION_MIXED><<<blocks, kWideBlock, 0, s>>>(p, mc, V, map, pass);
-    } else {
-        if (Vo)
-            k_pool_wide_step<BIN, HAM, PAIRS, HG_PRECISION_FP64>
-                <<<blocks, kWideBlock, 0, s>>>(p, mc, V, *Vo, map, pass, half, dt);
-        else
-            k_pool_wide_force<BIN, HAM, PAIRS, HG_PRECISION_FP64><<<blocks, kWideBlock, 0, s>>>(p, mc, V, map, pass);
+hipError_t launch_tile_steps(const hg_params &p, const pool_view &V, const pool_view &VB, const wide_block *map,
+                                    unsigned blocks, uint32_t len, bool facets, double half, double dt,
+                                    hipStream_t s) {
+    const pool_view *in = len % 2 ? &VB : &V, *out = len % 2 ? &V : &VB;
+    hipError_t e = launch_tile_kick(V, *in, map, blocks, p.pair_mode, half, dt, s);
+    for (uint32_t k = 0; k < len && e == hipSuccess; k++) {
+        e = launch_tile(p, *in, *out, map, blocks, k + 1 < len ? TILE_STEP : TILE_LAST, facets, half, dt, s);
+        const pool_view *t = in;
+        in = out;
+        out = t;
     }
-    return hipGetLastError();
+    return e;
 }
 
-template <int PAIRS>
-hipError_t launch_wide_force_p(const hg_params &p, const pool_view &V, const wide_block *map, unsigned blocks,
-                               int pass, hipStream_t s, const pool_view *Vo = nullptr, double half = 0.0,
-                               double dt = 0.0) {
-#define HG_WCASE(B, H)                                                                                 \
-    if (p.binary_model == B && p.hamaker_model == H)                                                   \
-        return launch_wide_force_t<B, H, PAIRS>(p, V, map, blocks, pass, s, Vo, half, dt);
-    HG_WCASE(HG_BINARY_NONE, HG_HAMAKER_NONE)
-    HG_WCASE(HG_BINARY_NONE, HG_HAMAKER_FULL)
-    HG_WCASE(HG_BINARY_NONE, HG_HAMAKER_LIMITED)
-    HG_WCASE(HG_BINARY_NONE, HG_HAMAKER_SIMPLIFIED)
-    HG_WCASE(HG_BINARY_CONTACT, HG_HAMAKER_NONE)
-    HG_WCASE(HG_BINARY_CONTACT, HG_HAMAKER_FULL)
-    HG_WCASE(HG_BINARY_CONTACT, HG_HAMAKER_LIMITED)
-    HG_WCASE(HG_BINARY_CONTACT, HG_HAMAKER_SIMPLIFIED)
-    HG_WCASE(HG_BINARY_SINTER, HG_HAMAKER_NONE)
-    HG_WCASE(HG_BINARY_SINTER, HG_HAMAKER_FULL)
-    HG_WCASE(HG_BINARY_SINTER, HG_HAMAKER_LIMITED)
-    HG_WCASE(HG_BINARY_SINTER, HG_HAMAKER_SIMPLIFIED)
-#undef HG_WCASE
-    return hipErrorInvalidValue;
-}
+namespace {
 
 }  // namespace
 }  // namespace hg
@@ -1015,14 +282,14 @@ struct hg_pool {
     size_t energy_cap = 0;
     hipStream_t stream = nullptr;
     double *x = nullptr, *v = nullptr, *th = nullptr, *w = nullptr, *a = nullptr, *al = nullptr;
-    double *xb = nullptr, *vb = nullptr, *wb = nullptr;  // second x, v, omega for the fused wide steps
+    double *xb = nullptr, *vb = nullptr, *wb = nullptr;  // second x, v, omega for the per-step launches
     uint32_t cap_n = 0, *nb = nullptr, *ncnt = nullptr;
     uint32_t cap_s = 0, *pj[2] = {nullptr, nullptr}, *pcnt[2] = {nullptr, nullptr};
     uint32_t *bj = nullptr, *bcnt = nullptr;  // neck strengths (sinter_breaking)
     double *bstr = nullptr;
     double *ps[2] = {nullptr, nullptr};
     uint32_t *owner = nullptr;
-    facet_dev *facets = nullptr;
+    facet_dev *facets = nullptr, *facets_b = nullptr;  // facets_b: the second set of the per-step launches
     double *ss = nullptr;
     pool_meta *meta_d = nullptr;
     std::vector<pool_meta> meta;
@@ -1060,7 +327,7 @@ struct hg_pool {
     size_t tune_pos = 0;
     hipGraphExec_t wg_exec = nullptr;
     uint32_t wg_len = 0;
-    bool wg_fused = false;
+    bool wg_facets = false;
     unsigned wg_blocks = 0;
     double wg_dt = 0.0;
     hipEvent_t wev[3] = {nullptr, nullptr, nullptr};
@@ -1187,6 +454,7 @@ pool_view make_pool_view(hg_pool *Q) {
     V.cap_n = Q->cap_n;
     V.facets = Q->facets;
     V.max_facets = uint32_t(Q->MF);
+    V.facet_steps = 1;
     V.ss = Q->ss;
     V.meta = Q->meta_d;
     V.stride = Q->P;
@@ -1406,11 +674,12 @@ hg_status hg_pool_create(const hg_params *params, size_t max_particles, size_t m
         PG_HIPC(hipMemcpy(Q->owner, none.data(), P * 4, hipMemcpyHostToDevice));
     }
     PG_TRYC(palloc(Q, &Q->facets, std::max<size_t>(1, Q->S * std::max<size_t>(Q->MF, 1))));
+    PG_TRYC(palloc(Q, &Q->facets_b, std::max<size_t>(1, Q->S * std::max<size_t>(Q->MF, 1))));
     if (Q->MF) PG_TRYC(palloc(Q, &Q->ss, Q->MF * 9 * P));
     PG_TRYC(palloc(Q, &Q->meta_d, Q->S));
     PG_TRYC(palloc(Q, &Q->order_d, Q->S));
     PG_TRYC(palloc(Q, &Q->packs_d, Q->S));
-    Q->wide_map_cap = Q->P / kWideBlock + Q->S + 1;
+    Q->wide_map_cap = Q->P / size_t(tile_width(Q->p.pair_mode)) + Q->S + 1;
     PG_TRYC(palloc(Q, &Q->wide_map_d, Q->wide_map_cap));
     PG_TRYC(palloc(Q, &Q->counter_d, 1));
     PG_TRYC(palloc(Q, &Q->flags, FLAG_COUNT));
@@ -1743,10 +1012,13 @@ hg_status refresh_order(hg_pool *Q) {
     std::stable_sort(Q->order.begin(), Q->order.end(),
                      [&](uint32_t a, uint32_t b) { return Q->meta[a].n > Q->meta[b].n; });
     std::vector<wide_block> map;
+    const uint32_t width = uint32_t(tile_width(Q->p.pair_mode));
     size_t first_narrow = 0;
     while (first_narrow < Q->order.size() && Q->wide_min && Q->meta[Q->order[first_narrow]].n >= Q->wide_min) {
         const uint32_t s = Q->order[first_narrow++];
-        for (uint32_t st = 0; st < Q->meta[s].n; st += kWideBlock) map.push_back(wide_block{s, st});
+        const pool_meta &M = Q->meta[s];
+        for (uint32_t st = 0; st < M.n; st += width)
+            map.push_back(wide_block{s, st, M.offset, M.n | (M.cur ? kBondBit : 0u)});
     }
     if (map.size() > Q->wide_map_cap) return fail(HG_ERR_INVALID, "hg_pool_step: wide map overflow");
     Q->narrow_count = uint32_t(Q->order.size() - first_narrow);
@@ -1929,67 +1201,26 @@ hg_status pool_begin(hg_pool *Q, double dt, uint64_t max_len, uint32_t rebuild_e
         hipStream_t s2 = split ? Q->stream_w : Q->stream;
         if (split) HG_HIP(hipStreamWaitEvent(Q->stream_w, Q->ev[1], 0));
         HG_HIP(hipEventRecord(Q->wev[0], s2));
-        auto force = [&](int pass) {
-            return nl ? launch_wide_force_p<HG_PAIRS_NEIGHBOR_LIST>(Q->p, V, Q->wide_map_d, Q->wide_blocks, pass, s2)
-                      : launch_wide_force_p<HG_PAIRS_ALL>(Q->p, V, Q->wide_map_d, Q->wide_blocks, pass, s2);
-        };
-        if (any_wide_initial) {
-            HG_HIP(force(-1));
-            Q->last_wide_launches++;
-        }
-        // Without wide facets the steps are fused: the first kick/drift, then
-        // one launch per step doing its pass and the next step's kick/drift,
-        // x, v and omega alternating between the pool's buffers (A) and the
-        // second set (B), the last pass alone and a final kick that leaves
-        // the state in A: len + 2 launches instead of 2 len + 1.
         bool wide_facets = false;
         for (size_t k = 0; k < Q->order.size() - count; k++) wide_facets |= Q->meta[Q->order[k]].nf > 0;
-        const bool fused = !wide_facets;
+        if (any_wide_initial) {
+            HG_HIP(launch_tile(Q->p, V, V, Q->wide_map_d, Q->wide_blocks, TILE_FORCE, wide_facets, half, dt, s2));
+            Q->last_wide_launches++;
+        }
         pool_view VB = V;
         VB.x = Q->xb;
         VB.v = Q->vb;
         VB.w = Q->wb;
-        auto enqueue_fused = [&](hipStream_t st_) -> hipError_t {
-            k_pool_wide_kick_drift<<<Q->wide_blocks, kWideBlock, 0, st_>>>(V, Q->wide_map_d, 0, half, dt);
-            hipError_t e = hipGetLastError();
-            if (e != hipSuccess) return e;
-            for (uint32_t st = 0; st + 1 < len; st++) {
-                const pool_view &Vi = st % 2 ? VB : V, &Vo = st % 2 ? V : VB;
-                e = nl ? launch_wide_force_p<HG_PAIRS_NEIGHBOR_LIST>(Q->p, Vi, Q->wide_map_d, Q->wide_blocks,
-                                                                     int(st), st_, &Vo, half, dt)
-                       : launch_wide_force_p<HG_PAIRS_ALL>(Q->p, Vi, Q->wide_map_d, Q->wide_blocks, int(st), st_,
-                                                           &Vo, half, dt);
-                if (e != hipSuccess) return e;
-            }
-            const pool_view &Vl = (len - 1) % 2 ? VB : V;
-            e = nl ? launch_wide_force_p<HG_PAIRS_NEIGHBOR_LIST>(Q->p, Vl, Q->wide_map_d, Q->wide_blocks,
-                                                                 int(len - 1), st_)
-                   : launch_wide_force_p<HG_PAIRS_ALL>(Q->p, Vl, Q->wide_map_d, Q->wide_blocks, int(len - 1), st_);
-            if (e != hipSuccess) return e;
-            k_pool_wide_final_kick_io<<<Q->wide_blocks, kWideBlock, 0, st_>>>(Vl, V, Q->wide_map_d, half);
-            return hipGetLastError();
-        };
+        VB.facets = Q->facets_b;
         // the interval's launches: recorded once into a HIP graph per
-        // (interval length, dt, wide set, fused or not) and replayed;
+        // (interval length, dt, wide set, facets or not) and replayed;
         // launched one by one when graphs are off
-        auto enqueue = [&](hipStream_t st_) -> hipError_t {
-            if (fused) return enqueue_fused(st_);
-            for (uint32_t st = 0; st < len; st++) {
-                k_pool_wide_kick_drift<<<Q->wide_blocks, kWideBlock, 0, st_>>>(V, Q->wide_map_d, st > 0 ? 1 : 0,
-                                                                                half, dt);
-                hipError_t e = hipGetLastError();
-                if (e != hipSuccess) return e;
-                e = nl ? launch_wide_force_p<HG_PAIRS_NEIGHBOR_LIST>(Q->p, V, Q->wide_map_d, Q->wide_blocks,
-                                                                     int(st), st_)
-                       : launch_wide_force_p<HG_PAIRS_ALL>(Q->p, V, Q->wide_map_d, Q->wide_blocks, int(st), st_);
-                if (e != hipSuccess) return e;
-            }
-            k_pool_wide_final_kick<<<Q->wide_blocks, kWideBlock, 0, st_>>>(V, Q->wide_map_d, half, dt);
-            return hipGetLastError();
+        auto enqueue = [&](hipStream_t st_) {
+            return launch_tile_steps(Q->p, V, VB, Q->wide_map_d, Q->wide_blocks, len, wide_facets, half, dt, st_);
         };
         if (Q->wide_graph) {
             if (!Q->wg_exec || Q->wg_len != len || Q->wg_dt != dt || Q->wg_blocks != Q->wide_blocks ||
-                Q->wg_fused != fused) {
+                Q->wg_facets != wide_facets) {
                 if (Q->wg_exec) HG_HIP(hipGraphExecDestroy(Q->wg_exec));
                 Q->wg_exec = nullptr;
                 hipGraph_t graph = nullptr;
@@ -2002,7 +1233,7 @@ hg_status pool_begin(hg_pool *Q, double dt, uint64_t max_len, uint32_t rebuild_e
                 (void)hipGraphDestroy(graph);
                 HG_HIP(ei);
                 Q->wg_len = len;
-                Q->wg_fused = fused;
+                Q->wg_facets = wide_facets;
                 Q->wg_dt = dt;
                 Q->wg_blocks = Q->wide_blocks;
             }
@@ -2010,7 +1241,7 @@ hg_status pool_begin(hg_pool *Q, double dt, uint64_t max_len, uint32_t rebuild_e
         } else {
             HG_HIP(enqueue(s2));
         }
-        Q->last_wide_launches += fused ? len + 2 : 2 * len + 1;
+        Q->last_wide_launches += len + 1;
         HG_HIP(hipEventRecord(Q->wev[1], s2));
     }
     if (count) {
@@ -2019,11 +1250,10 @@ hg_status pool_begin(hg_pool *Q, double dt, uint64_t max_len, uint32_t rebuild_e
         HG_HIP(hipEventRecord(Q->ev[2], sc));
         bool facets = false;
         for (size_t k = Q->order.size() - count; k < Q->order.size(); k++) facets |= Q->meta[Q->order[k]].nf > 0;
-        hipError_t e = nl ? launch_chunk_p<HG_PAIRS_NEIGHBOR_LIST>(Q->p, V, Q->order_d, Q->packs_d, Q->pack_count,
-                                                                   Q->counter_d, len, dt, g, Q->lds_cap, facets,
-                                                                   Q->chunk_tpb, sc)
-                          : launch_chunk_p<HG_PAIRS_ALL>(Q->p, V, Q->order_d, Q->packs_d, Q->pack_count, Q->counter_d,
-                                                         len, dt, g, Q->lds_cap, facets, Q->chunk_tpb, sc);
+        const chunk_launch c{Q->order_d, Q->packs_d, Q->pack_count, Q->counter_d, len,
+                             dt,         g,          Q->lds_cap,    facets,       Q->chunk_tpb};
+        hipError_t e = nl ? launch_chunk_p<HG_PAIRS_NEIGHBOR_LIST>(Q->p, V, c, sc)
+                          : launch_chunk_p<HG_PAIRS_ALL>(Q->p, V, c, sc);
         HG_HIP(e);
         HG_HIP(hipEventRecord(Q->ev[3], sc));
     }
@@ -2048,15 +1278,17 @@ hg_status pool_end(hg_pool *Q, std::vector<int32_t> &faulted) {
     HG_HIP(hipStreamSynchronize(Q->stream));
     // host mirror of what the kernels did to each system, before any fault is
     // read, so that the systems that go on keep a true mirror
-    for (uint32_t s : Q->order) {
+    const size_t wide = Q->order.size() - Q->fl.count;  // the first ones; their tables are updated in place
+    for (size_t k = 0; k < Q->order.size(); k++) {
+        const uint32_t s = Q->order[k];
         pool_meta &M = Q->meta[s];
-        if (Q->cap_s) {
+        if (Q->cap_s && k >= wide) {
             if (!M.acc_valid) M.cur ^= 1u;
             M.cur ^= (len & 1u);
         }
         M.acc_valid = 1;
         Q->step_index[s] += len;
-        for (uint32_t k = 0; k < len; k++) Q->t[s] = Q->t[s] + dt;
+        for (uint32_t q = 0; q < len; q++) Q->t[s] = Q->t[s] + dt;
     }
     Q->meta_dirty = true;
     PG_TRY(collect_faults(Q, faulted));

@@ -1,0 +1,513 @@
+// Per-step kernels over many workgroups: one launch per time step for a whole
+// set of systems (the wide systems of a pool, or one hg_system), each
+// workgroup carrying a tile of W particles.
+//
+// One lane per particle walking its partners in turn leaves most of the chip
+// idle at the sizes a single aggregate has (20,000 particles are 313
+// wavefronts for 1,024 SIMDs) and makes a step as long as the longest chain of
+// dependent pair evaluations. Here a workgroup spreads its tile's ordered
+// pairs over all its threads: the listed partners are read k by k, matched
+// against the particle's table row and queued in LDS, bonded pairs apart from
+// the others, so that a wavefront evaluates one kind; each pair leaves its
+// term in LDS at its place in the list, and one thread per particle adds the
+// terms in list order, which gives the sums of the walk bit for bit. The same
+// thread then completes the step and drifts the particle into the other set
+// of x, v, omega buffers (other workgroups still read this one), so a step is
+// one launch.
+//
+// The pair-state rows are updated in place: a spring goes back to the slot it
+// came from. A row changes only when a contact begins or ends (or a bond
+// breaks); its owner thread then removes the ended entries and puts the new
+// ones in order before the launch ends, so the table is canonical between
+// launches.
+#pragma once
+
+#include "force_device.h"
+#include "pool_device.h"
+
+namespace hg {
+
+// One pair's functors, in the expressions and order of pair_fold_vw (FP64)
+// and pair_fold_mx (mixed).
+template <int PREC>
+struct prec_types {
+    using term = double;
+    using vec = d3;
+};
+template <>
+struct prec_types<HG_PRECISION_MIXED> {
+    using term = float;
+    using vec = f3;
+};
+
+// hamaker_eval, lr_hamaker_eval and simplified_hamaker_eval of r = xj - xi,
+// with the distance taken once.
+template <int HAM>
+__device__ __forceinline__ d3 hamaker_lin(const hg_hamaker_params &p, d3 r) {
+    if constexpr (HAM == HG_HAMAKER_NONE) return zero3();
+    const double z = dot(r, r), dist = sqrt(z);
+    if (HAM == HG_HAMAKER_LIMITED && dist > p.r_cutoff) return zero3();
+    double h = dist - 2.0 * p.r_part;
+    if (h < p.h0) h = p.h0;
+    const d3 u = z > 0.0 ? r / dist : r;
+    d3 f;
+    if constexpr (HAM == HG_HAMAKER_SIMPLIFIED) f = 2.0 * p.A * p.r_part / sq(h) * u;
+    else f = hamaker_scalar(p.A, p.r_part, h) * u;
+    return f / p.mass;
+}
+
+template <int HAM, int PREC>
+struct pair_eval {
+    using vec = typename prec_types<PREC>::vec;
+    const hg_params &p;
+    const mixed_consts &m;
+    double touch2;  // squared contact distance and a margin far above rounding
+
+    __device__ __forceinline__ pair_eval(const hg_params &P, const mixed_consts &M) : p(P), m(M) {
+        const double reach = 2.0 * P.contact.r_part;
+        touch2 = reach * reach * (1.0 + 1e-12);
+    }
+    // A bonded pair: its term and new springs; true when the bond breaks
+    // (this evaluation is still the bonded one).
+    template <class NECK>
+    __device__ __forceinline__ bool bonded(d3 xi, d3 vi, d3 wi, d3 xj, d3 vj, d3 wj, spring9 &sp, NECK &&neck,
+                                           vec &lin, vec &ang) const {
+        bool broke = false;
+        if constexpr (PREC == HG_PRECISION_FP64) {
+            d3 ftot;
+            const acc6 b = sinter_eval(p.sinter, xi, xj, vi, vj, wi, wj, sp, ftot);
+            if (p.sinter_breaking) broke = norm(ftot) > neck();
+            lin = HAM != HG_HAMAKER_NONE ? b.lin + hamaker_lin<HAM>(p.hamaker, xj - xi) : b.lin;
+            ang = b.ang;
+        } else {
+            double dist;
+            d3 n64;
+            f3 n;
+            pair_kinematics_mx(xi, xj, dist, n64, n);
+            bool keep;
+            const accf b = bonded_or_contact_mx<true>(
+                m, dist, n64, n, vi, wi, [&](d3 &v, d3 &w) { v = vj, w = wj; }, sp, keep);
+            if (m.s_breaking) broke = sqrtf(dotf(b.lin, b.lin)) * m.s_m > float(neck());
+            f3 h = zerof();
+            if constexpr (HAM != HG_HAMAKER_NONE) h = hamaker_mx<HAM>(m, dist, n);
+            lin = b.lin + h;
+            ang = b.ang;
+        }
+        return broke;
+    }
+    // The Hamaker term of an unbonded pair and, with CONTACT, whether the
+    // pair is in contact.
+    template <bool CONTACT>
+    __device__ __forceinline__ bool free(d3 xi, d3 xj, vec &lin) const {
+        bool touching = false;
+        if constexpr (PREC == HG_PRECISION_FP64) {
+            if constexpr (CONTACT) {
+                const d3 d = xi - xj;
+                if (!(dot(d, d) > touch2)) {  // beyond touch2 the overlap is negative
+                    const double overlap = 2.0 * p.contact.r_part - dot(d, normalized(d));
+                    touching = !(overlap <= 0);
+                }
+            }
+            lin = hamaker_lin<HAM>(p.hamaker, xj - xi);
+        } else {
+            const d3 d = xi - xj;
+            const double d2 = dotm(d, d);
+            lin = zerof();
+            if (!(d2 > m.far2)) {
+                double dist;
+                d3 n64;
+                f3 n;
+                pair_kinematics_mx(xi, xj, dist, n64, n);
+                if constexpr (CONTACT) touching = !(m.c_r2 - dist <= 0.0);
+                if constexpr (HAM != HG_HAMAKER_NONE) lin = hamaker_mx<HAM>(m, dist, n);
+            } else {
+                if constexpr (HAM != HG_HAMAKER_NONE) lin = hamaker_far_mx<HAM>(m, d, d2);
+            }
+        }
+        return touching;
+    }
+    // The contact functor of a touching pair (without its Hamaker term).
+    __device__ __forceinline__ void contact(d3 xi, d3 vi, d3 wi, d3 xj, d3 vj, d3 wj, spring9 &sp, vec &lin,
+                                            vec &ang) const {
+        bool keep;
+        auto vw = [&](d3 &v, d3 &w) { v = vj, w = wj; };
+        if constexpr (PREC == HG_PRECISION_FP64) {
+            const acc6 b = contact_eval_vw(p.contact, xi, xj, vi, wi, vw, sp, keep);
+            lin = b.lin;
+            ang = b.ang;
+        } else {
+            double dist;
+            d3 n64;
+            f3 n;
+            pair_kinematics_mx(xi, xj, dist, n64, n);
+            const accf b = bonded_or_contact_mx<false>(m, dist, n64, n, vi, wi, vw, sp, keep);
+            lin = b.lin;
+            ang = b.ang;
+        }
+    }
+};
+
+namespace {
+
+// LDS of a tile: own state, the terms of KC list positions per particle
+// (position kk of particle i at [kk * W + i]), the queue of those positions'
+// pairs, and the rows' counts.
+template <int W, int KC, int PREC, bool FAC>
+struct tile_lds {
+    using term = typename prec_types<PREC>::term;
+    double s[9][W];  // x, v, omega
+    term T[6][KC * W];
+    uint2 Q[KC * W];  // partner, and i | kk << 8 | row slot << 20
+    uint16_t CW[KC * W];
+    uint32_t rows[W], dirty[W];
+    uint32_t nB[kTileThreads / 64], nO[kTileThreads / 64];
+    uint32_t contacts, ended;
+    typename prec_types<PREC>::term F[FAC ? 6 : 1][W];
+    term A[6][W < 64 ? W : 1];
+};
+
+constexpr uint32_t kNoRowSlot = 0xFFFu;
+
+// What a launch does after the pass: TILE_FORCE stores the accelerations of
+// the systems that have none; TILE_STEP completes the step, kicks and drifts
+// into the other buffers; TILE_LAST completes the last step.
+template <int BIN, int HAM, int PAIRS, int PREC, bool FAC>
+__global__ void __launch_bounds__(kTileThreads)
+    k_tile_step(hg_params P, mixed_consts MC, pool_view Vi, pool_view Vo, const wide_block *map, int mode, double half,
+                double dt) {
+    constexpr int W = tile_width(PAIRS), KC = kTilePairs / W, ROWS = kTileThreads / W, WAVES = kTileThreads / 64;
+    using term = typename prec_types<PREC>::term;
+    using vec = typename prec_types<PREC>::vec;
+    __shared__ tile_lds<W, KC, PREC, FAC> L;
+    const wide_block b = map[blockIdx.x];
+    const uint32_t n = b.n & kIdxMask, cur = b.n >> 31, base = b.offset + b.start;
+    const uint32_t nt = n - b.start < uint32_t(W) ? n - b.start : uint32_t(W);
+    const uint32_t tid = threadIdx.x, wv = tid >> 6, lane = tid & 63u;
+    if (mode == TILE_FORCE && Vi.meta[b.slot].acc_valid) return;
+    const size_t stride = Vi.stride;
+    uint32_t *pj = cur ? Vi.pj1 : Vi.pj0, *pcnt = cur ? Vi.pcnt1 : Vi.pcnt0;
+    double *ps = cur ? Vi.ps1 : Vi.ps0;
+    const pair_eval<HAM, PREC> ev(P, MC);
+
+    const uint32_t i = tid % W, r0 = tid / W;  // own particle of the tile, first list row
+    const uint32_t g = base + (i < nt ? i : 0);
+    uint32_t cnt = 0, c_old = 0;
+    if (i < nt) {
+        cnt = PAIRS == HG_PAIRS_NEIGHBOR_LIST ? Vi.ncnt[g] : n - 1u;
+        if constexpr (BIN != HG_BINARY_NONE) c_old = pcnt[g];
+    }
+    for (uint32_t q = tid; q < 3u * W; q += kTileThreads) {
+        const uint32_t f = q / W, t = q % W;
+        if (t < nt) {
+            const d3 a = ld3(f == 0 ? Vi.x : (f == 1 ? Vi.v : Vi.w), base + t);
+            L.s[3 * f][t] = a.x;
+            L.s[3 * f + 1][t] = a.y;
+            L.s[3 * f + 2][t] = a.z;
+        }
+    }
+    if (tid < uint32_t(W)) {
+        L.rows[tid] = c_old;
+        L.dirty[tid] = 0;
+    }
+    if (tid == 0) L.contacts = L.ended = 0;
+    auto own = [&](int f, uint32_t t) { return d3{L.s[3 * f][t], L.s[3 * f + 1][t], L.s[3 * f + 2][t]}; };
+
+    const uint32_t seg = wv * 64u * (KC / ROWS);  // this wavefront's part of the queue
+    vec accv{};          // W == 64: wavefront 0 sums forces, wavefront 1 torques
+    term acct = term(0);  // W < 64: thread c * W + i sums component c
+    for (uint32_t k0 = 0;; k0 += KC) {
+        // queue the pairs of list positions k0 .. k0 + KC - 1: bonded ones
+        // from the front of the wavefront's part, the others from its back
+        uint32_t tags[4];
+        if constexpr (BIN != HG_BINARY_NONE) {
+#pragma unroll
+            for (uint32_t s = 0; s < 4; s++) tags[s] = s < c_old ? pj[size_t(s) * stride + g] : kNoEntry;
+        }
+        uint32_t js[KC / ROWS];
+#pragma unroll
+        for (uint32_t q = 0; q < KC / ROWS; q++) {
+            const uint32_t k = k0 + r0 + q * ROWS;
+            if constexpr (PAIRS == HG_PAIRS_NEIGHBOR_LIST) js[q] = k < cnt ? Vi.nb[size_t(k) * stride + g] : kNoEntry;
+            else js[q] = k < cnt ? b.offset + k + (k >= b.start + i ? 1u : 0u) : kNoEntry;
+        }
+        uint32_t nB = 0, nO = 0;
+#pragma unroll
+        for (uint32_t q = 0; q < KC / ROWS; q++) {
+            const uint32_t j = js[q];
+            const bool on = j != kNoEntry;
+            uint32_t slot = kNoRowSlot;
+            bool bond = false;
+            if constexpr (BIN != HG_BINARY_NONE) {
+                if (on) {
+#pragma unroll
+                    for (uint32_t s = 0; s < 4; s++)
+                        if ((tags[s] & kIdxMask) == j) {
+                            slot = s;
+                            bond = (tags[s] & kBondBit) != 0;
+                        }
+                    for (uint32_t s = 4; s < c_old; s++) {
+                        const uint32_t t = pj[size_t(s) * stride + g];
+                        if ((t & kIdxMask) == j) {
+                            slot = s;
+                            bond = (t & kBondBit) != 0;
+                        }
+                    }
+                }
+            }
+            const uint64_t mb = __ballot(on && bond), mo = __ballot(on && !bond), below = (1ull << lane) - 1ull;
+            if (on) {
+                const uint32_t at = bond ? nB + uint32_t(__popcll(mb & below))
+                                         : 64u * (KC / ROWS) - 1u - (nO + uint32_t(__popcll(mo & below)));
+                L.Q[seg + at] = uint2{j, i | ((r0 + q * ROWS) << 8) | (slot << 20)};
+            }
+            nB += uint32_t(__popcll(mb));
+            nO += uint32_t(__popcll(mo));
+        }
+        if (lane == 0) {
+            L.nB[wv] = nB;
+            L.nO[wv] = nO;
+        }
+        __syncthreads();
+
+        // evaluate: the bonded pairs, then from the next wavefront on the others
+        uint32_t tB = 0, tO = 0;
+#pragma unroll
+        for (int w = 0; w < WAVES; w++) {
+            tB += L.nB[w];
+            tO += L.nO[w];
+        }
+        const uint32_t tBp = (tB + 63u) & ~63u;
+        for (uint32_t idx = tid; idx < tBp + tO; idx += kTileThreads) {
+            const bool bond = idx < tBp;
+            if (bond && idx >= tB) continue;
+            uint32_t rest = bond ? idx : idx - tBp, w = 0;
+            for (; w + 1 < WAVES; w++) {
+                const uint32_t c = bond ? L.nB[w] : L.nO[w];
+                if (rest < c) break;
+                rest -= c;
+            }
+            const uint32_t at = w * 64u * (KC / ROWS) + (bond ? rest : 64u * (KC / ROWS) - 1u - rest);
+            const uint2 e = L.Q[at];
+            const uint32_t t = e.y & 0xFFu, pos = ((e.y >> 8) & 0xFFFu) * W + t, slot = e.y >> 20, j = e.x;
+            const d3 xi = own(0, t), xj = ld3(Vi.x, j);
+            vec lin, ang{};
+            if (BIN == HG_BINARY_SINTER && bond) {
+                double *rec = ps + (size_t(slot) * stride + base + t) * kSpringRec;
+                spring9 sp = ld_rec(rec);
+                const bool broke = ev.bonded(
+                    xi, own(1, t), own(2, t), xj, ld3(Vi.v, j), ld3(Vi.w, j), sp,
+                    [&] {
+                        double r = __builtin_huge_val();
+                        if (Vi.bcnt)
+                            for (uint32_t s = 0; s < Vi.bcnt[base + t]; s++)
+                                if (Vi.bj[size_t(s) * stride + base + t] == j) r = Vi.bstr[size_t(s) * stride + base + t];
+                        return r;
+                    },
+                    lin, ang);
+                st_rec(rec, sp);
+                if (broke) {
+                    pj[size_t(slot) * stride + base + t] = kNoEntry;
+                    L.dirty[t] = L.ended = 1;
+                }
+            } else {
+                const bool touching = ev.template free<BIN != HG_BINARY_NONE>(xi, xj, lin);
+                if constexpr (BIN != HG_BINARY_NONE) {
+                    if (touching) {
+                        L.CW[atomicAdd(&L.contacts, 1u)] = uint16_t(at);
+                    } else if (slot != kNoRowSlot) {
+                        pj[size_t(slot) * stride + base + t] = kNoEntry;
+                        L.dirty[t] = L.ended = 1;
+                    }
+                }
+            }
+            L.T[0][pos] = lin.x;
+            L.T[1][pos] = lin.y;
+            L.T[2][pos] = lin.z;
+            L.T[3][pos] = ang.x;
+            L.T[4][pos] = ang.y;
+            L.T[5][pos] = ang.z;
+        }
+        if constexpr (FAC) {
+            // the facets' forces, by the last wavefront beside the pairs
+            const uint32_t nf = k0 == 0 ? Vi.meta[b.slot].nf : 0u;
+            if (nf && tid >= kTileThreads - uint32_t(W) && i < nt) {
+                const facet_dev *F = Vi.facets + size_t(b.slot) * Vi.max_facets;
+                auto put = [&](const auto &f) {
+                    L.F[0][i] = f.lin.x;
+                    L.F[1][i] = f.lin.y;
+                    L.F[2][i] = f.lin.z;
+                    L.F[3][i] = f.ang.x;
+                    L.F[4][i] = f.ang.y;
+                    L.F[5][i] = f.ang.z;
+                };
+                if constexpr (PREC == HG_PRECISION_FP64)
+                    put(facet_fold(P, F, int(nf), Vi.ss, stride, g, own(0, i), own(1, i), own(2, i)));
+                else
+                    put(facet_fold_mx(P, MC, F, int(nf), Vi.ss, stride, g, own(0, i), own(1, i), own(2, i)));
+            }
+        }
+        __syncthreads();
+        if constexpr (BIN != HG_BINARY_NONE) {
+            const uint32_t nc = L.contacts;
+            if (nc || L.ended) {  // uniform
+                // ended entries leave their rows before new contacts claim slots
+                if (tid < nt && L.dirty[tid]) {
+                    const uint32_t c = L.rows[tid], gi = base + tid;
+                    uint32_t q = 0;
+                    for (uint32_t s = 0; s < c; s++) {
+                        const uint32_t tag = pj[size_t(s) * stride + gi];
+                        if (tag == kNoEntry) continue;
+                        if (q != s) {
+                            pj[size_t(q) * stride + gi] = tag;
+                            st_rec(ps + (size_t(q) * stride + gi) * kSpringRec,
+                                   ld_rec(ps + (size_t(s) * stride + gi) * kSpringRec));
+                        }
+                        q++;
+                    }
+                    L.rows[tid] = q;
+                }
+                __syncthreads();
+                for (uint32_t c = tid; c < nc; c += kTileThreads) {
+                    const uint2 e = L.Q[L.CW[c]];
+                    const uint32_t t = e.y & 0xFFu, pos = ((e.y >> 8) & 0xFFFu) * W + t, j = e.x, gi = base + t;
+                    uint32_t slot = kNoRowSlot;
+                    if ((e.y >> 20) != kNoRowSlot) {  // it may have moved just now
+                        const uint32_t rc = L.rows[t] < Vi.cap_s ? L.rows[t] : Vi.cap_s;
+                        for (uint32_t s = 0; s < rc; s++)
+                            if ((pj[size_t(s) * stride + gi] & kIdxMask) == j) slot = s;
+                    }
+                    spring9 sp = zero_spring();
+                    if (slot != kNoRowSlot) sp = ld_rec(ps + (size_t(slot) * stride + gi) * kSpringRec);
+                    vec lin, ang;
+                    ev.contact(own(0, t), own(1, t), own(2, t), ld3(Vi.x, j), ld3(Vi.v, j), ld3(Vi.w, j), sp, lin, ang);
+                    if (slot == kNoRowSlot) {
+                        slot = atomicAdd(&L.rows[t], 1u);
+                        L.dirty[t] = 2;
+                        if (slot < Vi.cap_s) pj[size_t(slot) * stride + gi] = j;
+                    }
+                    if (slot < Vi.cap_s) st_rec(ps + (size_t(slot) * stride + gi) * kSpringRec, sp);
+                    if constexpr (HAM != HG_HAMAKER_NONE) lin = lin + vec{L.T[0][pos], L.T[1][pos], L.T[2][pos]};
+                    L.T[0][pos] = lin.x;
+                    L.T[1][pos] = lin.y;
+                    L.T[2][pos] = lin.z;
+                    L.T[3][pos] = ang.x;
+                    L.T[4][pos] = ang.y;
+                    L.T[5][pos] = ang.z;
+                }
+                __syncthreads();
+                if (tid < nt && L.dirty[tid]) {
+                    const uint32_t gi = base + tid;
+                    uint32_t c = L.rows[tid];
+                    if (c > Vi.cap_s) {
+                        atomicOr(&Vi.flags[FLAG_PAIR_OVERFLOW], 1);
+                        atomicMax(&Vi.flags[FLAG_PAIR_MAXCOUNT], int(c));
+                        if (Vi.sflags) atomicOr(&Vi.sflags[b.slot], HG_FAULT_PAIR_CAPACITY);
+                        c = Vi.cap_s;
+                        L.rows[tid] = c;
+                    }
+                    if (L.dirty[tid] == 2)  // new entries are at the row's end: insert them in order
+                        for (uint32_t s = 1; s < c; s++) {
+                            const uint32_t tag = pj[size_t(s) * stride + gi];
+                            uint32_t q = s;
+                            if ((pj[size_t(s - 1) * stride + gi] & kIdxMask) < (tag & kIdxMask)) continue;
+                            const spring9 sp = ld_rec(ps + (size_t(s) * stride + gi) * kSpringRec);
+                            while (q > 0) {
+                                const uint32_t prev = pj[size_t(q - 1) * stride + gi];
+                                if ((prev & kIdxMask) < (tag & kIdxMask)) break;
+                                pj[size_t(q) * stride + gi] = prev;
+                                st_rec(ps + (size_t(q) * stride + gi) * kSpringRec,
+                                       ld_rec(ps + (size_t(q - 1) * stride + gi) * kSpringRec));
+                                q--;
+                            }
+                            pj[size_t(q) * stride + gi] = tag;
+                            st_rec(ps + (size_t(q) * stride + gi) * kSpringRec, sp);
+                        }
+                    pcnt[gi] = c;
+                    L.dirty[tid] = 0;
+                }
+                if (tid == 0) L.contacts = L.ended = 0;
+            }
+        }
+        // the terms of this part of the lists, in list order
+        if constexpr (W == 64) {
+            if (wv < 2) {
+                const uint32_t left = cnt > k0 ? cnt - k0 : 0u, end = left < uint32_t(KC) ? left : uint32_t(KC);
+                for (uint32_t kk = 0; kk < end; kk++)
+                    accv = accv + vec{L.T[3 * wv][kk * W + i], L.T[3 * wv + 1][kk * W + i], L.T[3 * wv + 2][kk * W + i]};
+            }
+            if (!__any(cnt > k0 + KC)) break;  // every wavefront sees the same 64 counts
+        } else {
+            const uint32_t all = n - 1u, left = all > k0 ? all - k0 : 0u,
+                           end = left < uint32_t(KC) ? left : uint32_t(KC);
+            if (tid < 6u * W)
+                for (uint32_t kk = 0; kk < end; kk++) acct = acct + L.T[r0][kk * W + i];
+            if (k0 + KC >= all) break;
+        }
+        __syncthreads();
+        if constexpr (BIN != HG_BINARY_NONE) c_old = L.rows[i];
+    }
+    if constexpr (W < 64) {
+        if (tid < 6u * W) L.A[r0][i] = acct;
+        __syncthreads();
+    }
+    if constexpr (FAC) {
+        // the other set of facets for the next launch, moved by this step
+        if (b.start == 0 && tid == kTileThreads - 1 && mode != TILE_FORCE) {
+            const uint32_t nf = Vi.meta[b.slot].nf;
+            const facet_dev *F = Vi.facets + size_t(b.slot) * Vi.max_facets;
+            facet_dev *O = Vo.facets + size_t(b.slot) * Vo.max_facets;
+            for (uint32_t f = 0; f < nf; f++) O[f] = F[f];
+            if (Vi.facet_steps) advance_facets(O, int(nf), dt);
+        }
+    }
+    // wavefront (or row) 0: force, velocity and position; 1: torque, angular
+    // velocity and orientation
+    if (r0 >= 2 || i >= nt) return;
+    vec a;
+    if constexpr (W == 64) a = accv;
+    else a = vec{L.A[3 * r0][i], L.A[3 * r0 + 1][i], L.A[3 * r0 + 2][i]};
+    if constexpr (FAC)
+        if (Vi.meta[b.slot].nf) a = a + vec{L.F[3 * r0][i], L.F[3 * r0 + 1][i], L.F[3 * r0 + 2][i]};
+    d3 a64;
+    if constexpr (PREC == HG_PRECISION_FP64) a64 = a;
+    else a64 = tod(a);
+    if (mode != TILE_STEP) st3(r0 ? Vi.al : Vi.a, g, a64);
+    if (mode == TILE_FORCE) return;
+    d3 u = own(1 + int(r0), i);
+    u = u + a64 * half;
+    if (mode == TILE_STEP) {
+        u = u + a64 * half;
+        if (r0 == 0) st3(Vo.x, g, own(0, i) + u * dt);
+        else st3(Vi.th, g, ld3(Vi.th, g) + u * dt);
+    } else {
+        if (r0 == 0) st3(Vo.x, g, own(0, i));
+        if (nonfinite(u, u)) {
+            atomicOr(&Vi.flags[FLAG_NUMERIC], 1);
+            if (Vi.sflags) atomicOr(&Vi.sflags[b.slot], HG_FAULT_NUMERIC);
+        }
+    }
+    st3(r0 ? Vo.w : Vo.v, g, u);
+}
+
+// The first kick and drift of an interval, from the systems' own buffers into
+// Vo (the same buffers or the other set); the facets are copied along.
+__global__ void __launch_bounds__(64) k_tile_kick(pool_view V, pool_view Vo, const wide_block *map, uint32_t width,
+                                                  double half, double dt) {
+    const wide_block b = map[blockIdx.x];
+    const uint32_t n = b.n & kIdxMask;
+    if (Vo.facets != V.facets && b.start == 0 && threadIdx.x == 0) {
+        const uint32_t nf = V.meta[b.slot].nf;
+        for (uint32_t f = 0; f < nf; f++)
+            Vo.facets[size_t(b.slot) * V.max_facets + f] = V.facets[size_t(b.slot) * V.max_facets + f];
+    }
+    if (threadIdx.x >= width || b.start + threadIdx.x >= n) return;
+    const uint32_t g = b.offset + b.start + threadIdx.x;
+    const d3 v = ld3(V.v, g) + ld3(V.a, g) * half, w = ld3(V.w, g) + ld3(V.al, g) * half;
+    st3(Vo.x, g, ld3(V.x, g) + v * dt);
+    st3(V.th, g, ld3(V.th, g) + w * dt);
+    st3(Vo.v, g, v);
+    st3(Vo.w, g, w);
+}
+
+}  // namespace
+}  // namespace hg
