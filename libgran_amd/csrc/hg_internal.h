@@ -195,12 +195,15 @@ hipError_t launch_final_kick(double *v, double *w, const double *a, const double
                              facet_dev *facets, int nf, double facet_dt, int *flags, hipStream_t s);
 hipError_t launch_neighbor_build(hg_system_impl &S, hipStream_t s);
 hipError_t launch_advance_facet(facet_dev *f, const double *v, double dt, hipStream_t s);
-// nsteps steps of a system of at most 256 particles (FP64) in one workgroup
-// (see k_small_steps); `even`/`odd` are the views whose pair-state tables the
-// even/odd steps read. Systems of at most kTinySystemMax particles (all
-// pairs, or lists of capacity cap_n with n*cap_n <= 768) evaluate their pairs
-// in parallel (k_tiny_steps) when `scratch` holds n*max(n, cap_n)*kSpringRec
-// doubles.
+// nsteps steps of a small FP64 system in one workgroup; `even`/`odd` are the
+// views whose pair-state tables the even/odd steps read. Systems of at most
+// kTinySystemMax particles evaluate their pairs in parallel (k_tiny_steps;
+// `scratch` holds n*max(n, cap_n)*kSpringRec doubles). Legacy sinter_functor
+// systems of at most kSmallSystemMax take k_small_steps. The line for the
+// other functors lies at kTinySystemMax because one workgroup with a particle
+// per thread is slower than a launch per step over tiles from there on: 16
+// against 8.8 us per step at 30 particles, 22 against 10.9 at 200 (lists of
+// 3.9, FP64); with all pairs 49 against 9.0 and 199 against 14.3.
 constexpr uint32_t kSmallSystemMax = 256, kTinySystemMax = 27;
 hipError_t launch_small_steps(const hg_params &p, const sys_view &even, const sys_view &odd, double *x, double *v,
                               double *th, double *w, facet_dev *facets, uint32_t nsteps, bool pending_first,

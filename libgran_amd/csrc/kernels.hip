@@ -202,8 +202,8 @@ __global__ void __launch_bounds__(256) k_final_kick(double *v, double *w, const 
     final_kick_one(v, w, a, al, i, half, flags);
 }
 
-// nsteps steps of a system of at most kTile particles in one workgroup, one
-// particle per thread: per step the kick/drift (with the legacy connector
+// nsteps steps of a legacy sinter_functor system of at most kTile particles in
+// one workgroup, one particle per thread: per step the kick/drift (with the legacy connector
 // moves), a barrier, the acceleration pass, a barrier, as the per-step
 // launches of k_kick_drift, k_legacy_move and k_force_nl / k_force_all do it,
 // through the same device code. The pass reads pair-state table `even` on
@@ -743,8 +743,7 @@ hipError_t launch_small_steps_t(const hg_params &p, const sys_view &even, const 
                                 double *th, double *w, facet_dev *facets, uint32_t nsteps, bool pending_first,
                                 bool final_kick, double half, double dt, int nf_advance, double *lconn,
                                 const uint32_t *bcnt, double *scratch, hipStream_t s) {
-    const uint32_t slots = p.pair_mode == HG_PAIRS_NEIGHBOR_LIST ? even.cap_n : even.n;
-    if (scratch && even.n <= kTinyMax && even.n * slots <= kTinyThreads) {
+    if (even.n <= kTinyMax) {
         if (p.pair_mode == HG_PAIRS_NEIGHBOR_LIST)
             k_tiny_steps<BIN, HAM, true><<<1, kTinyThreads, 0, s>>>(p, even, odd, x, v, th, w, facets, nsteps,
                                                                     pending_first ? 1 : 0, final_kick ? 1 : 0, half,
@@ -755,16 +754,22 @@ hipError_t launch_small_steps_t(const hg_params &p, const sys_view &even, const 
                                                                      dt, nf_advance, scratch, lconn, bcnt);
         return hipGetLastError();
     }
-    k_small_steps<BIN, HAM><<<1, kTile, 0, s>>>(p, even, odd, x, v, th, w, facets, nsteps, pending_first ? 1 : 0,
-                                                final_kick ? 1 : 0, half, dt, nf_advance, lconn, bcnt);
-    return hipGetLastError();
+    if constexpr (BIN == HG_BINARY_SINTER_LEGACY) {
+        k_small_steps<BIN, HAM><<<1, kTile, 0, s>>>(p, even, odd, x, v, th, w, facets, nsteps, pending_first ? 1 : 0,
+                                                    final_kick ? 1 : 0, half, dt, nf_advance, lconn, bcnt);
+        return hipGetLastError();
+    }
+    return hipErrorInvalidValue;
 }
 
 hipError_t launch_small_steps(const hg_params &p, const sys_view &even, const sys_view &odd, double *x, double *v,
                               double *th, double *w, facet_dev *facets, uint32_t nsteps, bool pending_first,
                               bool final_kick, double half, double dt, int nf_advance, double *lconn,
                               const uint32_t *bcnt, double *scratch, hipStream_t s) {
-    if (even.n == 0 || even.n > uint32_t(kTile) || p.precision != HG_PRECISION_FP64) return hipErrorInvalidValue;
+    const uint32_t slots = p.pair_mode == HG_PAIRS_NEIGHBOR_LIST ? even.cap_n : even.n;
+    if (even.n == 0 || even.n > uint32_t(kTile) || p.precision != HG_PRECISION_FP64 ||
+        (even.n <= kTinyMax && (!scratch || even.n * slots > kTinyThreads)))
+        return hipErrorInvalidValue;
 #define HG_CASE(B, H)                                                                                            \
     if (p.binary_model == B && p.hamaker_model == H)                                                             \
         return launch_small_steps_t<B, H>(p, even, odd, x, v, th, w, facets, nsteps, pending_first, final_kick, \

@@ -618,11 +618,12 @@ hg_status step_impl(hg_system *S, double dt, uint64_t nsteps, uint32_t rebuild_e
     const uint32_t n = uint32_t(S->n);
     const bool nl = S->p.pair_mode == HG_PAIRS_NEIGHBOR_LIST;
     const int nf_advance = S->p.facet_advance ? 0 : S->nf;  // facets the step moves itself
-    if (n <= kSmallSystemMax && S->p.precision == HG_PRECISION_FP64 && !S->profiling && !S->per_step &&
-        !S->track_diss) {
+    const bool legacy = S->p.binary_model == HG_BINARY_SINTER_LEGACY;
+    if (n <= (legacy ? kSmallSystemMax : kTinySystemMax) && S->p.precision == HG_PRECISION_FP64 && !S->profiling &&
+        !S->per_step && !S->track_diss) {
         // small systems: the steps between list rebuilds in one launch of one
-        // workgroup instead of three dependent launches per step
-        if (S->p.binary_model == HG_BINARY_SINTER_LEGACY && !S->legacy_ready)
+        // workgroup instead of a launch or more per step
+        if (legacy && !S->legacy_ready)
             return fail(HG_ERR_INVALID, "the legacy sinter_functor's connectors are not set (hg_set_legacy_connectors)");
         if (n <= kTinySystemMax && !S->tiny) HG_TRY(dalloc(S, &S->tiny, size_t(n) * std::max(n, S->cap_n) * kSpringRec));
         uint64_t s = 0;
