@@ -359,11 +359,12 @@ size_t hg_pool_bytes_per_particle(const hg_params *params, size_t max_facets);
 hg_status hg_pool_last_step_profile(hg_pool *pool, double *chunk_ms, double *rebuild_ms, uint64_t *chunks,
                                     uint64_t *chunk_steps);
 /* Systems of at least wide_min particles (default 2048; 0: none) are stepped
- * by per-step launches over all their particles, one thread each, on a second
- * stream beside the chunk kernel, instead of by one workgroup: a large system
- * then no longer sets the critical path of the interval. The per-particle
- * operations are the same, so results do not change. Takes effect at the next
- * hg_pool_step. */
+ * by per-step launches over all their particles, instead of by one workgroup:
+ * a large system then no longer sets the critical path of the interval. With
+ * wide_min > 0 smaller systems take these launches too where that is the
+ * faster split for the sizes in the pool (few systems, or few large ones).
+ * The per-particle operations are the same, so results do not change. Takes
+ * effect at the next hg_pool_step. */
 hg_status hg_pool_set_wide_threshold(hg_pool *pool, size_t wide_min);
 /* While both kinds of systems are present, the chunk kernel's persistent grid
  * shrinks to wg_per_cu * (CUs - wide_cus) workgroups, leaving room worth
@@ -481,8 +482,8 @@ hg_status hg_server_get_stats(hg_server *srv, hg_server_stats *out);
  * their own, [2] neighbour rebuild (all of its kernels), [3] reserved. */
 hg_status hg_profile_enable(hg_system *sys, int enable);
 hg_status hg_profile_read(hg_system *sys, uint64_t *launches, double *device_ms);
-/* Small FP64 systems (up to 256 particles) step through one launch per
- * rebuild interval; enable = 1 makes hg_step use the per-step launches (the
+/* Small FP64 systems (up to 27 particles, with the legacy functor 256) step
+ * through one launch per rebuild interval; enable = 1 makes hg_step use the per-step launches (the
  * path every larger system takes) without the event timing of
  * hg_profile_enable, enable = 0 restores the choice by size. Results are the
  * same either way. Not in the reference (one code path per functor there):

@@ -1003,6 +1003,55 @@ hg_status hg_pool_set_facets(hg_pool *Q, int32_t slot, size_t nf, const double *
 
 namespace {
 
+// How many of the active systems, largest first, take the wide launches: all
+// of at least wide_min particles, and as many of the others as the estimates
+// below favour (none when wide_min = 0).
+//
+// A step of the wide launches costs a launch's latency or the chip's rate over
+// their particles, whichever is more; the chunk kernel's costs its longest
+// item (a workgroup goes through its system a particle per thread at a time)
+// or the sum of its items over the workgroups. Measured on MI355X, lists of
+// 3.9: per-step launches 8 us up to 30,000 particles, then 0.24 ns (mixed) or
+// 0.33 ns (FP64) a particle; a round of a 512-thread workgroup 20 us (mixed) or
+// 42 us (FP64), of a 256-thread one 12 and 25. So a system of 4,000 particles
+// held a launch of 50 steps for 176 us a step (mixed) where the tiles take 8,
+// and the chunk kernel's better rate (0.15 ns mixed, the same 0.33 ns in FP64)
+// only shows once every workgroup has work: 635,000 particles in 1,024
+// systems, mixed, took 206 us a step with the line at 4,096, 128 at 1,536 and
+// 166 at 512; 210,000 in 333, FP64, 291 us at 2,048 and 75 all wide.
+// With all pairs a round costs 0.5 us a partner and the tiles 0.1 ns a pair.
+size_t split_order(const hg_pool *Q) {
+    const size_t count = Q->order.size();
+    if (!Q->wide_min) return 0;
+    const bool mixed = Q->p.precision == HG_PRECISION_MIXED, all = Q->p.pair_mode == HG_PAIRS_ALL;
+    const double tpb = Q->chunk_tpb, wgs = Q->grid, round_us = mixed ? 0.032 * tpb + 4.0 : 0.068 * tpb + 7.0;
+    auto tile_us = [&](double n) { return all ? 1e-4 * n * n : (mixed ? 0.24e-3 : 0.33e-3) * n; };
+    auto item_us = [&](double n) { return std::max(1.0, n / tpb) * (all ? 0.5 * n : round_us); };
+    // a system smaller than a workgroup shares it with others (lists only)
+    auto share_us = [&](double n) { return all || n >= tpb ? item_us(n) : round_us * n / tpb; };
+    double chunk = 0.0;
+    for (uint32_t s : Q->order) chunk += share_us(Q->meta[s].n);
+    size_t best = 0;
+    double best_us = 0.0, wide = 0.0;
+    for (size_t k = 0; k <= count; k++) {
+        const double longest = k < count ? item_us(Q->meta[Q->order[k]].n) : 0.0;
+        const bool required = k < count && Q->meta[Q->order[k]].n >= Q->wide_min;
+        const bool boundary = k == 0 || k == count || Q->meta[Q->order[k]].n != Q->meta[Q->order[k - 1]].n;
+        if (!required && boundary) {
+            const double us = (k ? std::max(8.0, wide) : 0.0) + std::max(longest, chunk / wgs);
+            if (best_us == 0.0 || us < best_us) {
+                best_us = us;
+                best = k;
+            }
+        }
+        if (k < count) {
+            wide += tile_us(Q->meta[Q->order[k]].n);
+            chunk = std::max(0.0, chunk - share_us(Q->meta[Q->order[k]].n));
+        }
+    }
+    return best;
+}
+
 // Sorts the active systems largest first, splits off those that take the
 // wide launches and uploads the chunk kernel's queue and the wide block map.
 hg_status refresh_order(hg_pool *Q) {
@@ -1013,9 +1062,9 @@ hg_status refresh_order(hg_pool *Q) {
                      [&](uint32_t a, uint32_t b) { return Q->meta[a].n > Q->meta[b].n; });
     std::vector<wide_block> map;
     const uint32_t width = uint32_t(tile_width(Q->p.pair_mode));
-    size_t first_narrow = 0;
-    while (first_narrow < Q->order.size() && Q->wide_min && Q->meta[Q->order[first_narrow]].n >= Q->wide_min) {
-        const uint32_t s = Q->order[first_narrow++];
+    const size_t first_narrow = split_order(Q);
+    for (size_t k = 0; k < first_narrow; k++) {
+        const uint32_t s = Q->order[k];
         const pool_meta &M = Q->meta[s];
         for (uint32_t st = 0; st < M.n; st += width)
             map.push_back(wide_block{s, st, M.offset, M.n | (M.cur ? kBondBit : 0u)});

@@ -172,7 +172,7 @@ constexpr uint32_t kNoRowSlot = 0xFFFu;
 // the systems that have none; TILE_STEP completes the step, kicks and drifts
 // into the other buffers; TILE_LAST completes the last step.
 template <int BIN, int HAM, int PAIRS, int PREC, bool FAC>
-__global__ void __launch_bounds__(kTileThreads)
+__global__ void __launch_bounds__(kTileThreads, PREC == HG_PRECISION_MIXED && PAIRS == HG_PAIRS_NEIGHBOR_LIST ? 3 : 2)
     k_tile_step(hg_params P, mixed_consts MC, pool_view Vi, pool_view Vo, const wide_block *map, int mode, double half,
                 double dt) {
     constexpr int W = tile_width(PAIRS), KC = kTilePairs / W, ROWS = kTileThreads / W, WAVES = kTileThreads / 64;
