@@ -218,10 +218,10 @@ class System:
         _abi.check(_abi.lib().hg_step_async(self._h, dt, nsteps, rebuild_every))
 
     def state(self):
-        arrs = [np.zeros((self.n, 3)) for _ in range(4)]
+        arrs = [np.empty((self.n, 3)) for _ in range(4)]
         _abi.check(_abi.lib().hg_get_state(self._h, *[_abi.dptr(a) for a in arrs]))
         out = dict(zip(("x", "v", "theta", "omega"), arrs))
-        a, al = np.zeros((self.n, 3)), np.zeros((self.n, 3))
+        a, al = np.empty((self.n, 3)), np.empty((self.n, 3))
         _abi.check(_abi.lib().hg_get_accelerations(self._h, _abi.dptr(a), _abi.dptr(al)))
         out["a"], out["alpha"] = a, al
         return out
@@ -412,7 +412,7 @@ class Pool:
 
     def state(self, slot):
         n = self.info(slot)[0]
-        arrs = [np.zeros((n, 3)) for _ in range(6)]
+        arrs = [np.empty((n, 3)) for _ in range(6)]
         _abi.check(_abi.lib().hg_pool_get_state(self._h, slot, *[_abi.dptr(a) for a in arrs[:4]]))
         _abi.check(_abi.lib().hg_pool_get_accelerations(self._h, slot, _abi.dptr(arrs[4]), _abi.dptr(arrs[5])))
         return dict(zip(("x", "v", "theta", "omega", "a", "alpha"), arrs))

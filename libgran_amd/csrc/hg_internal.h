@@ -98,6 +98,48 @@ struct sys_view {
     double *diss = nullptr;  // dissipated work, 4 per particle (when tracked)
 };
 
+// slot: the system's own index, naming its fault word in pool_view::sflags.
+struct pool_meta {
+    uint32_t offset, n, cur, acc_valid, nf, rebuild, slot, pad1;
+};
+
+// Cell-list scratch and the lists it builds (launch_cell_lists), for the
+// particles [0, count) of an array of row stride `stride`.
+struct cell_rec {  // a binned particle: its position, index and system in one 32-byte read
+    double x, y, z;
+    uint32_t j, slot;
+};
+struct list_build {
+    const double *x;
+    // null, or a particle whose position the cells are laid from: a system far
+    // from the origin keeps exact cell coordinates (its positions' differences
+    // are exact where their quotients by a cell are not)
+    const double *origin;
+    uint32_t count;
+    size_t stride;
+    double r_verlet;
+    // owner[g]: the particle's system (kNoEntry: none); meta: the systems,
+    // of which those with `rebuild` set are listed. Both null: one system.
+    const uint32_t *owner;
+    const pool_meta *meta;
+    uint32_t hash_size;               // a power of two
+    uint32_t *buckets;                // 2 * hash_size words: counts, then fill positions
+    uint32_t *bucket_start, *scan_tmp;
+    uint32_t *cell_of;                // count words
+    cell_rec *recs;                   // count records
+    uint32_t *nb, *ncnt;              // slot k of particle g at nb[k * stride + g]
+    uint32_t cap;
+    int *flags, *sflags;              // sflags: per-system fault words, may be null
+};
+hipError_t launch_cell_lists(const list_build &B, hipStream_t s);
+
+// Pinned host memory that read-backs go through (read_fields).
+struct host_stage {
+    double *p = nullptr;
+    size_t cap = 0;  // doubles
+    ~host_stage();
+};
+
 struct hg_system_impl {
     hg_params p{};
     size_t n = 0;
@@ -128,9 +170,8 @@ struct hg_system_impl {
     uint32_t *nb = nullptr, *ncnt = nullptr;
     // cell-list scratch
     uint32_t hash_size = 0;
-    uint32_t *cell_of = nullptr, *bucket_count = nullptr, *bucket_start = nullptr, *bucket_fill = nullptr,
-             *cell_items = nullptr, *scan_tmp = nullptr;
-    double *bbox = nullptr;  // lo[3], hi[3]
+    uint32_t *cell_of = nullptr, *buckets = nullptr, *bucket_start = nullptr, *scan_tmp = nullptr;
+    cell_rec *cell_recs = nullptr;
     // facets
     int nf = 0;
     facet_dev *facets = nullptr;
@@ -138,6 +179,7 @@ struct hg_system_impl {
     // flags
     int *flags = nullptr;
     int *flags_host = nullptr;  // pinned
+    host_stage stage;
     // reductions
     double *red = nullptr;
     double *energy = nullptr;  // per-particle ledger terms, 8 per particle (allocated on first use)
@@ -194,6 +236,8 @@ hipError_t launch_kick_drift(double *x, double *v, double *th, double *w, const 
 hipError_t launch_final_kick(double *v, double *w, const double *a, const double *al, uint32_t n, double half,
                              facet_dev *facets, int nf, double facet_dt, int *flags, hipStream_t s);
 hipError_t launch_neighbor_build(hg_system_impl &S, hipStream_t s);
+// Systems of at most this many particles list every pair by brute force.
+constexpr uint32_t kBruteListMax = 8192;
 hipError_t launch_advance_facet(facet_dev *f, const double *v, double dt, hipStream_t s);
 // nsteps steps of a small FP64 system in one workgroup; `even`/`odd` are the
 // views whose pair-state tables the even/odd steps read. Systems of at most
@@ -217,6 +261,19 @@ hipError_t launch_legacy_move(const double *x, const double *v, const double *w,
 // Exclusive scan of count words; tmp holds scan_tmp_words(count) words.
 hipError_t launch_exclusive_scan(const uint32_t *in, uint32_t *out, uint32_t count, uint32_t *tmp, hipStream_t s);
 uint32_t scan_tmp_words(uint32_t count);
+// Copies `count` words by a kernel, e.g. into pinned host memory: a copy
+// command of a few bytes takes several times as long.
+hipError_t launch_copy_words(const int *src, int *dst, int count, hipStream_t s);
+// The first three components of n 4-double records of each of `count` <= 4
+// arrays, one array's n triples after the other's, into `out` (pinned host
+// memory).
+hipError_t launch_pack3(const double *const *src, int count, size_t n, double *out, hipStream_t s);
+// Reads back the n particles of `count` <= 4 fields as triples (a null dst
+// skips a field): one kernel that packs them into pinned memory and one wait,
+// where a copy command and a wait per field took 25 us each. Large n goes
+// through the stage in parts.
+hg_status read_fields(host_stage &stage, const double *const *src, double *const *dst, int count, size_t n,
+                      hipStream_t s);
 hipError_t launch_zero_u32(uint32_t *p, size_t count, hipStream_t s);
 hipError_t launch_zero_f64(double *p, size_t count, hipStream_t s);
 hipError_t launch_diagnostics(const double *x, const double *v, const double *w, uint32_t n, double mass,

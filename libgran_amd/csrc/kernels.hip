@@ -258,58 +258,21 @@ __global__ void k_zero_f64(double *p, size_t count) {
         p[k] = 0.0;
 }
 
+__global__ void __launch_bounds__(64) k_copy_words(const int *src, int *dst, int count) {
+    for (int k = int(threadIdx.x); k < count; k += 64) dst[k] = src[k];
+}
+
+// Bound by the link to the host: consecutive lanes write consecutive words.
+struct pack_src {
+    const double *f[4];
+};
+__global__ void __launch_bounds__(256) k_pack3(pack_src F, size_t words, double *out) {
+    const double *src = F.f[blockIdx.y];
+    for (size_t q = blockIdx.x * size_t(blockDim.x) + threadIdx.x; q < words; q += size_t(gridDim.x) * blockDim.x)
+        out[blockIdx.y * words + q] = src[q / 3 * 4 + q % 3];
+}
+
 // ---------------------------------------------------- neighbour rebuild -----
-// Single-block bounding box of the positions: bbox = lo[3], hi[3].
-__global__ void __launch_bounds__(1024) k_bbox(const double *x, uint32_t n, double *bbox) {
-    __shared__ double red[6][1024];
-    double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
-    for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) {
-        d3 q = ld3(x, i);
-        lo[0] = fmin(lo[0], q.x); lo[1] = fmin(lo[1], q.y); lo[2] = fmin(lo[2], q.z);
-        hi[0] = fmax(hi[0], q.x); hi[1] = fmax(hi[1], q.y); hi[2] = fmax(hi[2], q.z);
-    }
-    for (int c = 0; c < 3; c++) {
-        red[c][threadIdx.x] = lo[c];
-        red[3 + c][threadIdx.x] = hi[c];
-    }
-    __syncthreads();
-    for (uint32_t s = blockDim.x / 2; s > 0; s >>= 1) {
-        if (threadIdx.x < s)
-            for (int c = 0; c < 3; c++) {
-                red[c][threadIdx.x] = fmin(red[c][threadIdx.x], red[c][threadIdx.x + s]);
-                red[3 + c][threadIdx.x] = fmax(red[3 + c][threadIdx.x], red[3 + c][threadIdx.x + s]);
-            }
-        __syncthreads();
-    }
-    if (threadIdx.x < 6) bbox[threadIdx.x] = red[threadIdx.x][0];
-}
-
-__device__ __forceinline__ uint32_t cell_hash(long long cx, long long cy, long long cz, uint32_t mask) {
-    uint64_t h = uint64_t(cx) * 73856093ull ^ uint64_t(cy) * 19349663ull ^ uint64_t(cz) * 83492791ull;
-    h ^= h >> 29;
-    h *= 0xbf58476d1ce4e5b9ull;
-    h ^= h >> 32;
-    return uint32_t(h) & mask;
-}
-
-__device__ __forceinline__ void cell_coords(d3 q, const double *bbox, double cs, long long &cx, long long &cy,
-                                            long long &cz) {
-    cx = (long long)((q.x - bbox[0]) / cs);
-    cy = (long long)((q.y - bbox[1]) / cs);
-    cz = (long long)((q.z - bbox[2]) / cs);
-}
-
-__global__ void __launch_bounds__(256) k_cell_count(const double *x, uint32_t n, const double *bbox, double cs,
-                                                    uint32_t mask, uint32_t *cell_of, uint32_t *bucket_count) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    long long cx, cy, cz;
-    cell_coords(ld3(x, i), bbox, cs, cx, cy, cz);
-    const uint32_t h = cell_hash(cx, cy, cz, mask);
-    cell_of[i] = h;
-    atomicAdd(&bucket_count[h], 1u);
-}
-
 // Exclusive scan in three launches: per-block scan of kScanChunk words with
 // block totals, a single-block scan of the totals, then the offsets added.
 constexpr uint32_t kScanThreads = 256, kScanPer = 8, kScanChunk = kScanThreads * kScanPer;
@@ -367,62 +330,210 @@ __global__ void __launch_bounds__(kScanThreads) k_scan_add(uint32_t *out, uint32
     for (uint32_t k = threadIdx.x; k < kScanChunk && base + k < count; k += blockDim.x) out[base + k] += add;
 }
 
-__global__ void __launch_bounds__(256) k_cell_fill(uint32_t n, const uint32_t *cell_of, const uint32_t *bucket_start,
-                                                   uint32_t *bucket_fill, uint32_t *cell_items) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const uint32_t h = cell_of[i];
-    cell_items[bucket_start[h] + atomicAdd(&bucket_fill[h], 1u)] = i;
+__device__ __forceinline__ uint32_t cell_hash(uint32_t slot, long long cx, long long cy, long long cz, uint32_t mask) {
+    uint64_t h = uint64_t(cx) * 73856093ull ^ uint64_t(cy) * 19349663ull ^ uint64_t(cz) * 83492791ull ^
+                 uint64_t(slot) * 2654435761ull;
+    h ^= h >> 29;
+    h *= 0xbf58476d1ce4e5b9ull;
+    h ^= h >> 32;
+    return uint32_t(h) & mask;
 }
 
-// Per particle: the 27 surrounding cells' buckets (deduplicated, since two
-// cells may share a bucket), candidates filtered by the reference predicate
-// norm(x_i - x_j) < r_verlet, inserted in ascending j.
-__global__ void __launch_bounds__(256) k_nl_fill(const double *x, uint32_t n, const double *bbox, double cs,
-                                                 uint32_t mask, double r_verlet, const uint32_t *bucket_count,
-                                                 const uint32_t *bucket_start, const uint32_t *cell_items,
-                                                 uint32_t *nb, uint32_t *ncnt, uint32_t cap, int *flags) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const d3 xi = ld3(x, i);
-    long long cx, cy, cz;
-    cell_coords(xi, bbox, cs, cx, cy, cz);
-    uint32_t seen[27];
-    int nseen = 0;
-    uint32_t cnt = 0;
-    for (int dz = -1; dz <= 1; dz++)
-        for (int dy = -1; dy <= 1; dy++)
-            for (int dx = -1; dx <= 1; dx++) {
-                const uint32_t h = cell_hash(cx + dx, cy + dy, cz + dz, mask);
-                bool dup = false;
-                for (int s = 0; s < nseen; s++) dup |= seen[s] == h;
-                if (dup) continue;
-                seen[nseen++] = h;
-                const uint32_t b = bucket_start[h], e = b + bucket_count[h];
-                for (uint32_t q = b; q < e; q++) {
-                    const uint32_t j = cell_items[q];
-                    if (j == i) continue;
-                    if (norm(xi - ld3(x, j)) < r_verlet) {
-                        if (cnt < cap) {
-                            // insertion into the ascending slot list
-                            uint32_t pos = cnt;
-                            while (pos > 0) {
-                                const uint32_t prev = nb[size_t(pos - 1) * n + i];
-                                if (prev < j) break;
-                                nb[size_t(pos) * n + i] = prev;
-                                pos--;
-                            }
-                            nb[size_t(pos) * n + i] = j;
-                        }
-                        cnt++;
-                    }
-                }
-            }
-    ncnt[i] = cnt < cap ? cnt : cap;
-    if (cnt > cap) {
-        atomicOr(&flags[FLAG_NL_OVERFLOW], 1);
-        atomicMax(&flags[FLAG_NL_MAXCOUNT], int(cnt));
+__device__ __forceinline__ d3 cell_origin(const list_build &B) {
+    if (!B.origin) return zero3();
+    const d3 o = ld3(B.origin, 0);
+    return nonfinite(o, o) ? zero3() : o;
+}
+
+__device__ __forceinline__ void cell_coords(d3 q, double cs, long long &cx, long long &cy, long long &cz) {
+    cx = (long long)floor(q.x / cs);
+    cy = (long long)floor(q.y / cs);
+    cz = (long long)floor(q.z / cs);
+}
+
+__global__ void __launch_bounds__(256) k_cell_count(list_build B, double cs) {
+    const uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
+    if (g >= B.count) return;
+    const uint32_t slot = B.owner ? B.owner[g] : 0u;
+    if (slot == kNoEntry || (B.meta && !B.meta[slot].rebuild)) {
+        B.cell_of[g] = kNoEntry;
+        return;
     }
+    long long cx, cy, cz;
+    cell_coords(ld3(B.x, g) - cell_origin(B), cs, cx, cy, cz);
+    const uint32_t h = cell_hash(slot, cx, cy, cz, B.hash_size - 1);
+    B.cell_of[g] = h;
+    atomicAdd(&B.buckets[h], 1u);
+}
+
+__global__ void __launch_bounds__(256) k_cell_fill(list_build B) {
+    const uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
+    if (g >= B.count) return;
+    const uint32_t h = B.cell_of[g];
+    if (h == kNoEntry) return;
+    const d3 p = ld3(B.x, g);
+    B.recs[B.bucket_start[h] + atomicAdd(&B.buckets[B.hash_size + h], 1u)] =
+        cell_rec{p.x, p.y, p.z, g, B.owner ? B.owner[g] : 0u};
+}
+
+// The reference predicate norm(x_i - x_j) < r_verlet behind a squared-distance
+// prefilter: a correctly rounded sqrt(d2) < r_verlet implies d2 < r_verlet^2
+// (1 + 2^-52), so this bound drops no pair the exact test keeps.
+struct in_range {
+    double r, d2_max;
+    __device__ __forceinline__ in_range(double r_verlet) : r(r_verlet), d2_max(r_verlet * r_verlet * (1.0 + 1e-12)) {}
+    __device__ __forceinline__ bool operator()(d3 d) const { return dot(d, d) < d2_max && norm(d) < r; }
+};
+
+__device__ __forceinline__ void close_list(const list_build &B, uint32_t g, uint32_t slot, uint32_t cnt) {
+    B.ncnt[g] = cnt < B.cap ? cnt : B.cap;
+    if (cnt > B.cap) {
+        atomicOr(&B.flags[FLAG_NL_OVERFLOW], 1);
+        atomicMax(&B.flags[FLAG_NL_MAXCOUNT], int(cnt));
+        if (B.sflags) atomicOr(&B.sflags[slot], HG_FAULT_NEIGHBOR_CAPACITY);
+    }
+}
+
+// Lists from the cell records, eight lanes a particle. Cells are twice the
+// list radius wide, so a partner lies in the particle's own cell or the
+// neighbour on the side of the half the particle sits in, along each axis: 2 x
+// 2 x 2 cells, one for each lane. (In cell units a partner is less than 0.5 (1
+// - 1e-9) away; a particle in the lower half, u - floor(u) < 0.5, has its
+// partners in floor(u) - 1 .. floor(u), one in the upper half in floor(u) ..
+// floor(u) + 1.) The matches go to LDS and from there to their rank among
+// them, so the list ascends. One lane walking all eight buckets took 104 us at
+// 20,000 particles, each bucket a chain of dependent reads.
+constexpr uint32_t kListLanes = 8, kListParts = 256 / kListLanes, kListMost = 96, kRecBatch = 4;
+__global__ void __launch_bounds__(256) k_list_fill(list_build B, double cs) {
+    __shared__ uint32_t s_cnt[kListParts];
+    __shared__ uint32_t s_list[kListParts][kListMost];
+    const uint32_t lane = threadIdx.x % kListLanes, p = threadIdx.x / kListLanes;
+    const uint32_t g = blockIdx.x * kListParts + p;
+    const bool on = g < B.count && B.cell_of[g] != kNoEntry;
+    if (lane == 0) s_cnt[p] = 0;
+    __syncthreads();
+    const uint32_t slot = on && B.owner ? B.owner[g] : 0u;
+    const d3 xi = on ? ld3(B.x, g) : zero3();
+    const in_range near(B.r_verlet);
+    long long bx, by, bz;
+    const d3 u = xi - cell_origin(B);
+    cell_coords(u, cs, bx, by, bz);
+    bx -= u.x / cs - double(bx) < 0.5 ? 1 : 0;
+    by -= u.y / cs - double(by) < 0.5 ? 1 : 0;
+    bz -= u.z / cs - double(bz) < 0.5 ? 1 : 0;
+    // calls match(j) for every partner in the bucket of cell c of the eight
+    auto scan = [&](uint32_t h, auto &&match) {
+        const uint32_t b = B.bucket_start[h], e = b + B.buckets[h];
+        for (uint32_t q = b; q < e; q += kRecBatch) {
+            // records loaded together (the last one again past the end) overlap
+            cell_rec c[kRecBatch];
+#pragma unroll
+            for (uint32_t k = 0; k < kRecBatch; k++) c[k] = B.recs[q + k < e ? q + k : e - 1];
+#pragma unroll
+            for (uint32_t k = 0; k < kRecBatch; k++)
+                if (q + k < e && c[k].j != g && c[k].slot == slot && near(xi - d3{c[k].x, c[k].y, c[k].z}))
+                    match(c[k].j);
+        }
+    };
+    auto hash_of = [&](uint32_t c) {
+        return cell_hash(slot, bx + (c & 1), by + (c >> 1 & 1), bz + (c >> 2), B.hash_size - 1);
+    };
+    const uint32_t h = hash_of(lane);
+    bool dup = false;  // a bucket shared by two of the cells is scanned once
+    for (uint32_t c = 0; c < kListLanes - 1; c++) {
+        const uint32_t hc = uint32_t(__shfl(int(h), int(c), int(kListLanes)));
+        dup |= c < lane && hc == h;
+    }
+    if (on && !dup)
+        scan(h, [&](uint32_t j) {
+            const uint32_t at = atomicAdd(&s_cnt[p], 1u);
+            if (at < kListMost) s_list[p][at] = j;
+        });
+    __syncthreads();
+    if (!on) return;
+    const uint32_t cnt = s_cnt[p];
+    if (cnt <= kListMost) {
+        for (uint32_t e = lane; e < cnt; e += kListLanes) {
+            const uint32_t j = s_list[p][e];
+            uint32_t rank = 0;
+            for (uint32_t f = 0; f < cnt; f++) rank += s_list[p][f] < j ? 1u : 0u;
+            if (rank < B.cap) B.nb[size_t(rank) * B.stride + g] = j;
+        }
+    } else if (lane == 0) {
+        // a list longer than the LDS row: by insertion, one lane
+        uint32_t n = 0;
+        for (uint32_t c = 0; c < kListLanes; c++) {
+            const uint32_t hc = hash_of(c);
+            bool seen = false;
+            for (uint32_t q = 0; q < c; q++) seen |= hash_of(q) == hc;
+            if (seen) continue;
+            scan(hc, [&](uint32_t j) {
+                uint32_t pos = n < B.cap ? n : B.cap;
+                if (pos == B.cap) {  // full: j displaces the largest kept one, or is dropped
+                    if (B.cap == 0 || B.nb[size_t(B.cap - 1) * B.stride + g] < j) {
+                        n++;
+                        return;
+                    }
+                    pos--;
+                }
+                while (pos > 0 && B.nb[size_t(pos - 1) * B.stride + g] > j) {
+                    B.nb[size_t(pos) * B.stride + g] = B.nb[size_t(pos - 1) * B.stride + g];
+                    pos--;
+                }
+                B.nb[size_t(pos) * B.stride + g] = j;
+                n++;
+            });
+        }
+    }
+    if (lane == 0) close_list(B, g, slot, cnt);
+}
+
+// Every pair tested: one launch instead of the cell list's seven, whose
+// latency a small system pays in full. A wavefront lists four particles, 64
+// candidates at a time from LDS; the ballot gives each match its place, in
+// ascending order. Work grows with n^2 and is hidden behind the cell list's
+// launches up to kBruteListMax.
+constexpr uint32_t kBruteEach = 4, kBruteParts = 4 * kBruteEach;
+__global__ void __launch_bounds__(256) k_list_brute(list_build B) {
+    __shared__ double sx[3][256];
+    const uint32_t lane = threadIdx.x & 63u, first = blockIdx.x * kBruteParts + (threadIdx.x >> 6) * kBruteEach;
+    const in_range near(B.r_verlet);
+    d3 xi[kBruteEach];
+    uint32_t cnt[kBruteEach];
+#pragma unroll
+    for (uint32_t q = 0; q < kBruteEach; q++) {
+        xi[q] = first + q < B.count ? ld3(B.x, first + q) : zero3();
+        cnt[q] = 0;
+    }
+    for (uint32_t base = 0; base < B.count; base += 256) {
+        __syncthreads();
+        if (base + threadIdx.x < B.count) {
+            const d3 a = ld3(B.x, base + threadIdx.x);
+            sx[0][threadIdx.x] = a.x;
+            sx[1][threadIdx.x] = a.y;
+            sx[2][threadIdx.x] = a.z;
+        }
+        __syncthreads();
+        for (uint32_t t = lane; t < 256u && base + t - lane < B.count; t += 64) {
+            const uint32_t j = base + t;
+            const bool live = j < B.count;
+            const d3 xj = live ? d3{sx[0][t], sx[1][t], sx[2][t]} : zero3();
+#pragma unroll
+            for (uint32_t q = 0; q < kBruteEach; q++) {
+                const uint32_t i = first + q;
+                const bool hit = live && i < B.count && j != i && near(xi[q] - xj);
+                const uint64_t m = __ballot(hit);
+                if (hit) {
+                    const uint32_t at = cnt[q] + uint32_t(__popcll(m & ((1ull << lane) - 1ull)));
+                    if (at < B.cap) B.nb[size_t(at) * B.stride + i] = j;
+                }
+                cnt[q] += uint32_t(__popcll(m));
+            }
+        }
+    }
+#pragma unroll
+    for (uint32_t q = 0; q < kBruteEach; q++)
+        if (lane == 0 && first + q < B.count) close_list(B, first + q, 0, cnt[q]);
 }
 
 // ---------------------------------------------------------- diagnostics -----
@@ -829,6 +940,20 @@ hipError_t launch_zero_u32(uint32_t *p, size_t count, hipStream_t s) {
     return hipGetLastError();
 }
 
+hipError_t launch_copy_words(const int *src, int *dst, int count, hipStream_t s) {
+    k_copy_words<<<1, 64, 0, s>>>(src, dst, count);
+    return hipGetLastError();
+}
+
+hipError_t launch_pack3(const double *const *src, int count, size_t n, double *out, hipStream_t s) {
+    if (count == 0 || n == 0) return hipSuccess;
+    pack_src F{};
+    for (int k = 0; k < count; k++) F.f[k] = src[k];
+    const unsigned nb = unsigned(std::min<size_t>(512, (3 * n + 255) / 256));
+    k_pack3<<<dim3(nb, unsigned(count)), 256, 0, s>>>(F, 3 * n, out);
+    return hipGetLastError();
+}
+
 hipError_t launch_zero_f64(double *p, size_t count, hipStream_t s) {
     if (count == 0) return hipSuccess;
     unsigned nb = unsigned(std::min<size_t>(1024, (count + 255) / 256));
@@ -847,21 +972,26 @@ hipError_t launch_exclusive_scan(const uint32_t *in, uint32_t *out, uint32_t cou
 
 uint32_t scan_tmp_words(uint32_t count) { return (count + kScanChunk - 1) / kScanChunk + 1; }
 
+hipError_t launch_cell_lists(const list_build &B, hipStream_t s) {
+    if (B.count == 0) return hipSuccess;
+    const double cs = 2.0 * B.r_verlet * (1.0 + 1e-9);  // two list radii: 2 x 2 x 2 cells per particle
+    hipError_t e;
+    if ((e = launch_zero_u32(B.buckets, size_t(2) * B.hash_size, s)) != hipSuccess) return e;
+    k_cell_count<<<blocks_for(B.count, 256), 256, 0, s>>>(B, cs);
+    if ((e = launch_exclusive_scan(B.buckets, B.bucket_start, B.hash_size, B.scan_tmp, s)) != hipSuccess) return e;
+    k_cell_fill<<<blocks_for(B.count, 256), 256, 0, s>>>(B);
+    k_list_fill<<<blocks_for(B.count, kListParts), 256, 0, s>>>(B, cs);
+    return hipGetLastError();
+}
+
 hipError_t launch_neighbor_build(hg_system_impl &S, hipStream_t s) {
     const uint32_t n = uint32_t(S.n);
     if (n == 0) return hipSuccess;
-    const double cs = S.p.r_verlet * (1.0 + 1e-9);
-    const uint32_t mask = S.hash_size - 1;
-    hipError_t e;
-    if ((e = launch_zero_u32(S.bucket_count, S.hash_size, s)) != hipSuccess) return e;
-    if ((e = launch_zero_u32(S.bucket_fill, S.hash_size, s)) != hipSuccess) return e;
-    k_bbox<<<1, 1024, 0, s>>>(S.x, n, S.bbox);
-    k_cell_count<<<blocks_for(n, 256), 256, 0, s>>>(S.x, n, S.bbox, cs, mask, S.cell_of, S.bucket_count);
-    if ((e = launch_exclusive_scan(S.bucket_count, S.bucket_start, S.hash_size, S.scan_tmp, s)) != hipSuccess)
-        return e;
-    k_cell_fill<<<blocks_for(n, 256), 256, 0, s>>>(n, S.cell_of, S.bucket_start, S.bucket_fill, S.cell_items);
-    k_nl_fill<<<blocks_for(n, 64), 64, 0, s>>>(S.x, n, S.bbox, cs, mask, S.p.r_verlet, S.bucket_count,
-                                               S.bucket_start, S.cell_items, S.nb, S.ncnt, S.cap_n, S.flags);
+    const list_build B{S.x,       S.x,    n,            S.n,        S.p.r_verlet, nullptr,     nullptr,
+                       S.hash_size, S.buckets, S.bucket_start, S.scan_tmp, S.cell_of,  S.cell_recs, S.nb,
+                       S.ncnt,      S.cap_n,   S.flags,        nullptr};
+    if (n > kBruteListMax) return launch_cell_lists(B, s);
+    k_list_brute<<<blocks_for(n, kBruteParts), 256, 0, s>>>(B);
     return hipGetLastError();
 }
 

@@ -65,162 +65,6 @@ __global__ void __launch_bounds__(64) k_energy_sum(const double *terms, uint32_t
     }
 }
 
-// ------------------------------------------------------ batched rebuild -----
-__device__ __forceinline__ uint32_t pool_hash(uint32_t slot, long long cx, long long cy, long long cz, uint32_t mask) {
-    uint64_t h = uint64_t(cx) * 73856093ull ^ uint64_t(cy) * 19349663ull ^ uint64_t(cz) * 83492791ull ^
-                 uint64_t(slot) * 2654435761ull;
-    h ^= h >> 29;
-    h *= 0xbf58476d1ce4e5b9ull;
-    h ^= h >> 32;
-    return uint32_t(h) & mask;
-}
-
-__device__ __forceinline__ void pool_cell(d3 q, double cs, long long &cx, long long &cy, long long &cz) {
-    cx = (long long)floor(q.x / cs);
-    cy = (long long)floor(q.y / cs);
-    cz = (long long)floor(q.z / cs);
-}
-
-__global__ void __launch_bounds__(256) k_pool_cell_count(const double *x, const uint32_t *owner, const pool_meta *meta,
-                                                         uint32_t hw, double cs, uint32_t mask, uint32_t *cell_of,
-                                                         uint32_t *bucket_count) {
-    const uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= hw) return;
-    const uint32_t slot = owner[g];
-    if (slot == kNoEntry || !meta[slot].rebuild) {
-        cell_of[g] = kNoEntry;
-        return;
-    }
-    long long cx, cy, cz;
-    pool_cell(ld3(x, g), cs, cx, cy, cz);
-    const uint32_t h = pool_hash(slot, cx, cy, cz, mask);
-    cell_of[g] = h;
-    atomicAdd(&bucket_count[h], 1u);
-}
-
-// A binned particle as the list fill reads it: its position, index and
-// system in one 32-byte record, so that a bucket's candidates are one
-// contiguous read each rather than an index followed by two gathers.
-struct cell_rec {
-    double x, y, z;
-    uint32_t j, slot;
-};
-
-__global__ void __launch_bounds__(256) k_pool_cell_fill(const double *x, const uint32_t *owner, uint32_t hw,
-                                                        const uint32_t *cell_of, const uint32_t *bucket_start,
-                                                        uint32_t *bucket_fill, cell_rec *recs) {
-    const uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= hw) return;
-    const uint32_t h = cell_of[g];
-    if (h == kNoEntry) return;
-    const d3 p = ld3(x, g);
-    recs[bucket_start[h] + atomicAdd(&bucket_fill[h], 1u)] = cell_rec{p.x, p.y, p.z, g, owner[g]};
-}
-
-constexpr uint32_t kListRegs = 16;
-constexpr uint32_t kRecBatch = 4;
-__global__ void __launch_bounds__(256) k_pool_nl_fill(const double *x, const uint32_t *owner, const uint32_t *cell_of,
-                                                      uint32_t hw, double cs, uint32_t mask, double r_verlet,
-                                                      const uint32_t *bucket_count, const uint32_t *bucket_start,
-                                                      const cell_rec *recs, uint32_t *nb, uint32_t *ncnt,
-                                                      size_t stride, uint32_t cap, int *flags, int *sflags) {
-    const uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= hw || cell_of[g] == kNoEntry) return;
-    const uint32_t slot = owner[g];
-    const d3 xi = ld3(x, g);
-    long long cx, cy, cz;
-    pool_cell(xi, cs, cx, cy, cz);
-    // squared-distance prefilter: a correctly rounded sqrt(d2) < r_verlet
-    // implies d2 < r_verlet^2 (1 + 2^-52), so this bound drops no pair the
-    // exact test keeps
-    const double d2_max = r_verlet * r_verlet * (1.0 + 1e-12);
-    // The list is kept sorted in registers (indices fixed at compile time,
-    // so no scratch memory) while it has at most kListRegs entries, and in
-    // nb itself by insertion once it grows past that.
-    uint32_t r[kListRegs];
-#pragma unroll
-    for (uint32_t s = 0; s < kListRegs; s++) r[s] = 0;
-    uint32_t cnt = 0;
-    bool spilled = false;
-    auto insert = [&](uint32_t j) {
-        if (!spilled && cnt == kListRegs) {
-#pragma unroll
-            for (uint32_t s = 0; s < kListRegs; s++)
-                if (s < cap) nb[size_t(s) * stride + g] = r[s];
-            spilled = true;
-        }
-        if (spilled) {
-            if (cnt < cap) {
-                uint32_t pos = cnt;
-                while (pos > 0) {
-                    const uint32_t prev = nb[size_t(pos - 1) * stride + g];
-                    if (prev < j) break;
-                    nb[size_t(pos) * stride + g] = prev;
-                    pos--;
-                }
-                nb[size_t(pos) * stride + g] = j;
-            }
-        } else {
-            uint32_t pos = 0;
-#pragma unroll
-            for (uint32_t s = 0; s < kListRegs; s++) pos += (s < cnt && r[s] < j) ? 1u : 0u;
-#pragma unroll
-            for (uint32_t s = kListRegs - 1; s >= 1; s--) r[s] = s > pos ? r[s - 1] : (s == pos ? j : r[s]);
-            r[0] = pos == 0 ? j : r[0];
-        }
-        cnt++;
-    };
-    // Cells are twice the list radius wide, so a partner lies in the
-    // particle's own cell or the neighbour on the side of the half the
-    // particle sits in, along each axis: 2 x 2 x 2 cells. (In cell units a
-    // partner is less than 0.5 (1 - 1e-9) away; a particle in the lower half,
-    // u - floor(u) < 0.5, has its partners in floor(u) - 1 .. floor(u), one in
-    // the upper half in floor(u) .. floor(u) + 1.) The cells are unrolled, so
-    // the hashes already visited (a bucket shared by two cells is scanned
-    // once) sit in registers too.
-    const long long bx = cx - (xi.x / cs - double(cx) < 0.5 ? 1 : 0);
-    const long long by = cy - (xi.y / cs - double(cy) < 0.5 ? 1 : 0);
-    const long long bz = cz - (xi.z / cs - double(cz) < 0.5 ? 1 : 0);
-    uint32_t seen[8];
-#pragma unroll
-    for (int c = 0; c < 8; c++) {
-        const uint32_t h = pool_hash(slot, bx + (c & 1), by + (c >> 1 & 1), bz + (c >> 2), mask);
-        seen[c] = h;
-        bool dup = false;
-#pragma unroll
-        for (int s = 0; s < c; s++) dup |= seen[s] == h;
-        if (dup) continue;
-        const uint32_t b = bucket_start[h], e = b + bucket_count[h];
-        // kRecBatch records loaded together (the last one again past the
-        // end), then tested in bucket order: the loads overlap one another
-        // instead of each waiting for the previous test
-        for (uint32_t q = b; q < e; q += kRecBatch) {
-            cell_rec c[kRecBatch];
-#pragma unroll
-            for (uint32_t k = 0; k < kRecBatch; k++) c[k] = recs[q + k < e ? q + k : e - 1];
-#pragma unroll
-            for (uint32_t k = 0; k < kRecBatch; k++) {
-                const uint32_t j = c[k].j;
-                if (q + k >= e || j == g || c[k].slot != slot) continue;
-                const d3 d = xi - d3{c[k].x, c[k].y, c[k].z};
-                if (!(dot(d, d) < d2_max)) continue;
-                if (norm(d) < r_verlet) insert(j);
-            }
-        }
-    }
-    if (!spilled) {
-#pragma unroll
-        for (uint32_t s = 0; s < kListRegs; s++)
-            if (s < cnt && s < cap) nb[size_t(s) * stride + g] = r[s];
-    }
-    ncnt[g] = cnt < cap ? cnt : cap;
-    if (cnt > cap) {
-        atomicOr(&flags[FLAG_NL_OVERFLOW], 1);
-        atomicMax(&flags[FLAG_NL_MAXCOUNT], int(cnt));
-        atomicOr(&sflags[slot], HG_FAULT_NEIGHBOR_CAPACITY);
-    }
-}
-
 // Zeroes `rows` strided rows [offset, offset+n) of an array with row stride.
 __global__ void k_zero_rows_f64(double *p, size_t stride, size_t offset, size_t n, uint32_t rows) {
     const size_t total = rows * n;
@@ -335,10 +179,10 @@ struct hg_pool {
     uint64_t last_wide_launches = 0;
     bool order_dirty = true;
     bool meta_dirty = true;
-    uint32_t hash_size = 0, *cell_of = nullptr, *bucket_count = nullptr, *bucket_start = nullptr,
-             *bucket_fill = nullptr, *scan_tmp = nullptr;
+    uint32_t hash_size = 0, *cell_of = nullptr, *buckets = nullptr, *bucket_start = nullptr, *scan_tmp = nullptr;
     cell_rec *cell_recs = nullptr;
     int *flags = nullptr, *flags_host = nullptr;
+    host_stage stage;
     // per-system fault words set by the kernels (device, cleared after every
     // read) and the faults recorded so far (host, per slot)
     int *sflags = nullptr, *sflags_host = nullptr;
@@ -403,13 +247,12 @@ uint32_t pool_cap_s(const hg_params &p) {
     return std::max<uint32_t>(p.pair_capacity ? p.pair_capacity : 24u, kTagPrefetch);
 }
 
-// Reads the flag words of the launches queued so far. When one is raised, the
+// Looks at the flag words that pool_begin copied back after its launches (the
+// stream has been waited for). When one is raised, the
 // per-system fault words say which systems tripped it: they are added to
 // Q->fault (those systems are no longer stepped) and pushed onto `faulted`,
 // and both the flags and the fault words are cleared on the device.
 hg_status collect_faults(hg_pool *Q, std::vector<int32_t> &faulted) {
-    HG_HIP(hipMemcpyAsync(Q->flags_host, Q->flags, FLAG_COUNT * sizeof(int), hipMemcpyDeviceToHost, Q->stream));
-    HG_HIP(hipStreamSynchronize(Q->stream));
     const int *f = Q->flags_host;
     if (!f[FLAG_NL_OVERFLOW] && !f[FLAG_PAIR_OVERFLOW] && !f[FLAG_NUMERIC]) return HG_OK;
     if (f[FLAG_NL_OVERFLOW]) Q->fault_nl_need = std::max(Q->fault_nl_need, f[FLAG_NL_MAXCOUNT]);
@@ -493,21 +336,10 @@ hg_status download_rows(hg_pool *Q, const T *dev, uint32_t offset, uint32_t n, u
 hg_status rebuild_due(hg_pool *Q) {
     const uint32_t hw = Q->high_water;
     if (hw == 0) return HG_OK;
-    const double cs = 2.0 * Q->p.r_verlet * (1.0 + 1e-9);  // two list radii: 2 x 2 x 2 cells per particle
-    const uint32_t mask = Q->hash_size - 1;
-    HG_HIP(launch_zero_u32(Q->bucket_count, Q->hash_size, Q->stream));
-    HG_HIP(launch_zero_u32(Q->bucket_fill, Q->hash_size, Q->stream));
-    k_pool_cell_count<<<nblk(hw, 256), 256, 0, Q->stream>>>(Q->x, Q->owner, Q->meta_d, hw, cs, mask, Q->cell_of,
-                                                           Q->bucket_count);
-    HG_HIP(hipGetLastError());
-    HG_HIP(launch_exclusive_scan(Q->bucket_count, Q->bucket_start, Q->hash_size, Q->scan_tmp, Q->stream));
-    k_pool_cell_fill<<<nblk(hw, 256), 256, 0, Q->stream>>>(Q->x, Q->owner, hw, Q->cell_of, Q->bucket_start,
-                                                          Q->bucket_fill, Q->cell_recs);
-    HG_HIP(hipGetLastError());
-    k_pool_nl_fill<<<nblk(hw, 64), 64, 0, Q->stream>>>(Q->x, Q->owner, Q->cell_of, hw, cs, mask, Q->p.r_verlet,
-                                                      Q->bucket_count, Q->bucket_start, Q->cell_recs, Q->nb,
-                                                      Q->ncnt, Q->P, Q->cap_n, Q->flags, Q->sflags);
-    HG_HIP(hipGetLastError());
+    const list_build B{Q->x,         nullptr,     hw,          Q->P,       Q->p.r_verlet, Q->owner, Q->meta_d, Q->hash_size, Q->buckets,
+                       Q->bucket_start, Q->scan_tmp, Q->cell_of, Q->cell_recs,  Q->nb,    Q->ncnt,   Q->cap_n,     Q->flags,
+                       Q->sflags};
+    HG_HIP(launch_cell_lists(B, Q->stream));
     return HG_OK;
 }
 
@@ -650,9 +482,8 @@ hg_status hg_pool_create(const hg_params *params, size_t max_particles, size_t m
         Q->hash_size = hs;
         PG_TRYC(palloc(Q, &Q->cell_of, P));
         PG_TRYC(palloc(Q, &Q->cell_recs, P));
-        PG_TRYC(palloc(Q, &Q->bucket_count, hs));
+        PG_TRYC(palloc(Q, &Q->buckets, size_t(2) * hs));
         PG_TRYC(palloc(Q, &Q->bucket_start, hs));
-        PG_TRYC(palloc(Q, &Q->bucket_fill, hs));
         PG_TRYC(palloc(Q, &Q->scan_tmp, scan_tmp_words(hs)));
     }
     if (Q->cap_s) {
@@ -934,18 +765,10 @@ hg_status pool_release(hg_pool *Q, int32_t slot, hipStream_t cs) {
 hg_status pool_read_state(hg_pool *Q, int32_t slot, double *x, double *v, double *theta, double *omega,
                           hipStream_t cs) {
     PG_TRY(valid_slot(Q, slot));
-    const uint32_t off = Q->meta[slot].offset, n = Q->meta[slot].n;
-    std::vector<double> buf(4 * size_t(n));
-    const double *src[4] = {Q->x, Q->v, Q->th, Q->w};
+    const size_t off = 4 * size_t(Q->meta[slot].offset);
+    const double *src[4] = {Q->x + off, Q->v + off, Q->th + off, Q->w + off};
     double *dst[4] = {x, v, theta, omega};
-    for (int f = 0; f < 4; f++) {
-        if (!dst[f]) continue;
-        HG_HIP(hipMemcpyAsync(buf.data(), src[f] + 4 * size_t(off), buf.size() * 8, hipMemcpyDeviceToHost, cs));
-        HG_HIP(hipStreamSynchronize(cs));
-        for (uint32_t i = 0; i < n; i++)
-            for (int c = 0; c < 3; c++) dst[f][3 * i + c] = buf[4 * i + c];
-    }
-    return HG_OK;
+    return read_fields(Q->stage, src, dst, 4, Q->meta[slot].n, cs);
 }
 
 hipStream_t pool_copy_stream(hg_pool *Q) { return Q->stream_c; }
@@ -1308,6 +1131,7 @@ hg_status pool_begin(hg_pool *Q, double dt, uint64_t max_len, uint32_t rebuild_e
     }
     if (split) HG_HIP(hipStreamWaitEvent(Q->stream, Q->wev[1], 0));
     HG_HIP(hipEventRecord(Q->evb[1], Q->stream));
+    HG_HIP(launch_copy_words(Q->flags, Q->flags_host, FLAG_COUNT, Q->stream));
     Q->fl.active = true;
     Q->fl.len = len;
     Q->fl.count = count;
@@ -1411,8 +1235,7 @@ hg_status hg_pool_step(hg_pool *Q, double dt, uint64_t nsteps, uint32_t rebuild_
         PG_TRY(pool_end(Q, faulted));
         done += len;
     }
-    PG_TRY(upload_meta(Q));
-    return pool_fault_status(Q, faulted, "hg_pool_step");
+    return pool_fault_status(Q, faulted, "hg_pool_step");  // the next pool_begin uploads the meta
 }
 
 hg_status hg_pool_fault(hg_pool *Q, int32_t slot, int *fault) {
@@ -1497,19 +1320,7 @@ hg_status hg_pool_last_wide_profile(hg_pool *Q, double *wide_ms, uint64_t *launc
 }
 
 hg_status hg_pool_get_state(hg_pool *Q, int32_t slot, double *x, double *v, double *theta, double *omega) {
-    PG_TRY(valid_slot(Q, slot));
-    const uint32_t off = Q->meta[slot].offset, n = Q->meta[slot].n;
-    std::vector<double> buf(4 * size_t(n));
-    const double *src[4] = {Q->x, Q->v, Q->th, Q->w};
-    double *dst[4] = {x, v, theta, omega};
-    for (int f = 0; f < 4; f++) {
-        if (!dst[f]) continue;
-        HG_HIP(hipMemcpyAsync(buf.data(), src[f] + 4 * size_t(off), buf.size() * 8, hipMemcpyDeviceToHost, Q->stream));
-        HG_HIP(hipStreamSynchronize(Q->stream));
-        for (uint32_t i = 0; i < n; i++)
-            for (int c = 0; c < 3; c++) dst[f][3 * i + c] = buf[4 * i + c];
-    }
-    return HG_OK;
+    return pool_read_state(Q, slot, x, v, theta, omega, Q ? Q->stream : nullptr);
 }
 
 hg_status hg_pool_energy(hg_pool *Q, int32_t slot, double mass, double inertia, double *out) {
@@ -1567,18 +1378,10 @@ hg_status hg_pool_energy_noalloc(hg_pool *Q, int32_t slot, double mass, double i
 
 hg_status hg_pool_get_accelerations(hg_pool *Q, int32_t slot, double *a, double *alpha) {
     PG_TRY(valid_slot(Q, slot));
-    const uint32_t off = Q->meta[slot].offset, n = Q->meta[slot].n;
-    std::vector<double> buf(4 * size_t(n));
-    const double *src[2] = {Q->a, Q->al};
+    const size_t off = 4 * size_t(Q->meta[slot].offset);
+    const double *src[2] = {Q->a + off, Q->al + off};
     double *dst[2] = {a, alpha};
-    for (int f = 0; f < 2; f++) {
-        if (!dst[f]) continue;
-        HG_HIP(hipMemcpyAsync(buf.data(), src[f] + 4 * size_t(off), buf.size() * 8, hipMemcpyDeviceToHost, Q->stream));
-        HG_HIP(hipStreamSynchronize(Q->stream));
-        for (uint32_t i = 0; i < n; i++)
-            for (int c = 0; c < 3; c++) dst[f][3 * i + c] = buf[4 * i + c];
-    }
-    return HG_OK;
+    return read_fields(Q->stage, src, dst, 2, Q->meta[slot].n, Q->stream);
 }
 
 hg_status hg_pool_get_neighbors(hg_pool *Q, int32_t slot, uint64_t *offsets, uint32_t *idx, size_t cap,

@@ -12,11 +12,6 @@
 namespace hg {
 
 
-// slot: the system's own index, naming its fault word in pool_view::sflags.
-struct pool_meta {
-    uint32_t offset, n, cur, acc_valid, nf, rebuild, slot, pad1;
-};
-
 struct pool_view {
     double *x, *v, *th, *w, *a, *al;
     const uint32_t *nb;

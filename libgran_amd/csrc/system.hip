@@ -20,6 +20,42 @@ namespace {
 thread_local std::string g_err;
 }
 
+host_stage::~host_stage() {
+    if (p) (void)hipHostFree(p);
+}
+
+hg_status read_fields(host_stage &stage, const double *const *src, double *const *dst, int count, size_t n,
+                      hipStream_t s) {
+    constexpr size_t kMost = size_t(1) << 20;  // doubles: 8 MB
+    const double *from[4];
+    double *to[4];
+    int m = 0;
+    for (int f = 0; f < count; f++)
+        if (dst[f]) {
+            from[m] = src[f];
+            to[m++] = dst[f];
+        }
+    if (m == 0 || n == 0) return HG_OK;
+    const size_t part = std::min(n, kMost / (3 * size_t(m)));
+    if (stage.cap < part * 3 * size_t(m)) {
+        if (stage.p) HG_HIP(hipHostFree(stage.p));
+        stage.p = nullptr;
+        stage.cap = 0;
+        const size_t cap = std::min(std::max<size_t>(part * 12, 1024), kMost);
+        HG_HIP(hipHostMalloc(reinterpret_cast<void **>(&stage.p), cap * sizeof(double)));
+        stage.cap = cap;
+    }
+    for (size_t i = 0; i < n; i += part) {
+        const size_t c = std::min(part, n - i);
+        const double *at[4];
+        for (int f = 0; f < m; f++) at[f] = from[f] + 4 * i;
+        HG_HIP(launch_pack3(at, m, c, stage.p, s));
+        HG_HIP(hipStreamSynchronize(s));
+        for (int f = 0; f < m; f++) std::memcpy(to[f] + 3 * i, stage.p + size_t(f) * 3 * c, 3 * c * sizeof(double));
+    }
+    return HG_OK;
+}
+
 void set_error(const std::string &msg) { g_err = msg; }
 hg_status fail(hg_status st, const std::string &msg) {
     g_err = msg;
@@ -71,16 +107,7 @@ std::vector<double> pack4(const double *src, size_t n) {
 }
 
 hg_status download3(hg_system *S, const double *dev, double *host3) {
-    if (!host3) return HG_OK;
-    std::vector<double> tmp(4 * S->n);
-    HG_HIP(hipMemcpyAsync(tmp.data(), dev, tmp.size() * sizeof(double), hipMemcpyDeviceToHost, S->stream));
-    HG_HIP(hipStreamSynchronize(S->stream));
-    for (size_t i = 0; i < S->n; i++) {
-        host3[3 * i] = tmp[4 * i];
-        host3[3 * i + 1] = tmp[4 * i + 1];
-        host3[3 * i + 2] = tmp[4 * i + 2];
-    }
-    return HG_OK;
+    return read_fields(S->stage, &dev, &host3, 1, S->n, S->stream);
 }
 
 hg_status upload3(hg_system *S, double *dev, const double *host3) {
@@ -137,7 +164,7 @@ hg_status collect_profile(hg_system *S) {
 // Device flags -> status. Clears them for the next call.
 hg_status check_flags(hg_system *S, const char *where) {
     S->flags_unchecked = false;
-    HG_HIP(hipMemcpyAsync(S->flags_host, S->flags, FLAG_COUNT * sizeof(int), hipMemcpyDeviceToHost, S->stream));
+    HG_HIP(launch_copy_words(S->flags, S->flags_host, FLAG_COUNT, S->stream));
     HG_HIP(hipStreamSynchronize(S->stream));
     if (!S->pending.empty()) {
         hg_status st = collect_profile(S);
@@ -480,14 +507,14 @@ hg_status create_impl(const hg_params *params, size_t n, const double *x0, const
         S->cap_n = uint32_t(std::max<uint64_t>(cap, 1));
         HG_TRYC(dalloc(S, &S->nb, size_t(S->cap_n) * n));
         HG_TRYC(dalloc(S, &S->ncnt, n));
-        S->hash_size = next_pow2(std::max<uint64_t>(2 * n, 1024));
-        HG_TRYC(dalloc(S, &S->cell_of, n));
-        HG_TRYC(dalloc(S, &S->cell_items, n));
-        HG_TRYC(dalloc(S, &S->bucket_count, S->hash_size));
-        HG_TRYC(dalloc(S, &S->bucket_start, S->hash_size));
-        HG_TRYC(dalloc(S, &S->bucket_fill, S->hash_size));
-        HG_TRYC(dalloc(S, &S->scan_tmp, scan_tmp_words(S->hash_size)));
-        HG_TRYC(dalloc(S, &S->bbox, 8));
+        if (n > kBruteListMax) {
+            S->hash_size = next_pow2(2 * n);
+            HG_TRYC(dalloc(S, &S->cell_of, n));
+            HG_TRYC(dalloc(S, &S->cell_recs, n));
+            HG_TRYC(dalloc(S, &S->buckets, size_t(2) * S->hash_size));
+            HG_TRYC(dalloc(S, &S->bucket_start, S->hash_size));
+            HG_TRYC(dalloc(S, &S->scan_tmp, scan_tmp_words(S->hash_size)));
+        }
         HG_HIPC(launch_neighbor_build(*S, S->stream));
         HG_TRYC(check_flags(S, "hg_create"));
     }
@@ -714,11 +741,9 @@ extern "C" {
 hg_status hg_get_state(hg_system *S, double *x, double *v, double *theta, double *omega) {
     if (!S) return fail(HG_ERR_INVALID, "system is null");
     HG_TRY(settle(S, "hg_get_state"));
-    HG_TRY(download3(S, S->x, x));
-    HG_TRY(download3(S, S->v, v));
-    HG_TRY(download3(S, S->th, theta));
-    HG_TRY(download3(S, S->w, omega));
-    return HG_OK;
+    const double *src[4] = {S->x, S->v, S->th, S->w};
+    double *dst[4] = {x, v, theta, omega};
+    return read_fields(S->stage, src, dst, 4, S->n, S->stream);
 }
 
 hg_status hg_set_state(hg_system *S, const double *x, const double *v, const double *theta, const double *omega) {
@@ -735,9 +760,9 @@ hg_status hg_set_state(hg_system *S, const double *x, const double *v, const dou
 hg_status hg_get_accelerations(hg_system *S, double *a, double *alpha) {
     if (!S) return fail(HG_ERR_INVALID, "system is null");
     HG_TRY(settle(S, "hg_get_accelerations"));
-    HG_TRY(download3(S, S->a, a));
-    HG_TRY(download3(S, S->al, alpha));
-    return HG_OK;
+    const double *src[2] = {S->a, S->al};
+    double *dst[2] = {a, alpha};
+    return read_fields(S->stage, src, dst, 2, S->n, S->stream);
 }
 
 hg_status hg_reset_accelerations(hg_system *S) {
