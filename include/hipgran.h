@@ -482,7 +482,7 @@ hg_status hg_server_get_stats(hg_server *srv, hg_server_stats *out);
  * their own, [2] neighbour rebuild (all of its kernels), [3] reserved. */
 hg_status hg_profile_enable(hg_system *sys, int enable);
 hg_status hg_profile_read(hg_system *sys, uint64_t *launches, double *device_ms);
-/* Small FP64 systems (up to 27 particles, with the legacy functor 256) step
+/* Small FP64 systems (up to 32 particles, with the legacy functor 256) step
  * through one launch per rebuild interval; enable = 1 makes hg_step use the per-step launches (the
  * path every larger system takes) without the event timing of
  * hg_profile_enable, enable = 0 restores the choice by size. Results are the

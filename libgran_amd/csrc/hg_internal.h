@@ -164,6 +164,7 @@ struct hg_system_impl {
     // legacy sinter_functor connectors (pair_table::lconn / lslot)
     double *lconn = nullptr;
     uint32_t *lslot = nullptr;
+    uint32_t lmax = 0;  // the most legacy bonds of a particle
     bool legacy_ready = false;
     // neighbour list
     uint32_t cap_n = 0;
@@ -183,7 +184,6 @@ struct hg_system_impl {
     // reductions
     double *red = nullptr;
     double *energy = nullptr;  // per-particle ledger terms, 8 per particle (allocated on first use)
-    double *tiny = nullptr;    // per-pair springs of the pair-parallel pass (n*n*kSpringRec, on first use)
     // per-step launches (tile_step.h), on first use: the second x, v, omega
     // and facets, the system's meta and its tiles
     double *tile_state = nullptr;
@@ -239,20 +239,20 @@ hipError_t launch_neighbor_build(hg_system_impl &S, hipStream_t s);
 // Systems of at most this many particles list every pair by brute force.
 constexpr uint32_t kBruteListMax = 8192;
 hipError_t launch_advance_facet(facet_dev *f, const double *v, double dt, hipStream_t s);
-// nsteps steps of a small FP64 system in one workgroup; `even`/`odd` are the
-// views whose pair-state tables the even/odd steps read. Systems of at most
-// kTinySystemMax particles evaluate their pairs in parallel (k_tiny_steps;
-// `scratch` holds n*max(n, cap_n)*kSpringRec doubles). Legacy sinter_functor
-// systems of at most kSmallSystemMax take k_small_steps. The line for the
-// other functors lies at kTinySystemMax because one workgroup with a particle
-// per thread is slower than a launch per step over tiles from there on: 16
-// against 8.8 us per step at 30 particles, 22 against 10.9 at 200 (lists of
-// 3.9, FP64); with all pairs 49 against 9.0 and 199 against 14.3.
-constexpr uint32_t kSmallSystemMax = 256, kTinySystemMax = 27;
+// nsteps steps of a small FP64 system in one workgroup. Systems of at most
+// kTinySystemMax particles whose pairs fit LDS (tiny_steps_fit; maxb: the most
+// legacy bonds of a particle) take k_tiny_steps, which reads the table of
+// `even` and writes its other half once, whatever the step count. Larger legacy
+// sinter_functor systems, up to kSmallSystemMax, take k_small_steps; `even` /
+// `odd` are the views whose tables the even / odd steps read. For the other
+// functors a launch per step over tiles is faster than k_small_steps from there
+// on: 8.8 against 16 us per step at 30 particles, 10.9 against 22 at 200 (lists
+// of 3.9, FP64); with all pairs 9.0 against 49 and 14.3 against 199.
+constexpr uint32_t kSmallSystemMax = 256, kTinySystemMax = 32;
+bool tiny_steps_fit(uint32_t n, uint32_t maxb);
 hipError_t launch_small_steps(const hg_params &p, const sys_view &even, const sys_view &odd, double *x, double *v,
-                              double *th, double *w, facet_dev *facets, uint32_t nsteps, bool pending_first,
-                              bool final_kick, double half, double dt, int nf_advance, double *lconn,
-                              const uint32_t *bcnt, double *scratch, hipStream_t s);
+                              double *th, double *w, facet_dev *facets, uint32_t nsteps, double half, double dt,
+                              int nf_advance, double *lconn, const uint32_t *bcnt, uint32_t maxb, hipStream_t s);
 // sinter_step_handler's connector moves after a drift (x and v already
 // advanced): each of particle i's connectors follows dx = v_i dt, then turns
 // by dtheta = w_i dt about the new x_i.

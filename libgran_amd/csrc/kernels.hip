@@ -16,8 +16,8 @@
 //     so spring state survives neighbour rebuilds with no separate merge.
 #include <hip/hip_runtime.h>
 
-#include "force_device.h"
 #include "hg_internal.h"
+#include "pair_eval.h"
 
 namespace hg {
 
@@ -695,110 +695,325 @@ hipError_t launch_force(const hg_params &p, const sys_view &sv, hipStream_t s) {
     return hipErrorInvalidValue;
 }
 
-// nsteps steps of a system of at most kTinyMax particles in one workgroup of
-// kTinyThreads, one thread per ordered pair (all pairs, or particle i's
-// listed partner slot k): each pair's functors evaluated at once (its old
-// springs looked up in the pair-state row of i), its term kept in LDS and its
-// new springs in `scratch` (kSpringRec doubles per pair: the 9 components,
-// then keep | bonded << 1). Then one thread per particle adds its terms in
-// partner order and writes its new row as the walker of the per-particle
-// pass does: old entries of partners not evaluated are carried in place, an
-// evaluated partner's entry is replaced by its kept springs. So the sums and
-// tables are those of k_force_all / k_force_nl. Contact, alt_sinter (bonds
-// broken past their neck strength drop their entry), the legacy
-// sinter_functor (its connectors moved after each drift, as k_legacy_move
-// does) or no binary functor.
-constexpr uint32_t kTinyMax = 27, kTinyThreads = 768;
+// ------------------------------------------------------- tiny systems -----
+// All steps between two list rebuilds of a system of a few dozen particles, by
+// one workgroup, with everything a step touches in LDS: state, the springs and
+// terms of every evaluated ordered pair, connectors, facets. Pair (i, k-th
+// partner) has the place i * row + k. A step is three phases: which unbonded
+// pairs touch; every pair's term; each particle's sum, kick and drift.
+//
+// What bounds a step is the longest chain of dependent arithmetic, so a pair
+// with springs (bonded or touching) is evaluated by four lanes: three for its
+// tangential, rolling and torsion springs, one for its Hamaker term, joined by
+// quad permutes; lane c < 3 then finishes component c. In the last phase a
+// thread owns one component of one particle. The expressions and their order
+// are those of sinter_eval, contact_eval and the per-particle walk.
+//
+// Measured against one thread per pair with state, rows and springs in global
+// memory: 19 particles, contact and Hamaker, list rebuilt every 20 steps 20.7
+// -> 5.0 us a step, all pairs 15.2 -> 4.2; the legacy 27-particle lattice 19.0
+// -> 4.8.
+constexpr uint32_t kTinyThreads = 512;
 
-template <int BIN, int HAM, bool NL>
+// Doubles (then words) of LDS a system of n particles needs; maxb: the most
+// legacy bonds a particle has (0 without the legacy functor).
+struct tiny_layout {
+    uint32_t n, row, places, maxb;
+    __host__ __device__ tiny_layout(uint32_t n_, uint32_t maxb_)
+        : n(n_), row((n_ > 1 ? n_ - 1 : 1) | 1u), places(n_ * ((n_ > 1 ? n_ - 1 : 1) | 1u)), maxb(maxb_) {}
+    // state (x, v, omega, theta, a, alpha), terms, springs, facet terms, connectors
+    __host__ __device__ size_t doubles() const {
+        return size_t(18) * n + size_t(15) * places + size_t(6) * n + size_t(15) * maxb * n;
+    }
+    // entries, bonded list, touching list, flags
+    __host__ __device__ size_t bytes() const { return doubles() * 8 + size_t(places) * (4 + 2 + 2 + 1) + 16; }
+};
+
+template <int CTRL>
+__device__ __forceinline__ double quad_bcast(double v) {
+    union {
+        double d;
+        int w[2];
+    } a, r;
+    a.d = v;
+    r.w[0] = __builtin_amdgcn_mov_dpp(a.w[0], CTRL, 0xF, 0xF, true);
+    r.w[1] = __builtin_amdgcn_mov_dpp(a.w[1], CTRL, 0xF, 0xF, true);
+    return r.d;
+}
+// Component c (0..2) of the vector that lane LANE of this lane's quad holds.
+template <int LANE>
+__device__ __forceinline__ double quad_comp(d3 v, uint32_t c) {
+    const double x = quad_bcast<LANE * 0x55>(v.x), y = quad_bcast<LANE * 0x55>(v.y), z = quad_bcast<LANE * 0x55>(v.z);
+    return c == 0 ? x : (c == 1 ? y : z);
+}
+
+// TINY_BROKEN: a bond that broke in this step's pass, an unbonded pair from the
+// next one on.
+enum : uint8_t { TINY_NONE = 0, TINY_FREE, TINY_CONTACT, TINY_BOND, TINY_BROKEN, TINY_LEGACY };
+
+template <int BIN, int HAM>
 __global__ void __launch_bounds__(kTinyThreads)
-    k_tiny_steps(hg_params P, sys_view even, sys_view odd, double *x, double *v, double *th, double *w,
-                 facet_dev *facets, uint32_t nsteps, int pending_first, int final_kick, double half, double dt,
-                 int nf_advance, double *scratch, double *lconn, const uint32_t *bcnt) {
-    __shared__ double terms[kTinyThreads * 6];
-    const uint32_t t = threadIdx.x;
-    const uint32_t n = even.n;
-    constexpr bool nl = NL;
-    const uint32_t slots = nl ? even.cap_n : n;  // pair threads per particle
+    k_tiny_steps(hg_params P, sys_view S, double *gx, double *gv, double *gth, double *gw, facet_dev *facets,
+                 uint32_t nsteps, double half, double dt, int nf_advance, double *lconn, uint32_t maxb) {
+    extern __shared__ double tiny_lds[];
+    __shared__ facet_dev F[kMaxFacets];
+    __shared__ uint32_t s_bonds, s_touch;
+    __shared__ uint32_t s_cnt[kTinySystemMax], s_legacy[kTinySystemMax];  // partners and legacy bonds
+    const tiny_layout Y(S.n, maxb);
+    const uint32_t n = Y.n, row = Y.row, places = Y.places, tid = threadIdx.x;
+    const bool nl = P.pair_mode == HG_PAIRS_NEIGHBOR_LIST;
+    double *X = tiny_lds;                        // 18 components of n
+    double *T = X + size_t(18) * n;              // 6 components of every place
+    double *SP = T + size_t(6) * places;         // 9 components of every place
+    double *FT = SP + size_t(9) * places;        // 6 components of n
+    double *C = FT + size_t(6) * n;              // connectors: 15 per (particle, bond slot)
+    uint32_t *E = reinterpret_cast<uint32_t *>(C + size_t(15) * maxb * n);  // i | j << 8 | legacy slots: i's << 16, j's << 24
+    uint16_t *LB = reinterpret_cast<uint16_t *>(E + places), *LC = LB + places;
+    uint8_t *K = reinterpret_cast<uint8_t *>(LC + places);
+    auto vec = [&](uint32_t f, uint32_t i) {
+        const double *q = X + size_t(3 * f) * n + i;
+        return d3{q[0], q[n], q[2 * n]};
+    };
+    auto spring = [&](uint32_t at, uint32_t c) {
+        const double *q = SP + size_t(3 * c) * places + at;
+        return d3{q[0], q[places], q[2 * places]};
+    };
+    auto set_spring = [&](uint32_t at, uint32_t c, d3 a) {
+        double *q = SP + size_t(3 * c) * places + at;
+        q[0] = a.x;
+        q[places] = a.y;
+        q[2 * places] = a.z;
+    };
+
+    // in: state, facets, connectors, then the pairs with their springs
+    const double *fields[6] = {gx, gv, gw, gth, S.a, S.al};
+    for (uint32_t q = tid; q < 18u * n; q += kTinyThreads) {
+        const uint32_t c = q / n, i = q % n;
+        X[q] = fields[c / 3][4 * i + c % 3];
+    }
+    if (tid < uint32_t(S.nf)) F[tid] = facets[tid];
+    if (tid == 0) s_bonds = s_touch = 0;
+    if (tid < n) {
+        s_cnt[tid] = nl ? S.ncnt[tid] : n - 1u;
+        s_legacy[tid] = BIN == HG_BINARY_SINTER_LEGACY ? S.pt.bcnt[tid] : 0u;
+    }
+    if constexpr (BIN == HG_BINARY_SINTER_LEGACY)
+        for (uint32_t q = tid; q < 15u * maxb * n; q += kTinyThreads) {
+            const uint32_t e = q / 15, i = e / maxb, s = e % maxb;
+            if (s < S.pt.bcnt[i]) C[q] = lconn[(size_t(s) * n + i) * kConnRec + q % 15];
+        }
+    __syncthreads();
+    for (uint32_t at = tid; at < places; at += kTinyThreads) {
+        const uint32_t i = at / row, k = at % row;
+        const bool on = k < s_cnt[i];
+        uint8_t kind = TINY_NONE;
+        if (on) {
+            const uint32_t j = nl ? S.nb[size_t(k) * n + i] : k + (k >= i ? 1u : 0u);
+            uint32_t ls = 0;
+            kind = TINY_FREE;
+            if constexpr (BIN == HG_BINARY_SINTER_LEGACY)
+                for (uint32_t q = 0; q < s_legacy[i]; q++)
+                    if (S.pt.bj[size_t(q) * n + i] == j) {
+                        kind = TINY_LEGACY;
+                        ls = q | (S.pt.lslot[size_t(q) * n + i] << 8);
+                    }
+            E[at] = i | (j << 8) | (ls << 16);
+            if constexpr (BIN != HG_BINARY_NONE) {
+                const uint32_t cnt = S.pt.pcnt_old[i];
+                for (uint32_t q = 0; q < cnt; q++) {
+                    const uint32_t tag = S.pt.pj_old[size_t(q) * n + i];
+                    if ((tag & kIdxMask) != j) continue;
+                    kind = (tag & kBondBit) ? TINY_BOND : TINY_CONTACT;
+                    const spring9 sp = ld_rec(S.pt.ps_old + (size_t(q) * n + i) * kSpringRec);
+                    for (uint32_t c = 0; c < 3; c++) set_spring(at, c, sp.s[c]);
+                }
+            }
+            if (kind == TINY_BOND || kind == TINY_LEGACY) LB[atomicAdd(&s_bonds, 1u)] = uint16_t(at);
+        }
+        K[at] = kind;
+    }
+    // the first kick and drift
+    for (uint32_t q = tid; q < 6u * n; q += kTinyThreads) {
+        const uint32_t c = q / n, i = q % n, ang = c >= 3, d = c % 3;
+        double *u = X + size_t(3 + c) * n + i, *o = X + size_t((ang ? 9 : 0) + d) * n + i;
+        *u = *u + X[size_t(12 + c) * n + i] * half;
+        *o = *o + *u * dt;
+    }
+    const double touch = 2.0 * P.contact.r_part, touch2 = touch * touch * (1.0 + 1e-12);
     for (uint32_t s = 0; s < nsteps; s++) {
-        const int pending = (s > 0 || pending_first) ? 1 : 0;
-        if (pending && t == 0) advance_facets(facets, nf_advance, dt);
-        if (t < n) {
-            kick_drift_one(x, v, th, w, even.a, even.al, t, pending, half, half, dt);
-            if constexpr (BIN == HG_BINARY_SINTER_LEGACY) legacy_move_one(x, v, w, n, t, dt, lconn, bcnt);
-        }
         __syncthreads();
-        const sys_view &S = (s & 1u) ? odd : even;
-        if (t < n * slots) {
-            const uint32_t i = t / slots, k = t % slots;
-            bool eval;
-            uint32_t j;
-            if (nl) {
-                eval = k < S.ncnt[i];
-                j = eval ? S.nb[size_t(k) * n + i] : 0u;
-            } else {
-                eval = k != i;
-                j = k;
+        if constexpr (BIN == HG_BINARY_SINTER_LEGACY) {
+            // sinter_step_handler: a connector follows its particle, then turns with it
+            for (uint32_t q = tid; q < 5u * maxb * n; q += kTinyThreads) {
+                const uint32_t e = q / 5, i = e / maxb;
+                if (e % maxb >= s_legacy[i]) continue;
+                double *r = C + size_t(3) * q;
+                const d3 p = d3{r[0], r[1], r[2]} + vec(1, i) * dt;
+                const d3 moved = p + cross(vec(2, i) * dt, p - vec(0, i));
+                r[0] = moved.x;
+                r[1] = moved.y;
+                r[2] = moved.z;
             }
-            if (eval) {
-                const d3 xi = ld3(S.x, i), vi = ld3(S.v, i), wi = ld3(S.w, i);
-                const d3 xj = ld3(S.x, j), vj = ld3(S.v, j), wj = ld3(S.w, j);
-                acc6 b{zero3(), zero3()};
-                spring9 sp = zero_spring();
-                bool bonded = false, keep = false;
-                uint32_t ls = kNoEntry;  // the legacy bond's slot in i's list
-                if constexpr (BIN == HG_BINARY_SINTER_LEGACY)
-                    for (uint32_t q = 0; q < S.pt.bcnt[i]; q++)
-                        if (S.pt.bj[size_t(q) * n + i] == j) ls = q;
-                if (ls != kNoEntry) {
-                    // sinter_bridge.h:222-223: its five connector springs; the
-                    // pair has no table entry (keep stays false)
-                    const double *ri = S.pt.lconn + (size_t(ls) * n + i) * kConnRec;
-                    const double *rj = S.pt.lconn + (size_t(S.pt.lslot[size_t(ls) * n + i]) * n + j) * kConnRec;
-                    d3 ci[5], cj[5];
-                    for (int q = 0; q < 5; q++) {
-                        ci[q] = d3{ri[3 * q], ri[3 * q + 1], ri[3 * q + 2]};
-                        cj[q] = d3{rj[3 * q], rj[3 * q + 1], rj[3 * q + 2]};
+        }
+        if constexpr (BIN != HG_BINARY_NONE)
+            for (uint32_t at = tid; at < places; at += kTinyThreads) {
+                const uint8_t kind = K[at];
+                if (kind != TINY_FREE && kind != TINY_CONTACT && kind != TINY_BROKEN) continue;
+                const uint32_t e = E[at];
+                const d3 d = vec(0, e & 0xFFu) - vec(0, (e >> 8) & 0xFFu);
+                bool touching = false;
+                if (!(dot(d, d) > touch2)) touching = !(2.0 * P.contact.r_part - dot(d, normalized(d)) <= 0);
+                if (touching) {
+                    LC[atomicAdd(&s_touch, 1u)] = uint16_t(at);
+                    if (kind != TINY_CONTACT) {
+                        for (uint32_t c = 0; c < 3; c++) set_spring(at, c, zero3());
+                        K[at] = TINY_CONTACT;
                     }
-                    b = legacy_bonded_eval(P.sinter.k, P.sinter.gamma_n, P.contact.r_part, P.contact.mass,
-                                           P.contact.inertia, ci, cj, xi, xj, vi, vj, wi, wj);
-                } else if constexpr (BIN != HG_BINARY_NONE) {
-                    const uint32_t cnt = S.pt.pcnt_old[i];
-                    for (uint32_t q = 0; q < cnt; q++) {
-                        const uint32_t tag = S.pt.pj_old[size_t(q) * n + i];
-                        if ((tag & kIdxMask) == j) {
-                            sp = ld_rec(S.pt.ps_old + (size_t(q) * n + i) * kSpringRec);
-                            bonded = (tag & kBondBit) != 0;
-                        }
-                    }
-                    // the bond's neck strength, as walker_t::neck finds it
-                    auto neck = [&] {
-                        double r = __builtin_huge_val();
+                } else {
+                    K[at] = TINY_FREE;
+                }
+            }
+        __syncthreads();
+        // terms: bonded quads, touching quads, the other pairs, facets, each
+        // kind from a wavefront of its own
+        const uint32_t bonds = s_bonds, touching = s_touch, per = BIN == HG_BINARY_SINTER_LEGACY ? 1u : 4u;
+        const uint32_t e1 = (bonds * per + 63u) & ~63u, e2 = e1 + ((touching * 4u + 63u) & ~63u),
+                       e3 = e2 + ((places + 63u) & ~63u), e4 = e3 + (S.nf > 0 ? n : 0u);
+        for (uint32_t q = tid; q < e4; q += kTinyThreads) {
+            if (q >= e3) {
+                const uint32_t i = q - e3;
+                const acc6 f = facet_fold(P, F, S.nf, S.ss, n, i, vec(0, i), vec(1, i), vec(2, i));
+                const double r[6] = {f.lin.x, f.lin.y, f.lin.z, f.ang.x, f.ang.y, f.ang.z};
+                for (uint32_t c = 0; c < 6; c++) FT[size_t(c) * n + i] = r[c];
+            } else if (q >= e2) {
+                const uint32_t at = q - e2;
+                if (at >= places || K[at] != TINY_FREE) continue;
+                const uint32_t e = E[at];
+                const d3 h = hamaker_lin<HAM>(P.hamaker, vec(0, (e >> 8) & 0xFFu) - vec(0, e & 0xFFu));
+                T[at] = h.x;
+                T[places + at] = h.y;
+                T[2 * places + at] = h.z;
+                for (uint32_t c = 3; c < 6; c++) T[c * places + at] = 0.0;
+            } else if (BIN == HG_BINARY_SINTER_LEGACY && q < e1) {
+                if (q >= bonds) continue;
+                const uint32_t at = LB[q], e = E[at], i = e & 0xFFu, j = (e >> 8) & 0xFFu, ls = (e >> 16) & 0xFFu;
+                // sinter_bridge.h:222-223: the bond's connectors, i's at its
+                // slot for j, j's at its slot for i
+                const double *ri = C + (size_t(i) * maxb + ls) * 15;
+                const double *rj = C + (size_t(j) * maxb + (e >> 24)) * 15;
+                d3 ci[5], cj[5];
+                for (int c = 0; c < 5; c++) {
+                    ci[c] = d3{ri[3 * c], ri[3 * c + 1], ri[3 * c + 2]};
+                    cj[c] = d3{rj[3 * c], rj[3 * c + 1], rj[3 * c + 2]};
+                }
+                const acc6 b = legacy_bonded_eval(P.sinter.k, P.sinter.gamma_n, P.contact.r_part, P.contact.mass,
+                                                  P.contact.inertia, ci, cj, vec(0, i), vec(0, j), vec(1, i), vec(1, j),
+                                                  vec(2, i), vec(2, j));
+                d3 lin = b.lin;
+                if constexpr (HAM != HG_HAMAKER_NONE) lin = lin + hamaker_lin<HAM>(P.hamaker, vec(0, j) - vec(0, i));
+                const double r[6] = {lin.x, lin.y, lin.z, b.ang.x, b.ang.y, b.ang.z};
+                for (uint32_t c = 0; c < 6; c++) T[c * places + at] = r[c];
+            } else if constexpr (BIN == HG_BINARY_CONTACT || BIN == HG_BINARY_SINTER || BIN == HG_BINARY_SINTER_LEGACY) {
+                const bool bond = BIN == HG_BINARY_SINTER && q < e1;
+                const uint32_t item = (bond ? q : q - e1) >> 2, c = q & 3u;
+                if (item >= (bond ? bonds : touching)) continue;
+                const uint32_t at = bond ? LB[item] : LC[item], e = E[at], i = e & 0xFFu, j = (e >> 8) & 0xFFu;
+                if (bond && K[at] != TINY_BOND) continue;  // broken: the pair is among the others
+                const d3 xi = vec(0, i), xj = vec(0, j), vi = vec(1, i), vj = vec(1, j), wi = vec(2, i), wj = vec(2, j);
+                const hg_contact_params &pc = P.contact;
+                const hg_sinter_params &ps = P.sinter;
+                const double r = bond ? ps.r_part : pc.r_part;
+                const d3 d = xi - xj, nn = normalized(d);
+                const double overlap = 2.0 * r - dot(d, nn), rpp = r - overlap / 2.0, v_n = -dot(vi - vj, nn);
+                const double f_n = (bond ? ps.k : pc.k) * overlap + (bond ? ps.gamma_n : pc.gamma_n) * v_n;
+                const d3 cwi = cross(nn, wi), cwj = cross(nn, wj);
+                const d3 v_ij = ((vi - vj) + rpp * cwi) + rpp * cwj;
+                const d3 v_t = v_ij - dot(v_ij, nn) * nn, v_r = (-rpp) * (cwi - cwj),
+                         v_o = (r * (dot(nn, wi) - dot(nn, wj))) * nn;
+                auto pick = [&](auto a, auto b, auto o) { return c == 0 ? a : (c == 1 ? b : o); };
+                const d3 rel{pick(v_t.x, v_r.x, v_o.x), pick(v_t.y, v_r.y, v_o.y), pick(v_t.z, v_r.z, v_o.z)};
+                d3 f;
+                if (c == 3) {
+                    f = hamaker_lin<HAM>(P.hamaker, xj - xi);
+                } else {
+                    d3 sp = spring(at, c);
+                    if (bond)
+                        f = shear_sinter(sp, nn, pick(ps.k_t, ps.k_r, ps.k_o), pick(ps.gamma_t, ps.gamma_r, ps.gamma_o),
+                                         rel, ps.dt);
+                    else
+                        f = shear_contact(sp, nn, pick(pc.k_t, pc.k_r, pc.k_o), pick(pc.gamma_t, pc.gamma_r, pc.gamma_o),
+                                          f_n, pick(pc.mu_s, pc.mu_r, pc.mu_o), pick(pc.phi_d, pc.phi_r, pc.phi_o), rel,
+                                          pc.dt);
+                    set_spring(at, c, sp);
+                }
+                const d3 cr = cross(nn, f);
+                const d3 tau = c == 0 ? rpp * cr : (c == 1 ? r * cr : r * f);
+                const double ft = quad_comp<0>(f, c), h = quad_comp<3>(f, c), tt = quad_comp<0>(tau, c),
+                             tr = quad_comp<1>(tau, c), to = quad_comp<2>(tau, c);
+                if (bond && P.sinter_breaking) {
+                    // alt_breaking_sinter_bridge.h:117-119; lane 0 holds f_t
+                    const d3 ftot = f_n * nn + f;
+                    if (c == 0) {
+                        double neck = __builtin_huge_val();
                         if (S.pt.bcnt)
-                            for (uint32_t q = 0; q < S.pt.bcnt[i]; q++)
-                                if (S.pt.bj[size_t(q) * n + i] == j) r = S.pt.bstr[size_t(q) * n + i];
-                        return r;
-                    };
-                    b = pair_binary<BIN>(P, xi, xj, vi, wi, [&](d3 &v, d3 &w) { v = vj, w = wj; }, sp, bonded,
-                                         keep, neck);
+                            for (uint32_t b = 0; b < S.pt.bcnt[i]; b++)
+                                if (S.pt.bj[size_t(b) * n + i] == j) neck = S.pt.bstr[size_t(b) * n + i];
+                        if (norm(ftot) > neck) K[at] = TINY_BROKEN;
+                    }
                 }
-                const acc6 e = pair_term<BIN, HAM>(b, pair_hamaker<HAM>(P, xi, xj));
-                double *tm = terms + size_t(t) * 6;
-                tm[0] = e.lin.x; tm[1] = e.lin.y; tm[2] = e.lin.z;
-                tm[3] = e.ang.x; tm[4] = e.ang.y; tm[5] = e.ang.z;
-                if constexpr (BIN != HG_BINARY_NONE) {
-                    double *r = scratch + size_t(t) * kSpringRec;
-                    st_rec(r, sp);
-                    r[9] = double((keep ? 1 : 0) | (bonded ? 2 : 0));
+                if (c < 3) {
+                    const double nc = c == 0 ? nn.x : (c == 1 ? nn.y : nn.z);
+                    double lin = (f_n * nc + ft) / (bond ? ps.mass : pc.mass);
+                    if constexpr (HAM != HG_HAMAKER_NONE) lin = lin + h;
+                    T[c * places + at] = lin;
+                    T[(3 + c) * places + at] = ((-tt + tr) + to) / (bond ? ps.inertia : pc.inertia);
                 }
             }
         }
         __syncthreads();
-        if (t < n) {
-            const uint32_t i = t;
-            acc6 acc{zero3(), zero3()};
+        if (tid == 0) {
+            s_touch = 0;
+            advance_facets(F, nf_advance, dt);
+        }
+        // sums in partner order, then the kicks and the drift, a component a thread
+        const bool last = s + 1 == nsteps;
+        for (uint32_t q = tid; q < 6u * n; q += kTinyThreads) {
+            const uint32_t c = q / n, i = q % n, ang = c >= 3, d = c % 3;
+            const uint32_t m = s_cnt[i];
+            const double *t = T + size_t(c) * places + size_t(i) * row;
+            double acc = 0.0;
+#pragma unroll 6
+            for (uint32_t k = 0; k < m; k++) acc = acc + t[k];
+            if (S.nf > 0) acc = acc + FT[q];
+            double *u = X + size_t(3 + c) * n + i, *o = X + size_t((ang ? 9 : 0) + d) * n + i;
+            double w = *u + acc * half;
+            if (last) {
+                X[size_t(12 + c) * n + i] = acc;
+            } else {
+                w = w + acc * half;
+                *o = *o + w * dt;
+            }
+            *u = w;
+        }
+    }
+    __syncthreads();
+    double *back[6] = {gx, gv, gw, gth, S.a, S.al};
+    for (uint32_t q = tid; q < 18u * n; q += kTinyThreads) {
+        const uint32_t c = q / n, i = q % n;
+        back[c / 3][4 * i + c % 3] = X[q];
+        if (c >= 3 && c < 9 && !__builtin_isfinite(X[q])) atomicOr(&S.flags[FLAG_NUMERIC], 1);
+    }
+    if (tid < uint32_t(S.nf)) facets[tid] = F[tid];
+    if constexpr (BIN == HG_BINARY_SINTER_LEGACY)
+        for (uint32_t q = tid; q < 15u * maxb * n; q += kTinyThreads) {
+            const uint32_t e = q / 15, i = e / maxb, s = e % maxb;
+            if (s < S.pt.bcnt[i]) lconn[(size_t(s) * n + i) * kConnRec + q % 15] = C[q];
+        }
+    // the rows as the walk leaves them: entries of partners not listed carried in place
+    if constexpr (BIN != HG_BINARY_NONE) {
+        if (tid < n) {
+            const uint32_t i = tid, cnt_old = S.pt.pcnt_old[i], m = s_cnt[i];
             uint32_t q = 0, p = 0;
-            const uint32_t cnt_old = BIN != HG_BINARY_NONE ? S.pt.pcnt_old[i] : 0u;
             auto put = [&](uint32_t tag, const spring9 &sp) {
                 if (q < S.pt.cap) {
                     S.pt.pj_new[size_t(q) * n + i] = tag;
@@ -806,85 +1021,61 @@ __global__ void __launch_bounds__(kTinyThreads)
                 }
                 q++;
             };
-            auto carry_below = [&](uint32_t j) {  // old entries of partners before j
+            auto carry_below = [&](uint32_t j) {
                 while (p < cnt_old && (S.pt.pj_old[size_t(p) * n + i] & kIdxMask) < j) {
                     put(S.pt.pj_old[size_t(p) * n + i], ld_rec(S.pt.ps_old + (size_t(p) * n + i) * kSpringRec));
                     p++;
                 }
             };
-            const uint32_t m = nl ? S.ncnt[i] : n;
             for (uint32_t k = 0; k < m; k++) {
-                const uint32_t j = nl ? S.nb[size_t(k) * n + i] : k;
-                if (!nl && j == i) continue;
-                const double *tm = terms + size_t(i * slots + k) * 6;
-                acc.lin = acc.lin + d3{tm[0], tm[1], tm[2]};
-                acc.ang = acc.ang + d3{tm[3], tm[4], tm[5]};
-                if constexpr (BIN != HG_BINARY_NONE) {
-                    if constexpr (NL) {  // with all pairs every partner is evaluated: nothing to carry
-                        carry_below(j);
-                        if (p < cnt_old && (S.pt.pj_old[size_t(p) * n + i] & kIdxMask) == j) p++;  // replaced
-                    }
-                    const double *r = scratch + size_t(i * slots + k) * kSpringRec;
-                    const int flags = int(r[9]);
-                    if (flags & 1) put(j | ((flags & 2) ? kBondBit : 0u), ld_rec(r));
-                }
+                const uint32_t at = i * row + k, j = (E[at] >> 8) & 0xFFu;
+                carry_below(j);
+                if (p < cnt_old && (S.pt.pj_old[size_t(p) * n + i] & kIdxMask) == j) p++;  // replaced
+                if (K[at] == TINY_CONTACT || K[at] == TINY_BOND)
+                    put(j | (K[at] == TINY_BOND ? kBondBit : 0u),
+                        spring9{{spring(at, 0), spring(at, 1), spring(at, 2)}});
             }
-            if constexpr (BIN != HG_BINARY_NONE) {
-                if constexpr (NL) carry_below(kNoEntry);
-                S.pt.pcnt_new[i] = q < S.pt.cap ? q : S.pt.cap;
-                if (q > S.pt.cap) {
-                    atomicOr(&S.flags[FLAG_PAIR_OVERFLOW], 1);
-                    atomicMax(&S.flags[FLAG_PAIR_MAXCOUNT], int(q));
-                }
+            carry_below(kNoEntry & kIdxMask);
+            S.pt.pcnt_new[i] = q < S.pt.cap ? q : S.pt.cap;
+            if (q > S.pt.cap) {
+                atomicOr(&S.flags[FLAG_PAIR_OVERFLOW], 1);
+                atomicMax(&S.flags[FLAG_PAIR_MAXCOUNT], int(q));
             }
-            if (S.nf > 0) acc = acc + facet_fold(P, S.facets, S.nf, S.ss, S.n, i, ld3(S.x, i), ld3(S.v, i), ld3(S.w, i));
-            st3(S.a, i, acc.lin);
-            st3(S.al, i, acc.ang);
         }
-        __syncthreads();
-    }
-    if (final_kick) {
-        if (t == 0) advance_facets(facets, nf_advance, dt);
-        if (t < n) final_kick_one(v, w, even.a, even.al, t, half, even.flags);
     }
 }
 
+bool tiny_steps_fit(uint32_t n, uint32_t maxb) { return tiny_layout(n, maxb).bytes() <= size_t(154) * 1024; }
+
 template <int BIN, int HAM>
 hipError_t launch_small_steps_t(const hg_params &p, const sys_view &even, const sys_view &odd, double *x, double *v,
-                                double *th, double *w, facet_dev *facets, uint32_t nsteps, bool pending_first,
-                                bool final_kick, double half, double dt, int nf_advance, double *lconn,
-                                const uint32_t *bcnt, double *scratch, hipStream_t s) {
-    if (even.n <= kTinyMax) {
-        if (p.pair_mode == HG_PAIRS_NEIGHBOR_LIST)
-            k_tiny_steps<BIN, HAM, true><<<1, kTinyThreads, 0, s>>>(p, even, odd, x, v, th, w, facets, nsteps,
-                                                                    pending_first ? 1 : 0, final_kick ? 1 : 0, half,
-                                                                    dt, nf_advance, scratch, lconn, bcnt);
-        else
-            k_tiny_steps<BIN, HAM, false><<<1, kTinyThreads, 0, s>>>(p, even, odd, x, v, th, w, facets, nsteps,
-                                                                     pending_first ? 1 : 0, final_kick ? 1 : 0, half,
-                                                                     dt, nf_advance, scratch, lconn, bcnt);
+                                double *th, double *w, facet_dev *facets, uint32_t nsteps, double half, double dt,
+                                int nf_advance, double *lconn, const uint32_t *bcnt, uint32_t maxb, hipStream_t s) {
+    if (even.n <= kTinySystemMax && tiny_steps_fit(even.n, maxb)) {
+        const uint32_t bytes = uint32_t(tiny_layout(even.n, maxb).bytes());
+        const auto kernel = &k_tiny_steps<BIN, HAM>;
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, int(bytes));
+        if (e != hipSuccess) return e;
+        kernel<<<1, kTinyThreads, bytes, s>>>(p, even, x, v, th, w, facets, nsteps, half, dt, nf_advance, lconn, maxb);
         return hipGetLastError();
     }
     if constexpr (BIN == HG_BINARY_SINTER_LEGACY) {
-        k_small_steps<BIN, HAM><<<1, kTile, 0, s>>>(p, even, odd, x, v, th, w, facets, nsteps, pending_first ? 1 : 0,
-                                                    final_kick ? 1 : 0, half, dt, nf_advance, lconn, bcnt);
+        k_small_steps<BIN, HAM><<<1, kTile, 0, s>>>(p, even, odd, x, v, th, w, facets, nsteps, 0, 1, half, dt, nf_advance,
+                                                    lconn, bcnt);
         return hipGetLastError();
     }
     return hipErrorInvalidValue;
 }
 
 hipError_t launch_small_steps(const hg_params &p, const sys_view &even, const sys_view &odd, double *x, double *v,
-                              double *th, double *w, facet_dev *facets, uint32_t nsteps, bool pending_first,
-                              bool final_kick, double half, double dt, int nf_advance, double *lconn,
-                              const uint32_t *bcnt, double *scratch, hipStream_t s) {
-    const uint32_t slots = p.pair_mode == HG_PAIRS_NEIGHBOR_LIST ? even.cap_n : even.n;
-    if (even.n == 0 || even.n > uint32_t(kTile) || p.precision != HG_PRECISION_FP64 ||
-        (even.n <= kTinyMax && (!scratch || even.n * slots > kTinyThreads)))
-        return hipErrorInvalidValue;
-#define HG_CASE(B, H)                                                                                            \
-    if (p.binary_model == B && p.hamaker_model == H)                                                             \
-        return launch_small_steps_t<B, H>(p, even, odd, x, v, th, w, facets, nsteps, pending_first, final_kick, \
-                                          half, dt, nf_advance, lconn, bcnt, scratch, s);
+                              double *th, double *w, facet_dev *facets, uint32_t nsteps, double half, double dt,
+                              int nf_advance, double *lconn, const uint32_t *bcnt, uint32_t maxb, hipStream_t s) {
+    if (even.n == 0 || even.n > kSmallSystemMax || p.precision != HG_PRECISION_FP64) return hipErrorInvalidValue;
+#define HG_CASE(B, H)                                                                                                \
+    if (p.binary_model == B && p.hamaker_model == H)                                                                 \
+        return launch_small_steps_t<B, H>(p, even, odd, x, v, th, w, facets, nsteps, half, dt, nf_advance, lconn, bcnt, \
+                                          maxb, s);
     HG_CASE(HG_BINARY_NONE, HG_HAMAKER_NONE)
     HG_CASE(HG_BINARY_NONE, HG_HAMAKER_FULL)
     HG_CASE(HG_BINARY_NONE, HG_HAMAKER_LIMITED)

@@ -456,6 +456,7 @@ hg_status create_impl(const hg_params *params, size_t n, const double *x0, const
             return cleanup_on(fail(HG_ERR_CAPACITY, "a particle has " + std::to_string(mb) +
                                                         " sinter bonds; at most " +
                                                         std::to_string(kMaxBondsPerParticle)));
+        S->lmax = uint32_t(mb);
         S->bcap = kMaxBondsPerParticle;
         std::vector<uint32_t> bj(size_t(S->bcap) * n, kNoEntry), cnt(n, 0), slot(size_t(S->bcap) * n, 0);
         for (size_t i = 0; i < n; i++) {  // rows come out ascending: bonds are in row order
@@ -646,13 +647,13 @@ hg_status step_impl(hg_system *S, double dt, uint64_t nsteps, uint32_t rebuild_e
     const bool nl = S->p.pair_mode == HG_PAIRS_NEIGHBOR_LIST;
     const int nf_advance = S->p.facet_advance ? 0 : S->nf;  // facets the step moves itself
     const bool legacy = S->p.binary_model == HG_BINARY_SINTER_LEGACY;
-    if (n <= (legacy ? kSmallSystemMax : kTinySystemMax) && S->p.precision == HG_PRECISION_FP64 && !S->profiling &&
+    const bool tiny = n <= kTinySystemMax && tiny_steps_fit(n, S->lmax);
+    if ((tiny || (legacy && n <= kSmallSystemMax)) && S->p.precision == HG_PRECISION_FP64 && !S->profiling &&
         !S->per_step && !S->track_diss) {
         // small systems: the steps between list rebuilds in one launch of one
         // workgroup instead of a launch or more per step
         if (legacy && !S->legacy_ready)
             return fail(HG_ERR_INVALID, "the legacy sinter_functor's connectors are not set (hg_set_legacy_connectors)");
-        if (n <= kTinySystemMax && !S->tiny) HG_TRY(dalloc(S, &S->tiny, size_t(n) * std::max(n, S->cap_n) * kSpringRec));
         uint64_t s = 0;
         while (s < nsteps) {
             if (nl && rebuild_every && (S->step_index % rebuild_every) == 0)
@@ -664,10 +665,9 @@ hg_status step_impl(hg_system *S, double dt, uint64_t nsteps, uint32_t rebuild_e
             S->cur ^= 1;
             const sys_view odd = make_view(S);
             S->cur ^= 1;
-            HG_HIP(launch_small_steps(S->p, even, odd, S->x, S->v, S->th, S->w, S->facets, uint32_t(len), s > 0,
-                                      s + len == nsteps, half, dt, nf_advance, S->lconn, S->bcnt, S->tiny,
-                                      S->stream));
-            if (S->p.binary_model != HG_BINARY_NONE) S->cur ^= int(len & 1u);
+            HG_HIP(launch_small_steps(S->p, even, odd, S->x, S->v, S->th, S->w, S->facets, uint32_t(len), half, dt,
+                                      nf_advance, S->lconn, S->bcnt, S->lmax, S->stream));
+            if (S->p.binary_model != HG_BINARY_NONE) S->cur ^= tiny ? 1 : int(len & 1u);
             for (uint64_t k = 0; k < len; k++) S->t = S->t + dt;
             S->step_index += len;
             s += len;
