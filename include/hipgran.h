@@ -383,14 +383,13 @@ hg_status hg_pool_set_wide_graph(hg_pool *pool, int enable);
  * gives every system a workgroup of its own. */
 hg_status hg_pool_set_packing(hg_pool *pool, int enable);
 /* Online autotuner: from the next hg_pool_step on, first the chunk kernel's
- * shape (256 threads x 2 workgroups per CU, or 512 x 1) at the current launch
- * split, then the launch split at the better shape (wide threshold 0, or
- * 1024..8192 up to the largest system, run one after the other or beside the
- * chunk kernel with room for CUs/32, /16, /8 or /4). Each
- * candidate runs two rebuild intervals of live steps, scored by the second
- * one's host-measured time per step; the fastest is kept. Neither choice
- * changes results, so no step is wasted. enable = 0 stops it and keeps the
- * current setting. */
+ * shape (256 threads x 2 workgroups per CU, or 512 x 1), then, at the better
+ * shape, whether the wide launches run one after the other with the chunk
+ * kernel or beside it with room for CUs/8 or /4. Each candidate runs two
+ * rebuild intervals of live steps, scored by the second one's host-measured
+ * time per step; the fastest is kept. Neither choice changes results, so no
+ * step is wasted. Nothing is tuned where every system takes the wide launches.
+ * enable = 0 stops it and keeps the current setting. */
 hg_status hg_pool_autotune(hg_pool *pool, int enable);
 /* Current split and whether the autotuner has finished (tuned = 1). */
 hg_status hg_pool_get_tuning(hg_pool *pool, size_t *wide_min, int *wide_cus, int *tuned);

@@ -363,24 +363,28 @@ __device__ __forceinline__ void pair_fold(const hg_params &P, uint32_t j, d3 xi,
     pair_fold_vw<BIN, HAM>(P, j, xi, vi, wi, xj, [&](d3 &v, d3 &w) { v = vj, w = wj; }, W, acc);
 }
 
-// Unary container over facets (unary_force_container.h:20-32, a right fold),
-// each facet folding its surface functors (triangular_facet.h:32-51). Surface
-// springs of facet f for particle i at ss + f*9*stride + i.
+// One facet's surface functors on particle i (triangular_facet.h:32-51);
+// surface springs of facet f for particle i at ss + f*9*stride + i.
+__device__ __forceinline__ acc6 facet_term(const hg_params &P, const facet_dev &F, int f, double *ss, size_t stride,
+                                           uint32_t i, d3 xi, d3 vi, d3 wi) {
+    d3 xf = closest_point_on_triangle(F, xi);
+    acc6 c{zero3(), zero3()}, h{zero3(), zero3()};
+    if (P.facet_contact) {
+        double *b = ss + size_t(f) * 9 * stride + i;
+        spring9 sp = ld_spring(b, stride);
+        c = surface_contact_eval(P.surface_contact, xf, F.v_facet, xi, vi, wi, sp);
+        st_spring(b, stride, sp);
+    }
+    if (P.facet_hamaker) h = surface_hamaker_eval(P.surface_hamaker, xf, xi);
+    return (P.facet_contact && P.facet_hamaker) ? c + h : (P.facet_contact ? c : h);
+}
+// Unary container over facets (unary_force_container.h:20-32, a right fold).
 __device__ __forceinline__ acc6 facet_fold(const hg_params &P, const facet_dev *facets, int nf, double *ss,
                                            size_t stride, uint32_t i, d3 xi, d3 vi, d3 wi) {
     acc6 s{zero3(), zero3()};
     for (int f = nf - 1; f >= 0; f--) {
         const facet_dev F = facets[f];
-        d3 xf = closest_point_on_triangle(F, xi);
-        acc6 c{zero3(), zero3()}, h{zero3(), zero3()};
-        if (P.facet_contact) {
-            double *b = ss + size_t(f) * 9 * stride + i;
-            spring9 sp = ld_spring(b, stride);
-            c = surface_contact_eval(P.surface_contact, xf, F.v_facet, xi, vi, wi, sp);
-            st_spring(b, stride, sp);
-        }
-        if (P.facet_hamaker) h = surface_hamaker_eval(P.surface_hamaker, xf, xi);
-        acc6 e = (P.facet_contact && P.facet_hamaker) ? c + h : (P.facet_contact ? c : h);
+        acc6 e = facet_term(P, F, f, ss, stride, i, xi, vi, wi);
         s = (f == nf - 1) ? e : e + s;
     }
     return s;
@@ -434,19 +438,31 @@ __device__ __forceinline__ void pair_fold_mx(const mixed_consts &m, uint32_t j, 
     acc.ang = acc.ang + b.ang;
 }
 
+// One facet's contact term c and Hamaker term h, mixed precision.
+__device__ __forceinline__ void facet_term_mx(const hg_params &P, const mixed_consts &m, const facet_dev &F, int f,
+                                              double *ss, size_t stride, uint32_t i, d3 xi, d3 vi, d3 wi, accf &c,
+                                              f3 &h) {
+    const d3 xf = closest_point_on_triangle(F, xi);
+    c = accf{zerof(), zerof()};
+    h = zerof();
+    if (P.facet_contact) {
+        double *b = ss + size_t(f) * 9 * stride + i;
+        spring9 sp = ld_spring(b, stride);
+        c = surface_contact_mx(m, xf, F.v_facet, xi, vi, wi, sp);
+        st_spring(b, stride, sp);
+    }
+    if (P.facet_hamaker) h = surface_hamaker_mx(m, xf, xi);
+}
 __device__ __forceinline__ accf facet_fold_mx(const hg_params &P, const mixed_consts &m, const facet_dev *facets,
                                               int nf, double *ss, size_t stride, uint32_t i, d3 xi, d3 vi, d3 wi) {
     accf s{zerof(), zerof()};
     for (int f = nf - 1; f >= 0; f--) {
         const facet_dev F = facets[f];
-        const d3 xf = closest_point_on_triangle(F, xi);
-        if (P.facet_contact) {
-            double *b = ss + size_t(f) * 9 * stride + i;
-            spring9 sp = ld_spring(b, stride);
-            s = s + surface_contact_mx(m, xf, F.v_facet, xi, vi, wi, sp);
-            st_spring(b, stride, sp);
-        }
-        if (P.facet_hamaker) s.lin = s.lin + surface_hamaker_mx(m, xf, xi);
+        accf c;
+        f3 h;
+        facet_term_mx(P, m, F, f, ss, stride, i, xi, vi, wi, c, h);
+        if (P.facet_contact) s = s + c;
+        if (P.facet_hamaker) s.lin = s.lin + h;
     }
     return s;
 }

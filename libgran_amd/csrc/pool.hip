@@ -952,35 +952,28 @@ hg_status refresh_order(hg_pool *Q) {
 
 // Online tuner, in two stages: the chunk kernel's shape (256 threads, two
 // workgroups per CU; 512 threads, one: the same waves per SIMD with twice the
-// LDS per system) at the current launch split, then the launch split (wide
-// threshold and the CUs left for the wide launches) at the better shape.
-// Every candidate runs two intervals (the first may record a graph); the
-// second one's host-measured time per step is its score. Neither choice
-// changes any result, so tuning happens on live steps.
+// LDS per system), then whether the wide launches run ahead of the chunk kernel
+// or beside it, with room for CUs/8 or CUs/4; which systems go wide is
+// split_order's choice. Every candidate runs two intervals (the first may
+// record a graph); the second one's host-measured time per step is its score.
+// Neither choice changes any result, so tuning happens on live steps. A pool
+// whose systems all go wide has nothing to tune.
 void tune_splits(hg_pool *Q) {
     Q->tune_cands.clear();
-    size_t largest = 0;
-    for (size_t s = 0; s < Q->S; s++)
-        if (Q->active[s]) largest = std::max<size_t>(largest, Q->meta[s].n);
-    Q->tune_cands.push_back({0u, Q->wide_cus, Q->chunk_tpb, Q->wg_per_cu});
-    for (uint32_t wm : {1024u, 2048u, 4096u, 8192u}) {
-        if (wm > largest) break;  // no system would go wide
-        Q->tune_cands.push_back({wm, 0, Q->chunk_tpb, Q->wg_per_cu});  // one after the other
-        for (int frac : {32, 16, 8, 4})
-            Q->tune_cands.push_back({wm, std::max(1, Q->n_cus / frac), Q->chunk_tpb, Q->wg_per_cu});
-    }
+    for (int cus : {0, Q->n_cus / 8, Q->n_cus / 4})
+        Q->tune_cands.push_back({uint32_t(Q->wide_min), cus, Q->chunk_tpb, Q->wg_per_cu});
     Q->tune_stage = 1;
     Q->tune_scores.assign(Q->tune_cands.size(), 0.0);
     Q->tune_pos = 0;
-    Q->tune_phase = Q->tune_cands.size() > 1 ? TUNE_RUNNING : TUNE_DONE;
-    if (Q->tune_phase == TUNE_DONE) {
-        Q->wide_min = 0;
-        Q->order_dirty = true;
-    }
+    Q->tune_phase = TUNE_RUNNING;
 }
 
 void tune_begin(hg_pool *Q) {
     const uint32_t wm = uint32_t(Q->wide_min);
+    if (Q->narrow_count == 0) {
+        Q->tune_phase = TUNE_DONE;
+        return;
+    }
     Q->tune_cands = {{wm, Q->wide_cus, 256, 2}, {wm, Q->wide_cus, 512, 1}};
     Q->tune_stage = 0;
     Q->tune_scores.assign(Q->tune_cands.size(), 0.0);
@@ -1023,10 +1016,13 @@ namespace hg {
 hg_status pool_begin(hg_pool *Q, double dt, uint64_t max_len, uint32_t rebuild_every, uint32_t *len_out) {
     *len_out = 0;
     if (Q->fl.active) return fail(HG_ERR_INVALID, "pool: an interval is already queued");
-    if (Q->tune_phase == TUNE_START) tune_begin(Q);
-    if (Q->tune_phase == TUNE_RUNNING) tune_select(Q);
     if (Q->order_dirty) PG_TRY(refresh_order(Q));
     if (Q->order.empty() || max_len == 0) return HG_OK;
+    if (Q->tune_phase == TUNE_START) tune_begin(Q);
+    if (Q->tune_phase == TUNE_RUNNING) {
+        tune_select(Q);
+        if (Q->order_dirty) PG_TRY(refresh_order(Q));
+    }
     const bool nl = Q->p.pair_mode == HG_PAIRS_NEIGHBOR_LIST;
     const bool cadence = nl && rebuild_every;
     const pool_view V = make_pool_view(Q);

@@ -44,7 +44,7 @@ struct wide_block {
     uint32_t slot, start, offset, n;
 };
 constexpr uint32_t kTileThreads = 256, kTilePairs = 1024;
-constexpr int tile_width(int pairs) { return pairs == HG_PAIRS_NEIGHBOR_LIST ? 64 : 4; }
+constexpr int tile_width(int pairs) { return pairs == HG_PAIRS_NEIGHBOR_LIST ? 64 : 1; }
 enum { TILE_FORCE = 0, TILE_STEP = 1, TILE_LAST = 2 };
 
 // The launches of one binary functor and pair mode (pool_chunk.hip), by

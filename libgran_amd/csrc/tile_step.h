@@ -42,17 +42,28 @@ struct tile_lds {
     uint32_t rows[W], dirty[W];
     uint32_t nB[kTileThreads / 64], nO[kTileThreads / 64];
     uint32_t contacts, ended;
-    typename prec_types<PREC>::term F[FAC ? 6 : 1][W];
+    // the terms of four facets: FP64 the 6 components of each, mixed the
+    // contact's 6 and the Hamaker term's 3
+    typename prec_types<PREC>::term F[FAC ? 4 : 1][9][W];
     term A[6][W < 64 ? W : 1];
 };
 
 constexpr uint32_t kNoRowSlot = 0xFFFu;
 
+// Wavefronts per SIMD that the registers leave room for. Listed tiles, many to
+// a CU, hide one pair's latency behind another's: mixed 151 us a step at
+// 635,000 particles with three, 187 with two (four spill: 241). All pairs come
+// in few blocks, and two cost them registers: 33 us a step at 522 particles
+// against 28.
+constexpr int tile_waves(int pairs, int prec) {
+    return pairs != HG_PAIRS_NEIGHBOR_LIST ? 1 : (prec == HG_PRECISION_MIXED ? 3 : 2);
+}
+
 // What a launch does after the pass: TILE_FORCE stores the accelerations of
 // the systems that have none; TILE_STEP completes the step, kicks and drifts
 // into the other buffers; TILE_LAST completes the last step.
 template <int BIN, int HAM, int PAIRS, int PREC, bool FAC>
-__global__ void __launch_bounds__(kTileThreads, PREC == HG_PRECISION_MIXED && PAIRS == HG_PAIRS_NEIGHBOR_LIST ? 3 : 2)
+__global__ void __launch_bounds__(kTileThreads, tile_waves(PAIRS, PREC))
     k_tile_step(hg_params P, mixed_consts MC, pool_view Vi, pool_view Vo, const wide_block *map, int mode, double half,
                 double dt) {
     constexpr int W = tile_width(PAIRS), KC = kTilePairs / W, ROWS = kTileThreads / W, WAVES = kTileThreads / 64;
@@ -91,6 +102,62 @@ __global__ void __launch_bounds__(kTileThreads, PREC == HG_PRECISION_MIXED && PA
     }
     if (tid == 0) L.contacts = L.ended = 0;
     auto own = [&](int f, uint32_t t) { return d3{L.s[3 * f][t], L.s[3 * f + 1][t], L.s[3 * f + 2][t]}; };
+
+    // Facets f0 .. f0 + 3, one per wavefront (W == 64) or thread group: their
+    // terms to LDS, where fold_facets adds them to the right fold over f.
+    const uint32_t nf = FAC ? Vi.meta[b.slot].nf : 0u;
+    auto facet_terms = [&](uint32_t f0) {
+        if constexpr (FAC) {
+            const uint32_t q = W == 64 ? wv : r0, f = f0 + q;
+            if (q < 4 && f < nf && i < nt) {
+                const facet_dev fd = Vi.facets[size_t(b.slot) * Vi.max_facets + f];
+                auto put = [&](uint32_t c, vec u) {
+                    L.F[q][c][i] = u.x;
+                    L.F[q][c + 1][i] = u.y;
+                    L.F[q][c + 2][i] = u.z;
+                };
+                if constexpr (PREC == HG_PRECISION_FP64) {
+                    const acc6 e = facet_term(P, fd, int(f), Vi.ss, stride, g, own(0, i), own(1, i), own(2, i));
+                    put(0, e.lin);
+                    put(3, e.ang);
+                } else {
+                    accf c;
+                    f3 h;
+                    facet_term_mx(P, MC, fd, int(f), Vi.ss, stride, g, own(0, i), own(1, i), own(2, i), c, h);
+                    put(0, c.lin);
+                    put(3, c.ang);
+                    put(6, h);
+                }
+            }
+        }
+    };
+    vec fsum{};  // rows 0 and 1: this thread's half (force, torque) of the fold so far
+    auto fold_facets = [&](uint32_t f0) {
+        if constexpr (FAC) {
+            if (r0 >= 2) return;
+            for (int f = int(min(f0 + 4u, nf)) - 1; f >= int(f0); f--) {
+                const auto &t = L.F[f - int(f0)];
+                const vec e{t[3 * r0][i], t[3 * r0 + 1][i], t[3 * r0 + 2][i]};
+                if constexpr (PREC == HG_PRECISION_FP64) {
+                    fsum = f == int(nf) - 1 ? e : e + fsum;
+                } else {
+                    if (P.facet_contact) fsum = fsum + e;
+                    if (P.facet_hamaker && r0 == 0) fsum = fsum + vec{t[6][i], t[7][i], t[8][i]};
+                }
+            }
+        }
+    };
+    if constexpr (FAC) {
+        if (nf > 4) {  // all but the first four ahead of the pairs
+            __syncthreads();
+            for (uint32_t f0 = (nf - 1) & ~3u; f0 > 0; f0 -= 4) {
+                facet_terms(f0);
+                __syncthreads();
+                fold_facets(f0);
+                __syncthreads();
+            }
+        }
+    }
 
     const uint32_t seg = wv * 64u * (KC / ROWS);  // this wavefront's part of the queue
     vec accv{};          // W == 64: wavefront 0 sums forces, wavefront 1 torques
@@ -207,25 +274,8 @@ __global__ void __launch_bounds__(kTileThreads, PREC == HG_PRECISION_MIXED && PA
             L.T[4][pos] = ang.y;
             L.T[5][pos] = ang.z;
         }
-        if constexpr (FAC) {
-            // the facets' forces, by the last wavefront beside the pairs
-            const uint32_t nf = k0 == 0 ? Vi.meta[b.slot].nf : 0u;
-            if (nf && tid >= kTileThreads - uint32_t(W) && i < nt) {
-                const facet_dev *F = Vi.facets + size_t(b.slot) * Vi.max_facets;
-                auto put = [&](const auto &f) {
-                    L.F[0][i] = f.lin.x;
-                    L.F[1][i] = f.lin.y;
-                    L.F[2][i] = f.lin.z;
-                    L.F[3][i] = f.ang.x;
-                    L.F[4][i] = f.ang.y;
-                    L.F[5][i] = f.ang.z;
-                };
-                if constexpr (PREC == HG_PRECISION_FP64)
-                    put(facet_fold(P, F, int(nf), Vi.ss, stride, g, own(0, i), own(1, i), own(2, i)));
-                else
-                    put(facet_fold_mx(P, MC, F, int(nf), Vi.ss, stride, g, own(0, i), own(1, i), own(2, i)));
-            }
-        }
+        if constexpr (FAC)
+            if (k0 == 0) facet_terms(0);
         __syncthreads();
         if constexpr (BIN != HG_BINARY_NONE) {
             const uint32_t nc = L.contacts;
@@ -333,7 +383,6 @@ __global__ void __launch_bounds__(kTileThreads, PREC == HG_PRECISION_MIXED && PA
     if constexpr (FAC) {
         // the other set of facets for the next launch, moved by this step
         if (b.start == 0 && tid == kTileThreads - 1 && mode != TILE_FORCE) {
-            const uint32_t nf = Vi.meta[b.slot].nf;
             const facet_dev *F = Vi.facets + size_t(b.slot) * Vi.max_facets;
             facet_dev *O = Vo.facets + size_t(b.slot) * Vo.max_facets;
             for (uint32_t f = 0; f < nf; f++) O[f] = F[f];
@@ -347,7 +396,10 @@ __global__ void __launch_bounds__(kTileThreads, PREC == HG_PRECISION_MIXED && PA
     if constexpr (W == 64) a = accv;
     else a = vec{L.A[3 * r0][i], L.A[3 * r0 + 1][i], L.A[3 * r0 + 2][i]};
     if constexpr (FAC)
-        if (Vi.meta[b.slot].nf) a = a + vec{L.F[3 * r0][i], L.F[3 * r0 + 1][i], L.F[3 * r0 + 2][i]};
+        if (nf) {
+            fold_facets(0);
+            a = a + fsum;
+        }
     d3 a64;
     if constexpr (PREC == HG_PRECISION_FP64) a64 = a;
     else a64 = tod(a);

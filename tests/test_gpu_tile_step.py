@@ -1,6 +1,7 @@
 """The per-step tile kernel against the CPU oracle at the edges of its tiles
-(64 listed particles, 4 with all pairs), with lists longer than the 16
-positions it handles at once and contacts that begin and end. FP64, so state
+(64 listed particles, one with all pairs), with lists longer than the 16
+positions it handles at once (1,024 with all pairs) and contacts that begin and
+end. FP64, so state
 and springs must be equal to the last bit."""
 import numpy as np
 import pytest
@@ -23,7 +24,7 @@ def hot_cloud(n, seed):
 
 
 @pytest.mark.parametrize("pairs", ["all", "list"])
-@pytest.mark.parametrize("n", [1, 3, 4, 5, 63, 64, 65, 129, 257])
+@pytest.mark.parametrize("n", [1, 3, 4, 5, 63, 64, 65, 129, 257, 1024, 1025, 1026])
 def test_tiles_equal_oracle(n, pairs):
     import libgran_amd as L
     print(f"[tile] n {n}, pairs {pairs}", flush=True)
@@ -39,7 +40,7 @@ def test_tiles_equal_oracle(n, pairs):
     every = 20 if pairs == "list" else 0
     changed = 0
     last = None
-    for steps in (1, 2, 97, 60):  # odd and even intervals: both buffers hold the last input
+    for steps in (1, 2, 97, 60) if n < 1000 else (1, 2, 7, 20):  # odd and even intervals: both buffers hold the last input
         o.step(1e-13, steps, rebuild_every=every)
         s.step(1e-13, steps, rebuild_every=every)
         a, b = o.state(), s.state()
@@ -50,8 +51,42 @@ def test_tiles_equal_oracle(n, pairs):
         np.testing.assert_array_equal(s2, s1)
         changed += last is not None and (len(last) != len(ij1) or not np.array_equal(last, ij1))
         last = ij1
-    if n >= 63:
+    if 63 <= n < 1000:
         assert changed  # contacts began or ended between the looks
+    s.close()
+
+
+@pytest.mark.parametrize("terms", ["both", "contact", "hamaker"])
+@pytest.mark.parametrize("pairs", [0, 1])
+@pytest.mark.parametrize("nf", [1, 4, 5, 9])
+def test_facet_terms_in_fours(nf, pairs, terms):
+    """Facets four at a time over the threads of a tile: the right fold over
+    all of them, in tiles of both kinds."""
+    import libgran_amd as L
+    from libgran_amd import workloads
+    import _scenarios as S
+    print(f"[tile] {nf} facets, pairs {pairs}, {terms}", flush=True)
+    x = L.generate_aggregate(70, R, 1.8, 1.3, 3)
+    v = np.random.default_rng(3).normal(0.0, 1.0, x.shape)
+    c, sn, h = S.aggregate_params()
+    sets = [workloads.plates(x, R, 5.0 + 0.5 * q) for q in range(3)]
+    verts = np.concatenate([q[0] for q in sets])[:nf]
+    vel = np.concatenate([q[1] for q in sets])[:nf]
+    fac = dict(facet_contact=int(terms != "hamaker"), facet_hamaker=int(terms != "contact"), surface_contact=c,
+               surface_hamaker=h)
+    kw = dict(r_verlet=3.2 * R) if pairs else {}
+    o = O.OracleSystem(O.system_params(O.BIN_SINTER, O.HAM_LIMITED, neighbor_mode=pairs, contact=c, sinter=sn,
+                                       hamaker=h, **kw, **fac), x, v)
+    s = L.System(L.make_params(L.BINARY_SINTER, L.HAMAKER_LIMITED, pair_mode=pairs, contact=c, sinter=sn, hamaker=h,
+                               **kw, **fac), x, v)
+    s.per_step_launches(True)
+    o.set_facets(verts, vel)
+    s.set_facets(verts, vel)
+    o.step(1e-13, 60, rebuild_every=20 * pairs)
+    s.step(1e-13, 60, rebuild_every=20 * pairs)
+    a, b = o.state(), s.state()
+    for k in ("x", "v", "theta", "omega", "a", "alpha"):
+        np.testing.assert_array_equal(b[k], a[k], err_msg=k)
     s.close()
 
 
