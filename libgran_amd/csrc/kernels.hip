@@ -542,8 +542,11 @@ __global__ void __launch_bounds__(1024) k_diag(const double *x, const double *v,
                                                double mass, double inertia, double *out) {
     __shared__ double red[8][1024];
     double acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};  // 2*KE_trans, 2*KE_rot, sum v (3), L (3)
+    d3 cmsum = zero3();
+#pragma unroll 4
     for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) {
         d3 vi = ld3(v, i), wi = ld3(w, i), xi = ld3(x, i);
+        cmsum = cmsum + xi;
         acc[0] += mass * dot(vi, vi);
         acc[1] += inertia * dot(wi, wi);
         acc[2] += vi.x; acc[3] += vi.y; acc[4] += vi.z;
@@ -557,8 +560,6 @@ __global__ void __launch_bounds__(1024) k_diag(const double *x, const double *v,
             for (int c = 0; c < 8; c++) red[c][threadIdx.x] += red[c][threadIdx.x + s];
         __syncthreads();
     }
-    d3 cmsum = zero3();
-    for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) cmsum = cmsum + ld3(x, i);
     __syncthreads();
     double k0 = red[0][0], k1 = red[1][0];
     d3 P{red[2][0], red[3][0], red[4][0]}, L{red[5][0], red[6][0], red[7][0]};
@@ -573,6 +574,7 @@ __global__ void __launch_bounds__(1024) k_diag(const double *x, const double *v,
     const d3 cm = d3{red[0][0], red[1][0], red[2][0]} / double(n);
     __syncthreads();
     double rg = 0.0;
+#pragma unroll 4
     for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) {
         d3 dd = ld3(x, i) - cm;
         rg += dot(dd, dd);
@@ -600,24 +602,41 @@ __global__ void __launch_bounds__(1024) k_diag(const double *x, const double *v,
 // split evenly between the two particles of a pair and each ordered pair's
 // springs carry half of that pair's spring energy, so the sums over all
 // particles count every pair once.
+//
+// Eight lanes share a particle: each takes every eighth row entry and partner,
+// and the eight contributions are added in the order of one lane walking them,
+// so the sums do not depend on the split. One lane per particle left 79
+// wavefronts at 5,000 particles, each a chain of 13 dependent partners.
 __global__ void __launch_bounds__(256) k_energy(hg_params P, energy_view E, double mass, double inertia,
                                                 double *out) {
-    const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
+    constexpr uint32_t G = 8;
+    const uint32_t k = (blockIdx.x * blockDim.x + threadIdx.x) / G, l = threadIdx.x % G;
     if (k >= E.n) return;
     const uint32_t g = E.offset + k;
     const d3 xi = ld3(E.x, g), vi = ld3(E.v, g), wi = ld3(E.w, g);
     double e[8] = {0.5 * mass * dot(vi, vi), 0.5 * inertia * dot(wi, wi), 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    auto add = [&](double &to, double term) {
+#pragma unroll
+        for (uint32_t q = 0; q < G; q++) to += __shfl(term, int(q), int(G));
+    };
     const uint32_t cnt = E.pcnt ? E.pcnt[g] : 0u;
-    for (uint32_t s = 0; s < cnt; s++) {
-        const bool bonded = (E.pj[size_t(s) * E.stride + g] & kBondBit) != 0;
-        const spring9 sp = ld_rec(E.ps + (size_t(s) * E.stride + g) * kSpringRec);
-        const double kt = bonded ? P.sinter.k_t : P.contact.k_t, kr = bonded ? P.sinter.k_r : P.contact.k_r,
-                     ko = bonded ? P.sinter.k_o : P.contact.k_o;
-        e[3] += 0.25 * kt * dot(sp.s[0], sp.s[0]);
-        e[4] += 0.25 * kr * dot(sp.s[1], sp.s[1]);
-        e[5] += 0.25 * ko * dot(sp.s[2], sp.s[2]);
+    for (uint32_t s0 = 0; s0 < cnt; s0 += G) {
+        const uint32_t s = s0 + l;
+        double t[3] = {0.0, 0.0, 0.0};
+        if (s < cnt) {
+            const bool bonded = (E.pj[size_t(s) * E.stride + g] & kBondBit) != 0;
+            const spring9 sp = ld_rec(E.ps + (size_t(s) * E.stride + g) * kSpringRec);
+            const double kt = bonded ? P.sinter.k_t : P.contact.k_t, kr = bonded ? P.sinter.k_r : P.contact.k_r,
+                         ko = bonded ? P.sinter.k_o : P.contact.k_o;
+            t[0] = 0.25 * kt * dot(sp.s[0], sp.s[0]);
+            t[1] = 0.25 * kr * dot(sp.s[1], sp.s[1]);
+            t[2] = 0.25 * ko * dot(sp.s[2], sp.s[2]);
+        }
+        for (int c = 0; c < 3; c++) add(e[3 + c], t[c]);
     }
-    auto pair = [&](uint32_t j) {
+    // a partner's share of the bond energies in row order, and of the Hamaker
+    // potential; a legacy bond adds five of the first kind
+    auto pair = [&](uint32_t j, double (&bond)[5], double &ham) {
         const double dist = norm(xi - ld3(E.x, j));
         uint32_t ls = kNoEntry;
         if (E.lconn)
@@ -631,7 +650,7 @@ __global__ void __launch_bounds__(256) k_energy(hg_params P, energy_view E, doub
             for (int q = 0; q < 5; q++) {
                 const d3 sq = d3{rj[3 * q], rj[3 * q + 1], rj[3 * q + 2]} - d3{ri[3 * q], ri[3 * q + 1], ri[3 * q + 2]};
                 const double d = (q < 4 ? 2.0 * P.contact.r_part : 0.0) - norm(sq);
-                e[2] += 0.25 * P.sinter.k * d * d;
+                bond[q] = 0.25 * P.sinter.k * d * d;
             }
         } else if (P.binary_model != HG_BINARY_NONE) {
             bool bonded = false;
@@ -641,22 +660,32 @@ __global__ void __launch_bounds__(256) k_energy(hg_params P, energy_view E, doub
             }
             if (bonded) {
                 const double ov = 2.0 * P.sinter.r_part - dist;
-                e[2] += 0.25 * P.sinter.k * ov * ov;
+                bond[0] = 0.25 * P.sinter.k * ov * ov;
             } else {
                 const double ov = 2.0 * P.contact.r_part - dist;
-                if (ov > 0.0) e[2] += 0.25 * P.contact.k * ov * ov;
+                if (ov > 0.0) bond[0] = 0.25 * P.contact.k * ov * ov;
             }
         }
-        if (P.hamaker_model != HG_HAMAKER_NONE) e[6] += 0.5 * hamaker_potential(P.hamaker_model, P.hamaker, dist);
+        if (P.hamaker_model != HG_HAMAKER_NONE) ham = 0.5 * hamaker_potential(P.hamaker_model, P.hamaker, dist);
     };
-    if (E.nb) {
-        const uint32_t m = E.ncnt[g];
-        for (uint32_t q = 0; q < m; q++) pair(E.nb[size_t(q) * E.stride + g]);
-    } else {
-        for (uint32_t j = E.offset; j < E.offset + E.n; j++)
-            if (j != g) pair(j);
+    const uint32_t m = E.nb ? E.ncnt[g] : E.n;
+    for (uint32_t q0 = 0; q0 < m; q0 += G) {
+        const uint32_t q = q0 + l;
+        double bond[5] = {0.0, 0.0, 0.0, 0.0, 0.0}, ham = 0.0;
+        if (q < m) {
+            const uint32_t j = E.nb ? E.nb[size_t(q) * E.stride + g] : E.offset + q;
+            if (j != g) pair(j, bond, ham);
+        }
+        if (E.lconn) {
+            for (uint32_t t = 0; t < G; t++)
+                for (int c = 0; c < 5; c++) e[2] += __shfl(bond[c], int(t), int(G));
+        } else {
+            add(e[2], bond[0]);
+        }
+        add(e[6], ham);
     }
-    for (int c = 0; c < 8; c++) out[8 * size_t(k) + c] = e[c];
+    if (l == 0)
+        for (int c = 0; c < 8; c++) out[8 * size_t(k) + c] = e[c];
 }
 
 inline unsigned blocks_for(size_t n, unsigned bs) { return unsigned((n + bs - 1) / bs); }
@@ -1195,7 +1224,7 @@ hipError_t launch_diagnostics(const double *x, const double *v, const double *w,
 hipError_t launch_energy(const hg_params &p, const energy_view &E, double mass, double inertia, double *out,
                          hipStream_t s) {
     if (E.n == 0) return hipSuccess;
-    k_energy<<<blocks_for(E.n, 256), 256, 0, s>>>(p, E, mass, inertia, out);
+    k_energy<<<blocks_for(8 * size_t(E.n), 256), 256, 0, s>>>(p, E, mass, inertia, out);
     return hipGetLastError();
 }
 

@@ -24,9 +24,22 @@ host_stage::~host_stage() {
     if (p) (void)hipHostFree(p);
 }
 
+// Doubles of stage that n particles' four fields, energy terms or diagnostics
+// take, up to kStageMost: one allocation serves them all.
+size_t stage_size(size_t n) { return std::min(std::max<size_t>(n * 12, 1024), kStageMost); }
+
+hg_status need_stage(host_stage &stage, size_t doubles) {
+    if (stage.cap >= doubles) return HG_OK;
+    if (stage.p) HG_HIP(hipHostFree(stage.p));
+    stage.p = nullptr;
+    stage.cap = 0;
+    HG_HIP(hipHostMalloc(reinterpret_cast<void **>(&stage.p), doubles * sizeof(double)));
+    stage.cap = doubles;
+    return HG_OK;
+}
+
 hg_status read_fields(host_stage &stage, const double *const *src, double *const *dst, int count, size_t n,
                       hipStream_t s) {
-    constexpr size_t kMost = size_t(1) << 20;  // doubles: 8 MB
     const double *from[4];
     double *to[4];
     int m = 0;
@@ -36,14 +49,10 @@ hg_status read_fields(host_stage &stage, const double *const *src, double *const
             to[m++] = dst[f];
         }
     if (m == 0 || n == 0) return HG_OK;
-    const size_t part = std::min(n, kMost / (3 * size_t(m)));
+    const size_t part = std::min(n, kStageMost / (3 * size_t(m)));
     if (stage.cap < part * 3 * size_t(m)) {
-        if (stage.p) HG_HIP(hipHostFree(stage.p));
-        stage.p = nullptr;
-        stage.cap = 0;
-        const size_t cap = std::min(std::max<size_t>(part * 12, 1024), kMost);
-        HG_HIP(hipHostMalloc(reinterpret_cast<void **>(&stage.p), cap * sizeof(double)));
-        stage.cap = cap;
+        const hg_status st = need_stage(stage, stage_size(n));
+        if (st != HG_OK) return st;
     }
     for (size_t i = 0; i < n; i += part) {
         const size_t c = std::min(part, n - i);
@@ -392,7 +401,6 @@ hg_status create_impl(const hg_params *params, size_t n, const double *x0, const
     HG_TRYC(dalloc(S, &S->flags, FLAG_COUNT));
     HG_HIPC(hipHostMalloc(reinterpret_cast<void **>(&S->flags_host), FLAG_COUNT * sizeof(int)));
     HG_HIPC(hipMemsetAsync(S->flags, 0, FLAG_COUNT * sizeof(int), S->stream));
-    HG_TRYC(dalloc(S, &S->red, 16));
 
     // Bond topology (alt_sinter ctor) and the initial pair-state table.
     std::vector<std::vector<uint32_t>> rows(n);
@@ -1030,16 +1038,16 @@ hg_status hg_set_neck_strengths(hg_system *S, const double *strengths) {
 hg_status hg_diagnostics(hg_system *S, double mass, double inertia, double *out) {
     if (!S || !out) return fail(HG_ERR_INVALID, "system and out are required");
     HG_TRY(settle(S, "hg_diagnostics"));
-    HG_HIP(launch_diagnostics(S->x, S->v, S->w, uint32_t(S->n), mass, inertia, S->red, S->stream));
-    HG_HIP(hipMemcpyAsync(out, S->red, 9 * sizeof(double), hipMemcpyDeviceToHost, S->stream));
+    HG_TRY(need_stage(S->stage, stage_size(S->n)));
+    HG_HIP(launch_diagnostics(S->x, S->v, S->w, uint32_t(S->n), mass, inertia, S->stage.p, S->stream));
     HG_HIP(hipStreamSynchronize(S->stream));
+    std::copy(S->stage.p, S->stage.p + 9, out);
     return HG_OK;
 }
 
 hg_status hg_energy(hg_system *S, double mass, double inertia, double *out) {
     if (!S || !out) return fail(HG_ERR_INVALID, "system and out are required");
     HG_TRY(settle(S, "hg_energy"));
-    if (!S->energy) HG_TRY(dalloc(S, &S->energy, size_t(8) * S->n));
     const bool nl = S->p.pair_mode == HG_PAIRS_NEIGHBOR_LIST, bin = S->p.binary_model != HG_BINARY_NONE;
     energy_view E{S->x,
                   S->v,
@@ -1058,6 +1066,15 @@ hg_status hg_energy(hg_system *S, double mass, double inertia, double *out) {
                   S->lconn};
     if (S->p.binary_model == HG_BINARY_SINTER_LEGACY && !S->legacy_ready)
         return fail(HG_ERR_INVALID, "hg_energy: the legacy sinter_functor's connectors are not set");
+    const size_t words = size_t(8) * S->n;
+    if (words <= kStageMost) {  // the terms straight into pinned memory
+        HG_TRY(need_stage(S->stage, stage_size(S->n)));
+        HG_HIP(launch_energy(S->p, E, mass, inertia, S->stage.p, S->stream));
+        HG_HIP(hipStreamSynchronize(S->stream));
+        sum_energy(S->stage.p, S->n, out);
+        return HG_OK;
+    }
+    if (!S->energy) HG_TRY(dalloc(S, &S->energy, words));
     HG_HIP(launch_energy(S->p, E, mass, inertia, S->energy, S->stream));
     std::vector<double> h(size_t(8) * S->n);
     HG_HIP(hipMemcpyAsync(h.data(), S->energy, h.size() * sizeof(double), hipMemcpyDeviceToHost, S->stream));

@@ -26,7 +26,7 @@ def check(x, r_list, capacity=0):
     return off1
 
 
-@pytest.mark.parametrize("n", [1, 2, 15, 16, 17, 63, 64, 65, 255, 256, 257, 513, 8192, 8193])
+@pytest.mark.parametrize("n", [1, 2, 15, 16, 17, 63, 64, 65, 255, 256, 257, 513, 2047, 2048, 2049, 9001])
 def test_lists_equal_oracle(n):
     rng = np.random.default_rng(n)
     side = 2.2 * R * n ** (1.0 / 3.0)
