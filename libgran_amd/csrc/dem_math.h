@@ -169,12 +169,11 @@ HGD d3 shear_sinter(d3 &xi, d3 n, double stiffness, double damping, d3 rel_v, do
 
 // ---- alt_sinter_bridge.h:92-129 (bonded branch; no overlap gate) ----------
 // ftot receives f_n n + f_t, the force alt_breaking_sinter_bridge.h:115-118
-// compares with the neck strength. TRACK: as contact_eval_vw.
+// compares with the neck strength. TRACK: as contact_eval_vw. d = xi - xj and n
+// its direction.
 template <bool TRACK = false>
-HGD acc6 sinter_eval(const hg_sinter_params &p, d3 xi, d3 xj, d3 vi, d3 vj, d3 wi, d3 wj, spring9 &sp, d3 &ftot,
-                     double *d4 = nullptr) {
-    d3 d = xi - xj;
-    d3 n = normalized(d);
+HGD acc6 sinter_eval_n(const hg_sinter_params &p, d3 d, d3 n, d3 vi, d3 vj, d3 wi, d3 wj, spring9 &sp, d3 &ftot,
+                       double *d4 = nullptr) {
     double overlap = 2.0 * p.r_part - dot(d, n);
     double rpp = p.r_part - overlap / 2.0;
     double v_n = -dot(vi - vj, n);
@@ -200,6 +199,12 @@ HGD acc6 sinter_eval(const hg_sinter_params &p, d3 xi, d3 xj, d3 vi, d3 vj, d3 w
     d3 tau_o = p.r_part * f_o;
     ftot = f_n * n + f_t;
     return {ftot / p.mass, ((-tau_t + tau_r) + tau_o) / p.inertia};
+}
+template <bool TRACK = false>
+HGD acc6 sinter_eval(const hg_sinter_params &p, d3 xi, d3 xj, d3 vi, d3 vj, d3 wi, d3 wj, spring9 &sp, d3 &ftot,
+                     double *d4 = nullptr) {
+    const d3 d = xi - xj;
+    return sinter_eval_n<TRACK>(p, d, normalized(d), vi, vj, wi, wj, sp, ftot, d4);
 }
 
 // ---- sinter_bridge.h:235-259 (legacy sinter_functor, bonded pair) --------

@@ -184,13 +184,12 @@ struct hg_system_impl {
     // reductions
     double *energy = nullptr;  // per-particle ledger terms, 8 per particle (allocated on first use)
     // per-step launches (tile_step.h), on first use: the second x, v, omega
-    // and facets, the system's meta and its tiles
+    // and facets, and the system's meta
     double *tile_state = nullptr;
     facet_dev *tile_facets = nullptr;
-    void *tile_meta = nullptr, *tile_map = nullptr;
+    void *tile_meta = nullptr;
     unsigned tile_blocks = 0;
-    int tile_cur = -1;  // the table half `tile_map` names
-    int tile_nf = -1;   // the facet count `tile_meta` holds
+    int tile_nf = -1;  // the facet count `tile_meta` holds
     // host copies of the topology
     std::vector<std::pair<uint32_t, uint32_t>> bonds;
     size_t bonds_skipped = 0;

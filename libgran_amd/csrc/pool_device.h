@@ -30,6 +30,7 @@ struct pool_view {
     size_t stride;
     int *flags;
     int *sflags;  // per-system fault words (HG_FAULT_* bits), indexed by slot
+    uint32_t alone;  // wide_block::n of a single system, whose tiles need no map
 };
 
 constexpr uint32_t kDefaultWideMin = 2048;
@@ -43,8 +44,13 @@ enum { TUNE_OFF = 0, TUNE_START = 1, TUNE_RUNNING = 2, TUNE_DONE = 3 };
 struct wide_block {
     uint32_t slot, start, offset, n;
 };
-constexpr uint32_t kTileThreads = 256, kTilePairs = 1024;
+constexpr uint32_t kTileThreads = 256;
 constexpr int tile_width(int pairs) { return pairs == HG_PAIRS_NEIGHBOR_LIST ? 64 : 1; }
+// List positions a tile takes at a time. Their terms take most of its LDS: with
+// twelve, an aggregate's longest lists (r_verlet of 3.2 radii) still fit one
+// round, and an FP64 tile takes 52 KB, 70 with facets (sixteen: 70 and 90, one
+// workgroup to a CU with facets).
+constexpr int tile_depth(int pairs) { return pairs == HG_PAIRS_NEIGHBOR_LIST ? 12 : 1024; }
 enum { TILE_FORCE = 0, TILE_STEP = 1, TILE_LAST = 2 };
 
 // The launches of one binary functor and pair mode (pool_chunk.hip), by

@@ -245,32 +245,23 @@ sys_view make_view(hg_system *S) {
 bool tiled(const hg_system *S) { return S->p.binary_model != HG_BINARY_SINTER_LEGACY && !S->track_diss; }
 
 // The views of a tiled system: its own buffers and the second set. What the
-// device needs beside them is made on first use and refreshed when the
-// current half of the table or the facet count has changed.
+// device needs beside them is made on first use and refreshed when the facet
+// count has changed.
 hg_status tile_views(hg_system *S, pool_view &V, pool_view &VB) {
     const size_t n = S->n, width = size_t(tile_width(S->p.pair_mode));
     if (!S->tile_state) {
         HG_TRY(dalloc(S, &S->tile_state, 12 * n));
         HG_TRY(dalloc(S, &S->tile_facets, kMaxFacets));
         S->tile_blocks = unsigned((n + width - 1) / width);
-        wide_block *map = nullptr;
         pool_meta *meta = nullptr;
-        HG_TRY(dalloc(S, &map, S->tile_blocks));
         HG_TRY(dalloc(S, &meta, 1));
-        S->tile_map = map;
         S->tile_meta = meta;
     }
     if (!S->facets) HG_TRY(dalloc(S, &S->facets, kMaxFacets));
-    if (S->tile_cur != S->cur || S->tile_nf != S->nf) {
-        std::vector<wide_block> map;
-        for (size_t st = 0; st < n; st += width)
-            map.push_back(wide_block{0, uint32_t(st), 0, uint32_t(n) | (S->cur ? kBondBit : 0u)});
-        const pool_meta M{0, uint32_t(n), uint32_t(S->cur), 0, uint32_t(S->nf), 0, 0, 0};
-        HG_HIP(hipMemcpyAsync(S->tile_map, map.data(), map.size() * sizeof(wide_block), hipMemcpyHostToDevice,
-                              S->stream));
+    if (S->tile_nf != S->nf) {
+        const pool_meta M{0, uint32_t(n), 0, 0, uint32_t(S->nf), 0, 0, 0};
         HG_HIP(hipMemcpyAsync(S->tile_meta, &M, sizeof(M), hipMemcpyHostToDevice, S->stream));
         HG_HIP(hipStreamSynchronize(S->stream));
-        S->tile_cur = S->cur;
         S->tile_nf = S->nf;
     }
     V = pool_view{};
@@ -292,6 +283,7 @@ hg_status tile_views(hg_system *S, pool_view &V, pool_view &VB) {
     V.meta = static_cast<const pool_meta *>(S->tile_meta);
     V.stride = n;
     V.flags = S->flags;
+    V.alone = uint32_t(n) | (S->cur ? kBondBit : 0u);
     VB = V;
     VB.x = S->tile_state;
     VB.v = S->tile_state + 4 * n;
@@ -308,8 +300,7 @@ hg_status force_pass(hg_system *S) {
         pool_view V, VB;
         HG_TRY(tile_views(S, V, VB));
         HG_HIP(timed(S, PHASE_FORCE, [&] {
-            return launch_tile(S->p, V, V, static_cast<const wide_block *>(S->tile_map), S->tile_blocks, TILE_FORCE,
-                               S->nf > 0, 0.0, 0.0, S->stream);
+            return launch_tile(S->p, V, V, nullptr, S->tile_blocks, TILE_FORCE, S->nf > 0, 0.0, 0.0, S->stream);
         }));
         return HG_OK;
     }
@@ -689,7 +680,6 @@ hg_status step_impl(hg_system *S, double dt, uint64_t nsteps, uint32_t rebuild_e
     if (tiled(S)) {
         pool_view V, VB;
         HG_TRY(tile_views(S, V, VB));
-        const wide_block *map = static_cast<const wide_block *>(S->tile_map);
         for (uint64_t s = 0; s < nsteps;) {
             if (nl && rebuild_every && (S->step_index % rebuild_every) == 0)
                 HG_HIP(timed(S, PHASE_REBUILD, [&] { return launch_neighbor_build(*S, S->stream); }));
@@ -700,11 +690,11 @@ hg_status step_impl(hg_system *S, double dt, uint64_t nsteps, uint32_t rebuild_e
             // its pass (one launch); the kick phase is the interval's first
             const pool_view *in = len % 2 ? &VB : &V, *out = len % 2 ? &V : &VB;
             HG_HIP(timed(S, PHASE_KICK, [&] {
-                return launch_tile_kick(V, *in, map, S->tile_blocks, S->p.pair_mode, half, dt, S->stream);
+                return launch_tile_kick(V, *in, nullptr, S->tile_blocks, S->p.pair_mode, half, dt, S->stream);
             }));
             for (uint64_t k = 0; k < len; k++) {
                 HG_HIP(timed(S, PHASE_FORCE, [&] {
-                    return launch_tile(S->p, *in, *out, map, S->tile_blocks, k + 1 < len ? TILE_STEP : TILE_LAST,
+                    return launch_tile(S->p, *in, *out, nullptr, S->tile_blocks, k + 1 < len ? TILE_STEP : TILE_LAST,
                                        S->nf > 0, half, dt, S->stream);
                 }));
                 std::swap(in, out);

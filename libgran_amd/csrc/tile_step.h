@@ -35,7 +35,7 @@ namespace {
 template <int W, int KC, int PREC, bool FAC>
 struct tile_lds {
     using term = typename prec_types<PREC>::term;
-    double s[9][W];  // x, v, omega
+    double s[12][W];  // x, v, omega, theta
     term T[6][KC * W];
     uint2 Q[KC * W];  // partner, and i | kk << 8 | row slot << 20
     uint16_t CW[KC * W];
@@ -50,6 +50,12 @@ struct tile_lds {
 
 constexpr uint32_t kNoRowSlot = 0xFFFu;
 
+// This workgroup's tile: from the map or, without one, of the view's only
+// system, so that a single system's tile waits for no load.
+__device__ __forceinline__ wide_block tile_block(const wide_block *map, const pool_view &V, uint32_t width) {
+    return map ? map[blockIdx.x] : wide_block{0, blockIdx.x * width, 0, V.alone};
+}
+
 // Wavefronts per SIMD that the registers leave room for. Listed tiles, many to
 // a CU, hide one pair's latency behind another's: mixed 151 us a step at
 // 635,000 particles with three, 187 with two (four spill: 241). All pairs come
@@ -59,6 +65,20 @@ constexpr int tile_waves(int pairs, int prec) {
     return pairs != HG_PAIRS_NEIGHBOR_LIST ? 1 : (prec == HG_PRECISION_MIXED ? 3 : 2);
 }
 
+// A launch's arguments (the parameter set, its mixed form and two views, 1.5 KB)
+// lie in memory that no cache holds yet. Read where they are used, they were
+// three or four round trips one after the other, 4,400 cycles; one word of each
+// 64-byte line read together at the start brings them all in for 1,250.
+template <size_t BYTES>
+__device__ __forceinline__ void touch_args() {
+    using words = const __attribute__((address_space(4))) uint32_t;
+    words *a = (words *)__builtin_amdgcn_kernarg_segment_ptr();
+    uint32_t any = 0;
+#pragma unroll
+    for (size_t q = 0; q < BYTES / 4; q += 16) any |= a[q];
+    asm volatile("" ::"s"(any));
+}
+
 // What a launch does after the pass: TILE_FORCE stores the accelerations of
 // the systems that have none; TILE_STEP completes the step, kicks and drifts
 // into the other buffers; TILE_LAST completes the last step.
@@ -66,11 +86,12 @@ template <int BIN, int HAM, int PAIRS, int PREC, bool FAC>
 __global__ void __launch_bounds__(kTileThreads, tile_waves(PAIRS, PREC))
     k_tile_step(hg_params P, mixed_consts MC, pool_view Vi, pool_view Vo, const wide_block *map, int mode, double half,
                 double dt) {
-    constexpr int W = tile_width(PAIRS), KC = kTilePairs / W, ROWS = kTileThreads / W, WAVES = kTileThreads / 64;
+    constexpr int W = tile_width(PAIRS), KC = tile_depth(PAIRS), ROWS = kTileThreads / W, WAVES = kTileThreads / 64;
     using term = typename prec_types<PREC>::term;
     using vec = typename prec_types<PREC>::vec;
     __shared__ tile_lds<W, KC, PREC, FAC> L;
-    const wide_block b = map[blockIdx.x];
+    touch_args<sizeof(hg_params) + sizeof(mixed_consts) + 2 * sizeof(pool_view)>();
+    const wide_block b = tile_block(map, Vi, W);
     const uint32_t n = b.n & kIdxMask, cur = b.n >> 31, base = b.offset + b.start;
     const uint32_t nt = n - b.start < uint32_t(W) ? n - b.start : uint32_t(W);
     const uint32_t tid = threadIdx.x, wv = tid >> 6, lane = tid & 63u;
@@ -82,20 +103,34 @@ __global__ void __launch_bounds__(kTileThreads, tile_waves(PAIRS, PREC))
 
     const uint32_t i = tid % W, r0 = tid / W;  // own particle of the tile, first list row
     const uint32_t g = base + (i < nt ? i : 0);
-    uint32_t cnt = 0, c_old = 0;
-    if (i < nt) {
-        cnt = PAIRS == HG_PAIRS_NEIGHBOR_LIST ? Vi.ncnt[g] : n - 1u;
-        if constexpr (BIN != HG_BINARY_NONE) c_old = pcnt[g];
+    // Everything that only the tile's place tells is loaded in one go: counts,
+    // tags, the first part of the list (whatever its length) and the state. With
+    // tags and list loaded once the counts and the state were there, they took
+    // another round trip or two of some 1,700 cycles. With the arguments above,
+    // the list's depth of 12 and the sums below: 200 particles, 500 steps 4.42 ->
+    // 3.98 ms; 213,000 in 333 systems, FP64, 76.6 -> 71.5 ms.
+    uint32_t cnt = n - 1u, c_old = 0;
+    if constexpr (PAIRS == HG_PAIRS_NEIGHBOR_LIST) cnt = Vi.ncnt[g];
+    if constexpr (BIN != HG_BINARY_NONE) c_old = pcnt[g];
+    uint32_t tags[4], js[KC / ROWS];
+    if constexpr (BIN != HG_BINARY_NONE) {
+#pragma unroll
+        for (uint32_t s = 0; s < 4; s++) tags[s] = pj[size_t(s < Vi.cap_s ? s : 0u) * stride + g];
     }
-    for (uint32_t q = tid; q < 3u * W; q += kTileThreads) {
-        const uint32_t f = q / W, t = q % W;
-        if (t < nt) {
-            const d3 a = ld3(f == 0 ? Vi.x : (f == 1 ? Vi.v : Vi.w), base + t);
-            L.s[3 * f][t] = a.x;
-            L.s[3 * f + 1][t] = a.y;
-            L.s[3 * f + 2][t] = a.z;
+    if constexpr (PAIRS == HG_PAIRS_NEIGHBOR_LIST) {
+#pragma unroll
+        for (uint32_t q = 0; q < KC / ROWS; q++) {
+            const uint32_t k = r0 + q * ROWS;
+            js[q] = Vi.nb[size_t(k < Vi.cap_n ? k : 0u) * stride + g];
         }
     }
+    if (r0 < 4) {
+        const d3 a = ld3(r0 == 0 ? Vi.x : (r0 == 1 ? Vi.v : (r0 == 2 ? Vi.w : Vi.th)), g);
+        L.s[3 * r0][i] = a.x;
+        L.s[3 * r0 + 1][i] = a.y;
+        L.s[3 * r0 + 2][i] = a.z;
+    }
+    if (i >= nt) cnt = c_old = 0;
     if (tid < uint32_t(W)) {
         L.rows[tid] = c_old;
         L.dirty[tid] = 0;
@@ -165,17 +200,16 @@ __global__ void __launch_bounds__(kTileThreads, tile_waves(PAIRS, PREC))
     for (uint32_t k0 = 0;; k0 += KC) {
         // queue the pairs of list positions k0 .. k0 + KC - 1: bonded ones
         // from the front of the wavefront's part, the others from its back
-        uint32_t tags[4];
         if constexpr (BIN != HG_BINARY_NONE) {
 #pragma unroll
-            for (uint32_t s = 0; s < 4; s++) tags[s] = s < c_old ? pj[size_t(s) * stride + g] : kNoEntry;
+            for (uint32_t s = 0; s < 4; s++)
+                if (s >= c_old) tags[s] = kNoEntry;
         }
-        uint32_t js[KC / ROWS];
 #pragma unroll
         for (uint32_t q = 0; q < KC / ROWS; q++) {
             const uint32_t k = k0 + r0 + q * ROWS;
-            if constexpr (PAIRS == HG_PAIRS_NEIGHBOR_LIST) js[q] = k < cnt ? Vi.nb[size_t(k) * stride + g] : kNoEntry;
-            else js[q] = k < cnt ? b.offset + k + (k >= b.start + i ? 1u : 0u) : kNoEntry;
+            if constexpr (PAIRS != HG_PAIRS_NEIGHBOR_LIST) js[q] = b.offset + k + (k >= b.start + i ? 1u : 0u);
+            if (k >= cnt) js[q] = kNoEntry;
         }
         uint32_t nB = 0, nO = 0;
 #pragma unroll
@@ -362,19 +396,59 @@ __global__ void __launch_bounds__(kTileThreads, tile_waves(PAIRS, PREC))
         if constexpr (W == 64) {
             if (wv < 2) {
                 const uint32_t left = cnt > k0 ? cnt - k0 : 0u, end = left < uint32_t(KC) ? left : uint32_t(KC);
-                for (uint32_t kk = 0; kk < end; kk++)
-                    accv = accv + vec{L.T[3 * wv][kk * W + i], L.T[3 * wv + 1][kk * W + i], L.T[3 * wv + 2][kk * W + i]};
+                for (uint32_t kk = 0; kk < end; kk += 4) {  // KC is a multiple of 4
+                    // a sum that starts at +0 is never -0: adding +0 for the
+                    // places past a list's end changes nothing
+                    vec t[4];
+#pragma unroll
+                    for (uint32_t u = 0; u < 4; u++) {
+                        t[u] = vec{L.T[3 * wv][(kk + u) * W + i], L.T[3 * wv + 1][(kk + u) * W + i],
+                                   L.T[3 * wv + 2][(kk + u) * W + i]};
+                        if (kk + u >= end) t[u] = vec{};
+                    }
+#pragma unroll
+                    for (uint32_t u = 0; u < 4; u++) accv = accv + t[u];
+                }
             }
             if (!__any(cnt > k0 + KC)) break;  // every wavefront sees the same 64 counts
         } else {
             const uint32_t all = n - 1u, left = all > k0 ? all - k0 : 0u,
                            end = left < uint32_t(KC) ? left : uint32_t(KC);
-            if (tid < 6u * W)
-                for (uint32_t kk = 0; kk < end; kk++) acct = acct + L.T[r0][kk * W + i];
+            if (tid < 6u * W) {
+                // sixteen terms fetched while the sixteen before are added: the
+                // adds are one chain, the fetches need not be
+                term t[16], u[16];
+                auto fetch = [&](term *to, uint32_t from) {
+#pragma unroll
+                    for (uint32_t q = 0; q < 16; q++) to[q] = L.T[r0][(from + q) * W + i];
+                };
+                const uint32_t full = end & ~15u;
+                if (full) fetch(t, 0);
+                for (uint32_t kk = 0; kk < full; kk += 16) {
+                    fetch(u, kk + 16 < full ? kk + 16 : 0u);
+#pragma unroll
+                    for (uint32_t q = 0; q < 16; q++) {
+                        acct = acct + t[q];
+                        t[q] = u[q];
+                    }
+                }
+                for (uint32_t kk = full; kk < end; kk++) acct = acct + L.T[r0][kk * W + i];
+            }
             if (k0 + KC >= all) break;
         }
         __syncthreads();
-        if constexpr (BIN != HG_BINARY_NONE) c_old = L.rows[i];
+        if constexpr (BIN != HG_BINARY_NONE) {
+            c_old = L.rows[i];
+#pragma unroll
+            for (uint32_t s = 0; s < 4; s++) tags[s] = pj[size_t(s < Vi.cap_s ? s : 0u) * stride + g];
+        }
+        if constexpr (PAIRS == HG_PAIRS_NEIGHBOR_LIST) {
+#pragma unroll
+            for (uint32_t q = 0; q < KC / ROWS; q++) {
+                const uint32_t k = k0 + KC + r0 + q * ROWS;
+                if (k < cnt) js[q] = Vi.nb[size_t(k) * stride + g];
+            }
+        }
     }
     if constexpr (W < 64) {
         if (tid < 6u * W) L.A[r0][i] = acct;
@@ -410,7 +484,7 @@ __global__ void __launch_bounds__(kTileThreads, tile_waves(PAIRS, PREC))
     if (mode == TILE_STEP) {
         u = u + a64 * half;
         if (r0 == 0) st3(Vo.x, g, own(0, i) + u * dt);
-        else st3(Vi.th, g, ld3(Vi.th, g) + u * dt);
+        else st3(Vi.th, g, own(3, i) + u * dt);
     } else {
         if (r0 == 0) st3(Vo.x, g, own(0, i));
         if (nonfinite(u, u)) {
@@ -425,7 +499,7 @@ __global__ void __launch_bounds__(kTileThreads, tile_waves(PAIRS, PREC))
 // Vo (the same buffers or the other set); the facets are copied along.
 __global__ void __launch_bounds__(64) k_tile_kick(pool_view V, pool_view Vo, const wide_block *map, uint32_t width,
                                                   double half, double dt) {
-    const wide_block b = map[blockIdx.x];
+    const wide_block b = tile_block(map, V, width);
     const uint32_t n = b.n & kIdxMask;
     if (Vo.facets != V.facets && b.start == 0 && threadIdx.x == 0) {
         const uint32_t nf = V.meta[b.slot].nf;

@@ -1,5 +1,5 @@
 """The per-step tile kernel against the CPU oracle at the edges of its tiles
-(64 listed particles, one with all pairs), with lists longer than the 16
+(64 listed particles, one with all pairs), with lists longer than the 12
 positions it handles at once (1,024 with all pairs) and contacts that begin and
 end. FP64, so state
 and springs must be equal to the last bit."""
@@ -111,6 +111,32 @@ def test_facets_move_with_the_tiles(steps):
     o.set_facets(verts, vel)
     s.set_facets(verts, vel)
     for _ in range(2):
+        o.step(1e-13, steps, rebuild_every=50)
+        s.step(1e-13, steps, rebuild_every=50)
+    a, b = o.state(), s.state()
+    for k in ("x", "v", "theta", "omega", "a", "alpha"):
+        np.testing.assert_array_equal(b[k], a[k], err_msg=k)
+    s.close()
+
+
+@pytest.mark.parametrize("capacity", [2, 3, 4])
+@pytest.mark.parametrize("n", [2, 65])
+def test_tables_narrower_than_the_tags_read_ahead(n, capacity):
+    """A bonded chain whose table and list hold fewer entries than a tile loads
+    ahead of their counts."""
+    import libgran_amd as L
+    import _scenarios as S
+    print(f"[tile] chain of {n}, table of {capacity}", flush=True)
+    x = np.zeros((n, 3))
+    x[:, 0] = 2.0 * R * np.arange(n)
+    v = np.random.default_rng(n).normal(0.0, 1.0, x.shape)
+    c, sn, h = S.aggregate_params()
+    o = O.OracleSystem(O.system_params(O.BIN_SINTER, O.HAM_LIMITED, neighbor_mode=1, r_verlet=3.2 * R, contact=c,
+                                       sinter=sn, hamaker=h), x, v)
+    s = L.System(L.make_params(L.BINARY_SINTER, L.HAMAKER_LIMITED, pair_mode=1, r_verlet=3.2 * R, contact=c, sinter=sn,
+                               hamaker=h, pair_capacity=capacity, neighbor_capacity=2), x, v)
+    s.per_step_launches(True)
+    for steps in (1, 50):
         o.step(1e-13, steps, rebuild_every=50)
         s.step(1e-13, steps, rebuild_every=50)
     a, b = o.state(), s.state()
