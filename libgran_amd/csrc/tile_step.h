@@ -58,11 +58,13 @@ __device__ __forceinline__ wide_block tile_block(const wide_block *map, const po
 
 // Wavefronts per SIMD that the registers leave room for. Listed tiles, many to
 // a CU, hide one pair's latency behind another's: mixed 151 us a step at
-// 635,000 particles with three, 187 with two (four spill: 241). All pairs come
-// in few blocks, and two cost them registers: 33 us a step at 522 particles
-// against 28.
-constexpr int tile_waves(int pairs, int prec) {
-    return pairs != HG_PAIRS_NEIGHBOR_LIST ? 1 : (prec == HG_PRECISION_MIXED ? 3 : 2);
+// 635,000 particles with three, 187 with two (four spill: 241); with the facet
+// terms three spill too: 24 plate tests of 1,000 steps 40.5 ms, 35.8 with two.
+// FP64 takes the same time with two and three (72.2 ms for 800 steps of 333
+// aggregates). All pairs come in few blocks, and two cost them registers: 33 us
+// a step at 522 particles against 28.
+constexpr int tile_waves(int pairs, int prec, bool fac) {
+    return pairs != HG_PAIRS_NEIGHBOR_LIST ? 1 : (prec == HG_PRECISION_MIXED && !fac ? 3 : 2);
 }
 
 // A launch's arguments (the parameter set, its mixed form and two views, 1.5 KB)
@@ -83,7 +85,7 @@ __device__ __forceinline__ void touch_args() {
 // the systems that have none; TILE_STEP completes the step, kicks and drifts
 // into the other buffers; TILE_LAST completes the last step.
 template <int BIN, int HAM, int PAIRS, int PREC, bool FAC>
-__global__ void __launch_bounds__(kTileThreads, tile_waves(PAIRS, PREC))
+__global__ void __launch_bounds__(kTileThreads, tile_waves(PAIRS, PREC, FAC))
     k_tile_step(hg_params P, mixed_consts MC, pool_view Vi, pool_view Vo, const wide_block *map, int mode, double half,
                 double dt) {
     constexpr int W = tile_width(PAIRS), KC = tile_depth(PAIRS), ROWS = kTileThreads / W, WAVES = kTileThreads / 64;
