@@ -502,7 +502,10 @@ hg_status hg_pool_create(const hg_params *params, size_t max_particles, size_t m
     PG_TRYC(palloc(Q, &Q->owner, P));
     {
         std::vector<uint32_t> none(P, kNoEntry);
-        PG_HIPC(hipMemcpy(Q->owner, none.data(), P * 4, hipMemcpyHostToDevice));
+        // not hipMemcpy: the default stream refuses it, and spoils the recording,
+        // while another thread's pool records a graph
+        PG_HIPC(hipMemcpyAsync(Q->owner, none.data(), P * 4, hipMemcpyHostToDevice, Q->stream));
+        PG_HIPC(hipStreamSynchronize(Q->stream));
     }
     PG_TRYC(palloc(Q, &Q->facets, std::max<size_t>(1, Q->S * std::max<size_t>(Q->MF, 1))));
     PG_TRYC(palloc(Q, &Q->facets_b, std::max<size_t>(1, Q->S * std::max<size_t>(Q->MF, 1))));
@@ -1082,11 +1085,14 @@ hg_status pool_begin(hg_pool *Q, double dt, uint64_t max_len, uint32_t rebuild_e
         VB.facets = Q->facets_b;
         // the interval's launches: recorded once into a HIP graph per
         // (interval length, dt, wide set, facets or not) and replayed;
-        // launched one by one when graphs are off
+        // launched one by one when graphs are off or no system is wide by the
+        // threshold: the host queues a launch in 2.7 us and a step takes 8, and
+        // a program that copies through the default stream in another thread
+        // while a pool of small systems steps must not meet a recording
         auto enqueue = [&](hipStream_t st_) {
             return launch_tile_steps(Q->p, V, VB, Q->wide_map_d, Q->wide_blocks, len, wide_facets, half, dt, st_);
         };
-        if (Q->wide_graph) {
+        if (Q->wide_graph && Q->meta[Q->order[0]].n >= Q->wide_min) {
             if (!Q->wg_exec || Q->wg_len != len || Q->wg_dt != dt || Q->wg_blocks != Q->wide_blocks ||
                 Q->wg_facets != wide_facets) {
                 if (Q->wg_exec) HG_HIP(hipGraphExecDestroy(Q->wg_exec));
