@@ -10,14 +10,9 @@
 
 #include "../../include/hipgran.h"
 #include "dem_math.h"
+#include "pair_row.h"
 
 namespace hg {
-
-// Pair-state table entry tag: bit 31 marks a bonded (alt_sinter) pair; the low
-// 31 bits are the partner index j.
-constexpr uint32_t kBondBit = 0x80000000u;
-constexpr uint32_t kIdxMask = 0x7fffffffu;
-constexpr uint32_t kNoEntry = 0xffffffffu;  // (kNoEntry & kIdxMask) exceeds every valid j
 
 // Device flag words (int32 each) written by kernels, read back by the host.
 // The MAXCOUNT words are raised only by lists that overflow, so they hold the

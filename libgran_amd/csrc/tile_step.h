@@ -48,8 +48,6 @@ struct tile_lds {
     term A[6][W < 64 ? W : 1];
 };
 
-constexpr uint32_t kNoRowSlot = 0xFFFu;
-
 // This workgroup's tile: from the map or, without one, of the view's only
 // system, so that a single system's tile waits for no load.
 __device__ __forceinline__ wide_block tile_block(const wide_block *map, const pool_view &V, uint32_t width) {
@@ -339,8 +337,7 @@ __global__ void __launch_bounds__(kTileThreads, tile_waves(PAIRS, PREC, FAC))
                     uint32_t slot = kNoRowSlot;
                     if ((e.y >> 20) != kNoRowSlot) {  // it may have moved just now
                         const uint32_t rc = L.rows[t] < Vi.cap_s ? L.rows[t] : Vi.cap_s;
-                        for (uint32_t s = 0; s < rc; s++)
-                            if ((pj[size_t(s) * stride + gi] & kIdxMask) == j) slot = s;
+                        slot = row_slot(rc, j, [&](uint32_t s) { return pj[size_t(s) * stride + gi]; });
                     }
                     spring9 sp = zero_spring();
                     if (slot != kNoRowSlot) sp = ld_rec(ps + (size_t(slot) * stride + gi) * kSpringRec);

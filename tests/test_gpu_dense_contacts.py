@@ -1,0 +1,107 @@
+"""Beds of touching, unbonded spheres under neighbour lists: every particle has
+up to twelve contacts, many of which begin or end in one step, so that a tile
+holds more touching pairs than it has threads. FP64: equal to the oracle to the
+last bit, in a System and in a Pool over tiles and in the chunk kernel; mixed:
+the tiles equal the chunk kernel."""
+import numpy as np
+import pytest
+
+import _oracle as O
+
+pytestmark = pytest.mark.gpu
+
+R = O.R_PART
+TILE, DEPTH, THREADS = 64, 12, 256  # particles, list positions at a time, threads of a tile
+
+
+def bed(n, seed):
+    """n spheres around the sites of a touching face-centred cubic lattice,
+    layer by layer, drawn together while they shake."""
+    rng = np.random.default_rng(seed)
+    m = int(np.ceil((n / 4.0) ** (1.0 / 3.0)))
+    g = np.stack(np.meshgrid(*[np.arange(m)] * 3, indexing="ij"), axis=-1).reshape(-1, 3)
+    sites = (g[:, None, :] + np.array([[0, 0, 0], [0.5, 0.5, 0], [0.5, 0, 0.5], [0, 0.5, 0.5]])).reshape(-1, 3)[:n]
+    x = sites * 2.0 * np.sqrt(2.0) * R + rng.normal(0.0, 0.003 * R, (n, 3))
+    return x, rng.normal(0.0, 100.0, (n, 3)) - 1e9 * (x - x.mean(axis=0)), rng.normal(0.0, 1e8, (n, 3))
+
+
+def touching_in_a_pass(x, offsets, ids):
+    """The most touching pairs that one tile has among the list positions it
+    takes at a time."""
+    n = len(x)
+    most = {}
+    for i in range(n):
+        for k, j in enumerate(ids[offsets[i]:offsets[i + 1]]):
+            if np.linalg.norm(x[i] - x[int(j)]) < 2.0 * R:
+                key = (i // TILE, k // DEPTH)
+                most[key] = most.get(key, 0) + 1
+    return max(most.values())
+
+
+def params(precision, r_list):
+    import libgran_amd as L
+    return L.make_params(L.BINARY_CONTACT, L.HAMAKER_FULL, pair_mode=1, r_verlet=r_list * R,
+                         contact=O.contact_params(), hamaker=O.hamaker_params(A=1e-20, h0=1e-9), precision=precision)
+
+
+def equal(a, b, what):
+    for k in ("x", "v", "theta", "omega", "a", "alpha"):
+        np.testing.assert_array_equal(b[k], a[k], err_msg=f"{what}: {k}")
+
+
+@pytest.mark.parametrize("r_list", [2.2, 2.6, 3.2])
+@pytest.mark.parametrize("n", [500, 777])
+def test_beds_equal_oracle(n, r_list):
+    import libgran_amd as L
+    print(f"[bed] n {n}, list {r_list} r", flush=True)
+    x, v, w = bed(n, n)
+    o = O.OracleSystem(O.system_params(O.BIN_CONTACT, O.HAM_FULL, neighbor_mode=1, r_verlet=r_list * R,
+                                       contact=O.contact_params(), hamaker=O.hamaker_params(A=1e-20, h0=1e-9)), x, v, w0=w)
+    o.rebuild()
+    assert touching_in_a_pass(x, *o.neighbors()) > THREADS
+    s = L.System(params(0, r_list), x, v, omega0=w)
+    pools = []
+    for wide_min in (1, 0):  # tiles, chunk kernel
+        pool = L.Pool(params(0, r_list), max_particles=1024, max_systems=2)
+        pool.set_wide_threshold(wide_min)
+        pools.append((pool, pool.add(x, v, omega0=w)))
+    last, both = set(), 0
+    for steps in (1, 14, 25, 20, 20):
+        for _ in range(steps):
+            o.step(1e-13, 1, rebuild_every=20)
+            now = set(map(tuple, o.springs(0)[0].tolist()))
+            both += len({i for i, _ in now - last} & {i for i, _ in last - now})
+            last = now
+        s.step(1e-13, steps, rebuild_every=20)
+        ij, sp = o.springs(0)
+        equal(o.state(), s.state(), f"system after {steps}")
+        got = s.springs(0)
+        np.testing.assert_array_equal(got[0], ij)
+        np.testing.assert_array_equal(got[1], sp)
+        for pool, slot in pools:
+            pool.step(1e-13, steps, rebuild_every=20)
+            equal(o.state(), pool.state(slot), f"pool after {steps}")
+            got = pool.springs(slot, 0)
+            np.testing.assert_array_equal(got[0], ij)
+            np.testing.assert_array_equal(got[1], sp)
+    assert both > 100  # a contact began and another ended at one particle in one step
+    s.close()
+    for pool, _ in pools:
+        pool.close()
+
+
+def test_mixed_beds_in_tiles_equal_the_chunk_kernel():
+    import libgran_amd as L
+    print("[bed] mixed", flush=True)
+    x, v, w = bed(777, 3)
+    out = []
+    for wide_min in (1, 0):
+        pool = L.Pool(params(1, 2.6), max_particles=1024, max_systems=2)
+        pool.set_wide_threshold(wide_min)
+        slot = pool.add(x, v, omega0=w)
+        pool.step(1e-13, 80, rebuild_every=20)
+        out.append((pool.state(slot), pool.springs(slot, 0)))
+        pool.close()
+    equal(out[1][0], out[0][0], "mixed")
+    np.testing.assert_array_equal(out[0][1][0], out[1][1][0])
+    np.testing.assert_array_equal(out[0][1][1], out[1][1][1])
