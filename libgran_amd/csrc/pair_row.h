@@ -19,7 +19,15 @@ constexpr uint32_t kBondBit = 0x80000000u;
 constexpr uint32_t kIdxMask = 0x7fffffffu;
 constexpr uint32_t kNoEntry = 0xffffffffu;  // (kNoEntry & kIdxMask) exceeds every valid j
 
-constexpr uint32_t kNoRowSlot = 0xFFFu;
+// A queued pair's place: its list position among those the tile takes at a time
+// and its particle (position * width + particle, at most kTilePlaces) and its
+// slot in the particle's row. A row holds distinct partners, so a slot of 22
+// bits is beyond what the tables of such a system would fit in memory.
+constexpr uint32_t kPlaceBits = 10, kTilePlaces = 1u << kPlaceBits;
+constexpr uint32_t kNoRowSlot = ~0u >> kPlaceBits;
+HG_ROW uint32_t queue_word(uint32_t place, uint32_t slot) { return place | (slot << kPlaceBits); }
+HG_ROW uint32_t queue_place(uint32_t word) { return word & (kTilePlaces - 1u); }
+HG_ROW uint32_t queue_slot(uint32_t word) { return word >> kPlaceBits; }
 
 // The slot of partner j in a row of `count` entries, tag(s) the tag of slot s.
 // It is the first match: removing ended entries leaves their old tags beyond

@@ -35,9 +35,10 @@ namespace {
 template <int W, int KC, int PREC, bool FAC>
 struct tile_lds {
     using term = typename prec_types<PREC>::term;
+    static_assert(KC * W <= int(kTilePlaces), "queue_word");
     double s[12][W];  // x, v, omega, theta
     term T[6][KC * W];
-    uint2 Q[KC * W];  // partner, and i | kk << 8 | row slot << 20
+    uint2 Q[KC * W];  // partner and queue_word
     uint16_t CW[KC * W];
     uint32_t rows[W], dirty[W];
     uint32_t nB[kTileThreads / 64], nO[kTileThreads / 64];
@@ -239,7 +240,7 @@ __global__ void __launch_bounds__(kTileThreads, tile_waves(PAIRS, PREC, FAC))
             if (on) {
                 const uint32_t at = bond ? nB + uint32_t(__popcll(mb & below))
                                          : 64u * (KC / ROWS) - 1u - (nO + uint32_t(__popcll(mo & below)));
-                L.Q[seg + at] = uint2{j, i | ((r0 + q * ROWS) << 8) | (slot << 20)};
+                L.Q[seg + at] = uint2{j, queue_word((r0 + q * ROWS) * W + i, slot)};
             }
             nB += uint32_t(__popcll(mb));
             nO += uint32_t(__popcll(mo));
@@ -269,7 +270,7 @@ __global__ void __launch_bounds__(kTileThreads, tile_waves(PAIRS, PREC, FAC))
             }
             const uint32_t at = w * 64u * (KC / ROWS) + (bond ? rest : 64u * (KC / ROWS) - 1u - rest);
             const uint2 e = L.Q[at];
-            const uint32_t t = e.y & 0xFFu, pos = ((e.y >> 8) & 0xFFFu) * W + t, slot = e.y >> 20, j = e.x;
+            const uint32_t pos = queue_place(e.y), t = pos % W, slot = queue_slot(e.y), j = e.x;
             const d3 xi = own(0, t), xj = ld3(Vi.x, j);
             vec lin, ang{};
             if (BIN == HG_BINARY_SINTER && bond) {
@@ -333,9 +334,9 @@ __global__ void __launch_bounds__(kTileThreads, tile_waves(PAIRS, PREC, FAC))
                 __syncthreads();
                 for (uint32_t c = tid; c < nc; c += kTileThreads) {
                     const uint2 e = L.Q[L.CW[c]];
-                    const uint32_t t = e.y & 0xFFu, pos = ((e.y >> 8) & 0xFFFu) * W + t, j = e.x, gi = base + t;
+                    const uint32_t pos = queue_place(e.y), t = pos % W, j = e.x, gi = base + t;
                     uint32_t slot = kNoRowSlot;
-                    if ((e.y >> 20) != kNoRowSlot) {  // it may have moved just now
+                    if (queue_slot(e.y) != kNoRowSlot) {  // it may have moved just now
                         const uint32_t rc = L.rows[t] < Vi.cap_s ? L.rows[t] : Vi.cap_s;
                         slot = row_slot(rc, j, [&](uint32_t s) { return pj[size_t(s) * stride + gi]; });
                     }

@@ -37,5 +37,14 @@ int main() {
     expect("not in the row", row, 4, 5, kNoRowSlot);
     expect("beyond the row", row, 3, 6, kNoRowSlot);
     expect("an empty row", row, 0, 1, kNoRowSlot);
+    // a slot comes back from the queue as it went in, however long the row
+    for (uint32_t place : {0u, 1u, kTilePlaces - 1u})
+        for (uint32_t slot : {0u, 1u, 4094u, 4095u, 4096u, 70000u, kNoRowSlot - 1u, kNoRowSlot}) {
+            const uint32_t word = queue_word(place, slot);
+            if (queue_place(word) == place && queue_slot(word) == slot) continue;
+            std::printf("place %u, slot %u came back as %u, %u\n", place, slot, queue_place(word), queue_slot(word));
+            wrong++;
+        }
+    if (kNoRowSlot <= 4095u) wrong++;
     return wrong;
 }

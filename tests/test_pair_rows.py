@@ -3,7 +3,6 @@ host."""
 import os
 import subprocess
 
-
 HERE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "cpp")
 
 
@@ -15,5 +14,6 @@ def run(name):
 
 def test_an_entry_is_found_in_its_own_slot():
     """An entry that stays is found in its slot while other threads claim the
-    slots behind the row, where its old tag may still stand."""
+    slots behind the row, where its old tag may still stand; slots of rows
+    longer than 4,095 entries keep their number in a tile's queue."""
     run("pair_row_check")
