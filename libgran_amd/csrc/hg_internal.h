@@ -106,10 +106,6 @@ struct cell_rec {  // a binned particle: its position, index and system in one 3
 };
 struct list_build {
     const double *x;
-    // null, or a particle whose position the cells are laid from: a system far
-    // from the origin keeps exact cell coordinates (its positions' differences
-    // are exact where their quotients by a cell are not)
-    const double *origin;
     uint32_t count;
     size_t stride;
     double r_verlet;

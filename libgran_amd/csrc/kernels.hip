@@ -339,12 +339,6 @@ __device__ __forceinline__ uint32_t cell_hash(uint32_t slot, long long cx, long 
     return uint32_t(h) & mask;
 }
 
-__device__ __forceinline__ d3 cell_origin(const list_build &B) {
-    if (!B.origin) return zero3();
-    const d3 o = ld3(B.origin, 0);
-    return nonfinite(o, o) ? zero3() : o;
-}
-
 __device__ __forceinline__ void cell_coords(d3 q, double cs, long long &cx, long long &cy, long long &cz) {
     cx = (long long)floor(q.x / cs);
     cy = (long long)floor(q.y / cs);
@@ -360,7 +354,7 @@ __global__ void __launch_bounds__(256) k_cell_count(list_build B, double cs) {
         return;
     }
     long long cx, cy, cz;
-    cell_coords(ld3(B.x, g) - cell_origin(B), cs, cx, cy, cz);
+    cell_coords(ld3(B.x, g), cs, cx, cy, cz);
     const uint32_t h = cell_hash(slot, cx, cy, cz, B.hash_size - 1);
     B.cell_of[g] = h;
     atomicAdd(&B.buckets[h], 1u);
@@ -400,7 +394,13 @@ __device__ __forceinline__ void close_list(const list_build &B, uint32_t g, uint
 // 2 x 2 cells, one for each lane. (In cell units a partner is less than 0.5 (1
 // - 1e-9) away; a particle in the lower half, u - floor(u) < 0.5, has its
 // partners in floor(u) - 1 .. floor(u), one in the upper half in floor(u) ..
-// floor(u) + 1.) The matches go to LDS and from there to their rank among
+// floor(u) + 1. That holds however far out the system lies: u is one correctly
+// rounded quotient, and rounding cannot carry a value past a whole or a half,
+// so a particle that the rounding moves to the upper half, from within half a
+// unit in the last place below it, has its partners at floor(u) or above after
+// rounding too. Cells laid from one of the particles, u = (x - o) / cs, round
+// twice, and where that particle is far away from the others pairs were
+// missed.) The matches go to LDS and from there to their rank among
 // them, so the list ascends. One lane walking all eight buckets took 104 us at
 // 20,000 particles, each bucket a chain of dependent reads.
 constexpr uint32_t kListLanes = 8, kListParts = 256 / kListLanes, kListMost = 96, kRecBatch = 4;
@@ -416,11 +416,10 @@ __global__ void __launch_bounds__(256) k_list_fill(list_build B, double cs) {
     const d3 xi = on ? ld3(B.x, g) : zero3();
     const in_range near(B.r_verlet);
     long long bx, by, bz;
-    const d3 u = xi - cell_origin(B);
-    cell_coords(u, cs, bx, by, bz);
-    bx -= u.x / cs - double(bx) < 0.5 ? 1 : 0;
-    by -= u.y / cs - double(by) < 0.5 ? 1 : 0;
-    bz -= u.z / cs - double(bz) < 0.5 ? 1 : 0;
+    cell_coords(xi, cs, bx, by, bz);
+    bx -= xi.x / cs - double(bx) < 0.5 ? 1 : 0;
+    by -= xi.y / cs - double(by) < 0.5 ? 1 : 0;
+    bz -= xi.z / cs - double(bz) < 0.5 ? 1 : 0;
     // calls match(j) for every partner in the bucket of cell c of the eight
     auto scan = [&](uint32_t h, auto &&match) {
         const uint32_t b = B.bucket_start[h], e = b + B.buckets[h];
@@ -1207,7 +1206,7 @@ hipError_t launch_cell_lists(const list_build &B, hipStream_t s) {
 hipError_t launch_neighbor_build(hg_system_impl &S, hipStream_t s) {
     const uint32_t n = uint32_t(S.n);
     if (n == 0) return hipSuccess;
-    const list_build B{S.x,       S.x,    n,            S.n,        S.p.r_verlet, nullptr,     nullptr,
+    const list_build B{S.x,       n,            S.n,        S.p.r_verlet, nullptr,     nullptr,
                        S.hash_size, S.buckets, S.bucket_start, S.scan_tmp, S.cell_of,  S.cell_recs, S.nb,
                        S.ncnt,      S.cap_n,   S.flags,        nullptr};
     if (n > kBruteListMax) return launch_cell_lists(B, s);

@@ -336,7 +336,7 @@ hg_status download_rows(hg_pool *Q, const T *dev, uint32_t offset, uint32_t n, u
 hg_status rebuild_due(hg_pool *Q) {
     const uint32_t hw = Q->high_water;
     if (hw == 0) return HG_OK;
-    const list_build B{Q->x,         nullptr,     hw,          Q->P,       Q->p.r_verlet, Q->owner, Q->meta_d, Q->hash_size, Q->buckets,
+    const list_build B{Q->x,         hw,          Q->P,       Q->p.r_verlet, Q->owner, Q->meta_d, Q->hash_size, Q->buckets,
                        Q->bucket_start, Q->scan_tmp, Q->cell_of, Q->cell_recs,  Q->nb,    Q->ncnt,   Q->cap_n,     Q->flags,
                        Q->sflags};
     HG_HIP(launch_cell_lists(B, Q->stream));

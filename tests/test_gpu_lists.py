@@ -47,3 +47,17 @@ def test_cell_lists_far_from_the_origin():
     n = 9000
     x = np.random.default_rng(6).uniform(0.0, 2.2 * R * n ** (1.0 / 3.0), (n, 3)) + np.array([1.0, -3.0, 0.1])
     check(x, 3.2 * R)
+
+
+@pytest.mark.parametrize("where", [1.0, -1.0, np.inf])
+def test_one_particle_far_away_leaves_the_others_listed(where):
+    """A first particle 1e8 m out (or lost) beside pairs just inside the list
+    radius: the cells of the others must not depend on it."""
+    rng = np.random.default_rng(8)
+    m, r_list = 1500, 3.2 * R
+    a = rng.uniform(0.0, 40.0 * r_list, (m, 3))
+    b = a.copy()
+    b[np.arange(m), rng.integers(0, 3, m)] += r_list * (1.0 - 1e-5)
+    out = where * np.array([[1e8, 0.7e8, -0.3e8]])
+    off = check(np.concatenate([out, a, b]), r_list)
+    assert off[-1] >= 2 * m
