@@ -372,10 +372,12 @@ __global__ void __launch_bounds__(256) k_cell_fill(list_build B) {
 
 // The reference predicate norm(x_i - x_j) < r_verlet behind a squared-distance
 // prefilter: a correctly rounded sqrt(d2) < r_verlet implies d2 < r_verlet^2
-// (1 + 2^-52), so this bound drops no pair the exact test keeps.
+// (1 + 2^-52), so this bound drops no pair the exact test keeps; squares below
+// the smallest normal number have few bits and go to the exact test.
 struct in_range {
     double r, d2_max;
-    __device__ __forceinline__ in_range(double r_verlet) : r(r_verlet), d2_max(r_verlet * r_verlet * (1.0 + 1e-12)) {}
+    __device__ __forceinline__ in_range(double r_verlet)
+        : r(r_verlet), d2_max(fmax(r_verlet * r_verlet * (1.0 + 1e-12), 0x1p-1022)) {}
     __device__ __forceinline__ bool operator()(d3 d) const { return dot(d, d) < d2_max && norm(d) < r; }
 };
 
@@ -867,7 +869,7 @@ __global__ void __launch_bounds__(kTinyThreads)
         *u = *u + X[size_t(12 + c) * n + i] * half;
         *o = *o + *u * dt;
     }
-    const double touch = 2.0 * P.contact.r_part, touch2 = touch * touch * (1.0 + 1e-12);
+    const contact_reach reach(P.contact.r_part);
     for (uint32_t s = 0; s < nsteps; s++) {
         __syncthreads();
         if constexpr (BIN == HG_BINARY_SINTER_LEGACY) {
@@ -890,7 +892,7 @@ __global__ void __launch_bounds__(kTinyThreads)
                 const uint32_t e = E[at];
                 const d3 d = vec(0, e & 0xFFu) - vec(0, (e >> 8) & 0xFFu);
                 bool touching = false;
-                if (!(dot(d, d) > touch2)) touching = !(2.0 * P.contact.r_part - dot(d, normalized(d)) <= 0);
+                if (!reach.beyond(dot(d, d))) touching = !(2.0 * P.contact.r_part - dot(d, normalized(d)) <= 0);
                 if (touching) {
                     LC[atomicAdd(&s_touch, 1u)] = uint16_t(at);
                     if (kind != TINY_CONTACT) {

@@ -40,17 +40,29 @@ __device__ __forceinline__ d3 hamaker_lin(const hg_hamaker_params &p, d3 r) {
     return hamaker_along<HAM>(p, dist, z > 0.0 ? r / dist : r);
 }
 
+// The contact functor's overlap is 2 r minus a distance, a square root and three
+// divisions away from the squared distance d2. Beyond the squared contact
+// distance and a margin far above rounding it is negative; the margin is at
+// least the smallest normal number, below which d2 has few bits, and an infinite
+// d2, whose direction is zero or not a number, takes the functor's own course.
+struct contact_reach {
+    double d2_max;
+    __device__ __forceinline__ explicit contact_reach(double r_part) {
+        const double reach = 2.0 * r_part;
+        d2_max = fmax(reach * reach * (1.0 + 1e-12), 0x1p-1022);
+    }
+    __device__ __forceinline__ bool beyond(double d2) const { return d2 > d2_max && d2 < __builtin_huge_val(); }
+};
+
 template <int HAM, int PREC>
 struct pair_eval {
     using vec = typename prec_types<PREC>::vec;
     const hg_params &p;
     const mixed_consts &m;
-    double touch2;  // squared contact distance and a margin far above rounding
+    contact_reach reach;
 
-    __device__ __forceinline__ pair_eval(const hg_params &P, const mixed_consts &M) : p(P), m(M) {
-        const double reach = 2.0 * P.contact.r_part;
-        touch2 = reach * reach * (1.0 + 1e-12);
-    }
+    __device__ __forceinline__ pair_eval(const hg_params &P, const mixed_consts &M)
+        : p(P), m(M), reach(P.contact.r_part) {}
     // A bonded pair: its term and new springs; true when the bond breaks
     // (this evaluation is still the bonded one).
     template <class NECK>
@@ -93,7 +105,7 @@ struct pair_eval {
         if constexpr (PREC == HG_PRECISION_FP64) {
             if constexpr (CONTACT) {
                 const d3 d = xi - xj;
-                if (!(dot(d, d) > touch2)) {  // beyond touch2 the overlap is negative
+                if (!reach.beyond(dot(d, d))) {
                     const double overlap = 2.0 * p.contact.r_part - dot(d, normalized(d));
                     touching = !(overlap <= 0);
                 }
