@@ -789,6 +789,7 @@ __global__ void __launch_bounds__(kTinyThreads)
     __shared__ facet_dev F[kMaxFacets];
     __shared__ uint32_t s_bonds, s_touch;
     __shared__ uint32_t s_cnt[kTinySystemMax], s_legacy[kTinySystemMax];  // partners and legacy bonds
+    __shared__ uint32_t s_carried[kTinySystemMax];  // row entries of partners that are not listed
     const tiny_layout Y(S.n, maxb);
     const uint32_t n = Y.n, row = Y.row, places = Y.places, tid = threadIdx.x;
     const bool nl = P.pair_mode == HG_PAIRS_NEIGHBOR_LIST;
@@ -826,6 +827,7 @@ __global__ void __launch_bounds__(kTinyThreads)
     if (tid < n) {
         s_cnt[tid] = nl ? S.ncnt[tid] : n - 1u;
         s_legacy[tid] = BIN == HG_BINARY_SINTER_LEGACY ? S.pt.bcnt[tid] : 0u;
+        s_carried[tid] = BIN != HG_BINARY_NONE ? S.pt.pcnt_old[tid] : 0u;
     }
     if constexpr (BIN == HG_BINARY_SINTER_LEGACY)
         for (uint32_t q = tid; q < 15u * maxb * n; q += kTinyThreads) {
@@ -854,6 +856,7 @@ __global__ void __launch_bounds__(kTinyThreads)
                     const uint32_t tag = S.pt.pj_old[size_t(q) * n + i];
                     if ((tag & kIdxMask) != j) continue;
                     kind = (tag & kBondBit) ? TINY_BOND : TINY_CONTACT;
+                    atomicSub(&s_carried[i], 1u);
                     const spring9 sp = ld_rec(S.pt.ps_old + (size_t(q) * n + i) * kSpringRec);
                     for (uint32_t c = 0; c < 3; c++) set_spring(at, c, sp.s[c]);
                 }
@@ -870,6 +873,7 @@ __global__ void __launch_bounds__(kTinyThreads)
         *o = *o + *u * dt;
     }
     const contact_reach reach(P.contact.r_part);
+    const bool rows_may_overflow = BIN != HG_BINARY_NONE && S.pt.cap + 1 < n;
     for (uint32_t s = 0; s < nsteps; s++) {
         __syncthreads();
         if constexpr (BIN == HG_BINARY_SINTER_LEGACY) {
@@ -1004,6 +1008,20 @@ __global__ void __launch_bounds__(kTinyThreads)
         if (tid == 0) {
             s_touch = 0;
             advance_facets(F, nf_advance, dt);
+        }
+        // a row that holds more entries than the table, if only for this step, is
+        // reported as the walk reports it; threads that the sums leave idle
+        const uint32_t ri = tid - kTinyThreads / 2;
+        if (rows_may_overflow && ri < n) {
+            uint32_t held = s_carried[ri];
+            for (uint32_t k = 0; k < s_cnt[ri]; k++) {
+                const uint8_t kind = K[ri * row + k];
+                held += kind == TINY_CONTACT || kind == TINY_BOND ? 1u : 0u;
+            }
+            if (held > S.pt.cap) {
+                atomicOr(&S.flags[FLAG_PAIR_OVERFLOW], 1);
+                atomicMax(&S.flags[FLAG_PAIR_MAXCOUNT], int(held));
+            }
         }
         // sums in partner order, then the kicks and the drift, a component a thread
         const bool last = s + 1 == nsteps;

@@ -39,3 +39,35 @@ def test_tiny_equals_oracle(n, pairs, r_list):
         np.testing.assert_array_equal(ij2, ij1)
         np.testing.assert_array_equal(s2, s1)
     s.close()
+
+
+@pytest.mark.parametrize("pairs", ["all", "list"])
+@pytest.mark.parametrize("per_step", [False, True])
+def test_a_row_that_overflows_for_a_while_is_reported(per_step, pairs):
+    """Two spheres bounce off a third from both sides within one call: for some
+    steps its row needs two entries, at the end of the call none."""
+    import libgran_amd as L
+    print(f"[tiny] passing overflow, per step {per_step}, {pairs}", flush=True)
+    gap = 2.0 * R + 2e-11
+    x = np.array([[0.0, 0.0, 0.0], [gap, 0.0, 0.0], [-gap, 0.0, 0.0]])
+    v = np.array([[0.0, 0.0, 0.0], [-10.0, 0.0, 0.0], [10.0, 0.0, 0.0]])
+    mode = 1 if pairs == "list" else 0
+    kw = dict(r_verlet=3.0 * R) if mode else {}
+    o = O.OracleSystem(O.system_params(O.BIN_CONTACT, O.HAM_NONE, neighbor_mode=mode, contact=O.contact_params(), **kw), x, v)
+    most = 0
+    for _ in range(200):
+        o.step(1e-13, 1)
+        most = max(most, int(np.bincount(o.springs(0)[0][:, 0], minlength=3)[0]))
+    assert most == 2 and len(o.springs(0)[0]) == 0
+    for capacity in (1, 2):
+        s = L.System(L.make_params(L.BINARY_CONTACT, L.HAMAKER_NONE, pair_mode=mode, contact=O.contact_params(),
+                                   pair_capacity=capacity, **kw), x, v)
+        s.per_step_launches(per_step)
+        if capacity == 1:
+            with pytest.raises(L.HipgranError, match="needs 2 slots per particle, capacity is 1") as e:
+                s.step(1e-13, 200)
+            assert e.value.status == 5  # HG_ERR_CAPACITY
+        else:
+            s.step(1e-13, 200)
+            np.testing.assert_array_equal(s.state()["x"], o.state()["x"])
+        s.close()
