@@ -155,7 +155,7 @@ struct hg_system_impl {
     // legacy sinter_functor connectors (pair_table::lconn / lslot)
     double *lconn = nullptr;
     uint32_t *lslot = nullptr;
-    uint32_t lmax = 0;  // the most legacy bonds of a particle
+    uint32_t lmax = 0;  // no particle's legacy row is longer, and no slot in one reaches it
     bool legacy_ready = false;
     // neighbour list
     uint32_t cap_n = 0;

@@ -832,7 +832,7 @@ __global__ void __launch_bounds__(kTinyThreads)
     if constexpr (BIN == HG_BINARY_SINTER_LEGACY)
         for (uint32_t q = tid; q < 15u * maxb * n; q += kTinyThreads) {
             const uint32_t e = q / 15, i = e / maxb, s = e % maxb;
-            if (s < S.pt.bcnt[i]) C[q] = lconn[(size_t(s) * n + i) * kConnRec + q % 15];
+            C[q] = lconn[(size_t(s) * n + i) * kConnRec + q % 15];
         }
     __syncthreads();
     for (uint32_t at = tid; at < places; at += kTinyThreads) {

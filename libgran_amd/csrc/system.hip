@@ -1227,7 +1227,10 @@ hg_status hg_load(const void *buf, size_t size, hg_system **out) {
         if (z.has_legacy) {
             std::vector<uint32_t> bj, sl;
             std::vector<double> lc;
-            if (max_count(z.leg_count) > S->bcap) return fail(HG_ERR_INVALID, "hg_load: bad legacy rows");
+            uint32_t most = max_count(z.leg_count);
+            for (uint32_t k : z.leg_slot) most = std::max(most, k < S->bcap ? k + 1 : S->bcap + 1);
+            if (most > S->bcap) return fail(HG_ERR_INVALID, "hg_load: bad legacy rows");
+            S->lmax = std::max(S->lmax, most);  // the rows count, whatever bonds the snapshot lists
             csr_to_rows(z.leg_count, z.leg_j, n, S->bcap, 1, 1, kNoEntry, bj);
             csr_to_rows(z.leg_count, z.leg_slot, n, S->bcap, 1, 1, 0u, sl);
             csr_to_rows(z.leg_count, z.leg_conn, n, S->bcap, kConnRec, 15, 0.0, lc);
