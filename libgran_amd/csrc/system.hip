@@ -249,14 +249,15 @@ bool tiled(const hg_system *S) { return S->p.binary_model != HG_BINARY_SINTER_LE
 // count has changed.
 hg_status tile_views(hg_system *S, pool_view &V, pool_view &VB) {
     const size_t n = S->n, width = size_t(tile_width(S->p.pair_mode));
-    if (!S->tile_state) {
-        HG_TRY(dalloc(S, &S->tile_state, 12 * n));
-        HG_TRY(dalloc(S, &S->tile_facets, kMaxFacets));
-        S->tile_blocks = unsigned((n + width - 1) / width);
+    // one by one: after a call that ran out of memory the next one goes on
+    if (!S->tile_state) HG_TRY(dalloc(S, &S->tile_state, 12 * n));
+    if (!S->tile_facets) HG_TRY(dalloc(S, &S->tile_facets, kMaxFacets));
+    if (!S->tile_meta) {
         pool_meta *meta = nullptr;
         HG_TRY(dalloc(S, &meta, 1));
         S->tile_meta = meta;
     }
+    S->tile_blocks = unsigned((n + width - 1) / width);
     if (!S->facets) HG_TRY(dalloc(S, &S->facets, kMaxFacets));
     if (S->tile_nf != S->nf) {
         const pool_meta M{0, uint32_t(n), 0, 0, uint32_t(S->nf), 0, 0, 0};
