@@ -19,7 +19,10 @@
 // came from. A row changes only when a contact begins or ends (or a bond
 // breaks); its owner thread then removes the ended entries and puts the new
 // ones in order before the launch ends, so the table is canonical between
-// launches.
+// launches. A row that is full when a contact begins may lose an entry to a
+// later part of the list: the new entry waits in the table's other half, which
+// these launches leave alone, and a row overflows only if it still waits at the
+// end.
 #pragma once
 
 #include "pair_eval.h"
@@ -41,6 +44,7 @@ struct tile_lds {
     uint2 Q[KC * W];  // partner and queue_word
     uint16_t CW[KC * W];
     uint32_t rows[W], dirty[W];
+    uint32_t more[W], spilled;  // a row's entries in the table's other half, and whether there are any
     uint32_t nB[kTileThreads / 64], nO[kTileThreads / 64];
     uint32_t contacts, ended;
     // the terms of four facets: FP64 the 6 components of each, mixed the
@@ -100,6 +104,8 @@ __global__ void __launch_bounds__(kTileThreads, tile_waves(PAIRS, PREC, FAC))
     const size_t stride = Vi.stride;
     uint32_t *pj = cur ? Vi.pj1 : Vi.pj0, *pcnt = cur ? Vi.pcnt1 : Vi.pcnt0;
     double *ps = cur ? Vi.ps1 : Vi.ps0;
+    uint32_t *pj_other = cur ? Vi.pj0 : Vi.pj1;
+    double *ps_other = cur ? Vi.ps0 : Vi.ps1;
     const pair_eval<HAM, PREC> ev(P, MC);
 
     const uint32_t i = tid % W, r0 = tid / W;  // own particle of the tile, first list row
@@ -134,9 +140,9 @@ __global__ void __launch_bounds__(kTileThreads, tile_waves(PAIRS, PREC, FAC))
     if (i >= nt) cnt = c_old = 0;
     if (tid < uint32_t(W)) {
         L.rows[tid] = c_old;
-        L.dirty[tid] = 0;
+        L.dirty[tid] = L.more[tid] = 0;
     }
-    if (tid == 0) L.contacts = L.ended = 0;
+    if (tid == 0) L.contacts = L.ended = L.spilled = 0;
     auto own = [&](int f, uint32_t t) { return d3{L.s[3 * f][t], L.s[3 * f + 1][t], L.s[3 * f + 2][t]}; };
 
     // Facets f0 .. f0 + 3, one per wavefront (W == 64) or thread group: their
@@ -347,7 +353,16 @@ __global__ void __launch_bounds__(kTileThreads, tile_waves(PAIRS, PREC, FAC))
                     if (slot == kNoRowSlot) {
                         slot = atomicAdd(&L.rows[t], 1u);
                         L.dirty[t] = 2;
-                        if (slot < Vi.cap_s) pj[size_t(slot) * stride + gi] = j;
+                        if (slot < Vi.cap_s) {
+                            pj[size_t(slot) * stride + gi] = j;
+                        } else {
+                            const uint32_t q = slot - Vi.cap_s + L.more[t];
+                            L.spilled = 1;
+                            if (q < Vi.cap_s) {
+                                pj_other[size_t(q) * stride + gi] = j;
+                                st_rec(ps_other + (size_t(q) * stride + gi) * kSpringRec, sp);
+                            }
+                        }
                     }
                     if (slot < Vi.cap_s) st_rec(ps + (size_t(slot) * stride + gi) * kSpringRec, sp);
                     if constexpr (HAM != HG_HAMAKER_NONE) lin = lin + vec{L.T[0][pos], L.T[1][pos], L.T[2][pos]};
@@ -362,14 +377,25 @@ __global__ void __launch_bounds__(kTileThreads, tile_waves(PAIRS, PREC, FAC))
                 if (tid < nt && L.dirty[tid]) {
                     const uint32_t gi = base + tid;
                     uint32_t c = L.rows[tid];
-                    if (c > Vi.cap_s) {
-                        atomicOr(&Vi.flags[FLAG_PAIR_OVERFLOW], 1);
-                        atomicMax(&Vi.flags[FLAG_PAIR_MAXCOUNT], int(c));
-                        if (Vi.sflags) atomicOr(&Vi.sflags[b.slot], HG_FAULT_PAIR_CAPACITY);
-                        c = Vi.cap_s;
+                    bool fresh = L.dirty[tid] == 2;
+                    if (L.spilled) {
+                        uint32_t more = L.more[tid];
+                        if (c > Vi.cap_s) {
+                            more += c - Vi.cap_s;
+                            c = Vi.cap_s;
+                        }
+                        // more than the other half holds: it overflows anyway
+                        for (; c < Vi.cap_s && more > 0 && more <= Vi.cap_s; c++) {
+                            more--;
+                            pj[size_t(c) * stride + gi] = pj_other[size_t(more) * stride + gi];
+                            st_rec(ps + (size_t(c) * stride + gi) * kSpringRec,
+                                   ld_rec(ps_other + (size_t(more) * stride + gi) * kSpringRec));
+                            fresh = true;
+                        }
+                        L.more[tid] = more;
                         L.rows[tid] = c;
                     }
-                    if (L.dirty[tid] == 2)  // new entries are at the row's end: insert them in order
+                    if (fresh)  // new entries are at the row's end: insert them in order
                         for (uint32_t s = 1; s < c; s++) {
                             const uint32_t tag = pj[size_t(s) * stride + gi];
                             uint32_t q = s;
@@ -450,6 +476,12 @@ __global__ void __launch_bounds__(kTileThreads, tile_waves(PAIRS, PREC, FAC))
             }
         }
     }
+    if constexpr (BIN != HG_BINARY_NONE)
+        if (L.spilled && tid < nt && L.more[tid]) {
+            atomicOr(&Vi.flags[FLAG_PAIR_OVERFLOW], 1);
+            atomicMax(&Vi.flags[FLAG_PAIR_MAXCOUNT], int(L.rows[tid] + L.more[tid]));
+            if (Vi.sflags) atomicOr(&Vi.sflags[b.slot], HG_FAULT_PAIR_CAPACITY);
+        }
     if constexpr (W < 64) {
         if (tid < 6u * W) L.A[r0][i] = acct;
         __syncthreads();

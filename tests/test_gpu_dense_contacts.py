@@ -105,3 +105,51 @@ def test_mixed_beds_in_tiles_equal_the_chunk_kernel():
     equal(out[1][0], out[0][0], "mixed")
     np.testing.assert_array_equal(out[0][1][0], out[1][1][0])
     np.testing.assert_array_equal(out[0][1][1], out[1][1][1])
+
+
+@pytest.mark.parametrize("first", ["begins", "ends"])
+def test_a_full_row_takes_one_contact_for_another(first):
+    """A table of one slot: in the step in which one contact of a particle ends
+    another begins. The two partners stand in different parts of a list longer
+    than a tile takes at a time, in either order."""
+    import libgran_amd as L
+    print(f"[bed] full row, {first} first", flush=True)
+    # particle `mid` between a partner that it leaves and one that comes; 16
+    # more within its list, none touching
+    k = np.arange(16) + 0.5
+    polar, turn = np.arccos(1.0 - 2.0 * k / 16), np.pi * (1.0 + np.sqrt(5.0)) * k
+    shell = 4.4 * R * np.stack([np.cos(turn) * np.sin(polar), np.sin(turn) * np.sin(polar), np.cos(polar)], axis=1)
+    shell = shell[np.abs(shell[:, 0]) < 3.9 * R]
+    assert len(shell) >= 12
+
+    def run(gap):
+        come, leave = [[2.0 * R + gap, 0.0, 0.0]], [[-2.0 * R * 0.999, 0.0, 0.0]]
+        ends = (come, leave) if first == "begins" else (leave, come)
+        x = np.concatenate([ends[0], [[0.0, 0.0, 0.0]], shell, ends[1]])
+        v = np.zeros_like(x)
+        c, q = (0, len(x) - 1) if first == "begins" else (len(x) - 1, 0)
+        v[c, 0] = -20.0
+        o = O.OracleSystem(O.system_params(O.BIN_CONTACT, O.HAM_NONE, neighbor_mode=1, r_verlet=5.0 * R,
+                                           contact=O.contact_params()), x, v)
+        held = []
+        for _ in range(60):
+            o.step(1e-13, 1)
+            ij = o.springs(0)[0]
+            held.append(sorted(int(j) for i, j in ij if i == 1))
+        return x, v, o, held, c, q
+
+    for gap in np.arange(0.0, 120e-12, 0.25e-12):
+        x, v, o, held, c, q = run(gap)
+        if any(held[s] == [q] and held[s + 1] == [c] for s in range(59)):
+            break
+    else:
+        raise AssertionError("no gap gives both in one step")
+    assert all(len(h) <= 1 for h in held)
+    s = L.System(L.make_params(L.BINARY_CONTACT, L.HAMAKER_NONE, pair_mode=1, r_verlet=5.0 * R,
+                               contact=O.contact_params(), pair_capacity=1), x, v)
+    s.per_step_launches(True)
+    s.step(1e-13, 60)
+    equal(o.state(), s.state(), first)
+    np.testing.assert_array_equal(s.springs(0)[0], o.springs(0)[0])
+    np.testing.assert_array_equal(s.springs(0)[1], o.springs(0)[1])
+    s.close()
