@@ -788,6 +788,7 @@ __global__ void __launch_bounds__(kTinyThreads)
     extern __shared__ double tiny_lds[];
     __shared__ facet_dev F[kMaxFacets];
     __shared__ uint32_t s_bonds, s_touch;
+    __shared__ uint32_t s_spare;  // with no more touching pairs than this no row overflows
     __shared__ uint32_t s_cnt[kTinySystemMax], s_legacy[kTinySystemMax];  // partners and legacy bonds
     __shared__ uint32_t s_carried[kTinySystemMax];  // row entries of partners that are not listed
     const tiny_layout Y(S.n, maxb);
@@ -823,7 +824,10 @@ __global__ void __launch_bounds__(kTinyThreads)
         X[q] = fields[c / 3][4 * i + c % 3];
     }
     if (tid < uint32_t(S.nf)) F[tid] = facets[tid];
-    if (tid == 0) s_bonds = s_touch = 0;
+    if (tid == 0) {
+        s_bonds = s_touch = 0;
+        s_spare = S.pt.cap + 1 < n ? S.pt.cap : kNoEntry;
+    }
     if (tid < n) {
         s_cnt[tid] = nl ? S.ncnt[tid] : n - 1u;
         s_legacy[tid] = BIN == HG_BINARY_SINTER_LEGACY ? S.pt.bcnt[tid] : 0u;
@@ -865,6 +869,8 @@ __global__ void __launch_bounds__(kTinyThreads)
         }
         K[at] = kind;
     }
+    if (BIN != HG_BINARY_NONE && tid < n && S.pt.cap + 1 < n)
+        atomicMin(&s_spare, S.pt.cap - (S.pt.pcnt_old[tid] < S.pt.cap ? S.pt.pcnt_old[tid] : S.pt.cap));
     // the first kick and drift
     for (uint32_t q = tid; q < 6u * n; q += kTinyThreads) {
         const uint32_t c = q / n, i = q % n, ang = c >= 3, d = c % 3;
@@ -873,7 +879,6 @@ __global__ void __launch_bounds__(kTinyThreads)
         *o = *o + *u * dt;
     }
     const contact_reach reach(P.contact.r_part);
-    const bool rows_may_overflow = BIN != HG_BINARY_NONE && S.pt.cap + 1 < n;
     for (uint32_t s = 0; s < nsteps; s++) {
         __syncthreads();
         if constexpr (BIN == HG_BINARY_SINTER_LEGACY) {
@@ -910,7 +915,7 @@ __global__ void __launch_bounds__(kTinyThreads)
         __syncthreads();
         // terms: bonded quads, touching quads, the other pairs, facets, each
         // kind from a wavefront of its own
-        const uint32_t bonds = s_bonds, touching = s_touch, per = BIN == HG_BINARY_SINTER_LEGACY ? 1u : 4u;
+        const uint32_t bonds = s_bonds, touching = s_touch, spare = s_spare, per = BIN == HG_BINARY_SINTER_LEGACY ? 1u : 4u;
         const uint32_t e1 = (bonds * per + 63u) & ~63u, e2 = e1 + ((touching * 4u + 63u) & ~63u),
                        e3 = e2 + ((places + 63u) & ~63u), e4 = e3 + (S.nf > 0 ? n : 0u);
         for (uint32_t q = tid; q < e4; q += kTinyThreads) {
@@ -1012,7 +1017,7 @@ __global__ void __launch_bounds__(kTinyThreads)
         // a row that holds more entries than the table, if only for this step, is
         // reported as the walk reports it; threads that the sums leave idle
         const uint32_t ri = tid - kTinyThreads / 2;
-        if (rows_may_overflow && ri < n) {
+        if (BIN != HG_BINARY_NONE && __builtin_expect(touching > spare, 0) && ri < n) {
             uint32_t held = s_carried[ri];
             for (uint32_t k = 0; k < s_cnt[ri]; k++) {
                 const uint8_t kind = K[ri * row + k];
