@@ -30,9 +30,9 @@ HG_ROW uint32_t queue_place(uint32_t word) { return word & (kTilePlaces - 1u); }
 HG_ROW uint32_t queue_slot(uint32_t word) { return word >> kPlaceBits; }
 
 // The slot of partner j in a row of `count` entries, tag(s) the tag of slot s.
-// It is the first match: removing ended entries leaves their old tags beyond
-// the row's end, and a slot there that another thread has claimed (`count`
-// includes it) holds such a tag, j's own perhaps, until the claimer has written
+// It is the first match: removing ended entries leaves old tags beyond the
+// row's end, and a slot there that another thread has claimed, should `count`
+// include it, holds such a tag, j's own perhaps, until the claimer has written
 // its own.
 template <class TAG>
 HG_ROW uint32_t row_slot(uint32_t count, uint32_t j, TAG &&tag) {

@@ -17,9 +17,13 @@
 //
 // The pair-state rows are updated in place: a spring goes back to the slot it
 // came from. A row changes only when a contact begins or ends (or a bond
-// breaks); its owner thread then removes the ended entries and puts the new
-// ones in order before the launch ends, so the table is canonical between
-// launches. A row that is full when a contact begins may lose an entry to a
+// breaks). Its owner thread fills the slot of an ended entry with the row's last
+// one, and new entries go to the row's end; in the last launch of an interval it
+// puts a row that is out of order in order, so the table is canonical whenever
+// anything but these launches reads it. Kept in order in every launch, a bed's
+// rows of twelve moved several records for each contact that began or ended: a
+// face-centred packing of 32,000, mixed, lists of 12, took 47 us a step, 32 so
+// (the walk of one lane a particle 42). A row that is full when a contact begins may lose an entry to a
 // later part of the list: the new entry waits in the table's other half, which
 // these launches leave alone, and a row overflows only if it still waits at the
 // end.
@@ -43,7 +47,8 @@ struct tile_lds {
     term T[6][KC * W];
     uint2 Q[KC * W];  // partner and queue_word
     uint16_t CW[KC * W];
-    uint32_t rows[W], dirty[W];
+    uint32_t rows[W], dirty[W];  // lengths; whether entries ended or began in this part of the lists
+    uint32_t holes[W], kept[W];  // slots of ended entries (kManyHoles: others from slot 31 on); lengths without them
     uint32_t more[W], spilled;  // a row's entries in the table's other half, and whether there are any
     uint32_t nB[kTileThreads / 64], nO[kTileThreads / 64];
     uint32_t contacts, ended;
@@ -52,6 +57,8 @@ struct tile_lds {
     typename prec_types<PREC>::term F[FAC ? 4 : 1][9][W];
     term A[6][W < 64 ? W : 1];
 };
+
+constexpr uint32_t kManyHoles = 1u << 31;
 
 // This workgroup's tile: from the map or, without one, of the view's only
 // system, so that a single system's tile waits for no load.
@@ -104,8 +111,6 @@ __global__ void __launch_bounds__(kTileThreads, tile_waves(PAIRS, PREC, FAC))
     const size_t stride = Vi.stride;
     uint32_t *pj = cur ? Vi.pj1 : Vi.pj0, *pcnt = cur ? Vi.pcnt1 : Vi.pcnt0;
     double *ps = cur ? Vi.ps1 : Vi.ps0;
-    uint32_t *pj_other = cur ? Vi.pj0 : Vi.pj1;
-    double *ps_other = cur ? Vi.ps0 : Vi.ps1;
     const pair_eval<HAM, PREC> ev(P, MC);
 
     const uint32_t i = tid % W, r0 = tid / W;  // own particle of the tile, first list row
@@ -140,7 +145,7 @@ __global__ void __launch_bounds__(kTileThreads, tile_waves(PAIRS, PREC, FAC))
     if (i >= nt) cnt = c_old = 0;
     if (tid < uint32_t(W)) {
         L.rows[tid] = c_old;
-        L.dirty[tid] = L.more[tid] = 0;
+        L.dirty[tid] = L.holes[tid] = L.more[tid] = 0;
     }
     if (tid == 0) L.contacts = L.ended = L.spilled = 0;
     auto own = [&](int f, uint32_t t) { return d3{L.s[3 * f][t], L.s[3 * f + 1][t], L.s[3 * f + 2][t]}; };
@@ -202,6 +207,18 @@ __global__ void __launch_bounds__(kTileThreads, tile_waves(PAIRS, PREC, FAC))
     }
 
     const uint32_t seg = wv * 64u * (KC / ROWS);  // this wavefront's part of the queue
+    bool unsorted = false;  // the particle's row, by this launch or those before it
+    uint32_t waiting = 0;   // its owner's copy of L.more
+    // an entry that ends in the evaluation
+    auto end_entry = [&](uint32_t t, uint32_t slot) {
+        if (slot < 31u) {
+            atomicOr(&L.holes[t], 1u << slot);
+        } else {
+            pj[size_t(slot) * stride + base + t] = kNoEntry;
+            atomicOr(&L.holes[t], kManyHoles);
+        }
+        L.dirty[t] = L.ended = 1;
+    };
     vec accv{};          // W == 64: wavefront 0 sums forces, wavefront 1 torques
     term acct = term(0);  // W < 64: thread c * W + i sums component c
     for (uint32_t k0 = 0;; k0 += KC) {
@@ -218,30 +235,43 @@ __global__ void __launch_bounds__(kTileThreads, tile_waves(PAIRS, PREC, FAC))
             if constexpr (PAIRS != HG_PAIRS_NEIGHBOR_LIST) js[q] = b.offset + k + (k >= b.start + i ? 1u : 0u);
             if (k >= cnt) js[q] = kNoEntry;
         }
+        // each pair's row entry: its slot, the bond bit above it
+        uint32_t held[KC / ROWS];
+#pragma unroll
+        for (uint32_t q = 0; q < KC / ROWS; q++) held[q] = kNoRowSlot;
+        if constexpr (BIN != HG_BINARY_NONE) {
+            auto match = [&](const uint32_t (&t)[4], uint32_t s0) {
+#pragma unroll
+                for (uint32_t q = 0; q < KC / ROWS; q++)
+#pragma unroll
+                    for (uint32_t s = 0; s < 4; s++)
+                        if ((t[s] & kIdxMask) == js[q]) held[q] = (s0 + s) | (t[s] & kBondBit);
+            };
+            match(tags, 0);
+            uint32_t before = tags[3] & kIdxMask;
+            for (uint32_t s = 1; s < 4; s++)
+                unsorted |= s < c_old && (tags[s] & kIdxMask) < (tags[s - 1] & kIdxMask);
+            // four at a time: one by one for every pair, with a search for every
+            // contact, the bed above took 50 us
+            for (uint32_t s0 = 4; s0 < c_old; s0 += 4) {
+                uint32_t t[4];
+#pragma unroll
+                for (uint32_t s = 0; s < 4; s++) t[s] = pj[size_t(s0 + s < c_old ? s0 + s : s0) * stride + g];
+#pragma unroll
+                for (uint32_t s = 1; s < 4; s++)
+                    if (s0 + s >= c_old) t[s] = kNoEntry;
+                match(t, s0);
+                for (uint32_t s = 0; s < 4 && s0 + s < c_old; s++) {
+                    unsorted |= (t[s] & kIdxMask) < before;
+                    before = t[s] & kIdxMask;
+                }
+            }
+        }
         uint32_t nB = 0, nO = 0;
 #pragma unroll
         for (uint32_t q = 0; q < KC / ROWS; q++) {
-            const uint32_t j = js[q];
-            const bool on = j != kNoEntry;
-            uint32_t slot = kNoRowSlot;
-            bool bond = false;
-            if constexpr (BIN != HG_BINARY_NONE) {
-                if (on) {
-#pragma unroll
-                    for (uint32_t s = 0; s < 4; s++)
-                        if ((tags[s] & kIdxMask) == j) {
-                            slot = s;
-                            bond = (tags[s] & kBondBit) != 0;
-                        }
-                    for (uint32_t s = 4; s < c_old; s++) {
-                        const uint32_t t = pj[size_t(s) * stride + g];
-                        if ((t & kIdxMask) == j) {
-                            slot = s;
-                            bond = (t & kBondBit) != 0;
-                        }
-                    }
-                }
-            }
+            const uint32_t j = js[q], slot = held[q] & kIdxMask;
+            const bool on = j != kNoEntry, bond = on && (held[q] & kBondBit) != 0;
             const uint64_t mb = __ballot(on && bond), mo = __ballot(on && !bond), below = (1ull << lane) - 1ull;
             if (on) {
                 const uint32_t at = bond ? nB + uint32_t(__popcll(mb & below))
@@ -293,18 +323,14 @@ __global__ void __launch_bounds__(kTileThreads, tile_waves(PAIRS, PREC, FAC))
                     },
                     lin, ang);
                 st_rec(rec, sp);
-                if (broke) {
-                    pj[size_t(slot) * stride + base + t] = kNoEntry;
-                    L.dirty[t] = L.ended = 1;
-                }
+                if (broke) end_entry(t, slot);
             } else {
                 const bool touching = ev.template free<BIN != HG_BINARY_NONE>(xi, xj, lin);
                 if constexpr (BIN != HG_BINARY_NONE) {
                     if (touching) {
                         L.CW[atomicAdd(&L.contacts, 1u)] = uint16_t(at);
                     } else if (slot != kNoRowSlot) {
-                        pj[size_t(slot) * stride + base + t] = kNoEntry;
-                        L.dirty[t] = L.ended = 1;
+                        end_entry(t, slot);
                     }
                 }
             }
@@ -321,50 +347,54 @@ __global__ void __launch_bounds__(kTileThreads, tile_waves(PAIRS, PREC, FAC))
         if constexpr (BIN != HG_BINARY_NONE) {
             const uint32_t nc = L.contacts;
             if (nc || L.ended) {  // uniform
-                // ended entries leave their rows before new contacts claim slots
-                if (tid < nt && L.dirty[tid]) {
-                    const uint32_t c = L.rows[tid], gi = base + tid;
-                    uint32_t q = 0;
-                    for (uint32_t s = 0; s < c; s++) {
-                        const uint32_t tag = pj[size_t(s) * stride + gi];
-                        if (tag == kNoEntry) continue;
-                        if (q != s) {
-                            pj[size_t(q) * stride + gi] = tag;
-                            st_rec(ps + (size_t(q) * stride + gi) * kSpringRec,
-                                   ld_rec(ps + (size_t(s) * stride + gi) * kSpringRec));
-                        }
-                        q++;
+                // ended entries leave their rows before new contacts claim slots,
+                // the highest slot first: what is above it stays
+                if (tid < nt && L.holes[tid]) {
+                    const uint32_t gi = base + tid;
+                    uint32_t h = L.holes[tid], c = L.rows[tid];
+                    auto drop = [&](uint32_t s) {
+                        if (s == --c) return;
+                        pj[size_t(s) * stride + gi] = pj[size_t(c) * stride + gi];
+                        st_rec(ps + (size_t(s) * stride + gi) * kSpringRec,
+                               ld_rec(ps + (size_t(c) * stride + gi) * kSpringRec));
+                    };
+                    if (h & kManyHoles)
+                        for (uint32_t s = c; s-- > 31u;)
+                            if (pj[size_t(s) * stride + gi] == kNoEntry) drop(s);
+                    for (h &= ~kManyHoles; h;) {
+                        const uint32_t s = 31u - uint32_t(__builtin_clz(h));
+                        h ^= 1u << s;
+                        drop(s);
                     }
-                    L.rows[tid] = q;
+                    L.rows[tid] = L.kept[tid] = c;
                 }
                 __syncthreads();
                 for (uint32_t c = tid; c < nc; c += kTileThreads) {
                     const uint2 e = L.Q[L.CW[c]];
                     const uint32_t pos = queue_place(e.y), t = pos % W, j = e.x, gi = base + t;
-                    uint32_t slot = kNoRowSlot;
-                    if (queue_slot(e.y) != kNoRowSlot) {  // it may have moved just now
-                        const uint32_t rc = L.rows[t] < Vi.cap_s ? L.rows[t] : Vi.cap_s;
-                        slot = row_slot(rc, j, [&](uint32_t s) { return pj[size_t(s) * stride + gi]; });
-                    }
+                    uint32_t slot = queue_slot(e.y);
+                    if (slot != kNoRowSlot && L.holes[t] && slot >= L.kept[t])  // it has moved just now
+                        slot = row_slot(L.kept[t], j, [&](uint32_t s) { return pj[size_t(s) * stride + gi]; });
                     spring9 sp = zero_spring();
                     if (slot != kNoRowSlot) sp = ld_rec(ps + (size_t(slot) * stride + gi) * kSpringRec);
                     vec lin, ang;
                     ev.contact(own(0, t), own(1, t), own(2, t), ld3(Vi.x, j), ld3(Vi.v, j), ld3(Vi.w, j), sp, lin, ang);
+                    double *to = ps;
                     if (slot == kNoRowSlot) {
                         slot = atomicAdd(&L.rows[t], 1u);
-                        L.dirty[t] = 2;
-                        if (slot < Vi.cap_s) {
-                            pj[size_t(slot) * stride + gi] = j;
-                        } else {
-                            const uint32_t q = slot - Vi.cap_s + L.more[t];
+                        L.dirty[t] = 1;
+                        if (slot >= Vi.cap_s) {
+                            slot = slot - Vi.cap_s + L.more[t];
                             L.spilled = 1;
-                            if (q < Vi.cap_s) {
-                                pj_other[size_t(q) * stride + gi] = j;
-                                st_rec(ps_other + (size_t(q) * stride + gi) * kSpringRec, sp);
+                            if (slot < Vi.cap_s) {
+                                (cur ? Vi.pj0 : Vi.pj1)[size_t(slot) * stride + gi] = j;
+                                to = cur ? Vi.ps0 : Vi.ps1;
                             }
+                        } else {
+                            pj[size_t(slot) * stride + gi] = j;
                         }
                     }
-                    if (slot < Vi.cap_s) st_rec(ps + (size_t(slot) * stride + gi) * kSpringRec, sp);
+                    if (slot < Vi.cap_s) st_rec(to + (size_t(slot) * stride + gi) * kSpringRec, sp);
                     if constexpr (HAM != HG_HAMAKER_NONE) lin = lin + vec{L.T[0][pos], L.T[1][pos], L.T[2][pos]};
                     L.T[0][pos] = lin.x;
                     L.T[1][pos] = lin.y;
@@ -377,7 +407,6 @@ __global__ void __launch_bounds__(kTileThreads, tile_waves(PAIRS, PREC, FAC))
                 if (tid < nt && L.dirty[tid]) {
                     const uint32_t gi = base + tid;
                     uint32_t c = L.rows[tid];
-                    bool fresh = L.dirty[tid] == 2;
                     if (L.spilled) {
                         uint32_t more = L.more[tid];
                         if (c > Vi.cap_s) {
@@ -387,33 +416,16 @@ __global__ void __launch_bounds__(kTileThreads, tile_waves(PAIRS, PREC, FAC))
                         // more than the other half holds: it overflows anyway
                         for (; c < Vi.cap_s && more > 0 && more <= Vi.cap_s; c++) {
                             more--;
-                            pj[size_t(c) * stride + gi] = pj_other[size_t(more) * stride + gi];
+                            pj[size_t(c) * stride + gi] = (cur ? Vi.pj0 : Vi.pj1)[size_t(more) * stride + gi];
                             st_rec(ps + (size_t(c) * stride + gi) * kSpringRec,
-                                   ld_rec(ps_other + (size_t(more) * stride + gi) * kSpringRec));
-                            fresh = true;
+                                   ld_rec((cur ? Vi.ps0 : Vi.ps1) + (size_t(more) * stride + gi) * kSpringRec));
                         }
-                        L.more[tid] = more;
+                        L.more[tid] = waiting = more;
                         L.rows[tid] = c;
                     }
-                    if (fresh)  // new entries are at the row's end: insert them in order
-                        for (uint32_t s = 1; s < c; s++) {
-                            const uint32_t tag = pj[size_t(s) * stride + gi];
-                            uint32_t q = s;
-                            if ((pj[size_t(s - 1) * stride + gi] & kIdxMask) < (tag & kIdxMask)) continue;
-                            const spring9 sp = ld_rec(ps + (size_t(s) * stride + gi) * kSpringRec);
-                            while (q > 0) {
-                                const uint32_t prev = pj[size_t(q - 1) * stride + gi];
-                                if ((prev & kIdxMask) < (tag & kIdxMask)) break;
-                                pj[size_t(q) * stride + gi] = prev;
-                                st_rec(ps + (size_t(q) * stride + gi) * kSpringRec,
-                                       ld_rec(ps + (size_t(q - 1) * stride + gi) * kSpringRec));
-                                q--;
-                            }
-                            pj[size_t(q) * stride + gi] = tag;
-                            st_rec(ps + (size_t(q) * stride + gi) * kSpringRec, sp);
-                        }
                     pcnt[gi] = c;
-                    L.dirty[tid] = 0;
+                    L.dirty[tid] = L.holes[tid] = 0;
+                    unsorted = true;
                 }
                 if (tid == 0) L.contacts = L.ended = 0;
             }
@@ -477,10 +489,30 @@ __global__ void __launch_bounds__(kTileThreads, tile_waves(PAIRS, PREC, FAC))
         }
     }
     if constexpr (BIN != HG_BINARY_NONE)
-        if (L.spilled && tid < nt && L.more[tid]) {
+        if (waiting) {
             atomicOr(&Vi.flags[FLAG_PAIR_OVERFLOW], 1);
-            atomicMax(&Vi.flags[FLAG_PAIR_MAXCOUNT], int(L.rows[tid] + L.more[tid]));
+            atomicMax(&Vi.flags[FLAG_PAIR_MAXCOUNT], int(L.rows[tid] + waiting));
             if (Vi.sflags) atomicOr(&Vi.sflags[b.slot], HG_FAULT_PAIR_CAPACITY);
+        }
+    if constexpr (BIN != HG_BINARY_NONE)
+        if (mode != TILE_STEP && unsorted && tid < nt) {
+            const uint32_t gi = base + tid, c = L.rows[tid];
+            for (uint32_t s = 1; s < c; s++) {
+                const uint32_t tag = pj[size_t(s) * stride + gi];
+                uint32_t q = s;
+                if ((pj[size_t(s - 1) * stride + gi] & kIdxMask) < (tag & kIdxMask)) continue;
+                const spring9 sp = ld_rec(ps + (size_t(s) * stride + gi) * kSpringRec);
+                while (q > 0) {
+                    const uint32_t prev = pj[size_t(q - 1) * stride + gi];
+                    if ((prev & kIdxMask) < (tag & kIdxMask)) break;
+                    pj[size_t(q) * stride + gi] = prev;
+                    st_rec(ps + (size_t(q) * stride + gi) * kSpringRec,
+                           ld_rec(ps + (size_t(q - 1) * stride + gi) * kSpringRec));
+                    q--;
+                }
+                pj[size_t(q) * stride + gi] = tag;
+                st_rec(ps + (size_t(q) * stride + gi) * kSpringRec, sp);
+            }
         }
     if constexpr (W < 64) {
         if (tid < 6u * W) L.A[r0][i] = acct;

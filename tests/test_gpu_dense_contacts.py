@@ -153,3 +153,33 @@ def test_a_full_row_takes_one_contact_for_another(first):
     np.testing.assert_array_equal(s.springs(0)[0], o.springs(0)[0])
     np.testing.assert_array_equal(s.springs(0)[1], o.springs(0)[1])
     s.close()
+
+
+@pytest.mark.parametrize("pairs", [0, 1])
+@pytest.mark.parametrize("n", [70, 130])
+def test_rows_of_more_than_31_entries(n, pairs):
+    """A cloud of spheres pressed into one another that flies apart: rows of
+    dozens of entries that end here and there, looked at after every few steps
+    and after many."""
+    import libgran_amd as L
+    print(f"[bed] long rows, n {n}, pairs {pairs}", flush=True)
+    rng = np.random.default_rng(n)
+    x = rng.uniform(0.0, 2.6 * R, (n, 3))
+    v, w = rng.normal(0.0, 300.0, (n, 3)), rng.normal(0.0, 1e8, (n, 3))
+    contact = O.contact_params(k=10.0)
+    kw = dict(r_verlet=6.0 * R) if pairs else {}
+    o = O.OracleSystem(O.system_params(O.BIN_CONTACT, O.HAM_NONE, neighbor_mode=pairs, contact=contact, **kw), x, v, w0=w)
+    s = L.System(L.make_params(L.BINARY_CONTACT, L.HAMAKER_NONE, pair_mode=pairs, contact=contact, pair_capacity=n,
+                               neighbor_capacity=n if pairs else 0, **kw), x, v, omega0=w)
+    s.per_step_launches(True)
+    rows = []
+    for steps in (1, 2, 5, 40, 40, 80, 80):
+        o.step(1e-13, steps, rebuild_every=20)
+        s.step(1e-13, steps, rebuild_every=20)
+        equal(o.state(), s.state(), f"after {steps}")
+        ij = o.springs(0)[0]
+        np.testing.assert_array_equal(s.springs(0)[0], ij)
+        np.testing.assert_array_equal(s.springs(0)[1], o.springs(0)[1])
+        rows.append(np.bincount(ij[:, 0], minlength=n))
+    assert rows[-1].max() > 40 and rows[0].sum() - rows[-1].sum() > 50
+    s.close()
