@@ -54,7 +54,7 @@ struct tile_lds {
     uint32_t contacts, ended;
     // the terms of four facets: FP64 the 6 components of each, mixed the
     // contact's 6 and the Hamaker term's 3
-    typename prec_types<PREC>::term F[FAC ? 4 : 1][9][W];
+    term F[FAC ? 4 : 1][FAC ? 9 : 1][FAC ? W : 1];
     term A[6][W < 64 ? W : 1];
 };
 
@@ -70,9 +70,10 @@ __device__ __forceinline__ wide_block tile_block(const wide_block *map, const po
 // a CU, hide one pair's latency behind another's: mixed 151 us a step at
 // 635,000 particles with three, 187 with two (four spill: 241); with the facet
 // terms three spill too: 24 plate tests of 1,000 steps 40.5 ms, 35.8 with two.
-// FP64 takes the same time with two and three (72.2 ms for 800 steps of 333
-// aggregates). All pairs come in few blocks, and two cost them registers: 33 us
-// a step at 522 particles against 28.
+// In FP64 nine registers spill with three: 213,000 particles in 333 systems
+// take 54.5 us a step, 61.7 with two, but 20,000 in one 14.0 against 13.3 and
+// 200 8.9 against 8.4. All pairs come in few blocks, and two cost them
+// registers: 33 us a step at 522 particles against 28.
 constexpr int tile_waves(int pairs, int prec, bool fac) {
     return pairs != HG_PAIRS_NEIGHBOR_LIST ? 1 : (prec == HG_PRECISION_MIXED && !fac ? 3 : 2);
 }
@@ -102,6 +103,8 @@ __global__ void __launch_bounds__(kTileThreads, tile_waves(PAIRS, PREC, FAC))
     using term = typename prec_types<PREC>::term;
     using vec = typename prec_types<PREC>::vec;
     __shared__ tile_lds<W, KC, PREC, FAC> L;
+    // a workgroup is a wavefront for each SIMD: the CU's LDS holds as many
+    static_assert(sizeof(L) * size_t(tile_waves(PAIRS, PREC, FAC)) <= 160u * 1024u, "LDS of the tiles on a CU");
     touch_args<sizeof(hg_params) + sizeof(mixed_consts) + 2 * sizeof(pool_view)>();
     const wide_block b = tile_block(map, Vi, W);
     const uint32_t n = b.n & kIdxMask, cur = b.n >> 31, base = b.offset + b.start;
