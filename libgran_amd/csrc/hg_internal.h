@@ -14,6 +14,20 @@
 
 namespace hg {
 
+// All-pairs systems of more particles than this are stepped by the walk, a lane
+// a particle, smaller ones by tiles, a workgroup a particle. A tile's step takes
+// 0.027 ns a pair with a contact and a Hamaker functor (FP64; 0.022 with one of
+// them; mixed 0.0125 and 0.012), so it grows with n^2; the walk's takes 0.8 us
+// (0.4; 0.34 and 0.25) times n while the chip has lanes left. FP64, both
+// functors: 15.3 against 19.2 ms at 24,000, 26.9 against 25.4 at 32,000, 60
+// against 38 at 48,000; contact alone 4.5 against 5.8 at 14,000, 7.3 both at
+// 18,000, 22.5 against 12.3 at 32,000.
+inline size_t all_pairs_tile_most(const hg_params &p) {
+    const bool both = p.binary_model != HG_BINARY_NONE && p.hamaker_model != HG_HAMAKER_NONE;
+    if (p.precision == HG_PRECISION_MIXED) return both ? 26000 : 20000;
+    return both ? 30000 : 18000;
+}
+
 // Device flag words (int32 each) written by kernels, read back by the host.
 // The MAXCOUNT words are raised only by lists that overflow, so they hold the
 // count the overflow needed. FLAG_NUMERIC: a velocity or angular velocity
@@ -215,8 +229,8 @@ hg_status fail(hg_status st, const std::string &msg);
     } while (0)
 
 // kernel launchers (kernels.hip)
-// The per-particle walk: the legacy functor, and the contact and alt_sinter
-// functors with dissipation tracking (sv.diss).
+// The per-particle walk: the legacy functor, the contact and alt_sinter
+// functors with dissipation tracking (sv.diss), and large all-pairs systems.
 hipError_t launch_force(const hg_params &p, const sys_view &sv, hipStream_t s);
 hipError_t launch_kick_drift(double *x, double *v, double *th, double *w, const double *a, const double *al,
                              uint32_t n, bool pending, double half_prev, double half, double dt, facet_dev *facets,

@@ -694,11 +694,14 @@ inline unsigned blocks_for(size_t n, unsigned bs) { return unsigned((n + bs - 1)
 template <int BIN, int HAM, bool TRACK>
 hipError_t launch_force_t(const hg_params &p, const sys_view &sv, hipStream_t s) {
     if (sv.n == 0) return hipSuccess;
-    // 64-lane blocks spread a modest particle count over more CUs.
-    if (p.pair_mode == HG_PAIRS_NEIGHBOR_LIST)
-        k_force_nl<BIN, HAM, TRACK><<<blocks_for(sv.n, 64), 64, 0, s>>>(p, sv);
-    else
+    if (p.pair_mode != HG_PAIRS_NEIGHBOR_LIST) {
         k_force_all<BIN, HAM, TRACK><<<blocks_for(sv.n, kTile), kTile, 0, s>>>(p, sv);
+    } else if constexpr (TRACK || BIN == HG_BINARY_SINTER_LEGACY) {
+        // 64-lane blocks spread a modest particle count over more CUs.
+        k_force_nl<BIN, HAM, TRACK><<<blocks_for(sv.n, 64), 64, 0, s>>>(p, sv);
+    } else {
+        return hipErrorInvalidValue;  // tiles
+    }
     return hipGetLastError();
 }
 
@@ -717,10 +720,16 @@ hipError_t launch_force(const hg_params &p, const sys_view &sv, hipStream_t s) {
     HG_CASE(HG_BINARY_SINTER, HG_HAMAKER_FULL, true)
     HG_CASE(HG_BINARY_SINTER, HG_HAMAKER_LIMITED, true)
     HG_CASE(HG_BINARY_SINTER, HG_HAMAKER_SIMPLIFIED, true)
-    HG_CASE(HG_BINARY_SINTER_LEGACY, HG_HAMAKER_NONE, false)
-    HG_CASE(HG_BINARY_SINTER_LEGACY, HG_HAMAKER_FULL, false)
-    HG_CASE(HG_BINARY_SINTER_LEGACY, HG_HAMAKER_LIMITED, false)
-    HG_CASE(HG_BINARY_SINTER_LEGACY, HG_HAMAKER_SIMPLIFIED, false)
+#define HG_CASES(B)                        \
+    HG_CASE(B, HG_HAMAKER_NONE, false)     \
+    HG_CASE(B, HG_HAMAKER_FULL, false)     \
+    HG_CASE(B, HG_HAMAKER_LIMITED, false)  \
+    HG_CASE(B, HG_HAMAKER_SIMPLIFIED, false)
+    HG_CASES(HG_BINARY_NONE)
+    HG_CASES(HG_BINARY_CONTACT)
+    HG_CASES(HG_BINARY_SINTER)
+    HG_CASES(HG_BINARY_SINTER_LEGACY)
+#undef HG_CASES
 #undef HG_CASE
     return hipErrorInvalidValue;
 }

@@ -241,8 +241,12 @@ sys_view make_view(hg_system *S) {
 
 // Whether the system's passes run as per-step launches over tiles
 // (tile_step.h): every functor but the legacy one, without dissipation
-// tracking; those take the per-particle walk of kernels.hip.
-bool tiled(const hg_system *S) { return S->p.binary_model != HG_BINARY_SINTER_LEGACY && !S->track_diss; }
+// tracking, and all pairs up to a size; the others take the per-particle walk of
+// kernels.hip.
+bool tiled(const hg_system *S) {
+    return S->p.binary_model != HG_BINARY_SINTER_LEGACY && !S->track_diss &&
+           (S->p.pair_mode == HG_PAIRS_NEIGHBOR_LIST || S->n <= all_pairs_tile_most(S->p));
+}
 
 // The views of a tiled system: its own buffers and the second set. What the
 // device needs beside them is made on first use and refreshed when the facet
