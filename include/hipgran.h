@@ -373,7 +373,8 @@ hg_status hg_pool_set_wide_threshold(hg_pool *pool, size_t wide_min);
  * the interval's wide steps, then the chunk kernel, each on the whole GPU.
  * 0 <= wide_cus < CU count. */
 hg_status hg_pool_set_wide_cus(hg_pool *pool, int wide_cus);
-/* The wide launches of one interval (one per step + 1) are recorded once into a
+/* The wide launches of one interval (one per step + 1, two for large systems
+ * with all pairs) are recorded once into a
  * HIP graph per (interval length, dt, wide set) and replayed; enable = 0
  * launches them one by one instead. Default on. */
 hg_status hg_pool_set_wide_graph(hg_pool *pool, int enable);

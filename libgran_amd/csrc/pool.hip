@@ -111,6 +111,44 @@ hipError_t launch_tile_steps(const hg_params &p, const pool_view &V, const pool_
 
 namespace {
 
+// The kicks of the walked systems (large all-pairs systems): before step s's
+// pass the kick and drift (with `pending` = s > 0 the completion of step s - 1
+// and the facets' move first), after the last pass its completion.
+__global__ void __launch_bounds__(kWalkBlock) k_walk_kick(pool_view V, const wide_block *map, int pending, double half,
+                                                          double dt) {
+    const wide_block b = map[blockIdx.x];
+    const pool_meta M = V.meta[b.slot];
+    if (pending && b.start == 0 && threadIdx.x == 0)
+        advance_facets(V.facets + size_t(b.slot) * V.max_facets, int(M.nf), dt);
+    const uint32_t g = M.offset + b.start + threadIdx.x;
+    if (g < M.offset + M.n) pool_kick_drift<STATE_GLOBAL>(V, M, pending != 0, half, dt, g, g + 1, 1);
+}
+__global__ void __launch_bounds__(kWalkBlock) k_walk_final(pool_view V, const wide_block *map, double half, double dt) {
+    const wide_block b = map[blockIdx.x];
+    const pool_meta M = V.meta[b.slot];
+    if (b.start == 0 && threadIdx.x == 0) advance_facets(V.facets + size_t(b.slot) * V.max_facets, int(M.nf), dt);
+    const uint32_t g = M.offset + b.start + threadIdx.x;
+    if (g < M.offset + M.n) pool_final_kick<STATE_GLOBAL>(V, M, half, g, g + 1, 1);
+}
+
+hipError_t launch_walk(const hg_params &p, const pool_view &V, const wide_block *map, unsigned blocks, int pass,
+                       hipStream_t s) {
+    if (p.binary_model == HG_BINARY_NONE) return launch_walk_b<HG_BINARY_NONE>(p, V, map, blocks, pass, s);
+    if (p.binary_model == HG_BINARY_CONTACT) return launch_walk_b<HG_BINARY_CONTACT>(p, V, map, blocks, pass, s);
+    if (p.binary_model == HG_BINARY_SINTER) return launch_walk_b<HG_BINARY_SINTER>(p, V, map, blocks, pass, s);
+    return hipErrorInvalidValue;
+}
+hipError_t launch_walk_steps(const hg_params &p, const pool_view &V, const wide_block *map, unsigned blocks,
+                             uint32_t len, double half, double dt, hipStream_t s) {
+    for (uint32_t k = 0; k < len; k++) {
+        k_walk_kick<<<blocks, kWalkBlock, 0, s>>>(V, map, k > 0 ? 1 : 0, half, dt);
+        const hipError_t e = launch_walk(p, V, map, blocks, int(k), s);
+        if (e != hipSuccess) return e;
+    }
+    k_walk_final<<<blocks, kWalkBlock, 0, s>>>(V, map, half, dt);
+    return hipGetLastError();
+}
+
 }  // namespace
 }  // namespace hg
 
@@ -153,7 +191,7 @@ struct hg_pool {
     wide_block *wide_map_d = nullptr;
     size_t wide_map_cap = 0;
     unsigned wide_blocks = 0;
-    bool wide_pending_initial = false;
+    bool wide_walk = false;  // the wide systems are walked, not tiled (all pairs)
     // with wide systems present the wide launches run on stream_w beside the
     // chunk kernel, whose grid then leaves room worth wide_cus CUs
     hipStream_t stream_w = nullptr;
@@ -171,7 +209,7 @@ struct hg_pool {
     size_t tune_pos = 0;
     hipGraphExec_t wg_exec = nullptr;
     uint32_t wg_len = 0;
-    bool wg_facets = false;
+    bool wg_facets = false, wg_walk = false;
     unsigned wg_blocks = 0;
     double wg_dt = 0.0;
     hipEvent_t wev[3] = {nullptr, nullptr, nullptr};
@@ -845,7 +883,8 @@ namespace {
 // only shows once every workgroup has work: 635,000 particles in 1,024
 // systems, mixed, took 206 us a step with the line at 4,096, 128 at 1,536 and
 // 166 at 512; 210,000 in 333, FP64, 291 us at 2,048 and 75 all wide.
-// With all pairs a round costs 0.5 us a partner and the tiles 0.1 ns a pair.
+// With all pairs a round costs 0.5 us a partner and the tiles 0.1 ns a pair at
+// 522 particles (0.03 from 3,000 on, and the walk takes over above).
 size_t split_order(const hg_pool *Q) {
     const size_t count = Q->order.size();
     if (!Q->wide_min) return 0;
@@ -887,8 +926,15 @@ hg_status refresh_order(hg_pool *Q) {
     std::stable_sort(Q->order.begin(), Q->order.end(),
                      [&](uint32_t a, uint32_t b) { return Q->meta[a].n > Q->meta[b].n; });
     std::vector<wide_block> map;
-    const uint32_t width = uint32_t(tile_width(Q->p.pair_mode));
     const size_t first_narrow = split_order(Q);
+    Q->wide_walk = false;
+    if (Q->p.pair_mode == HG_PAIRS_ALL && first_narrow) {
+        // tiles take a time per pair, the walk one per particle of the largest
+        double pairs = 0.0;
+        for (size_t k = 0; k < first_narrow; k++) pairs += double(Q->meta[Q->order[k]].n) * Q->meta[Q->order[k]].n;
+        Q->wide_walk = pairs > double(all_pairs_tile_most(Q->p)) * Q->meta[Q->order[0]].n;
+    }
+    const uint32_t width = Q->wide_walk ? kWalkBlock : uint32_t(tile_width(Q->p.pair_mode));
     for (size_t k = 0; k < first_narrow; k++) {
         const uint32_t s = Q->order[k];
         const pool_meta &M = Q->meta[s];
@@ -1075,7 +1121,9 @@ hg_status pool_begin(hg_pool *Q, double dt, uint64_t max_len, uint32_t rebuild_e
         bool wide_facets = false;
         for (size_t k = 0; k < Q->order.size() - count; k++) wide_facets |= Q->meta[Q->order[k]].nf > 0;
         if (any_wide_initial) {
-            HG_HIP(launch_tile(Q->p, V, V, Q->wide_map_d, Q->wide_blocks, TILE_FORCE, wide_facets, half, dt, s2));
+            HG_HIP(Q->wide_walk
+                       ? launch_walk(Q->p, V, Q->wide_map_d, Q->wide_blocks, -1, s2)
+                       : launch_tile(Q->p, V, V, Q->wide_map_d, Q->wide_blocks, TILE_FORCE, wide_facets, half, dt, s2));
             Q->last_wide_launches++;
         }
         pool_view VB = V;
@@ -1090,11 +1138,13 @@ hg_status pool_begin(hg_pool *Q, double dt, uint64_t max_len, uint32_t rebuild_e
         // a program that copies through the default stream in another thread
         // while a pool of small systems steps must not meet a recording
         auto enqueue = [&](hipStream_t st_) {
-            return launch_tile_steps(Q->p, V, VB, Q->wide_map_d, Q->wide_blocks, len, wide_facets, half, dt, st_);
+            return Q->wide_walk ? launch_walk_steps(Q->p, V, Q->wide_map_d, Q->wide_blocks, len, half, dt, st_)
+                                : launch_tile_steps(Q->p, V, VB, Q->wide_map_d, Q->wide_blocks, len, wide_facets, half,
+                                                    dt, st_);
         };
         if (Q->wide_graph && Q->meta[Q->order[0]].n >= Q->wide_min) {
             if (!Q->wg_exec || Q->wg_len != len || Q->wg_dt != dt || Q->wg_blocks != Q->wide_blocks ||
-                Q->wg_facets != wide_facets) {
+                Q->wg_facets != wide_facets || Q->wg_walk != Q->wide_walk) {
                 if (Q->wg_exec) HG_HIP(hipGraphExecDestroy(Q->wg_exec));
                 Q->wg_exec = nullptr;
                 hipGraph_t graph = nullptr;
@@ -1108,6 +1158,7 @@ hg_status pool_begin(hg_pool *Q, double dt, uint64_t max_len, uint32_t rebuild_e
                 HG_HIP(ei);
                 Q->wg_len = len;
                 Q->wg_facets = wide_facets;
+                Q->wg_walk = Q->wide_walk;
                 Q->wg_dt = dt;
                 Q->wg_blocks = Q->wide_blocks;
             }
@@ -1115,7 +1166,7 @@ hg_status pool_begin(hg_pool *Q, double dt, uint64_t max_len, uint32_t rebuild_e
         } else {
             HG_HIP(enqueue(s2));
         }
-        Q->last_wide_launches += len + 1;
+        Q->last_wide_launches += Q->wide_walk ? 2 * len + 1 : len + 1;
         HG_HIP(hipEventRecord(Q->wev[1], s2));
     }
     if (count) {
@@ -1153,11 +1204,12 @@ hg_status pool_end(hg_pool *Q, std::vector<int32_t> &faulted) {
     HG_HIP(hipStreamSynchronize(Q->stream));
     // host mirror of what the kernels did to each system, before any fault is
     // read, so that the systems that go on keep a true mirror
-    const size_t wide = Q->order.size() - Q->fl.count;  // the first ones; their tables are updated in place
+    // the first ones are wide; tiles update their tables in place
+    const size_t in_place = Q->wide_walk ? 0 : Q->order.size() - Q->fl.count;
     for (size_t k = 0; k < Q->order.size(); k++) {
         const uint32_t s = Q->order[k];
         pool_meta &M = Q->meta[s];
-        if (Q->cap_s && k >= wide) {
+        if (Q->cap_s && k >= in_place) {
             if (!M.acc_valid) M.cur ^= 1u;
             M.cur ^= (len & 1u);
         }

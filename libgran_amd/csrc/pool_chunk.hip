@@ -78,4 +78,29 @@ hipError_t launch_tile_b<HG_BIN, HG_PAIRS>(const hg_params &p, const pool_view &
     return hipErrorInvalidValue;
 }
 
+#if HG_PAIRS == 0
+static_assert(HG_PAIRS_ALL == 0, "the walk is all pairs'");
+template <>
+hipError_t launch_walk_b<HG_BIN>(const hg_params &p, const pool_view &V, const wide_block *map, unsigned blocks,
+                                 int pass, hipStream_t s) {
+    if (blocks == 0) return hipSuccess;
+    const mixed_consts mc = make_mixed_consts(p);
+#define HG_WCASE(H, PREC)                                                                  \
+    if (p.hamaker_model == H && p.precision == PREC) {                                     \
+        k_walk_force<HG_BIN, H, PREC><<<blocks, kWalkBlock, 0, s>>>(p, mc, V, map, pass);  \
+        return hipGetLastError();                                                          \
+    }
+    HG_WCASE(HG_HAMAKER_NONE, HG_PRECISION_FP64)
+    HG_WCASE(HG_HAMAKER_FULL, HG_PRECISION_FP64)
+    HG_WCASE(HG_HAMAKER_LIMITED, HG_PRECISION_FP64)
+    HG_WCASE(HG_HAMAKER_SIMPLIFIED, HG_PRECISION_FP64)
+    HG_WCASE(HG_HAMAKER_NONE, HG_PRECISION_MIXED)
+    HG_WCASE(HG_HAMAKER_FULL, HG_PRECISION_MIXED)
+    HG_WCASE(HG_HAMAKER_LIMITED, HG_PRECISION_MIXED)
+    HG_WCASE(HG_HAMAKER_SIMPLIFIED, HG_PRECISION_MIXED)
+#undef HG_WCASE
+    return hipErrorInvalidValue;
+}
+#endif
+
 }  // namespace hg

@@ -83,6 +83,15 @@ hipError_t launch_tile(const hg_params &p, const pool_view &Vi, const pool_view 
 hipError_t launch_tile_steps(const hg_params &p, const pool_view &V, const pool_view &VB, const wide_block *map,
                              unsigned blocks, uint32_t len, bool facets, double half, double dt, hipStream_t s);
 
+// Per-step launches of large all-pairs systems, a lane a particle
+// (all_pairs_tile_most): wide_block b carries [start, start + kWalkBlock), the
+// pair-state table alternates between its halves as in the chunk kernel.
+// pass < 0: the accelerations of the systems that have none.
+constexpr uint32_t kWalkBlock = 128;
+template <int BIN>
+hipError_t launch_walk_b(const hg_params &p, const pool_view &V, const wide_block *map, unsigned blocks, int pass,
+                         hipStream_t s);
+
 template <int PAIRS>
 inline hipError_t launch_chunk_p(const hg_params &p, const pool_view &V, const chunk_launch &c, hipStream_t s) {
     if (p.binary_model == HG_BINARY_NONE) return launch_chunk_b<HG_BINARY_NONE, PAIRS>(p, V, c, s);
@@ -242,8 +251,8 @@ __device__ __forceinline__ uint32_t block_max_u32(uint32_t v, uint32_t *s_red) {
 }
 
 // Acceleration pass for particles g = g_first, g_first + g_step, ... < g_end
-// of system M (a workgroup strides over the whole system; a wide launch gives
-// each thread one particle). With LIDS the partner ids come from the system's
+// of system M (a workgroup strides over the whole system; a pack and the walk of
+// large all-pairs systems give each thread one particle). With LIDS the partner ids come from the system's
 // LDS copy `lids` (lds_ids_fill).
 template <int BIN, int HAM, int PAIRS, int PREC, int LDS, bool LIDS = false, bool FAC = true>
 __device__ __forceinline__ void pool_force_phase(const hg_params &P, const mixed_consts &MC, const pool_view &V,
@@ -604,6 +613,19 @@ __global__ void __launch_bounds__(TPB, HG_CHUNK_MIN_BLOCKS)
         for (uint32_t k = 0; k < cnt; k++)
             run_one<BIN, HAM, PAIRS, PREC, FAC>(P, MC, V, order[first + k], nsteps, dt, lds_bytes, s_red);
     }
+}
+
+template <int BIN, int HAM, int PREC>
+__global__ void __launch_bounds__(kWalkBlock)
+    k_walk_force(hg_params P, mixed_consts MC, pool_view V, const wide_block *map, int pass) {
+    const wide_block b = map[blockIdx.x];
+    const pool_meta M = V.meta[b.slot];
+    if (pass < 0 && M.acc_valid) return;
+    const uint32_t passed = pass < 0 ? 0u : uint32_t(pass) + (M.acc_valid ? 0u : 1u);
+    const uint32_t g = M.offset + b.start + threadIdx.x;
+    if (g >= M.offset + M.n) return;
+    pool_force_phase<BIN, HAM, HG_PAIRS_ALL, PREC, STATE_GLOBAL>(
+        P, MC, V, M, M.cur ^ (passed & 1u), V.facets + size_t(b.slot) * V.max_facets, g, g + 1, 1);
 }
 
 }  // namespace
