@@ -440,6 +440,7 @@ size_t hg_pool_bytes_per_particle(const hg_params *p, size_t max_facets) {
     if (p->binary_model == HG_BINARY_SINTER && p->sinter_breaking)
         b += kMaxBondsPerParticle * 12 + 4;  // neck-strength lists
     if (p->pair_mode == HG_PAIRS_NEIGHBOR_LIST) b += 4 + 32 + 3 * 2 * 4 + 4;  // cell list scratch
+    else b += sizeof(wide_block);  // tiles of one particle
     return b;
 }
 
