@@ -51,7 +51,8 @@ def log(msg):
     """Progress of the legs, on stderr (the JSON line alone goes to stdout)."""
     print(f"[bench {time.perf_counter() - T_START:7.1f} s] {msg}", file=sys.stderr, flush=True)
 # The pool's autotuner scores each candidate over two rebuild intervals: two
-# chunk shapes, then 21 launch splits on this batch. With fewer warm-up steps
+# chunk shapes, then eight launch splits on this batch; 46 intervals leave the
+# chosen one some. With fewer warm-up steps
 # a fixed choice is set: 512 threads x 1 workgroup per CU (what the tuner
 # picks) and wide threshold 4096 with the wide steps run before the chunk
 # kernel rather than beside it (the fastest of a sweep of 14 splits, and the
@@ -119,7 +120,7 @@ def run_pool(L, precision, sizes, xs, vs, steps, warmup, split=None, chunk_shape
     tuning = pool.tuning()
     tuning["packing"] = packing
     # measured neighbour and spring counts on a sample of the chunk kernel's systems
-    wm = tuning["wide_min"]
+    wm = pool.split()["wide_from"]
     narrow = [s for s, n in zip(slots, sizes) if not wm or n < wm]
     sample = narrow[:: max(1, len(narrow) // 64)]
     npart = sum(pool.info(s)[0] for s in sample)

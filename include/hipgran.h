@@ -366,6 +366,12 @@ hg_status hg_pool_last_step_profile(hg_pool *pool, double *chunk_ms, double *reb
  * The per-particle operations are the same, so results do not change. Takes
  * effect at the next hg_pool_step. */
 hg_status hg_pool_set_wide_threshold(hg_pool *pool, size_t wide_min);
+/* enable = 0: the threshold alone decides, and exactly the systems of at least
+ * wide_min particles take the per-step launches. Default on. */
+hg_status hg_pool_set_split_estimate(hg_pool *pool, int enable);
+/* The split of the last hg_pool_step: the particles of the smallest system that
+ * took the per-step launches (0: none did), and whether the estimate is on. */
+hg_status hg_pool_get_split(hg_pool *pool, size_t *wide_from, int *estimated);
 /* While both kinds of systems are present, the chunk kernel's persistent grid
  * shrinks to wg_per_cu * (CUs - wide_cus) workgroups, leaving room worth
  * wide_cus CUs (default a quarter) for the wide launches that run beside it
@@ -385,12 +391,14 @@ hg_status hg_pool_set_wide_graph(hg_pool *pool, int enable);
 hg_status hg_pool_set_packing(hg_pool *pool, int enable);
 /* Online autotuner: from the next hg_pool_step on, first the chunk kernel's
  * shape (256 threads x 2 workgroups per CU, or 512 x 1), then, at the better
- * shape, whether the wide launches run one after the other with the chunk
- * kernel or beside it with room for CUs/8 or /4. Each candidate runs two
- * rebuild intervals of live steps, scored by the second one's host-measured
- * time per step; the fastest is kept. Neither choice changes results, so no
- * step is wasted. Nothing is tuned where every system takes the wide launches.
- * enable = 0 stops it and keeps the current setting. */
+ * shape, the launch split: the present one with the wide launches before the
+ * chunk kernel or beside it with room for CUs/8 or /4, and exact thresholds of 0
+ * and 1024..8192 up to the largest system. Each candidate runs two rebuild
+ * intervals of live steps, scored by the second one's host-measured time per
+ * step; the fastest is kept. Neither choice changes results, so no step is
+ * wasted. While every system takes the wide launches there is nothing to tune
+ * (tuned = 1); it starts with the first step in which one does not. enable = 0
+ * stops it and keeps the current setting. */
 hg_status hg_pool_autotune(hg_pool *pool, int enable);
 /* Current split and whether the autotuner has finished (tuned = 1). */
 hg_status hg_pool_get_tuning(hg_pool *pool, size_t *wide_min, int *wide_cus, int *tuned);

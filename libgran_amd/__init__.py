@@ -477,8 +477,21 @@ class Pool:
         return f.value
 
     def set_wide_threshold(self, wide_min):
-        """Systems of at least wide_min particles (0: none) use the wide launches."""
+        """Systems of at least wide_min particles (0: none) use the wide launches,
+        and smaller ones where an estimate favours it."""
         _abi.check(_abi.lib().hg_pool_set_wide_threshold(self._h, int(wide_min)))
+
+    def set_split_estimate(self, enable):
+        """Let the estimate send smaller systems wide (default) or go by the
+        threshold alone."""
+        _abi.check(_abi.lib().hg_pool_set_split_estimate(self._h, 1 if enable else 0))
+
+    def split(self):
+        """The last step's split: particles of the smallest system on the wide
+        launches (0: none), and whether the estimate is on."""
+        wf, est = C.c_size_t(0), C.c_int(0)
+        _abi.check(_abi.lib().hg_pool_get_split(self._h, C.byref(wf), C.byref(est)))
+        return dict(wide_from=wf.value, estimate=bool(est.value))
 
     def set_wide_cus(self, wide_cus):
         """CUs given to the wide launches while both kinds of systems run."""

@@ -140,6 +140,8 @@ SIGNATURES = {
     "hg_pool_save": (C.c_int, [_sysp, C.c_int32, C.c_void_p, C.c_size_t, _szp]),
     "hg_pool_load": (C.c_int, [_sysp, C.c_void_p, C.c_size_t, C.POINTER(C.c_int32)]),
     "hg_pool_set_wide_threshold": (C.c_int, [_sysp, C.c_size_t]),
+    "hg_pool_set_split_estimate": (C.c_int, [_sysp, C.c_int]),
+    "hg_pool_get_split": (C.c_int, [_sysp, _szp, C.POINTER(C.c_int)]),
     "hg_pool_last_wide_profile": (C.c_int, [_sysp, _dp, _u64p]),
     "hg_pool_last_busy": (C.c_int, [_sysp, _dp]),
     "hg_pool_set_wide_cus": (C.c_int, [_sysp, C.c_int]),

@@ -188,6 +188,10 @@ struct hg_pool {
     uint32_t pack_count = 0;
     bool packing = true;           // small systems share a workgroup (neighbour-list mode)
     uint32_t wide_min = 0;         // systems with n >= wide_min use the wide launches (0: none)
+    bool estimate = true;          // and others where split_order's estimate favours it
+    uint32_t asked_min = 0;        // the two as the caller set them, which the tuner starts from
+    bool asked_estimate = true;
+    uint32_t wide_from = 0;        // the smallest system that does, in the order last used (0: none)
     wide_block *wide_map_d = nullptr;
     size_t wide_map_cap = 0;
     unsigned wide_blocks = 0;
@@ -201,6 +205,7 @@ struct hg_pool {
     int tune_phase = 0;      // TUNE_*
     struct tune_cand {
         uint32_t wide_min;
+        bool estimate;
         int wide_cus, tpb, wgs;  // launch split, chunk shape
     };
     std::vector<tune_cand> tune_cands;
@@ -503,7 +508,7 @@ hg_status hg_pool_create(const hg_params *params, size_t max_particles, size_t m
     for (auto &e : Q->ev) PG_HIPC(hipEventCreate(&e));
     for (auto &e : Q->wev) PG_HIPC(hipEventCreate(&e));
     for (auto &e : Q->evb) PG_HIPC(hipEventCreate(&e));
-    Q->wide_min = kDefaultWideMin;
+    Q->wide_min = Q->asked_min = kDefaultWideMin;
     Q->wide_cus = int(std::lround(kDefaultWideCuFraction * Q->n_cus));
     PG_HIPC(hipStreamCreateWithFlags(&Q->stream_w, hipStreamNonBlocking));
     PG_HIPC(hipStreamCreateWithFlags(&Q->stream_c, hipStreamNonBlocking));
@@ -870,7 +875,7 @@ namespace {
 
 // How many of the active systems, largest first, take the wide launches: all
 // of at least wide_min particles, and as many of the others as the estimates
-// below favour (none when wide_min = 0).
+// below favour (none when wide_min = 0 or the estimate is off).
 //
 // A step of the wide launches costs a launch's latency or the chip's rate over
 // their particles, whichever is more; the chunk kernel's costs its longest
@@ -903,6 +908,7 @@ size_t split_order(const hg_pool *Q) {
         const double longest = k < count ? item_us(Q->meta[Q->order[k]].n) : 0.0;
         const bool required = k < count && Q->meta[Q->order[k]].n >= Q->wide_min;
         const bool boundary = k == 0 || k == count || Q->meta[Q->order[k]].n != Q->meta[Q->order[k - 1]].n;
+        if (!required && !Q->estimate) return k;
         if (!required && boundary) {
             const double us = (k ? std::max(8.0, wide) : 0.0) + std::max(longest, chunk / wgs);
             if (best_us == 0.0 || us < best_us) {
@@ -944,6 +950,7 @@ hg_status refresh_order(hg_pool *Q) {
     }
     if (map.size() > Q->wide_map_cap) return fail(HG_ERR_INVALID, "hg_pool_step: wide map overflow");
     Q->narrow_count = uint32_t(Q->order.size() - first_narrow);
+    Q->wide_from = first_narrow ? Q->meta[Q->order[first_narrow - 1]].n : 0u;
     Q->wide_blocks = unsigned(map.size());
     // The queue, largest first: each system of at least a workgroup's
     // threads alone, then (neighbour-list mode) the smaller ones packed best
@@ -1002,40 +1009,50 @@ hg_status refresh_order(hg_pool *Q) {
 
 // Online tuner, in two stages: the chunk kernel's shape (256 threads, two
 // workgroups per CU; 512 threads, one: the same waves per SIMD with twice the
-// LDS per system), then whether the wide launches run ahead of the chunk kernel
-// or beside it, with room for CUs/8 or CUs/4; which systems go wide is
-// split_order's choice. Every candidate runs two intervals (the first may
+// LDS per system), then the launch split: the one in use with the wide launches
+// ahead of the chunk kernel or beside it, with room for CUs/8 or CUs/4, and
+// thresholds that the estimate may have missed, none and those that divide the
+// pool's sizes, without it. Every candidate runs two intervals (the first may
 // record a graph); the second one's host-measured time per step is its score.
-// Neither choice changes any result, so tuning happens on live steps. A pool
-// whose systems all go wide has nothing to tune.
+// Neither choice changes any result, so tuning happens on live steps. While all
+// of a pool's systems go wide there is nothing to tune; it goes on once one does
+// not.
 void tune_splits(hg_pool *Q) {
     Q->tune_cands.clear();
     for (int cus : {0, Q->n_cus / 8, Q->n_cus / 4})
-        Q->tune_cands.push_back({uint32_t(Q->wide_min), cus, Q->chunk_tpb, Q->wg_per_cu});
+        Q->tune_cands.push_back({Q->asked_min, Q->asked_estimate, cus, Q->chunk_tpb, Q->wg_per_cu});
+    const uint32_t largest = Q->order.empty() ? 0u : Q->meta[Q->order.front()].n;
+    for (uint32_t wm : {0u, 1024u, 2048u, 4096u, 8192u})
+        if (wm <= largest && (wm != Q->asked_min || Q->asked_estimate))
+            Q->tune_cands.push_back({wm, false, 0, Q->chunk_tpb, Q->wg_per_cu});
     Q->tune_stage = 1;
     Q->tune_scores.assign(Q->tune_cands.size(), 0.0);
     Q->tune_pos = 0;
     Q->tune_phase = TUNE_RUNNING;
 }
 
-void tune_begin(hg_pool *Q) {
-    const uint32_t wm = uint32_t(Q->wide_min);
-    if (Q->narrow_count == 0) {
-        Q->tune_phase = TUNE_DONE;
-        return;
+hg_status tune_begin(hg_pool *Q) {
+    if (Q->wide_min != Q->asked_min || Q->estimate != Q->asked_estimate) {  // an earlier tuning's choice
+        Q->wide_min = Q->asked_min;
+        Q->estimate = Q->asked_estimate;
+        PG_TRY(refresh_order(Q));
     }
-    Q->tune_cands = {{wm, Q->wide_cus, 256, 2}, {wm, Q->wide_cus, 512, 1}};
+    if (Q->narrow_count == 0) {
+        Q->tune_phase = TUNE_IDLE;
+        return HG_OK;
+    }
+    Q->tune_cands = {{Q->wide_min, Q->estimate, Q->wide_cus, 256, 2}, {Q->wide_min, Q->estimate, Q->wide_cus, 512, 1}};
     Q->tune_stage = 0;
     Q->tune_scores.assign(Q->tune_cands.size(), 0.0);
     Q->tune_pos = 0;
     Q->tune_phase = TUNE_RUNNING;
+    return HG_OK;
 }
 
 void tune_apply(hg_pool *Q, const hg_pool::tune_cand &c) {
-    if (Q->wide_min != c.wide_min) {
-        Q->wide_min = c.wide_min;
-        Q->order_dirty = true;
-    }
+    if (Q->wide_min != c.wide_min || Q->estimate != c.estimate) Q->order_dirty = true;
+    Q->wide_min = c.wide_min;
+    Q->estimate = c.estimate;
     Q->wide_cus = c.wide_cus;
     if (Q->chunk_tpb != c.tpb) Q->order_dirty = true;  // the packs follow the threads per workgroup
     Q->chunk_tpb = c.tpb;
@@ -1068,7 +1085,7 @@ hg_status pool_begin(hg_pool *Q, double dt, uint64_t max_len, uint32_t rebuild_e
     if (Q->fl.active) return fail(HG_ERR_INVALID, "pool: an interval is already queued");
     if (Q->order_dirty) PG_TRY(refresh_order(Q));
     if (Q->order.empty() || max_len == 0) return HG_OK;
-    if (Q->tune_phase == TUNE_START) tune_begin(Q);
+    if (Q->tune_phase == TUNE_START || Q->tune_phase == TUNE_IDLE) PG_TRY(tune_begin(Q));
     if (Q->tune_phase == TUNE_RUNNING) {
         tune_select(Q);
         if (Q->order_dirty) PG_TRY(refresh_order(Q));
@@ -1303,7 +1320,7 @@ hg_status hg_pool_fault(hg_pool *Q, int32_t slot, int *fault) {
 hg_status hg_pool_set_wide_threshold(hg_pool *Q, size_t wide_min) {
     if (!Q) return fail(HG_ERR_INVALID, "pool is null");
     if (wide_min > 0xffffffffu) wide_min = 0;
-    Q->wide_min = uint32_t(wide_min);
+    Q->wide_min = Q->asked_min = uint32_t(wide_min);
     Q->order_dirty = true;
     return HG_OK;
 }
@@ -1318,7 +1335,21 @@ hg_status hg_pool_get_tuning(hg_pool *Q, size_t *wide_min, int *wide_cus, int *t
     if (!Q) return fail(HG_ERR_INVALID, "pool is null");
     if (wide_min) *wide_min = Q->wide_min;
     if (wide_cus) *wide_cus = Q->wide_cus;
-    if (tuned) *tuned = Q->tune_phase == TUNE_DONE ? 1 : 0;
+    if (tuned) *tuned = Q->tune_phase == TUNE_DONE || Q->tune_phase == TUNE_IDLE ? 1 : 0;
+    return HG_OK;
+}
+
+hg_status hg_pool_set_split_estimate(hg_pool *Q, int enable) {
+    if (!Q) return fail(HG_ERR_INVALID, "pool is null");
+    Q->estimate = Q->asked_estimate = enable != 0;
+    Q->order_dirty = true;
+    return HG_OK;
+}
+
+hg_status hg_pool_get_split(hg_pool *Q, size_t *wide_from, int *estimated) {
+    if (!Q) return fail(HG_ERR_INVALID, "pool is null");
+    if (wide_from) *wide_from = Q->wide_from;
+    if (estimated) *estimated = Q->estimate ? 1 : 0;
     return HG_OK;
 }
 

@@ -35,7 +35,8 @@ struct pool_view {
 
 constexpr uint32_t kDefaultWideMin = 2048;
 constexpr double kDefaultWideCuFraction = 0.25;
-enum { TUNE_OFF = 0, TUNE_START = 1, TUNE_RUNNING = 2, TUNE_DONE = 3 };
+// TUNE_IDLE: nothing to tune until a system takes the chunk kernel
+enum { TUNE_OFF = 0, TUNE_START = 1, TUNE_RUNNING = 2, TUNE_DONE = 3, TUNE_IDLE = 4 };
 
 // Per-step launches (tile_step.h): workgroup b carries the particles
 // [start, start + tile_width) of the system at [offset, offset + n) of the
