@@ -203,25 +203,23 @@ __global__ void __launch_bounds__(256) k_final_kick(double *v, double *w, const 
 }
 
 // nsteps steps of a legacy sinter_functor system of at most kTile particles in
-// one workgroup, one particle per thread: per step the kick/drift (with the legacy connector
-// moves), a barrier, the acceleration pass, a barrier, as the per-step
-// launches of k_kick_drift, k_legacy_move and k_force_nl / k_force_all do it,
-// through the same device code. The pass reads pair-state table `even` on
-// even steps and `odd` on odd ones (the two halves swap every pass).
-// pending_first: the first kick also completes a previous step; final_kick:
-// the last step's closing kick is applied (otherwise it is left pending, as
-// between the per-step launches).
+// one workgroup, one particle per thread: per step the kick/drift (with the
+// legacy connector moves), a barrier, the acceleration pass, a barrier, and at
+// the end the closing kick, as the per-step launches of k_kick_drift,
+// k_legacy_move, k_force_nl / k_force_all and k_final_kick do it, through the
+// same device code. The pass reads pair-state table `even` on even steps and
+// `odd` on odd ones (the two halves swap every pass).
 template <int BIN, int HAM>
 __global__ void __launch_bounds__(kTile) k_small_steps(hg_params P, sys_view even, sys_view odd, double *x, double *v,
                                                        double *th, double *w, facet_dev *facets, uint32_t nsteps,
-                                                       int pending_first, int final_kick, double half, double dt,
-                                                       int nf_advance, double *lconn, const uint32_t *bcnt) {
+                                                       double half, double dt, int nf_advance, double *lconn,
+                                                       const uint32_t *bcnt) {
     __shared__ tile_lds T;
     const uint32_t i = threadIdx.x;
     const uint32_t n = even.n;
     const bool live = i < n;
     for (uint32_t s = 0; s < nsteps; s++) {
-        const int pending = (s > 0 || pending_first) ? 1 : 0;
+        const bool pending = s > 0;
         if (pending && i == 0) advance_facets(facets, nf_advance, dt);
         if (live) {
             kick_drift_one(x, v, th, w, even.a, even.al, i, pending, half, half, dt);
@@ -235,10 +233,8 @@ __global__ void __launch_bounds__(kTile) k_small_steps(hg_params P, sys_view eve
         }
         __syncthreads();
     }
-    if (final_kick) {
-        if (i == 0) advance_facets(facets, nf_advance, dt);
-        if (live) final_kick_one(v, w, even.a, even.al, i, half, even.flags);
-    }
+    if (i == 0) advance_facets(facets, nf_advance, dt);
+    if (live) final_kick_one(v, w, even.a, even.al, i, half, even.flags);
 }
 
 // triangular_facet::update_positions with the driver's velocity (one lane).
@@ -1123,7 +1119,7 @@ hipError_t launch_small_steps_t(const hg_params &p, const sys_view &even, const 
         return hipGetLastError();
     }
     if constexpr (BIN == HG_BINARY_SINTER_LEGACY) {
-        k_small_steps<BIN, HAM><<<1, kTile, 0, s>>>(p, even, odd, x, v, th, w, facets, nsteps, 0, 1, half, dt, nf_advance,
+        k_small_steps<BIN, HAM><<<1, kTile, 0, s>>>(p, even, odd, x, v, th, w, facets, nsteps, half, dt, nf_advance,
                                                     lconn, bcnt);
         return hipGetLastError();
     }
