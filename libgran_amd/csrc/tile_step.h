@@ -48,7 +48,9 @@ struct tile_lds {
     uint2 Q[KC * W];  // partner and queue_word
     uint16_t CW[KC * W];
     uint32_t rows[W], dirty[W];  // lengths; whether entries ended or began in this part of the lists
-    uint32_t holes[W], kept[W];  // slots of ended entries (kManyHoles: others from slot 31 on); lengths without them
+    // slots of ended entries (kManyHoles: others from slot 31 on); the length
+    // without them of a row that has some
+    uint32_t holes[W], kept[W];
     uint32_t more[W], spilled;  // a row's entries in the table's other half, and whether there are any
     uint32_t nB[kTileThreads / 64], nO[kTileThreads / 64];
     uint32_t contacts, ended;
@@ -149,6 +151,7 @@ __global__ void __launch_bounds__(kTileThreads, tile_waves(PAIRS, PREC, FAC))
     if (tid < uint32_t(W)) {
         L.rows[tid] = c_old;
         L.dirty[tid] = L.holes[tid] = L.more[tid] = 0;
+        L.kept[tid] = kNoEntry;
     }
     if (tid == 0) L.contacts = L.ended = L.spilled = 0;
     auto own = [&](int f, uint32_t t) { return d3{L.s[3 * f][t], L.s[3 * f + 1][t], L.s[3 * f + 2][t]}; };
@@ -376,12 +379,14 @@ __global__ void __launch_bounds__(kTileThreads, tile_waves(PAIRS, PREC, FAC))
                     const uint2 e = L.Q[L.CW[c]];
                     const uint32_t pos = queue_place(e.y), t = pos % W, j = e.x, gi = base + t;
                     uint32_t slot = queue_slot(e.y);
-                    if (slot != kNoRowSlot && L.holes[t] && slot >= L.kept[t])  // it has moved just now
-                        slot = row_slot(L.kept[t], j, [&](uint32_t s) { return pj[size_t(s) * stride + gi]; });
+                    const uint32_t kept = L.kept[t];
+                    const d3 xj = ld3(Vi.x, j), vj = ld3(Vi.v, j), wj = ld3(Vi.w, j);
+                    if (slot != kNoRowSlot && slot >= kept)  // it has moved just now
+                        slot = row_slot(kept, j, [&](uint32_t s) { return pj[size_t(s) * stride + gi]; });
                     spring9 sp = zero_spring();
                     if (slot != kNoRowSlot) sp = ld_rec(ps + (size_t(slot) * stride + gi) * kSpringRec);
                     vec lin, ang;
-                    ev.contact(own(0, t), own(1, t), own(2, t), ld3(Vi.x, j), ld3(Vi.v, j), ld3(Vi.w, j), sp, lin, ang);
+                    ev.contact(own(0, t), own(1, t), own(2, t), xj, vj, wj, sp, lin, ang);
                     double *to = ps;
                     if (slot == kNoRowSlot) {
                         slot = atomicAdd(&L.rows[t], 1u);
@@ -428,6 +433,7 @@ __global__ void __launch_bounds__(kTileThreads, tile_waves(PAIRS, PREC, FAC))
                     }
                     pcnt[gi] = c;
                     L.dirty[tid] = L.holes[tid] = 0;
+                    L.kept[tid] = kNoEntry;
                     unsorted = true;
                 }
                 if (tid == 0) L.contacts = L.ended = 0;
