@@ -251,7 +251,7 @@ hipError_t launch_advance_facet(facet_dev *f, const double *v, double dt, hipStr
 // sinter_functor systems, up to kSmallSystemMax, take k_small_steps; `even` /
 // `odd` are the views whose tables the even / odd steps read. For the other
 // functors a launch per step over tiles is faster than k_small_steps from there
-// on: 8.8 against 16 us per step at 30 particles, 10.9 against 22 at 200 (lists
+// on: 8.8 against 16 us per step at 30 particles, 8.3 against 22 at 200 (lists
 // of 3.9, FP64); with all pairs 9.0 against 49 and 14.3 against 199.
 constexpr uint32_t kSmallSystemMax = 256, kTinySystemMax = 32;
 bool tiny_steps_fit(uint32_t n, uint32_t maxb);

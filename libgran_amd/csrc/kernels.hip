@@ -745,9 +745,9 @@ hipError_t launch_force(const hg_params &p, const sys_view &sv, hipStream_t s) {
 // are those of sinter_eval, contact_eval and the per-particle walk.
 //
 // Measured against one thread per pair with state, rows and springs in global
-// memory: 19 particles, contact and Hamaker, list rebuilt every 20 steps 20.7
-// -> 5.0 us a step, all pairs 15.2 -> 4.2; the legacy 27-particle lattice 19.0
-// -> 4.8.
+// memory: 19 particles, contact and Hamaker, list rebuilt every 20 steps 20.2
+// -> 5.6 us a step, all pairs 15.2 -> 5.6; the legacy 27-particle lattice 18.8
+// -> 4.9.
 constexpr uint32_t kTinyThreads = 512;
 
 // Doubles (then words) of LDS a system of n particles needs; maxb: the most

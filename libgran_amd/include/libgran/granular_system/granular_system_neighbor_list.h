@@ -2,7 +2,8 @@
 // neighbour list of radius r_verlet that the driver refreshes with
 // update_neighbor_list(). Same template parameters and constructor as the
 // reference (include/libgran/granular_system/granular_system_neighbor_list.h:26-87);
-// the list is built on the GPU by a cell list (kernels.hip: k_nl_fill).
+// the list is built on the GPU (kernels.hip: k_list_brute up to 2,048 particles,
+// k_list_fill's cells above).
 #ifndef LIBGRAN_GRANULAR_SYSTEM_NEIGHBOR_LIST_H
 #define LIBGRAN_GRANULAR_SYSTEM_NEIGHBOR_LIST_H
 
