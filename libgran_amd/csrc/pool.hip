@@ -1320,7 +1320,9 @@ hg_status hg_pool_fault(hg_pool *Q, int32_t slot, int *fault) {
 hg_status hg_pool_set_wide_threshold(hg_pool *Q, size_t wide_min) {
     if (!Q) return fail(HG_ERR_INVALID, "pool is null");
     if (wide_min > 0xffffffffu) wide_min = 0;
-    Q->wide_min = Q->asked_min = uint32_t(wide_min);
+    Q->asked_min = uint32_t(wide_min);
+    Q->wide_min = Q->asked_min;
+    Q->estimate = Q->asked_estimate;  // not an earlier tuning's
     Q->order_dirty = true;
     return HG_OK;
 }
@@ -1341,7 +1343,9 @@ hg_status hg_pool_get_tuning(hg_pool *Q, size_t *wide_min, int *wide_cus, int *t
 
 hg_status hg_pool_set_split_estimate(hg_pool *Q, int enable) {
     if (!Q) return fail(HG_ERR_INVALID, "pool is null");
-    Q->estimate = Q->asked_estimate = enable != 0;
+    Q->asked_estimate = enable != 0;
+    Q->wide_min = Q->asked_min;
+    Q->estimate = Q->asked_estimate;
     Q->order_dirty = true;
     return HG_OK;
 }

@@ -102,12 +102,11 @@ def test_the_tuner_tries_splits_and_starts_when_there_is_something_to_tune():
         while tune and not pool.tuning()["tuned"]:
             pool.step(DT, 50, rebuild_every=50)
             intervals += 1
-            seen.add((pool.split()["wide_from"], pool.tuning()["wide_cus"], pool.tuning()["chunk_threads"]))
+            seen.add(pool.split()["wide_from"])
             assert intervals < 40
         if tune:
             assert intervals == 2 * (2 + 3 + 3)  # shapes, the split, thresholds of 0, 1024 and 2048
-            assert {0, 1300, 2200} <= {w for w, _, _ in seen}
-            assert {256, 512} <= {t for _, _, t in seen} | {512}
+            assert {0, 1300, 2200} <= seen
         pool.step(DT, 50 * (20 - intervals), rebuild_every=50)
         outs.append([pool.state(s) for s in slots])
         pool.autotune(tune)  # from the caller's split again
@@ -116,6 +115,26 @@ def test_the_tuner_tries_splits_and_starts_when_there_is_something_to_tune():
             assert pool.split()["wide_from"] == 1300
     for a, b in zip(*outs):
         same(a, b, "tuned")
+
+
+def test_a_threshold_set_after_tuning_is_the_callers():
+    """Whatever the tuner chose, a threshold set later comes with the caller's
+    own choice of the estimate, and the estimate with the caller's threshold."""
+    print("[paths] after tuning", flush=True)
+    cases = [agg_case(n, 90 + k) for k, n in enumerate((3000, 1300, 150))]
+    for estimate in (False, True):
+        pool, slots = pool_of(nl_params(1), cases)
+        pool.set_wide_threshold(2000)
+        pool.set_split_estimate(False)  # something narrow to tune
+        pool.autotune(True)
+        while not pool.tuning()["tuned"] or pool.info(slots[0])[2] == 0:
+            pool.step(DT, 50, rebuild_every=50)
+        if estimate:
+            pool.set_split_estimate(True)
+            assert pool.tuning()["wide_min"] == 2000
+        pool.set_wide_threshold(1000)
+        pool.step(DT, 50, rebuild_every=50)
+        assert pool.split() == dict(wide_from=150 if estimate else 1300, estimate=estimate)
 
 
 def test_all_pairs_lattices_in_the_chunk_kernel():
