@@ -39,6 +39,12 @@ template <int HAM>
 hipError_t launch_tile_h(const hg_params &p, const pool_view &Vi, const pool_view &Vo, const wide_block *map,
                          unsigned blocks, int mode, bool facets, double half, double dt, hipStream_t s) {
     const mixed_consts mc = make_mixed_consts(p);
+    if constexpr (HG_PAIRS == HG_PAIRS_NEIGHBOR_LIST && HG_BIN != HG_BINARY_NONE)
+        if (p.precision == HG_PRECISION_FP64 && !facets && blocks > kTwoOnEachCu) {
+            k_tile_step<HG_BIN, HAM, HG_PAIRS, HG_PRECISION_FP64, false, 3>
+                <<<blocks, kTileThreads, 0, s>>>(p, mc, Vi, Vo, map, mode, half, dt);
+            return hipGetLastError();
+        }
 #define HG_KCASE(PREC, FAC)                                                       \
     if (p.precision == PREC && facets == FAC)                                     \
         k_tile_step<HG_BIN, HAM, HG_PAIRS, PREC, FAC>                             \

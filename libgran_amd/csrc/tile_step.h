@@ -72,13 +72,20 @@ __device__ __forceinline__ wide_block tile_block(const wide_block *map, const po
 // a CU, hide one pair's latency behind another's: mixed 151 us a step at
 // 635,000 particles with three, 187 with two (four spill: 241); with the facet
 // terms three spill too: 24 plate tests of 1,000 steps 40.5 ms, 35.8 with two.
-// In FP64 nine registers spill with three: 213,000 particles in 333 systems
-// take 54.5 us a step, 61.7 with two, but 20,000 in one 14.0 against 13.3 and
-// 200 8.9 against 8.4. All pairs come in few blocks, and two cost them
+// In FP64 nine registers spill with three, which pays where a CU has a third
+// workgroup to put beside two (kTwoOnEachCu). All pairs come in few blocks, and two cost them
 // registers: 33 us a step at 522 particles against 28.
 constexpr int tile_waves(int pairs, int prec, bool fac) {
     return pairs != HG_PAIRS_NEIGHBOR_LIST ? 1 : (prec == HG_PRECISION_MIXED && !fac ? 3 : 2);
 }
+
+// FP64 tiles with a binary functor and no facets in more workgroups than this are
+// held to three wavefronts per SIMD: what 256 CUs take two each of. Aggregates
+// with lists of 3.9 at 450 tiles 13.6 us a step with two, 14.3 with three; 550
+// 17.2 and 15.2; 1,000 22.4 and 22.3; 2,500 47.4 and 42.4. Beds with lists of
+// about 50 at 450 114 and 118, 600 175 and 141, 4,700 951 and 792, where the walk
+// takes 824. Without a binary functor the two take the same time.
+constexpr unsigned kTwoOnEachCu = 512;
 
 // A launch's arguments (the parameter set, its mixed form and two views, 1.5 KB)
 // lie in memory that no cache holds yet. Read where they are used, they were
@@ -97,8 +104,8 @@ __device__ __forceinline__ void touch_args() {
 // What a launch does after the pass: TILE_FORCE stores the accelerations of
 // the systems that have none; TILE_STEP completes the step, kicks and drifts
 // into the other buffers; TILE_LAST completes the last step.
-template <int BIN, int HAM, int PAIRS, int PREC, bool FAC>
-__global__ void __launch_bounds__(kTileThreads, tile_waves(PAIRS, PREC, FAC))
+template <int BIN, int HAM, int PAIRS, int PREC, bool FAC, int PER_SIMD = tile_waves(PAIRS, PREC, FAC)>
+__global__ void __launch_bounds__(kTileThreads, PER_SIMD)
     k_tile_step(hg_params P, mixed_consts MC, pool_view Vi, pool_view Vo, const wide_block *map, int mode, double half,
                 double dt) {
     constexpr int W = tile_width(PAIRS), KC = tile_depth(PAIRS), ROWS = kTileThreads / W, WAVES = kTileThreads / 64;
@@ -106,7 +113,7 @@ __global__ void __launch_bounds__(kTileThreads, tile_waves(PAIRS, PREC, FAC))
     using vec = typename prec_types<PREC>::vec;
     __shared__ tile_lds<W, KC, PREC, FAC> L;
     // a workgroup is a wavefront for each SIMD: the CU's LDS holds as many
-    static_assert(sizeof(L) * size_t(tile_waves(PAIRS, PREC, FAC)) <= 160u * 1024u, "LDS of the tiles on a CU");
+    static_assert(sizeof(L) * size_t(PER_SIMD) <= 160u * 1024u, "LDS of the tiles on a CU");
     touch_args<sizeof(hg_params) + sizeof(mixed_consts) + 2 * sizeof(pool_view)>();
     const wide_block b = tile_block(map, Vi, W);
     const uint32_t n = b.n & kIdxMask, cur = b.n >> 31, base = b.offset + b.start;

@@ -183,3 +183,45 @@ def test_rows_of_more_than_31_entries(n, pairs):
         rows.append(np.bincount(ij[:, 0], minlength=n))
     assert rows[-1].max() > 40 and rows[0].sum() - rows[-1].sum() > 50
     s.close()
+
+
+@pytest.mark.parametrize("n", [32768, 32769])
+def test_large_beds_equal_the_tracked_walk(n):
+    """512 tiles and one more, from where FP64 tiles run three to a CU;
+    dissipation tracking walks."""
+    import libgran_amd as L
+    print(f"[bed] n {n}", flush=True)
+    x, v, w = bed(n, 1)
+    out = []
+    for tracked in (True, False):
+        s = L.System(params(0, 2.6), x, v, omega0=w)
+        s.track_dissipation(tracked)
+        for steps in (1, 20, 12):
+            s.step(1e-13, steps, rebuild_every=20)
+        out.append((s.state(), s.springs(0)))
+        s.close()
+    equal(out[0][0], out[1][0], "tiles")
+    np.testing.assert_array_equal(out[1][1][0], out[0][1][0])
+    np.testing.assert_array_equal(out[1][1][1], out[0][1][1])
+
+
+def test_many_aggregates_in_tiles_equal_the_chunk_kernel():
+    """70 aggregates of 500 in 560 tiles."""
+    import libgran_amd as L
+    import _scenarios as S
+    print("[bed] 560 tiles of aggregates", flush=True)
+    c, sn, h = S.aggregate_params()
+    p = L.make_params(L.BINARY_SINTER, L.HAMAKER_LIMITED, pair_mode=1, r_verlet=3.2 * R, contact=c, sinter=sn, hamaker=h)
+    cases = [L.generate_aggregate(500, R, 1.8, 1.3, k) for k in range(70)]
+    out = []
+    for wide_min in (1, 0):
+        pool = L.Pool(p, max_particles=36000, max_systems=70)
+        pool.set_wide_threshold(wide_min)
+        slots = [pool.add(x, np.random.default_rng(k).normal(0.0, 1.0, x.shape)) for k, x in enumerate(cases)]
+        pool.step(1e-13, 120, rebuild_every=50)
+        assert (pool.last_step_profile()["chunks"] == 0) == (wide_min == 1)
+        out.append([(pool.state(s), pool.springs(s, 1)) for s in slots])
+        pool.close()
+    for (a, sa), (b, sb) in zip(*out):
+        equal(a, b, "aggregate")
+        np.testing.assert_array_equal(sb[1], sa[1])
