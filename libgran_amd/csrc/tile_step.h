@@ -73,10 +73,13 @@ __device__ __forceinline__ wide_block tile_block(const wide_block *map, const po
 // 635,000 particles with three, 187 with two (four spill: 241); with the facet
 // terms three spill too: 24 plate tests of 1,000 steps 40.5 ms, 35.8 with two.
 // In FP64 nine registers spill with three, which pays where a CU has a third
-// workgroup to put beside two (kTwoOnEachCu). All pairs come in few blocks, and two cost them
-// registers: 33 us a step at 522 particles against 28.
+// workgroup to put beside two (kTwoOnEachCu). All pairs in FP64 or with facets
+// are not held to any: two, asked for, cost 33 us a step at 522 particles against
+// 28. Mixed ones without facets fit three with a few registers to spare or
+// spilled, and take 10.1 ms a step at 24,000 particles with two, 7.2 with three.
 constexpr int tile_waves(int pairs, int prec, bool fac) {
-    return pairs != HG_PAIRS_NEIGHBOR_LIST ? 1 : (prec == HG_PRECISION_MIXED && !fac ? 3 : 2);
+    if (prec == HG_PRECISION_MIXED && !fac) return 3;
+    return pairs != HG_PAIRS_NEIGHBOR_LIST ? 1 : 2;
 }
 
 // FP64 tiles with a binary functor and no facets in more workgroups than this are
